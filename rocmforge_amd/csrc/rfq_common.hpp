@@ -114,6 +114,19 @@ RFQ_GEMV_PART_DECL(3)
 constexpr int GEMV_TRACE_STAMPS = 20;                    // readings per wavefront, see WaveTrace in rfq_gemv.hip
 int launch_gemv_traced(int fmt, const uint8_t *d_w, const float *d_x, float *d_y, int n, int k, unsigned long long *d_trace,
                        size_t capacity_waves, int *waves, hipStream_t s);
+// Few rows of activations on the matrix cores (rfq_skinny.hip, compiled in four parts): float16 a, rows or arranged.
+// The caller has checked formats, shapes and alignment.
+int launch_skinny_gemm(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, bool f16_out, int m, int n, int k,
+                       hipStream_t s);
+bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts);
+#define RFQ_SKINNY_PART_DECL(N)                                                                                              \
+    int launch_skinny_gemm_part##N(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, int f16_out, int m,   \
+                                   int n, int k, hipStream_t s);
+RFQ_SKINNY_PART_DECL(0)
+RFQ_SKINNY_PART_DECL(1)
+RFQ_SKINNY_PART_DECL(2)
+RFQ_SKINNY_PART_DECL(3)
+#undef RFQ_SKINNY_PART_DECL
 // y[n] = sum_l x[l] * Wd[l * n + j] over the flat stream of n * k elements (one row of x).
 int launch_gemv_kn(int fmt, const uint8_t *d_w, const float *d_x, float *d_y, int n, int k, hipStream_t s);
 int launch_gemv_fused(int fmt, const uint8_t *d_w, const uint8_t *d_w2, const float *d_x, const float *d_norm_w,

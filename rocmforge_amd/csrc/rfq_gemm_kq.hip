@@ -1017,6 +1017,20 @@ int launch_gemm_f16(int fmt, const uint8_t *d_w, const void *d_a, void *d_out, i
         return fail(RFQ_E_BADARG, "rfq_gemm_f16: activations must be 16-byte aligned with k a multiple of 8");
     if ((reinterpret_cast<uintptr_t>(d_w) & 3u) != 0)               // buffer loads of whole dwords
         return fail(RFQ_E_BADARG, "rfq_gemm_f16: weights must be 4-byte aligned");
+    // Few rows: the kernel that decodes each weight for all rows at once and needs neither the arrangement nor parts.
+    // (The tiled kernel cannot split k for arranged activations, so it is the slower one there up to more rows.  Q4_K, whose
+    // tiled kernel rounds q * scale to fp16 and whose few-row kernel does not, takes the same kernel from either entry point.)
+    const int rival_parts = d_arranged != nullptr && fmt != RFQ_Q4_K ? 1 : k_parts_for(m, n, k);
+    const bool known = fmt == RFQ_Q4_0 || fmt == RFQ_Q8_0 || fmt == RFQ_Q4_K || fmt == RFQ_Q6_K || fmt == RFQ_GGUF_Q4_0 ||
+                       fmt == RFQ_GGUF_Q8_0 || fmt == RFQ_GGUF_Q4_K || fmt == RFQ_GGUF_Q6_K;
+    const bool static_fits = !use_static_scratch || arranged_at_bytes(m, k) + arranged_s2_bytes(m, k) <= RFQ_STATIC_SCRATCH_BYTES;
+    // (From 256 rows on, a whole tile, plain activations keep the tiled kernel and with it the rule that a stream under
+    // capture must hold the call's temporary; arranged ones follow where both must give the same bits.)
+    const bool rows_in_range = m < BM || (d_arranged != nullptr && fmt != RFQ_Q4_K && k_parts_for(m, n, k) > 1);
+    if (known && (out_dtype & RFQ_GEMM_ONE_PLANE) == 0 && static_fits && rows_in_range &&
+        prefer_skinny_gemm(fmt, m, n, k, rival_parts))
+        return launch_skinny_gemm(fmt, d_w, static_cast<const uint8_t *>(d_arranged != nullptr ? d_arranged : d_a), d_arranged != nullptr,
+                                  d_out, out_dtype == RFQ_F16, m, n, k, s);
     switch (fmt) {
     case RFQ_Q4_0: return launch_fmt<RFQ_Q4_0>(d_w, d_a, d_out, out_dtype, m, n, k, st, d_arranged, s);
     case RFQ_Q8_0: return launch_fmt<RFQ_Q8_0>(d_w, d_a, d_out, out_dtype, m, n, k, st, d_arranged, s);

@@ -1,0 +1,169 @@
+// Launchers of the matrix-core kernels for few rows of activations (rfq_skinny.hpp).  Compiled RFQ_SKINNY_PARTS times
+// (-DRFQ_SKINNY_PART=0..3, the formats of skinny_part_of each), so that the formats build side by side; part 0 also holds
+// the entry points.
+#include <mutex>
+
+#include "rfq_skinny.hpp"
+
+#ifndef RFQ_SKINNY_PART
+#error "compile with -DRFQ_SKINNY_PART=0 .. 3 (see the Makefile)"
+#endif
+
+namespace rfq {
+
+constexpr int skinny_part_of(int fmt)
+{
+    switch (fmt) {
+    case RFQ_Q4_0: case RFQ_Q4_K: return 0;
+    case RFQ_Q8_0: case RFQ_GGUF_Q8_0: return 1;
+    case RFQ_Q6_K: case RFQ_GGUF_Q6_K: return 2;
+    case RFQ_GGUF_Q4_0: case RFQ_GGUF_Q4_K: return 3;
+    default: return -1;
+    }
+}
+
+namespace {
+
+using namespace skinny;
+
+// Wavefronts of a workgroup: they take the 128-element units of k in turn, so no more than there are units.
+int waves_for(int k, int most)
+{
+    const int units = (k / 32 + 3) / 4;
+    return units < most ? units : most;
+}
+
+template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES>
+int gemm_cfg(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int n, int k, int rows, int slices, hipStream_t s)
+{
+    constexpr bool STAGED = A16<W<FMT>::ORDER, W<FMT>::PAIRS, ARR>::STAGED;
+    constexpr int MOST_LDS = gemm_lds<MT, TJ, STAGED>(WAVES);
+    static_assert(MOST_LDS <= 160 * 1024, "LDS");
+    const int waves = waves_for(k, WAVES);
+    const size_t lds = (size_t)gemm_lds<MT, TJ, STAGED>(waves);
+    if constexpr (MOST_LDS > 64 * 1024) {
+        static std::once_flag once;
+        static hipError_t err = hipSuccess;
+        std::call_once(once, [] {
+            err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, MOST_LDS);
+        });
+        if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(gemm_skinny_kernel)");
+    }
+    hipLaunchKernelGGL((gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES>), dim3((n + 16 * TJ - 1) / (16 * TJ), slices), dim3(64 * waves), lds, s,
+                       w, a, y, f16_out, m, n, k, rows);
+    RFQ_LAUNCH_CHECK("gemm_skinny_kernel");
+    return RFQ_OK;
+}
+
+// Rows of a slice: at most 16 * most, the slices as even as 16 rows allow.
+struct Slices { int count, tiles; };
+Slices slices_of(int m, int most)
+{
+    const int tiles = (m + 15) / 16, count = (tiles + most - 1) / most;
+    return {count, (tiles + count - 1) / count};
+}
+// Eight 16-row operands per workgroup; four where two row tiles of the scale-only 4-bit layouts would spill registers
+// (Q4_0, 208 rows, 1792 -> 5713: 79.7 us with eight, 30 with four; the other formats hold eight).
+constexpr int most_tiles(int fmt, bool two) { return two && (fmt == RFQ_Q4_0 || fmt == RFQ_GGUF_Q4_0) ? 4 : 8; }
+// Two row tiles per workgroup from about one workgroup per CU on: a workgroup reads all activations of its slice whether
+// it multiplies 16 rows of W or 32 (Q8_0, k = 4096, 48 rows: n = 8192 23.5 -> 18.7 us, n = 14336 43.2 -> 32.7; with fewer
+// workgroups than CUs one tile is ahead, n = 4096 11.4 against 13.7 us).
+bool two_tiles(int m, int n) { return (n + 15) / 16 * slices_of(m, 8).count > device_cu_count() + device_cu_count() / 8; }
+
+template <int FMT, int TJ, bool ARR>
+int gemm_mt(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int n, int k, hipStream_t s)
+{
+    constexpr int MOST = most_tiles(FMT, TJ == 2);
+    const Slices sl = slices_of(m, MOST);
+    const int rows = 16 * sl.tiles, slices = sl.count;
+    // units of W in flight per wavefront: two, one where the registers of a unit leave no room for two
+    constexpr int D = TJ * W<FMT>::NR > 9 ? 1 : 2;
+    switch (sl.tiles) {
+    case 1: return gemm_cfg<FMT, 1, TJ, ARR, 2, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
+    case 2: return gemm_cfg<FMT, 2, TJ, ARR, 2, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
+    case 3: return gemm_cfg<FMT, 3, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
+    case 4: return gemm_cfg<FMT, 4, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
+    default:
+        if constexpr (MOST == 8) {
+            if (sl.tiles <= 6) return gemm_cfg<FMT, 6, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
+            return gemm_cfg<FMT, 8, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
+        }
+        return fail(RFQ_E_UNSUPPORTED, "rfq_gemm_f16: slices of %d rows", rows);
+    }
+}
+
+template <int FMT>
+int gemm_fmt(const uint8_t *w, const uint8_t *a, bool arranged, void *y, int f16_out, int m, int n, int k, hipStream_t s)
+{
+    if (two_tiles(m, n)) return arranged ? gemm_mt<FMT, 2, true>(w, a, y, f16_out, m, n, k, s) : gemm_mt<FMT, 2, false>(w, a, y, f16_out, m, n, k, s);
+    return arranged ? gemm_mt<FMT, 1, true>(w, a, y, f16_out, m, n, k, s) : gemm_mt<FMT, 1, false>(w, a, y, f16_out, m, n, k, s);
+}
+
+} // namespace
+
+#define RFQ_SKINNY_CAT2(a, b) a##b
+#define RFQ_SKINNY_CAT(a, b) RFQ_SKINNY_CAT2(a, b)
+#define RFQ_SKINNY_CASES(CALL)                                                                     \
+    return [&](auto part) -> int {                                                                  \
+        constexpr int P = decltype(part)::value;                                                    \
+        switch (fmt) {                                                                              \
+        case RFQ_Q4_0: if constexpr (skinny_part_of(RFQ_Q4_0) == P) return CALL(RFQ_Q4_0); break;   \
+        case RFQ_Q8_0: if constexpr (skinny_part_of(RFQ_Q8_0) == P) return CALL(RFQ_Q8_0); break;   \
+        case RFQ_Q4_K: if constexpr (skinny_part_of(RFQ_Q4_K) == P) return CALL(RFQ_Q4_K); break;   \
+        case RFQ_Q6_K: if constexpr (skinny_part_of(RFQ_Q6_K) == P) return CALL(RFQ_Q6_K); break;   \
+        case RFQ_GGUF_Q4_0: if constexpr (skinny_part_of(RFQ_GGUF_Q4_0) == P) return CALL(RFQ_GGUF_Q4_0); break; \
+        case RFQ_GGUF_Q8_0: if constexpr (skinny_part_of(RFQ_GGUF_Q8_0) == P) return CALL(RFQ_GGUF_Q8_0); break; \
+        case RFQ_GGUF_Q4_K: if constexpr (skinny_part_of(RFQ_GGUF_Q4_K) == P) return CALL(RFQ_GGUF_Q4_K); break; \
+        case RFQ_GGUF_Q6_K: if constexpr (skinny_part_of(RFQ_GGUF_Q6_K) == P) return CALL(RFQ_GGUF_Q6_K); break; \
+        default: break;                                                                             \
+        }                                                                                           \
+        return fail(RFQ_E_UNSUPPORTED, "no few-row kernel for format %d in this part of the build", fmt); \
+    }(std::integral_constant<int, RFQ_SKINNY_PART>{})
+
+int RFQ_SKINNY_CAT(launch_skinny_gemm_part, RFQ_SKINNY_PART)(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, int f16_out,
+                                                             int m, int n, int k, hipStream_t s)
+{
+#define RFQ_SKINNY_GEMM(F) gemm_fmt<F>(w, a, arranged, y, f16_out, m, n, k, s)
+    RFQ_SKINNY_CASES(RFQ_SKINNY_GEMM);
+}
+
+#if RFQ_SKINNY_PART == 0
+
+// Whether the few-row kernel is the faster one for a prompt, from estimates of both in microseconds fitted to 300 measured
+// shapes (Q4_K, Q8_0, GGUF_Q4_K, GGUF_Q6_K; n 768..14336, k 1024..14336, 16..256 rows).  The few-row kernel's time grows
+// with the 16-row operands a workgroup multiplies per 1024 k (all of them in every workgroup) and, beyond one workgroup
+// per CU, with the number of workgroups; the tiled kernel's is nearly flat up to 256 rows: a workgroup's own pass over k,
+// in `parts` parts, plus the f32 parts written and read again.  (tiled / few-row: Q8_0 16 x 4096 -> 4096 32.8 / 7.1 us,
+// 96 x 4096 -> 4096 35.9 / 20.6, 48 x 4096 -> 14336 66.5 / 32.7, 96 x 14336 -> 4096 65.8 / 63.1, 256 x 4096 -> 14336
+// 71.9 / 126.)  With parts == 1 the answer depends on the shape alone, so that arranged and plain activations take the
+// same kernel and give the same bits.
+bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts)
+{
+    const double cus = device_cu_count(), ku = k / 1024.0;
+    const bool two = two_tiles(m, n);
+    const Slices sl = slices_of(m, most_tiles(fmt, two));
+    const int row_tiles = (n + 15) / 16 * sl.count;
+    const double rounds = two ? 1.45 * (row_tiles / 2 > cus ? row_tiles / 2 / cus : 1.0) : 1.0;
+    const double few = 3.0 + ku * rounds * (0.5 + 0.7 * (sl.tiles <= 4 ? sl.tiles : sl.tiles <= 6 ? 6 : 8));
+    const double per_ku = fmt == RFQ_Q4_K ? 10.0 : fmt == RFQ_GGUF_Q4_K ? 13.0 : fmt == RFQ_GGUF_Q6_K ? 29.0 : 21.5;
+    const int groups = ((m + 255) / 256) * ((n + 127) / 128) * parts;
+    double tiled = 8.0 + per_ku * ku / parts * (groups > cus ? groups / cus : 1.0);
+    if (parts > 1) tiled += 4.0 + 8.0 * parts * m * (double)n / 5e6;
+    return few < tiled;
+}
+
+int launch_skinny_gemm(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, bool f16_out, int m, int n, int k, hipStream_t s)
+{
+    switch (skinny_part_of(fmt)) {
+    case 0: return launch_skinny_gemm_part0(fmt, w, a, arranged, y, f16_out, m, n, k, s);
+    case 1: return launch_skinny_gemm_part1(fmt, w, a, arranged, y, f16_out, m, n, k, s);
+    case 2: return launch_skinny_gemm_part2(fmt, w, a, arranged, y, f16_out, m, n, k, s);
+    case 3: return launch_skinny_gemm_part3(fmt, w, a, arranged, y, f16_out, m, n, k, s);
+    default: return fail(RFQ_E_UNSUPPORTED, "no few-row kernel for format %d", fmt);
+    }
+}
+
+#endif
+
+} // namespace rfq
