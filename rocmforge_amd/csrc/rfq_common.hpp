@@ -114,12 +114,17 @@ RFQ_GEMV_PART_DECL(3)
 constexpr int GEMV_TRACE_STAMPS = 20;                    // readings per wavefront, see WaveTrace in rfq_gemv.hip
 int launch_gemv_traced(int fmt, const uint8_t *d_w, const float *d_x, float *d_y, int n, int k, unsigned long long *d_trace,
                        size_t capacity_waves, int *waves, hipStream_t s);
-// Few rows of activations on the matrix cores (rfq_skinny.hip, compiled in four parts): float16 a, rows or arranged.
-// The caller has checked formats, shapes and alignment.
+// Few rows of activations on the matrix cores (rfq_skinny.hip, compiled in four parts): float32 x with m <= 8 (w2 != nullptr:
+// two matrices of one shape that share x), or float16 a (rows or arranged).  The caller has checked formats, shapes and
+// alignment (weights on multiples of 4, activations of 16).
+int launch_skinny_gemv(int fmt, const uint8_t *w, const uint8_t *w2, const float *x, float *y, float *y2, int m, int n, int k,
+                       hipStream_t s);
 int launch_skinny_gemm(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, bool f16_out, int m, int n, int k,
                        hipStream_t s);
 bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts);
 #define RFQ_SKINNY_PART_DECL(N)                                                                                              \
+    int launch_skinny_gemv_part##N(int fmt, const uint8_t *w, const uint8_t *w2, const float *x, float *y, float *y2, int m,  \
+                                   int n, int k, hipStream_t s);                                                             \
     int launch_skinny_gemm_part##N(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, int f16_out, int m,   \
                                    int n, int k, hipStream_t s);
 RFQ_SKINNY_PART_DECL(0)

@@ -7,7 +7,7 @@
 // 16-byte loads; a wavefront's 64 lanes fetch 64 neighbouring units, i.e. one
 // contiguous span of the row.
 //
-// Two kernels:
+// Kernels here (batches of two to eight vectors mostly go to the matrix-core kernel of rfq_skinny.hip, see few_rows_ahead):
 //   gemv_xreg    (m == 1): a team of WPR wavefronts owns a fixed set of k
 //                positions and walks down the rows; each lane keeps the x
 //                values of its units in registers for the whole kernel, so x is
@@ -2014,162 +2014,6 @@ gemv_idot_batch_kernel(const uint8_t *__restrict__ w, const float *__restrict__ 
     }
 }
 
-// ---- 2 <= m <= 8, Q8_0: the batch through the matrix cores ----------------------
-//
-// With M vectors in registers the integer-dot kernel above needs more than 250
-// registers per lane, one wavefront per SIMD, and cannot keep enough loads in
-// flight to stream the matrix.  Here the M vectors are the rows of a matrix
-// operand instead: v_mfma_f32_16x16x32_f16 multiplies a 16 x 32 tile of
-// activations (one unit of k; rows 0..7 are the high parts of the eight
-// vectors, rows 8..15 their low parts, see below) with a 32 x 16 tile of
-// weights (one unit of 16 rows).
-//
-// Exactness is kept as in the integer-dot scheme.  A small kernel first turns x
-// into block-fixed-point per unit and vector: a power of two s and integers
-// X_i = round(x_i / s), |X_i| <= 2^22, split as X = 2048 * hi + lo with
-// |hi| <= 2048 and 0 <= lo < 2048, both exact in fp16; the weights b - 128 are
-// exact in fp16 too, so every product and every 32-term sum is an exact
-// integer below 2^24 in the fp32 accumulator:
-//     sum_i (b_i - 128) x_i  =  s * (2048 * sum (b-128).hi + sum (b-128).lo).
-// Operand layout of the instruction: lane l holds row/column l % 16 and the
-// eight k values 8 * (l / 16) ..+8; the result's lane l holds column l % 16
-// (a weight row: the lane that loaded its bytes and its scale) and rows
-// 4 * (l / 16) ..+4 (vectors).
-//
-// A workgroup owns 16 weight rows; its 8 wavefronts take the units
-// w, w + 8, ... of those rows, sixteen at a time with all their loads issued up
-// front (64 KiB of weights in flight per CU), and add their partial results
-// through LDS.
-
-typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
-typedef _Float16 v2h_t __attribute__((ext_vector_type(2)));
-typedef float v4f_t __attribute__((ext_vector_type(4)));
-typedef uint32_t v2u_t __attribute__((ext_vector_type(2)));
-typedef uint32_t v4u_t __attribute__((ext_vector_type(4)));
-
-// parts: [unit][k octet 0..3][row 0..15][8 fp16] (1 KiB per unit; row i < 8 is
-// the high part of vector i, row i >= 8 the low part of vector i - 8; operand lane
-// 16 * q + i reads octet q, row i); sx: [unit][8] f32.  One workgroup per unit;
-// thread t: vector t / 32, element t % 32.
-__global__ void __launch_bounds__(256)
-gemv_mfma_prep_kernel(const float *__restrict__ x, _Float16 *__restrict__ parts, float *__restrict__ sx, int m, int k)
-{
-    const int u = blockIdx.x, v = threadIdx.x >> 5, kk = threadIdx.x & 31, lane = threadIdx.x & 63;
-    const float xv = v < m ? x[(size_t)v * k + u * 32 + kk] : 0.0f;
-    float mx = fabsf(xv);
-    const bool bad = !(mx <= 3.40282347e+38f);
-    const unsigned long long bad_mask = __ballot(bad);
-    const bool any_bad = ((bad_mask >> (lane & 32)) & 0xFFFFFFFFull) != 0;
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 32));
-    const int e = (int)(__float_as_uint(mx) >> 23);   // biased exponent of the largest |x|
-    int ie = 275 - e;                                 // 1/s = 2^(21 - (e - 127))
-    if (ie > 254) ie = 254;
-    const float inv_s = __uint_as_float((uint32_t)ie << 23);
-    float sc = ie == 254 ? __uint_as_float(0x00400000u) : __uint_as_float((uint32_t)(254 - ie) << 23);
-    if (any_bad) sc = __uint_as_float(0x7FC00000u);   // a non-finite x poisons its unit, as it would a float sum
-    const int X = any_bad ? 0 : (int)(__float_as_uint(__builtin_fmaf(xv, inv_s, 12582912.0f)) - 0x4B400000u);
-    const int hi = X >> 11, lo = X & 2047;
-    const size_t at = ((size_t)u * 64 + (kk >> 3) * 16 + v) * 8 + (kk & 7);
-    parts[at] = (_Float16)(float)hi;
-    parts[at + 8 * 8] = (_Float16)(float)lo;
-    if (kk == 0) sx[u * 8 + v] = sc;
-}
-
-constexpr int MFMA_NB = 16;                           // units of a wavefront in flight together
-constexpr int MFMA_WAVES = 8;
-
-// FMT: RFQ_Q8_0 (36-byte blocks: f32 scale, offset-binary bytes) or RFQ_GGUF_Q8_0 (34-byte
-// blocks: f16 scale, int8 bytes, flipped to offset binary with one XOR per dword).
-template <int FMT>
-__global__ void __launch_bounds__(64 * MFMA_WAVES)
-gemv_mfma_q8_0_kernel(const uint8_t *__restrict__ w, const _Float16 *__restrict__ parts, const float *__restrict__ sx,
-                      float *__restrict__ y, int m, int n, int k)
-{
-    constexpr int BB = Fmt<FMT>::BB, DOFF = FMT == RFQ_Q8_0 ? 4 : 2;
-    constexpr uint32_t FLIP = FMT == RFQ_Q8_0 ? 0u : 0x80808080u;
-    __shared__ float red[MFMA_WAVES * 2 * 16 * 8];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, q = lane >> 4;
-    const int units = k / 32, n0 = blockIdx.x * 16;
-
-    const int row = n0 + j < n ? n0 + j : n - 1;
-    const uint8_t *row_ptr = w + (size_t)row * units * BB;
-    // The weight bytes are fetched by four neighbouring lanes per row (32
-    // consecutive bytes: one request instead of four) and handed to the lane
-    // that holds them as an operand, lane 16 * q + j <- lane 4 * j + q.
-    const int row_c = n0 + (lane >> 2) < n ? n0 + (lane >> 2) : n - 1;
-    const uint8_t *row_ptr_c = w + (size_t)row_c * units * BB + DOFF + 8 * (lane & 3);
-    const int from_lane4 = 4 * (4 * j + q);
-    const v4u_t *parts_l = reinterpret_cast<const v4u_t *>(parts) + lane;     // (octet q, row j: 16 bytes per lane)
-    const v2h_t bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int base = wave; base < units; base += MFMA_WAVES * MFMA_NB) {
-        v2u_t wq[MFMA_NB];
-        float ws[MFMA_NB];
-        v4u_t xa[MFMA_NB];
-        v4f_t s4[MFMA_NB / 2];                          // (the x scales follow half a batch behind: registers)
-        auto load_s4 = [&](int b) {
-            const int u = base + MFMA_WAVES * b, uc = u < units ? u : units - 1;
-            s4[b % (MFMA_NB / 2)] = *reinterpret_cast<const v4f_t *>(sx + uc * 8 + 4 * (q & 1));
-        };
-#pragma unroll
-        for (int b = 0; b < MFMA_NB; b++) {
-            const int u = base + MFMA_WAVES * b, uc = u < units ? u : units - 1; // (past the end: a valid unit, weight scale 0)
-            const uint8_t *blk = row_ptr + (size_t)uc * BB;
-            wq[b] = ld<v2u_t>(row_ptr_c + (size_t)uc * BB);
-            ws[b] = FMT == RFQ_Q8_0 ? ld<float>(blk) : f16_bits_to_f32(ld<uint16_t>(blk));                    // (no branch around a load: it would wait for the others)
-            xa[b] = parts_l[(size_t)uc * 64];
-            if (b < MFMA_NB / 2) load_s4(b);
-        }
-        __builtin_amdgcn_sched_barrier(0);             // (every load of the batch is out before the first is used)
-#pragma unroll
-        for (int b = 0; b < MFMA_NB; b++) {
-            // bytes b0..b3 of a dword -> fp16 pairs (b0, b1), (b2, b3): 0x6400 | b reads 1024 + b
-            v4u_t wb;
-#pragma unroll
-            for (int d = 0; d < 2; d++) {
-                const uint32_t wd = (uint32_t)__builtin_amdgcn_ds_bpermute(from_lane4, (int)wq[b][d]) ^ FLIP;
-                const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, wd, 0x04010400u);
-                const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, wd, 0x04030402u);
-                v2h_t h0, h1;
-                __builtin_memcpy(&h0, &p0, 4);
-                __builtin_memcpy(&h1, &p1, 4);
-                h0 = h0 + bias;                        // 1024 + b - 1152 = b - 128
-                h1 = h1 + bias;
-                uint32_t o0, o1;
-                __builtin_memcpy(&o0, &h0, 4);
-                __builtin_memcpy(&o1, &h1, 4);
-                wb[2 * d] = o0;
-                wb[2 * d + 1] = o1;
-            }
-            v8h_t wf, ax;
-            __builtin_memcpy(&wf, &wb, 16);
-            __builtin_memcpy(&ax, &xa[b], 16);
-            const v4f_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-            // this lane's four results: weight row j times the high (q < 2) or low parts of vectors 4 (q & 1) ..+4
-            const v4f_t sp = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax, wf, zero, 0, 0, 0);
-            const float wsc = base + MFMA_WAVES * b < units ? ws[b] : 0.0f;
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(wsc * s4[b % (MFMA_NB / 2)][r], sp[r], acc[r]);
-            if (b + MFMA_NB / 2 < MFMA_NB) load_s4(b + MFMA_NB / 2);
-        }
-    }
-    // red[wavefront][part: 0 high, 1 low][weight row][vector]
-#pragma unroll
-    for (int r = 0; r < 4; r++) red[((wave * 2 + (q >> 1)) * 16 + j) * 8 + 4 * (q & 1) + r] = acc[r];
-    __syncthreads();
-    if (tid < 128) {
-        const int jj = tid >> 3, v = tid & 7;
-        float hi = 0.0f, lo = 0.0f;
-#pragma unroll
-        for (int wv = 0; wv < MFMA_WAVES; wv++) {
-            hi += red[((wv * 2 + 0) * 16 + jj) * 8 + v];
-            lo += red[((wv * 2 + 1) * 16 + jj) * 8 + v];
-        }
-        if (v < m && n0 + jj < n) y[(size_t)v * n + n0 + jj] = __builtin_fmaf(hi, 2048.0f, lo);
-    }
-}
-
 // ---- any m <= 8, any k: one row per wavefront ---------------------------------
 // BYTES: fetch blocks byte-exactly (a tensor that does not start on a multiple of 4, see load32_a2).
 template <int FMT, int M, bool BYTES = false>
@@ -2470,28 +2314,6 @@ int run_generic(const uint8_t *w, const float *x, float *y, int n, int k, hipStr
     return RFQ_OK;
 }
 
-template <int FMT>
-int run_mfma_q8_0(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStream_t s)
-{
-    const int units = k / 32;
-    const size_t parts_bytes = (size_t)units * 1024, sx_bytes = (size_t)units * 32;
-    uint8_t *tmp = nullptr;
-    bool transient = false;
-    if (int rc = workspace(s, parts_bytes + sx_bytes, &tmp, &transient)) return rc;
-    _Float16 *parts = reinterpret_cast<_Float16 *>(tmp);
-    float *sx = reinterpret_cast<float *>(tmp + parts_bytes);
-    note_kernel("gemv_mfma_prep_kernel + gemv_mfma_q8_0_kernel<%s>", FMT, 0, 0, 0);
-    hipLaunchKernelGGL(gemv_mfma_prep_kernel, dim3(units), dim3(256), 0, s, x, parts, sx, m, k);
-    hipLaunchKernelGGL(gemv_mfma_q8_0_kernel<FMT>, dim3((n + 15) / 16), dim3(64 * MFMA_WAVES), 0, s, w, parts, sx, y, m, n, k);
-    hipError_t launch_err = hipGetLastError();
-    if (transient) {
-        hipError_t free_err = hipFreeAsync(tmp, s);
-        if (launch_err == hipSuccess) launch_err = free_err;
-    }
-    if (launch_err != hipSuccess) return hip_fail(launch_err, "gemv_mfma_q8_0_kernel");
-    return RFQ_OK;
-}
-
 // m == 1, 16 < k / 32 <= 512: the kernels that keep x per lane.
 template <int FMT, bool FUSE>
 int run_rows(const uint8_t *w, const float *x, float *y, int n, int k, const GemvFuse &f, hipStream_t s)
@@ -2576,6 +2398,33 @@ int run_generic_m(const uint8_t *w, const float *x, float *y, int m, int n, int 
     }
 }
 
+// Whether a batch goes through the matrix-core kernel for few rows (rfq_skinny.hip) instead of the integer-dot batch kernel
+// (batch_fits) or, where a format or row length has none, one decode launch per vector or the one-row-per-wavefront
+// kernel.  Its time hardly depends on m; measured on 512..14336 rows of 768..13824 for every format (us, there / here):
+//   m >= 5: always (Q8_0 4096 x 4096 m = 8 11.4 / 9.7, Q4_0 13.0 / 8.8, Q4_K 14336 x 4096 30.7 / 23.6, GGUF_Q6_K
+//     4096 x 13824 82 / 23, Q6_K 14336 x 4096 82 / 23, MXFP6 4096 x 4096 42.6 / 12.4);
+//   m = 3, 4 against the batch kernel (which takes three as four): rows longer than 3000 with 12 or more of them per CU, up
+//     to 24 for the formats whose batch kernel streams well at many rows (4096 x 4096: Q8_0 9.5 / 8.3, GGUF_Q4_K 8.7 / 7.6;
+//     4096 x 8192 GGUF_Q6_K 12.9 / 14; 14336 x 4096: GGUF_Q4_0 18.4 / 15.7, but Q8_0 19.9 / 22.3, Q4_K 17.8 / 21.8);
+//   m = 3, 4 without a batch kernel: from four rows per CU on, or long rows (Q6_K 14336 x 4096 m = 4 42 / 21);
+//   m = 2: only without a batch kernel, for as many rows as make one launch cheaper than two (MXFP4 8192 x 4096 13.9 / 11.2;
+//     512 x 4096 5.8 / 7.0).  Q8_0 without one always (4096 x 13824 35 / 20).
+bool few_rows_ahead(int fmt, int m, int n, int ku, bool batch_fits)
+{
+    const int cus = device_cu_count();
+    if (m >= 5) return true;
+    const bool q8 = fmt == RFQ_Q8_0 || fmt == RFQ_GGUF_Q8_0;
+    if (m >= 3) {
+        if (batch_fits)
+            return ku >= 96 && n >= cus * 12 && (n <= cus * 24 || fmt == RFQ_Q4_0 || fmt == RFQ_GGUF_Q4_0 || fmt == RFQ_GGUF_Q4_K);
+        return q8 || n >= cus * 4 || ku > 256;
+    }
+    if (batch_fits) return false;
+    if (q8) return true;
+    if (fmt == RFQ_MXFP6_E2M3) return ku <= 32 && n >= cus * 12;
+    return n > cus * 16 || (n >= cus * 12 && ku <= 256);
+}
+
 template <int FMT>
 int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStream_t s)
 {
@@ -2585,18 +2434,16 @@ int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStre
     }
     if (m == 1 && ku > 16 && ku <= 512)                        // (shorter rows leave most of a wavefront's lanes without a unit)
         return run_rows<FMT, false>(w, x, y, n, k, GemvFuse{nullptr, nullptr, 0.0f, 0}, s);
-    if constexpr (FMT == RFQ_Q8_0 || FMT == RFQ_GGUF_Q8_0) {
-        // (the matrix-core kernel costs the same for any m; up to four vectors the integer-dot batch kernel below is
-        // faster where it applies -- 4096 x 4096: m = 2 7.1 against 11.8 us, m = 4 9.7 against 11.8, m = 8 14.3 against 11.8)
-        const bool idot_batch_fits = ku > 32 && ku <= 256;
-        if (m > (idot_batch_fits ? 4 : 1) && (reinterpret_cast<uintptr_t>(w) & (FMT == RFQ_Q8_0 ? 3u : 1u)) == 0)
-            return run_mfma_q8_0<FMT>(w, x, y, m, n, k, s);
+    const bool batch_fits = HasIdotBatch<FMT>::value && ku > 32 && ku <= 256;
+    if (m > 1 && (reinterpret_cast<uintptr_t>(w) & 3u) == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && few_rows_ahead(FMT, m, n, ku, batch_fits)) {
+        note_kernel("gemv_skinny_kernel<%s>", FMT, 0, 0, 0);
+        return launch_skinny_gemv(FMT, w, nullptr, x, y, nullptr, m, n, k, s);
     }
-    if (HasIdotBatch<FMT>::value && m > 1 && ku > 32 && ku <= 256) {
+    if (batch_fits && m > 1) {
         // the prepared vectors of a launch live in LDS (112 bytes per unit and vector): a batch that
         // does not fit goes out as launches of four or two vectors
         const size_t lds_limit = 160 * 1024 - 4096;
-        int mb = m <= 2 ? 2 : (m <= 4 ? 4 : 8);
+        int mb = m <= 2 ? 2 : 4;
         while (mb > 2 && (size_t)mb * ku * 112 > lds_limit) mb /= 2;
         for (int v0 = 0; v0 < m; v0 += mb) {
             const int mv = m - v0 < mb ? m - v0 : mb;
@@ -2604,8 +2451,7 @@ int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStre
             float *yv = y + (size_t)v0 * n;
             int rc;
             if (mb == 2) rc = run_idot_batch_k<FMT, 2>(w, xv, yv, mv, n, k, s);
-            else if (mb == 4) rc = run_idot_batch_k<FMT, 4>(w, xv, yv, mv, n, k, s);
-            else rc = run_idot_batch_k<FMT, 8>(w, xv, yv, mv, n, k, s);
+            else rc = run_idot_batch_k<FMT, 4>(w, xv, yv, mv, n, k, s);
             if (rc != RFQ_OK) return rc;
         }
         return RFQ_OK;

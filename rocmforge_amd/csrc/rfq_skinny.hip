@@ -16,8 +16,8 @@ constexpr int skinny_part_of(int fmt)
     switch (fmt) {
     case RFQ_Q4_0: case RFQ_Q4_K: return 0;
     case RFQ_Q8_0: case RFQ_GGUF_Q8_0: return 1;
-    case RFQ_Q6_K: case RFQ_GGUF_Q6_K: return 2;
-    case RFQ_GGUF_Q4_0: case RFQ_GGUF_Q4_K: return 3;
+    case RFQ_Q6_K: case RFQ_GGUF_Q6_K: case RFQ_MXFP4: return 2;
+    case RFQ_GGUF_Q4_0: case RFQ_GGUF_Q4_K: case RFQ_MXFP6_E2M3: return 3;
     default: return -1;
     }
 }
@@ -31,6 +31,38 @@ int waves_for(int k, int most)
 {
     const int units = (k / 32 + 3) / 4;
     return units < most ? units : most;
+}
+
+template <int FMT, int TJ, int MV, int D, int WAVES>
+int gemv_cfg(const uint8_t *w, const uint8_t *w2, const float *x, float *y, float *y2, int m, int n, int k, hipStream_t s)
+{
+    if constexpr (gemv_lds<TJ, MV>(WAVES) > 64 * 1024) {
+        static std::once_flag once;
+        static hipError_t err = hipSuccess;
+        std::call_once(once, [] {
+            err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_skinny_kernel<FMT, TJ, MV, D, WAVES>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, gemv_lds<TJ, MV>(WAVES));
+        });
+        if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(gemv_skinny_kernel)");
+    }
+    const int waves = waves_for(k, WAVES);
+    const size_t lds = (size_t)gemv_lds<TJ, MV>(waves);
+    hipLaunchKernelGGL((gemv_skinny_kernel<FMT, TJ, MV, D, WAVES>), dim3((n + 16 * TJ - 1) / (16 * TJ), w2 != nullptr ? 2 : 1),
+                       dim3(64 * waves), lds, s, w, x, y, m, n, k, w2, y2);
+    RFQ_LAUNCH_CHECK("gemv_skinny_kernel");
+    return RFQ_OK;
+}
+
+// Row tiles per workgroup: one up to 20 rows per CU, where a second tile would leave CUs without a workgroup, then two, four
+// from 52 on: every workgroup converts all of x (Q4_0, 8 vectors, k = 4096: n = 4096 8.8 / 10.7 / 14.5 us with 1 / 2 / 4,
+// n = 8192 12.7 / 11.5 / 14.9, n = 14336 23.4 / 18.8 / 18.4; MXFP4 n = 14336 22.8 / 22.1 / 18.8).
+template <int FMT, int MV>
+int gemv_fmt(const uint8_t *w, const uint8_t *w2, const float *x, float *y, float *y2, int m, int n, int k, hipStream_t s)
+{
+    const int rows = w2 != nullptr ? 2 * n : n, cus = device_cu_count();
+    if (rows >= 52 * cus) return gemv_cfg<FMT, 4, MV, 2, 8>(w, w2, x, y, y2, m, n, k, s);
+    if (rows > 20 * cus) return gemv_cfg<FMT, 2, MV, 2, 8>(w, w2, x, y, y2, m, n, k, s);
+    return gemv_cfg<FMT, 1, MV, 2, 8>(w, w2, x, y, y2, m, n, k, s);
 }
 
 template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES>
@@ -121,6 +153,17 @@ int gemm_fmt(const uint8_t *w, const uint8_t *a, bool arranged, void *y, int f16
         return fail(RFQ_E_UNSUPPORTED, "no few-row kernel for format %d in this part of the build", fmt); \
     }(std::integral_constant<int, RFQ_SKINNY_PART>{})
 
+int RFQ_SKINNY_CAT(launch_skinny_gemv_part, RFQ_SKINNY_PART)(int fmt, const uint8_t *w, const uint8_t *w2, const float *x, float *y,
+                                                             float *y2, int m, int n, int k, hipStream_t s)
+{
+#define RFQ_SKINNY_GEMV(F) (m <= 4 ? gemv_fmt<F, 4>(w, w2, x, y, y2, m, n, k, s) : gemv_fmt<F, 8>(w, w2, x, y, y2, m, n, k, s))
+    if constexpr (skinny_part_of(RFQ_MXFP4) == RFQ_SKINNY_PART)
+        if (fmt == RFQ_MXFP4) return RFQ_SKINNY_GEMV(RFQ_MXFP4);
+    if constexpr (skinny_part_of(RFQ_MXFP6_E2M3) == RFQ_SKINNY_PART)
+        if (fmt == RFQ_MXFP6_E2M3) return RFQ_SKINNY_GEMV(RFQ_MXFP6_E2M3);
+    RFQ_SKINNY_CASES(RFQ_SKINNY_GEMV);
+}
+
 int RFQ_SKINNY_CAT(launch_skinny_gemm_part, RFQ_SKINNY_PART)(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, int f16_out,
                                                              int m, int n, int k, hipStream_t s)
 {
@@ -151,6 +194,17 @@ bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts)
     double tiled = 8.0 + per_ku * ku / parts * (groups > cus ? groups / cus : 1.0);
     if (parts > 1) tiled += 4.0 + 8.0 * parts * m * (double)n / 5e6;
     return few < tiled;
+}
+
+int launch_skinny_gemv(int fmt, const uint8_t *w, const uint8_t *w2, const float *x, float *y, float *y2, int m, int n, int k, hipStream_t s)
+{
+    switch (skinny_part_of(fmt)) {
+    case 0: return launch_skinny_gemv_part0(fmt, w, w2, x, y, y2, m, n, k, s);
+    case 1: return launch_skinny_gemv_part1(fmt, w, w2, x, y, y2, m, n, k, s);
+    case 2: return launch_skinny_gemv_part2(fmt, w, w2, x, y, y2, m, n, k, s);
+    case 3: return launch_skinny_gemv_part3(fmt, w, w2, x, y, y2, m, n, k, s);
+    default: return fail(RFQ_E_UNSUPPORTED, "no few-row kernel for format %d", fmt);
+    }
 }
 
 int launch_skinny_gemm(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, bool f16_out, int m, int n, int k, hipStream_t s)

@@ -1,6 +1,8 @@
 // Matrix-core contraction for few rows of activations:  y[m, n] = x[m, k] . dequant(W)[n, k]^T, one launch, no temporary.
 //
-// float16 a, prompts up to about 160 rows (rfq_gemm_f16, rfq_gemm_f16_arranged; prefer_skinny_gemm draws the line).
+//   * float32 x, 2..8 rows  (decode batches, rfq_gemv)
+//   * float16 a, 9..160 rows (short prompts, rfq_gemm_f16 / rfq_gemm_f16_arranged)
+//
 // With so few rows every packed weight byte is wanted once and the matrix cores are nearly idle; what bounds the call is
 // the weight stream, the vector instructions that turn codes into operands, and the activations, which every workgroup
 // reads whole.  Hence:
@@ -13,12 +15,18 @@
 //     v_permlane16_swap until each holds its eight codes of every group.  Activations take the same way through LDS.
 //   * Mins (Q4_K): the sum of x over a group comes out of the same instruction with a weight operand of ones, already in
 //     the layout of the result: acc += min * sum(x).
+//   * float32 x is split into two fp16 parts hi + lo of 11 bits each under a power-of-two scale per wavefront and row that
+//     follows the largest |x| seen (slow path, rarely taken); both parts are multiplied, so 22 bits of x are kept.
 //   * No split of k over workgroups: the wavefronts of a workgroup share 16 * TJ weight rows, take the 128-element units
 //     of k in turn and add their results through LDS: one launch, nothing to allocate.
 // Measured (cold weights, captured launches; the tiled kernel with its arrangement and its parts -> this one):
 //   37 x 4096 -> 4096      Q8_0 33.6 -> 10.7 us   GGUF_Q4_K 25.8 -> 10.5   GGUF_Q6_K 43.0 -> 12.3   Q4_K 22.2 -> 12.6
 //   9 x 1024 -> 1000       Q8_0 27.5 -> 3.1       GGUF_Q4_K 20.0 -> 3.2    GGUF_Q6_K 36.0 -> 4.3    Q4_K 16.1 -> 3.9
 //   48 x 4096 -> 14336     Q8_0 66.5 -> 32.7      GGUF_Q4_K 42.5 -> 23.3   GGUF_Q6_K 77.9 -> 42.0   Q4_K 40.6 -> 34.7
+// and decode batches (integer-dot batch kernel, or a launch per vector -> this one):
+//   8 x 4096 -> 4096       Q8_0 11.4 -> 9.7 us    GGUF_Q4_K 13.9 -> 8.7    Q6_K 33.4 -> 10.1        MXFP4 34.1 -> 9.4
+//   5 x 13824 -> 5120      Q8_0 62 -> 31          GGUF_Q4_K 60 -> 28       GGUF_Q6_K 90 -> 42       Q4_K 75 -> 33
+//   error against 64 bits (2-norm): 8e-8 .. 2e-7, the integer-dot kernel 3e-7 .. 1e-6
 // (10.5 us for 37 rows of GGUF_Q4_K is 0.9 TB/s of weights: what bounds it is the activations, 384 KB per workgroup
 // through LDS, and the instructions, about 60 per unit and 16-row operand.)
 #pragma once
@@ -104,7 +112,7 @@ template <int NW> __device__ __forceinline__ void load_dwords(const uint8_t *a, 
 }
 // Which eight elements of a group lane row q holds, and in which order its four operand dwords hold them.
 enum { OCTET, OCTET_SWAPPED, HALVES, HALVES_SWAPPED };           // 8q..  |  8q'..  |  4q.. and 16+4q..  |  4q'.. and 16+4q'..   (q' = q with its bits swapped)
-enum { P04, P01, P02 };                                          // (0,4)(1,5)(2,6)(3,7) | (0,1)(2,3)(4,5)(6,7) | (0,2)(1,3)(4,6)(5,7)
+enum { P04, P01, P02, P26 };                                     // (0,4)(1,5)(2,6)(3,7) | (0,1)(2,3)(4,5)(6,7) | (0,2)(1,3)(4,6)(5,7) | (0,2)(4,6)(1,3)(5,7)
 
 // W<FMT>: load() fetches the dwords r[] that lane 4 * i + g holds of group g of the 128-element unit `u` of row i (four
 // neighbouring lanes on neighbouring bytes: a load whose neighbouring lanes sit in different rows runs at a quarter of the
@@ -380,6 +388,109 @@ template <> struct W<RFQ_GGUF_Q6_K> {
     __device__ __forceinline__ float mn(int) const { return 0.f; }
 };
 
+// The MXFP formats: the operand is the decoded code (MxfpBlock::decode_e2m1 / decode_e2m3, src/loader/mxfp.rs:234-293), a
+// multiple of 1/16 below 8 and exact in fp16.  The reference clamps value * 2^e to +-BOUND (mxfp.rs:196-203), which moves a
+// value only for e >= 1, and from e = 5 on every value but 0 sits at the bound: a wavefront that holds such a block (one
+// ballot) multiplies the block's operand by 2^min(e, 5), clamps it and gives the block the scale 1.
+template <int FMT> struct WMx {
+    static constexpr int ND = FMT == RFQ_MXFP4 ? 4 : 6;           // dwords of codes behind the exponent byte
+    static constexpr int ORDER = OCTET, PAIRS = FMT == RFQ_MXFP4 ? P26 : P01, NR = ND + 2;
+    static constexpr bool MINS = false, SPLIT16 = false;
+    uint32_t r[NR], q[8];
+    float sc4[4], up4[4];
+    bool clamp;
+    __device__ __forceinline__ void load(const uint8_t *row, int u, int g)
+    {
+        const uint8_t *p = row + (uint32_t)(4 * u + g) * (uint32_t)(1 + 4 * ND);
+        const uint32_t o = (uint32_t)(reinterpret_cast<uintptr_t>(p) & 3u);
+        uint32_t v[ND + 1];
+        load_dwords<ND + 1>(p - o, v);                            // (o + 1 + 4 ND <= 4 (ND + 1): each holds a byte of the block)
+#pragma unroll
+        for (int i = 0; i <= ND; i++) r[i] = v[i];
+        r[ND + 1] = o;
+    }
+    __device__ __forceinline__ void open(int, bool dead)
+    {
+        const uint32_t sel = 0x04030201u + __builtin_amdgcn_perm(0u, r[ND + 1], 0u);
+        uint32_t c[ND];
+#pragma unroll
+        for (int i = 0; i < ND; i++) c[i] = __builtin_amdgcn_perm(r[i + 1], r[i], sel);
+        const int e = (int)(int8_t)(r[0] >> (8u * r[ND + 1]));
+        clamp = __builtin_amdgcn_ballot_w64(e >= 1) != 0;
+        spread4(dead ? 0.f : e >= 1 ? 1.0f : mx_scale(e), sc4);
+        if (clamp) spread4(e >= 1 ? mx_scale(e < 5 ? e : 5) : 1.0f, up4);
+        if constexpr (FMT == RFQ_MXFP4) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) q[i] = c[i];
+            transpose4(q[0], q[1], q[2], q[3]);
+        } else {
+            // elements 4j .. 4j+3 at bits 10, 4, 14 and 24 of the 32 bits from bit 24 j (element 31 is never written: code 0)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int d = 24 * j / 32, sh = 24 * j % 32;
+                const uint32_t w = sh == 0 ? c[d] : __builtin_amdgcn_alignbit(d + 1 < ND ? c[d + 1] : 0u, c[d], sh);
+                q[j] = ((w >> 10) & 0x3Fu) | ((w << 4) & 0x3F00u) | ((w << 2) & 0x3F0000u) | (j < 7 ? w & 0x3F000000u : 0u);
+            }
+            transpose4(q[0], q[2], q[4], q[6]);
+            transpose4(q[1], q[3], q[5], q[7]);
+        }
+    }
+    // four E2M1 codes (one per byte) -> the high bytes of their fp16 values (the low bytes are zero)
+    static __device__ __forceinline__ uint32_t e2m1(uint32_t c)
+    {
+        const uint32_t at = c & 0x07070707u, s = (c >> 3) & 0x01010101u, neg = (s << 8) - s;
+        const uint32_t pos = __builtin_amdgcn_perm(0x48444440u, 0x403C3C00u, at), mns = __builtin_amdgcn_perm(0xC8C4C4C0u, 0xC0BCBCB8u, at);
+        return (neg & mns) | (~neg & pos);
+    }
+    // two E2M3 codes in the 16-bit halves -> fp16: 0x3800 + (code & 31) * 128 is (1 + m / 8) * 2^(x - 1); code 0 is zero
+    static __device__ __forceinline__ uint32_t e2m3(uint32_t p)
+    {
+        typedef uint16_t v2s __attribute__((ext_vector_type(2)));
+        const uint32_t h = (((p & 0x001F001Fu) << 7) + 0x38003800u) | ((p & 0x00200020u) << 10);
+        v2s a, b;
+        __builtin_memcpy(&a, &p, 4);
+        __builtin_memcpy(&b, &h, 4);
+        a = __builtin_elementwise_min(a, v2s{1, 1}) * b;
+        uint32_t o;
+        __builtin_memcpy(&o, &a, 4);
+        return o;
+    }
+    __device__ __forceinline__ v4u frag(int j) const
+    {
+        v4u o;
+        if constexpr (FMT == RFQ_MXFP4) {                         // element 2 b of an octet is the high nibble of byte b
+            const uint32_t ev = e2m1((q[j] >> 4) & 0x0F0F0F0Fu), od = e2m1(q[j] & 0x0F0F0F0Fu);
+            o = v4u{__builtin_amdgcn_perm(ev, ev, 0x010C000Cu), __builtin_amdgcn_perm(ev, ev, 0x030C020Cu),
+                    __builtin_amdgcn_perm(od, od, 0x010C000Cu), __builtin_amdgcn_perm(od, od, 0x030C020Cu)};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                o[2 * e] = e2m3(__builtin_amdgcn_perm(0u, q[2 * j + e], 0x0C010C00u));
+                o[2 * e + 1] = e2m3(__builtin_amdgcn_perm(0u, q[2 * j + e], 0x0C030C02u));
+            }
+        }
+        if (clamp) {
+            const _Float16 up = (_Float16)up4[j], bound = FMT == RFQ_MXFP4 ? (_Float16)8.0f : (_Float16)7.5f;
+            const v2h lim = {bound, bound};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                v2h h;
+                const uint32_t bits = o[i];
+                __builtin_memcpy(&h, &bits, 4);
+                h = __builtin_elementwise_max(__builtin_elementwise_min(h * v2h{up, up}, lim), -lim);
+                uint32_t t;
+                __builtin_memcpy(&t, &h, 4);
+                o[i] = t;
+            }
+        }
+        return o;
+    }
+    __device__ __forceinline__ float sc(int j, int) const { return sc4[j]; }
+    __device__ __forceinline__ float mn(int) const { return 0.f; }
+};
+template <> struct W<RFQ_MXFP4> : WMx<RFQ_MXFP4> {};
+template <> struct W<RFQ_MXFP6_E2M3> : WMx<RFQ_MXFP6_E2M3> {};
+
 // r[] of lane 4 * i + g -> lane 16 * g + i
 template <int FMT> __device__ __forceinline__ W<FMT> placed(const W<FMT> &raw, int from4)
 {
@@ -392,6 +503,19 @@ template <int FMT> __device__ __forceinline__ W<FMT> placed(const W<FMT> &raw, i
 __device__ __forceinline__ int row_part(int order, int q)         // the number of the octet / quarter-half of lane row q
 {
     return (order == OCTET_SWAPPED || order == HALVES_SWAPPED) ? ((q & 1) << 1) | (q >> 1) : q;
+}
+
+template <int PAIRS> __device__ __forceinline__ constexpr int pair_of(int r, int h)  // element h of operand dword r
+{
+    return PAIRS == P04 ? r + 4 * h : PAIRS == P01 ? 2 * r + h : PAIRS == P02 ? (r >> 1) * 4 + (r & 1) + 2 * h : (r & 1) * 4 + (r >> 1) + 2 * h;
+}
+
+__device__ __forceinline__ uint32_t pack2h(float a, float b)
+{
+    const v2h h = {(_Float16)a, (_Float16)b};
+    uint32_t o;
+    __builtin_memcpy(&o, &h, 4);
+    return o;
 }
 
 template <bool SPLIT16>
@@ -411,6 +535,237 @@ __device__ __forceinline__ void contract(const v4u &xa, const v4u &wf, v4f (&d)[
         __builtin_memcpy(&x8, &xa, 16);
         __builtin_memcpy(&w8, &wf, 16);
         d[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x8, w8, d[0], 0, 0, 0);
+    }
+}
+
+constexpr int MAX_WAVES = 16;
+
+// ---- float32 x, m <= 8 -----------------------------------------------------------------------------------------------
+// blockDim = 64 * waves; blockIdx.y: the second of two matrices of the same shape that share x (w2, y2), when there are two.
+// LDS: per wavefront x_bytes for its unit of x as fp16 parts (plane hi, plane lo; vector; operand
+// order), later the wavefronts' results.
+// x goes global -> registers (sixteen lanes per vector, eight elements each: consecutive lanes on consecutive bytes) ->
+// two fp16 parts -> LDS -> operands: every element is converted once per workgroup and unit.
+constexpr int XROW = 256 + 16;                                    // bytes of a vector's 128 elements, bank-skewed
+template <int MV> constexpr int x_bytes() { return 2 * MV * XROW; }
+template <int TJ, int MV> constexpr int gemv_lds(int waves) { return waves * (x_bytes<MV>() > MV * 16 * TJ * 4 ? x_bytes<MV>() : MV * 16 * TJ * 4); }
+
+// MV: 4 or 8 vectors, m <= MV.
+template <int FMT, int TJ, int MV, int D, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
+gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y, int m, int n, int k,
+                   const uint8_t *__restrict__ w2, float *__restrict__ y2)
+{
+    if (blockIdx.y != 0) {
+        w = w2;
+        y = y2;
+    }
+    typedef W<FMT> WF;
+    constexpr int P = MV / 4;                                     // octets of x per lane and unit
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
+    const int groups = k >> 5, units = (groups + 3) >> 2;
+    const int n0 = blockIdx.x * (16 * TJ);
+    const size_t row_bytes = (size_t)(k / Fmt<FMT>::BE) * Fmt<FMT>::BB;
+    const uint8_t *row[TJ];                                       // (weights: lane 4 * i + g fetches group g of row i)
+    const int lg = lane & 3, from4 = 4 * (4 * i + q);
+#pragma unroll
+    for (int t = 0; t < TJ; t++) {
+        const int r = n0 + 16 * t + (lane >> 2);
+        row[t] = w + (size_t)(r < n ? r : n - 1) * row_bytes;
+    }
+    // x: octet lane & 15 of the unit, vectors lane >> 4 and, with eight vectors, 4 + (lane >> 4)
+    const float *xl[P];
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+        const int v = 4 * p + q;
+        xl[p] = x + (size_t)(v < m ? v : m - 1) * k + 8 * i;
+    }
+    uint8_t *const area = lds + wave * x_bytes<MV>();
+    uint8_t *xw[P];
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+        const int o = i & 3;                                      // octet of group i >> 2
+        const int at = WF::ORDER <= OCTET_SWAPPED ? row_part(WF::ORDER, o) * 16 : (o >> 1) * 8;
+        xw[p] = area + (4 * p + q) * XROW + (i >> 2) * 64 + at;
+    }
+    // (halves: an octet is two operand halves, of the lane rows of parts 2 (o & 1) and 2 (o & 1) + 1)
+    const int h0 = WF::ORDER > OCTET_SWAPPED ? row_part(WF::ORDER, 2 * (i & 1)) * 16 : 0;
+    const int h1 = WF::ORDER > OCTET_SWAPPED ? row_part(WF::ORDER, 2 * (i & 1) + 1) * 16 : 0;
+    const uint8_t *const xrd = area + (i & (MV - 1)) * XROW + q * 16;
+
+    WF raw[D][TJ];
+    v4f xr[P][2];
+    auto load_w = [&](WF (&dst)[TJ], int u) __attribute__((always_inline)) {
+        const int uc = u < units ? u : units - 1;
+        const int g = 4 * uc + lg < groups ? lg : groups - 1 - 4 * uc;  // (past the row's end: its last group, with scale 0)
+#pragma unroll
+        for (int t = 0; t < TJ; t++) dst[t].load(row[t], uc, g);
+    };
+    auto load_x = [&](int u) __attribute__((always_inline)) {
+        const int uc = u < units ? u : units - 1;
+        const int at = 128 * uc + 8 * i < k ? 128 * uc : 128 * uc - 32 * (i >> 2);   // (past the end: the unit's first group)
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+            xr[p][0] = *reinterpret_cast<const v4f *>(xl[p] + at);
+            xr[p][1] = *reinterpret_cast<const v4f *>(xl[p] + at + 4);
+        }
+    };
+    float s[P], lim[P];                                           // this lane's vectors: scale, and the largest |x| it can take
+#pragma unroll
+    for (int p = 0; p < P; p++) { s[p] = 1.0f; lim[p] = 0.0f; }
+    float acc[TJ][4];
+#pragma unroll
+    for (int t = 0; t < TJ; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[t][r] = 0.0f;
+    const v4u ones = {0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
+
+    load_x(wave);
+#pragma unroll
+    for (int d = 0; d < D; d++) load_w(raw[d], wave + d * waves);
+
+    for (int u0 = wave; u0 < units; u0 += D * waves) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const int u = u0 + d * waves;
+            if (u < units) {
+                float e[P][8], mx[P];
+                bool over = false;
+                const bool past = 128 * u + 8 * i >= k;
+#pragma unroll
+                for (int p = 0; p < P; p++) {
+#pragma unroll
+                    for (int c = 0; c < 4; c++) { e[p][c] = xr[p][0][c]; e[p][4 + c] = xr[p][1][c]; }
+                    if (Fmt<FMT>::BE < 128 && past) {
+#pragma unroll
+                        for (int c = 0; c < 8; c++) e[p][c] = 0.0f;
+                    }
+                    mx[p] = fmaxf(fmaxf(fmaxf(fabsf(e[p][0]), fabsf(e[p][1])), fmaxf(fabsf(e[p][2]), fabsf(e[p][3]))),
+                                  fmaxf(fmaxf(fabsf(e[p][4]), fabsf(e[p][5])), fmaxf(fabsf(e[p][6]), fabsf(e[p][7]))));
+                    over |= mx[p] > lim[p];
+                }
+                load_x(u + waves);
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(over) != 0, 0)) {
+                    // |x| beyond what the scale takes: the vector's largest of this unit goes to 2^10 (up to 32 times as
+                    // much fits from then on), and what has been summed follows
+                    float f[P];
+#pragma unroll
+                    for (int p = 0; p < P; p++) {
+                        float t = mx[p];
+#pragma unroll
+                        for (int o = 1; o < 16; o <<= 1) t = fmaxf(t, __shfl_xor(t, o));
+                        f[p] = 1.0f;
+                        if (t > lim[p]) {
+                            const int ex = (int)(__float_as_uint(t) >> 23);  // biased exponent (255 for an infinity)
+                            int se = 264 - ex;                               // s = 2^(10 - (ex - 127))
+                            se = se > 252 ? 252 : se;
+                            const float s_new = __uint_as_float((uint32_t)se << 23);
+                            f[p] = s_new * (1.0f / s[p]);                    // (powers of two)
+                            s[p] = s_new;
+                            lim[p] = ex >= 249 ? 3.40282347e+38f : se == 252 ? __uint_as_float((uint32_t)17 << 23) : __uint_as_float((uint32_t)(ex + 5) << 23);
+                        }
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {                            // (vector 4 q + r is row r of lanes, octet set q)
+                        float fr = __shfl(f[0], 16 * r);
+                        if constexpr (P == 2) {
+                            const float f1 = __shfl(f[1], 16 * r);
+                            fr = (q & 1) ? f1 : fr;
+                        }
+#pragma unroll
+                        for (int t = 0; t < TJ; t++) acc[t][r] *= fr;
+                    }
+                }
+#pragma unroll
+                for (int p = 0; p < P; p++) {
+                    uint32_t hi[4], lo[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        float a = e[p][pair_of<WF::PAIRS>(r, 0)] * s[p], b = e[p][pair_of<WF::PAIRS>(r, 1)] * s[p];
+                        asm("" : "+v"(a), "+v"(b));               // (one conversion of each product, not one per use)
+                        const v2h h = {(_Float16)a, (_Float16)b};
+                        __builtin_memcpy(&hi[r], &h, 4);
+                        lo[r] = pack2h(a - (float)h[0], b - (float)h[1]);
+                    }
+                    if constexpr (WF::ORDER <= OCTET_SWAPPED) {
+                        *reinterpret_cast<v4u *>(xw[p]) = v4u{hi[0], hi[1], hi[2], hi[3]};
+                        *reinterpret_cast<v4u *>(xw[p] + MV * XROW) = v4u{lo[0], lo[1], lo[2], lo[3]};
+                    } else {
+                        *reinterpret_cast<v2u *>(xw[p] + h0) = v2u{hi[0], hi[1]};
+                        *reinterpret_cast<v2u *>(xw[p] + h1) = v2u{hi[2], hi[3]};
+                        *reinterpret_cast<v2u *>(xw[p] + MV * XROW + h0) = v2u{lo[0], lo[1]};
+                        *reinterpret_cast<v2u *>(xw[p] + MV * XROW + h1) = v2u{lo[2], lo[3]};
+                    }
+                }
+                WF cur[TJ];
+#pragma unroll
+                for (int t = 0; t < TJ; t++) {
+                    cur[t] = placed<FMT>(raw[d][t], from4);
+                    cur[t].open(u, Fmt<FMT>::BE < 128 && 4 * u + q >= groups);
+                }
+                // (a wavefront's LDS operations complete in order: no barrier between its writes and its reads)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const v4u hi = *reinterpret_cast<const v4u *>(xrd + j * 64);
+                    const v4u lo = *reinterpret_cast<const v4u *>(xrd + MV * XROW + j * 64);
+                    v4f xs[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                    if constexpr (WF::MINS) {
+                        contract<false>(lo, ones, xs);
+                        contract<false>(hi, ones, xs);
+                    }
+#pragma unroll
+                    for (int t = 0; t < TJ; t++) {
+                        const v4u wf = cur[t].frag(j);
+                        v4f p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                        contract<WF::SPLIT16>(lo, wf, p);
+                        contract<WF::SPLIT16>(hi, wf, p);
+                        const float s0 = cur[t].sc(j, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; r++) acc[t][r] = __builtin_fmaf(s0, p[0][r], acc[t][r]);
+                        if constexpr (WF::SPLIT16) {
+                            const float s1 = cur[t].sc(j, 1);
+#pragma unroll
+                            for (int r = 0; r < 4; r++) acc[t][r] = __builtin_fmaf(s1, p[1][r], acc[t][r]);
+                        }
+                        if constexpr (WF::MINS) {
+                            const float mn = cur[t].mn(j);
+#pragma unroll
+                            for (int r = 0; r < 4; r++) acc[t][r] = __builtin_fmaf(mn, xs[0][r], acc[t][r]);
+                        }
+                    }
+                }
+            }
+            load_w(raw[d], u + D * waves);
+        }
+    }
+    // red[wave][vector][16 * TJ rows]; lane rows 0 .. P - 1 hold vectors 0 .. MV - 1
+    float inv[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        inv[r] = __shfl(s[0], 16 * r);
+        if constexpr (P == 2) {
+            const float s1 = __shfl(s[1], 16 * r);
+            inv[r] = (q & 1) ? s1 : inv[r];
+        }
+        inv[r] = 1.0f / inv[r];                                   // (a power of two)
+    }
+    __syncthreads();
+    float *const red = reinterpret_cast<float *>(lds);
+    if (q < P) {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int t = 0; t < TJ; t++) red[(wave * MV + 4 * q + r) * (16 * TJ) + 16 * t + i] = acc[t][r] * inv[r];
+    }
+    __syncthreads();
+    for (int o = tid; o < MV * 16 * TJ; o += (int)blockDim.x) {
+        const int v = o / (16 * TJ), c = o % (16 * TJ);
+        if (v >= m || n0 + c >= n) continue;
+        float sum = 0.0f;
+        for (int wv = 0; wv < waves; wv++) sum += red[(wv * MV + v) * (16 * TJ) + c];
+        y[(size_t)v * n + n0 + c] = sum;
     }
 }
 

@@ -1,5 +1,5 @@
 """GPU: the matrix-core kernels for few rows of activations (short prompts through rfq_gemm_f16 and
-rfq_gemm_f16_arranged) at the edges of their tiles: rows per operand (16), rows
+rfq_gemm_f16_arranged, decode batches of 2 to 8 through rfq_gemv) at the edges of their tiles: rows per operand (16), rows
 per slice (128), weight rows per workgroup (16 and 32), 128-element units of k and their remainders, more and fewer units
 than wavefronts; against the float64 contraction of the decoded weights."""
 import numpy as np
@@ -43,3 +43,73 @@ def test_prompts(fmt, m, n, k, oracle, cuda):
         assert_close(got.cpu().numpy(), want, f"{Q.NAMES[fmt]} {m}x{n}x{k} {what}", tol=TOL, plain_tol=2e-4)
     f16 = ops.gemm_f16(fmt, dw, da, n, k)
     assert torch.equal(f16, plain.half())
+
+
+BATCH_FORMATS = FORMATS + [Q.MXFP4, Q.MXFP6_E2M3]
+
+
+@pytest.mark.parametrize("fmt", BATCH_FORMATS)
+@pytest.mark.parametrize("m,n,k", [(2, 4200, 544), (3, 1029, 1024), (4, 3100, 3072), (5, 15, 256), (5, 17, 32), (6, 33, 96), (7, 5201, 480), (8, 64, 4128),
+                                   (8, 13400, 768), (5, 200, 13824)])
+def test_decode_batches(fmt, m, n, k, oracle, cuda):
+    import torch
+    from rocmforge_amd import ops
+    if fmt in FORMATS:
+        n, k = shape_of(fmt, n, k)
+    w = Q.make_weights(fmt, n, k, seed=fmt + m)
+    x = np.random.default_rng(m * n).standard_normal((m, k)).astype(np.float32)
+    got = ops.gemv(fmt, torch.from_numpy(w).to(cuda), torch.from_numpy(x).to(cuda), n, k)
+    want = x.astype(np.float64) @ weights_of(oracle, fmt, w, n, k).T
+    assert_close(got.cpu().numpy(), want, f"{Q.NAMES[fmt]} {m}x{n}x{k}", tol=TOL, plain_tol=2e-4)
+
+
+@pytest.mark.parametrize("fmt", [Q.Q4_0, Q.GGUF_Q4_K, Q.Q6_K, Q.MXFP4])
+def test_decode_batch_of_any_magnitude(fmt, oracle, cuda):
+    """The fp16 parts of x follow its magnitude: vectors of very different size, sizes that grow and shrink by powers of
+    ten along k, zeros, subnormals; an infinity or a NaN turns its own vector's outputs into NaN and no other's."""
+    import torch
+    from rocmforge_amd import ops
+    m, n, k = 8, 48, 2048
+    w = Q.make_weights(fmt, n, k, seed=5)
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((m, k))
+    x[0] *= 1e30
+    x[1] *= 1e-30
+    x[2] *= 10.0 ** np.linspace(-8, 8, k)
+    x[3] *= 10.0 ** np.linspace(8, -8, k)
+    x[4, : k // 2] = 0
+    x[5] = 0
+    x[6] *= 1e-41
+    x = x.astype(np.float32)
+    dw = torch.from_numpy(w).to(cuda)
+    got = ops.gemv(fmt, dw, torch.from_numpy(x).to(cuda), n, k).cpu().numpy().astype(np.float64)
+    w64 = weights_of(oracle, fmt, w, n, k)
+    want = x.astype(np.float64) @ w64.T
+    for v in (0, 1, 2, 3, 4, 5, 7):
+        assert_close(got[v], want[v], f"{Q.NAMES[fmt]} vector {v}", tol=TOL, plain_tol=2e-4)
+    # (subnormal x: 2^-149 steps in the products' own sums)
+    assert np.all(np.abs(got[6] - want[6]) <= 2e-5 * np.abs(want[6]).max() + 64 * 2.0 ** -149)
+    for bad in (np.inf, -np.inf, np.nan):
+        y = x.copy()
+        y[2, 700] = bad
+        again = ops.gemv(fmt, dw, torch.from_numpy(y).to(cuda), n, k).cpu().numpy().astype(np.float64)
+        assert np.isnan(again[2]).all()
+        keep = [0, 1, 3, 4, 5, 6, 7]
+        assert np.array_equal(again[keep], got[keep])
+
+
+@pytest.mark.parametrize("fmt", [Q.MXFP4, Q.MXFP6_E2M3])
+def test_mx_exponents_beyond_the_clamp(fmt, oracle, cuda):
+    """Blocks whose exponent byte is 1..127 (the reference clamps value * 2^e) beside -128 and ordinary ones."""
+    import torch
+    from rocmforge_amd import ops
+    m, n, k = 8, 64, 1024
+    w = Q.make_weights(fmt, n, k, seed=9).copy()
+    blocks = w.reshape(-1, Q.BLOCK_BYTES[fmt])
+    rng = np.random.default_rng(10)
+    blocks[:, 0] = rng.choice(np.array([-128, -3, -1, 0, 1, 2, 3, 4, 5, 6, 127], np.int8), blocks.shape[0]).view(np.uint8)
+    blocks[:, 1:] = rng.integers(0, 256, blocks[:, 1:].shape, dtype=np.uint8)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    got = ops.gemv(fmt, torch.from_numpy(w).to(cuda), torch.from_numpy(x).to(cuda), n, k)
+    want = x.astype(np.float64) @ weights_of(oracle, fmt, w, n, k).T
+    assert_close(got.cpu().numpy(), want, Q.NAMES[fmt], tol=TOL, plain_tol=2e-4)
