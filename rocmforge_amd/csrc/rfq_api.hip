@@ -347,6 +347,8 @@ int rfq_rms_norm_gemv(int fmt, const void *d_w, size_t w_bytes, const float *d_x
     if (!d_scratch) return fail(RFQ_E_BADARG, "rfq_rms_norm_gemv: m=%d k=%d needs d_scratch (m * k floats)", m, k);
     if (k % 4 != 0 || !aligned16(d_x) || !aligned16(d_norm_weight) || !aligned16(d_scratch))
         return fail(RFQ_E_BADARG, "rfq_rms_norm_gemv: x, norm weight and scratch must be 16-byte aligned, k a multiple of 4");
+    rc = launch_skinny_gemv_fused(fmt, (const uint8_t *)d_w, nullptr, d_x, d_norm_weight, eps, d_y, m, n, k, s);
+    if (rc != RFQ_E_UNSUPPORTED) return rc;
     rc = launch_rms_norm(RFQ_TABLE_F32, d_x, d_norm_weight, d_scratch, m, k, eps, s);
     if (rc != RFQ_OK) return rc;
     return launch_gemv(fmt, (const uint8_t *)d_w, d_scratch, d_y, m, n, k, s);
@@ -392,10 +394,14 @@ int rfq_mlp_swiglu(int fmt_gate_up, const void *d_gate_w, const void *d_up_w, si
         rc = launch_gemv_fused(fmt_gate_up, (const uint8_t *)d_gate_w, (const uint8_t *)d_up_w, d_x, d_norm_weight, eps, h,
                                intermediate_size, hidden_size, s);
     if (rc == RFQ_E_UNSUPPORTED) {
+        if (d_norm_weight && (hidden_size % 4 != 0 || !aligned16(d_x) || !aligned16(d_norm_weight)))
+            return fail(RFQ_E_BADARG, "rfq_mlp_swiglu: x and norm weight must be 16-byte aligned, hidden_size a multiple of 4");
+        rc = launch_skinny_gemv_fused(fmt_gate_up, (const uint8_t *)d_gate_w, (const uint8_t *)d_up_w, d_x, d_norm_weight, eps, h, m,
+                                      intermediate_size, hidden_size, s);
+    }
+    if (rc == RFQ_E_UNSUPPORTED) {
         const float *xin = d_x;
         if (d_norm_weight) {
-            if (hidden_size % 4 != 0 || !aligned16(d_x) || !aligned16(d_norm_weight))
-                return fail(RFQ_E_BADARG, "rfq_mlp_swiglu: x and norm weight must be 16-byte aligned, hidden_size a multiple of 4");
             rc = launch_rms_norm(RFQ_TABLE_F32, d_x, d_norm_weight, xn, m, hidden_size, eps, s);
             if (rc != RFQ_OK) return rc;
             xin = xn;

@@ -114,17 +114,27 @@ RFQ_GEMV_PART_DECL(3)
 constexpr int GEMV_TRACE_STAMPS = 20;                    // readings per wavefront, see WaveTrace in rfq_gemv.hip
 int launch_gemv_traced(int fmt, const uint8_t *d_w, const float *d_x, float *d_y, int n, int k, unsigned long long *d_trace,
                        size_t capacity_waves, int *waves, hipStream_t s);
-// Few rows of activations on the matrix cores (rfq_skinny.hip, compiled in four parts): float32 x with m <= 8 (w2 != nullptr:
-// two matrices of one shape that share x), or float16 a (rows or arranged).  The caller has checked formats, shapes and
-// alignment (weights on multiples of 4, activations of 16).
-int launch_skinny_gemv(int fmt, const uint8_t *w, const uint8_t *w2, const float *x, float *y, float *y2, int m, int n, int k,
-                       hipStream_t s);
+// Few rows of activations on the matrix cores (rfq_skinny.hip, compiled in four parts): float32 x with m <= 8 (SkinnyGemv;
+// w2 != nullptr: y = swiglu over two matrices of one shape, norm_w != nullptr: x is RMSNorm(x) * norm_w), or float16 a (rows
+// or arranged).  The caller has checked formats, shapes and alignment (weights on multiples of 4, activations and the norm
+// weight of 16).
+struct SkinnyGemv {
+    const uint8_t *w, *w2;
+    const float *x, *norm_w;
+    float eps;
+    float *y;
+    int m, n, k;
+};
+int launch_skinny_gemv(int fmt, const SkinnyGemv &c, hipStream_t s);
+// Whether the above is the faster way for rows of x [m, k] and this matrix (m >= 2), alone and with what it takes along.
+bool few_rows_ahead(int fmt, int m, int n, int ku, bool batch_fits);
+int launch_skinny_gemv_fused(int fmt, const uint8_t *d_w, const uint8_t *d_w2, const float *d_x, const float *d_norm_w, float eps, float *d_y,
+                             int m, int n, int k, hipStream_t s);
 int launch_skinny_gemm(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, bool f16_out, int m, int n, int k,
                        hipStream_t s);
 bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts);
 #define RFQ_SKINNY_PART_DECL(N)                                                                                              \
-    int launch_skinny_gemv_part##N(int fmt, const uint8_t *w, const uint8_t *w2, const float *x, float *y, float *y2, int m,  \
-                                   int n, int k, hipStream_t s);                                                             \
+    int launch_skinny_gemv_part##N(int fmt, const SkinnyGemv &c, hipStream_t s);                                             \
     int launch_skinny_gemm_part##N(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, int f16_out, int m,   \
                                    int n, int k, hipStream_t s);
 RFQ_SKINNY_PART_DECL(0)

@@ -2398,33 +2398,6 @@ int run_generic_m(const uint8_t *w, const float *x, float *y, int m, int n, int 
     }
 }
 
-// Whether a batch goes through the matrix-core kernel for few rows (rfq_skinny.hip) instead of the integer-dot batch kernel
-// (batch_fits) or, where a format or row length has none, one decode launch per vector or the one-row-per-wavefront
-// kernel.  Its time hardly depends on m; measured on 512..14336 rows of 768..13824 for every format (us, there / here):
-//   m >= 5: always (Q8_0 4096 x 4096 m = 8 11.4 / 9.7, Q4_0 13.0 / 8.8, Q4_K 14336 x 4096 30.7 / 23.6, GGUF_Q6_K
-//     4096 x 13824 82 / 23, Q6_K 14336 x 4096 82 / 23, MXFP6 4096 x 4096 42.6 / 12.4);
-//   m = 3, 4 against the batch kernel (which takes three as four): rows longer than 3000 with 12 or more of them per CU, up
-//     to 24 for the formats whose batch kernel streams well at many rows (4096 x 4096: Q8_0 9.5 / 8.3, GGUF_Q4_K 8.7 / 7.6;
-//     4096 x 8192 GGUF_Q6_K 12.9 / 14; 14336 x 4096: GGUF_Q4_0 18.4 / 15.7, but Q8_0 19.9 / 22.3, Q4_K 17.8 / 21.8);
-//   m = 3, 4 without a batch kernel: from four rows per CU on, or long rows (Q6_K 14336 x 4096 m = 4 42 / 21);
-//   m = 2: only without a batch kernel, for as many rows as make one launch cheaper than two (MXFP4 8192 x 4096 13.9 / 11.2;
-//     512 x 4096 5.8 / 7.0).  Q8_0 without one always (4096 x 13824 35 / 20).
-bool few_rows_ahead(int fmt, int m, int n, int ku, bool batch_fits)
-{
-    const int cus = device_cu_count();
-    if (m >= 5) return true;
-    const bool q8 = fmt == RFQ_Q8_0 || fmt == RFQ_GGUF_Q8_0;
-    if (m >= 3) {
-        if (batch_fits)
-            return ku >= 96 && n >= cus * 12 && (n <= cus * 24 || fmt == RFQ_Q4_0 || fmt == RFQ_GGUF_Q4_0 || fmt == RFQ_GGUF_Q4_K);
-        return q8 || n >= cus * 4 || ku > 256;
-    }
-    if (batch_fits) return false;
-    if (q8) return true;
-    if (fmt == RFQ_MXFP6_E2M3) return ku <= 32 && n >= cus * 12;
-    return n > cus * 16 || (n >= cus * 12 && ku <= 256);
-}
-
 template <int FMT>
 int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStream_t s)
 {
@@ -2437,7 +2410,7 @@ int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStre
     const bool batch_fits = HasIdotBatch<FMT>::value && ku > 32 && ku <= 256;
     if (m > 1 && (reinterpret_cast<uintptr_t>(w) & 3u) == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && few_rows_ahead(FMT, m, n, ku, batch_fits)) {
         note_kernel("gemv_skinny_kernel<%s>", FMT, 0, 0, 0);
-        return launch_skinny_gemv(FMT, w, nullptr, x, y, nullptr, m, n, k, s);
+        return launch_skinny_gemv(FMT, SkinnyGemv{w, nullptr, x, nullptr, 0.0f, y, m, n, k}, s);
     }
     if (batch_fits && m > 1) {
         // the prepared vectors of a launch live in LDS (112 bytes per unit and vector): a batch that
@@ -2560,6 +2533,55 @@ int launch_gemv(int fmt, const uint8_t *d_w, const float *d_x, float *d_y, int m
 #endif
     default: return fail(RFQ_E_BADARG, "rfq_gemv: unknown format %d", fmt);
     }
+}
+
+// Whether a batch goes through the matrix-core kernel for few rows (rfq_skinny.hip) instead of the integer-dot batch kernel
+// (batch_fits) or, where a format or row length has none, one decode launch per vector or the one-row-per-wavefront
+// kernel.  Its time hardly depends on m; measured on 512..14336 rows of 768..13824 for every format (us, there / here):
+//   m >= 5: always (Q8_0 4096 x 4096 m = 8 11.4 / 9.7, Q4_0 13.0 / 8.8, Q4_K 14336 x 4096 30.7 / 23.6, GGUF_Q6_K
+//     4096 x 13824 82 / 23, Q6_K 14336 x 4096 82 / 23, MXFP6 4096 x 4096 42.6 / 12.4);
+//   m = 3, 4 against the batch kernel (which takes three as four): rows longer than 3000 with 12 or more of them per CU, up
+//     to 24 for the formats whose batch kernel streams well at many rows (4096 x 4096: Q8_0 9.5 / 8.3, GGUF_Q4_K 8.7 / 7.6;
+//     4096 x 8192 GGUF_Q6_K 12.9 / 14; 14336 x 4096: GGUF_Q4_0 18.4 / 15.7, but Q8_0 19.9 / 22.3, Q4_K 17.8 / 21.8);
+//   m = 3, 4 without a batch kernel: from four rows per CU on, or long rows (Q6_K 14336 x 4096 m = 4 42 / 21);
+//   m = 2: only without a batch kernel, for as many rows as make one launch cheaper than two (MXFP4 8192 x 4096 13.9 / 11.2;
+//     512 x 4096 5.8 / 7.0).  Q8_0 without one always (4096 x 13824 35 / 20).
+bool few_rows_ahead(int fmt, int m, int n, int ku, bool batch_fits)
+{
+    const int cus = device_cu_count();
+    if (m >= 5) return true;
+    const bool q8 = fmt == RFQ_Q8_0 || fmt == RFQ_GGUF_Q8_0;
+    if (m >= 3) {
+        if (batch_fits)
+            return ku >= 96 && n >= cus * 12 && (n <= cus * 24 || fmt == RFQ_Q4_0 || fmt == RFQ_GGUF_Q4_0 || fmt == RFQ_GGUF_Q4_K);
+        return q8 || n >= cus * 4 || ku > 256;
+    }
+    if (batch_fits) return false;
+    if (q8) return true;
+    if (fmt == RFQ_MXFP6_E2M3) return ku <= 32 && n >= cus * 12;
+    return n > cus * 16 || (n >= cus * 12 && ku <= 256);
+}
+
+// The same for two to eight vectors through the few-row kernel: RFQ_E_UNSUPPORTED (without an error text) where the
+// separate steps are ahead.  Besides where the plain batch takes that kernel it is taken where the launches it saves (about
+// 3 us for the norm, 8 for norm, second projection and activation) are worth more than the difference: a norm up to 16
+// or 20 rows per CU, two matrices up to 40 (two vectors) or at any size (three and more).
+int launch_skinny_gemv_fused(int fmt, const uint8_t *d_w, const uint8_t *d_w2, const float *d_x, const float *d_norm_w, float eps, float *d_y,
+                             int m, int n, int k, hipStream_t s)
+{
+    const int cf = canonical_format(fmt), ku = k / 32, cus = device_cu_count();
+    if (m < 2 || m > 8 || gemv_part_of(cf) < 0 || fmt_mm_variant(fmt)) return RFQ_E_UNSUPPORTED;
+    const uintptr_t ws = reinterpret_cast<uintptr_t>(d_w) | reinterpret_cast<uintptr_t>(d_w2);
+    const uintptr_t xs = reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_norm_w);
+    if ((ws & 3u) != 0 || (xs & 15u) != 0) return RFQ_E_UNSUPPORTED;
+    const bool per_vector = cf == RFQ_Q6_K || cf == RFQ_MXFP4 || cf == RFQ_MXFP6_E2M3;
+    const bool batch_fits = !per_vector && ku > 32 && ku <= 256;
+    // (with two vectors the batch kernel of these two formats is further ahead: GGUF_Q6_K 2 x 3072 -> 4864 12.5 / 14.2 us)
+    const int norm_rows = cus * (m >= 3 ? 20 : cf == RFQ_GGUF_Q6_K || cf == RFQ_Q4_K ? 8 : 16);
+    const bool taken = d_w2 != nullptr ? m >= 3 || n <= cus * 20 || few_rows_ahead(cf, m, n, ku, batch_fits)
+                                       : n <= norm_rows || few_rows_ahead(cf, m, n, ku, batch_fits);
+    if (!taken) return RFQ_E_UNSUPPORTED;
+    return launch_skinny_gemv(cf, SkinnyGemv{d_w, d_w2, d_x, d_norm_w, eps, d_y, m, n, k}, s);
 }
 
 // One launch for RMSNorm -> GEMV (norm_w != nullptr) and / or two GEMVs sharing

@@ -33,36 +33,40 @@ int waves_for(int k, int most)
     return units < most ? units : most;
 }
 
-template <int FMT, int TJ, int MV, int D, int WAVES>
-int gemv_cfg(const uint8_t *w, const uint8_t *w2, const float *x, float *y, float *y2, int m, int n, int k, hipStream_t s)
+constexpr int GEMV_WAVES = 8;
+
+template <int FMT, int TJ, int MV, bool NORM>
+int gemv_cfg(const SkinnyGemv &c, hipStream_t s)
 {
-    if constexpr (gemv_lds<TJ, MV>(WAVES) > 64 * 1024) {
-        static std::once_flag once;
-        static hipError_t err = hipSuccess;
-        std::call_once(once, [] {
-            err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_skinny_kernel<FMT, TJ, MV, D, WAVES>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, gemv_lds<TJ, MV>(WAVES));
-        });
-        if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(gemv_skinny_kernel)");
-    }
-    const int waves = waves_for(k, WAVES);
+    const int waves = waves_for(c.k, GEMV_WAVES);
+    constexpr int D = 2;                                          // units of W in flight per wavefront
+    static_assert(gemv_lds<TJ, MV>(GEMV_WAVES) <= 64 * 1024, "LDS a launch gets without asking");
     const size_t lds = (size_t)gemv_lds<TJ, MV>(waves);
-    hipLaunchKernelGGL((gemv_skinny_kernel<FMT, TJ, MV, D, WAVES>), dim3((n + 16 * TJ - 1) / (16 * TJ), w2 != nullptr ? 2 : 1),
-                       dim3(64 * waves), lds, s, w, x, y, m, n, k, w2, y2);
+    const int rows = c.w2 != nullptr ? 8 * TJ : 16 * TJ;
+    hipLaunchKernelGGL((gemv_skinny_kernel<FMT, TJ, MV, D, GEMV_WAVES, NORM>), dim3((c.n + rows - 1) / rows), dim3(64 * waves), lds, s, c.w, c.x,
+                       c.y, c.m, c.n, c.k, c.w2, c.norm_w, c.eps);
     RFQ_LAUNCH_CHECK("gemv_skinny_kernel");
     return RFQ_OK;
 }
 
 // Row tiles per workgroup: one up to 20 rows per CU, where a second tile would leave CUs without a workgroup, then two, four
 // from 52 on: every workgroup converts all of x (Q4_0, 8 vectors, k = 4096: n = 4096 8.8 / 10.7 / 14.5 us with 1 / 2 / 4,
-// n = 8192 12.7 / 11.5 / 14.9, n = 14336 23.4 / 18.8 / 18.4; MXFP4 n = 14336 22.8 / 22.1 / 18.8).
-template <int FMT, int MV>
-int gemv_fmt(const uint8_t *w, const uint8_t *w2, const float *x, float *y, float *y2, int m, int n, int k, hipStream_t s)
+// n = 8192 12.7 / 11.5 / 14.9, n = 14336 23.4 / 18.8 / 18.4; MXFP4 n = 14336 22.8 / 22.1 / 18.8).  Two matrices take an even
+// number.
+template <int FMT, int MV, bool NORM>
+int gemv_rows(const SkinnyGemv &c, hipStream_t s)
 {
-    const int rows = w2 != nullptr ? 2 * n : n, cus = device_cu_count();
-    if (rows >= 52 * cus) return gemv_cfg<FMT, 4, MV, 2, 8>(w, w2, x, y, y2, m, n, k, s);
-    if (rows > 20 * cus) return gemv_cfg<FMT, 2, MV, 2, 8>(w, w2, x, y, y2, m, n, k, s);
-    return gemv_cfg<FMT, 1, MV, 2, 8>(w, w2, x, y, y2, m, n, k, s);
+    const int cus = device_cu_count();
+    const long rows = c.w2 != nullptr ? 2L * c.n : c.n;
+    if (rows >= 52L * cus) return gemv_cfg<FMT, 4, MV, NORM>(c, s);
+    if (rows > 20L * cus || c.w2 != nullptr) return gemv_cfg<FMT, 2, MV, NORM>(c, s);
+    return gemv_cfg<FMT, 1, MV, NORM>(c, s);
+}
+
+template <int FMT> int gemv_fmt(const SkinnyGemv &c, hipStream_t s)
+{
+    if (c.norm_w != nullptr) return c.m <= 4 ? gemv_rows<FMT, 4, true>(c, s) : gemv_rows<FMT, 8, true>(c, s);
+    return c.m <= 4 ? gemv_rows<FMT, 4, false>(c, s) : gemv_rows<FMT, 8, false>(c, s);
 }
 
 template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES>
@@ -153,10 +157,9 @@ int gemm_fmt(const uint8_t *w, const uint8_t *a, bool arranged, void *y, int f16
         return fail(RFQ_E_UNSUPPORTED, "no few-row kernel for format %d in this part of the build", fmt); \
     }(std::integral_constant<int, RFQ_SKINNY_PART>{})
 
-int RFQ_SKINNY_CAT(launch_skinny_gemv_part, RFQ_SKINNY_PART)(int fmt, const uint8_t *w, const uint8_t *w2, const float *x, float *y,
-                                                             float *y2, int m, int n, int k, hipStream_t s)
+int RFQ_SKINNY_CAT(launch_skinny_gemv_part, RFQ_SKINNY_PART)(int fmt, const SkinnyGemv &c, hipStream_t s)
 {
-#define RFQ_SKINNY_GEMV(F) (m <= 4 ? gemv_fmt<F, 4>(w, w2, x, y, y2, m, n, k, s) : gemv_fmt<F, 8>(w, w2, x, y, y2, m, n, k, s))
+#define RFQ_SKINNY_GEMV(F) gemv_fmt<F>(c, s)
     if constexpr (skinny_part_of(RFQ_MXFP4) == RFQ_SKINNY_PART)
         if (fmt == RFQ_MXFP4) return RFQ_SKINNY_GEMV(RFQ_MXFP4);
     if constexpr (skinny_part_of(RFQ_MXFP6_E2M3) == RFQ_SKINNY_PART)
@@ -196,13 +199,13 @@ bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts)
     return few < tiled;
 }
 
-int launch_skinny_gemv(int fmt, const uint8_t *w, const uint8_t *w2, const float *x, float *y, float *y2, int m, int n, int k, hipStream_t s)
+int launch_skinny_gemv(int fmt, const SkinnyGemv &c, hipStream_t s)
 {
     switch (skinny_part_of(fmt)) {
-    case 0: return launch_skinny_gemv_part0(fmt, w, w2, x, y, y2, m, n, k, s);
-    case 1: return launch_skinny_gemv_part1(fmt, w, w2, x, y, y2, m, n, k, s);
-    case 2: return launch_skinny_gemv_part2(fmt, w, w2, x, y, y2, m, n, k, s);
-    case 3: return launch_skinny_gemv_part3(fmt, w, w2, x, y, y2, m, n, k, s);
+    case 0: return launch_skinny_gemv_part0(fmt, c, s);
+    case 1: return launch_skinny_gemv_part1(fmt, c, s);
+    case 2: return launch_skinny_gemv_part2(fmt, c, s);
+    case 3: return launch_skinny_gemv_part3(fmt, c, s);
     default: return fail(RFQ_E_UNSUPPORTED, "no few-row kernel for format %d", fmt);
     }
 }

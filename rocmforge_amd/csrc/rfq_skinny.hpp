@@ -68,6 +68,12 @@ __device__ __forceinline__ void spread4(float v, float (&out)[4])
     out[0] = __uint_as_float(a); out[1] = __uint_as_float(b); out[2] = __uint_as_float(c); out[3] = __uint_as_float(d);
 }
 
+__device__ __forceinline__ void spread4u(uint32_t v, uint32_t (&out)[4])
+{
+    out[0] = out[1] = out[2] = out[3] = v;
+    transpose4(out[0], out[1], out[2], out[3]);
+}
+
 __device__ __forceinline__ uint32_t add2h(uint32_t bits, float bias)
 {
     v2h h;
@@ -111,7 +117,7 @@ template <int NW> __device__ __forceinline__ void load_dwords(const uint8_t *a, 
     if (i < NW) d[i] = *reinterpret_cast<const uint32_t *>(a + 4 * i);
 }
 // Which eight elements of a group lane row q holds, and in which order its four operand dwords hold them.
-enum { OCTET, OCTET_SWAPPED, HALVES, HALVES_SWAPPED };           // 8q..  |  8q'..  |  4q.. and 16+4q..  |  4q'.. and 16+4q'..   (q' = q with its bits swapped)
+enum { OCTET, OCTET_SWAPPED, HALVES };                           // 8q..  |  8q'.. (q' = q with its bits swapped)  |  4q.. and 16+4q..
 enum { P04, P01, P02, P26 };                                     // (0,4)(1,5)(2,6)(3,7) | (0,1)(2,3)(4,5)(6,7) | (0,2)(1,3)(4,6)(5,7) | (0,2)(4,6)(1,3)(5,7)
 
 // W<FMT>: load() fetches the dwords r[] that lane 4 * i + g holds of group g of the 128-element unit `u` of row i (four
@@ -212,19 +218,19 @@ template <int FMT> struct W8 {                                   // Q8_0 (f32 sc
 template <> struct W<RFQ_Q8_0> : W8<RFQ_Q8_0> {};
 template <> struct W<RFQ_GGUF_Q8_0> : W8<RFQ_GGUF_Q8_0> {};
 
+// What the four lanes of a row share (scales, mins) is fetched as one dword per lane and spread: one load and one move to the
+// operand lanes instead of three or four of each.
 template <> struct W<RFQ_Q4_K> {                                 // 256-byte layout: 8 f16 scales, 8 i8 mins, nibbles at 32 + 28 * sb
-    static constexpr int ORDER = OCTET, PAIRS = P04, NR = 7;
+    static constexpr int ORDER = OCTET, PAIRS = P04, NR = 5;
     static constexpr bool MINS = true, SPLIT16 = false;
     struct U4 { uint32_t v[4]; };
-    uint32_t r[NR], q[4];
+    uint32_t r[NR], q[4], hd[4];
     __device__ __forceinline__ void load(const uint8_t *row, int u, int g)
     {
         const uint8_t *blk = row + (uint32_t)(u >> 1) * 256u;
         const int h = u & 1;
-        uint32_t s[2];
-        load_dwords<2>(blk + 8 * h, s);
-        r[4] = s[0]; r[5] = s[1];
-        r[6] = *reinterpret_cast<const uint32_t *>(blk + 16 + 4 * h);
+        // (lanes 0, 1: two scales each; lanes 2, 3: the unit's four mins)
+        r[4] = *reinterpret_cast<const uint32_t *>(blk + (g < 2 ? 8 * h + 4 * g : 16 + 4 * h));
         const U4 v = ld_once<U4>(blk + 32 + 28 * (4 * h + g));
 #pragma unroll
         for (int i = 0; i < 4; i++) r[i] = v.v[i];
@@ -234,42 +240,45 @@ template <> struct W<RFQ_Q4_K> {                                 // 256-byte lay
 #pragma unroll
         for (int i = 0; i < 4; i++) q[i] = r[i];
         transpose4(q[0], q[1], q[2], q[3]);
+        spread4u(r[4], hd);
     }
     __device__ __forceinline__ v4u frag(int j) const { return v4u{nib2h<0>(q[j], 0.f), nib2h<4>(q[j], 0.f), nib2h<8>(q[j], 0.f), nib2h<12>(q[j], 0.f)}; }
-    __device__ __forceinline__ float sc(int j, int) const { return f16_bits_to_f32((uint16_t)(r[4 + (j >> 1)] >> (16 * (j & 1)))); }
-    __device__ __forceinline__ float mn(int j) const { return (float)(int)(int8_t)(r[6] >> (8 * j)); }
+    __device__ __forceinline__ float sc(int j, int) const { return f16_bits_to_f32((uint16_t)(hd[j >> 1] >> (16 * (j & 1)))); }
+    __device__ __forceinline__ float mn(int j) const { return (float)(int)(int8_t)(hd[2] >> (8 * j)); }
 };
 
 template <> struct W<RFQ_GGUF_Q4_K> {
-    static constexpr int ORDER = OCTET_SWAPPED, PAIRS = P02, NR = 8;
+    static constexpr int ORDER = OCTET_SWAPPED, PAIRS = P02, NR = 5;
     static constexpr bool MINS = true, SPLIT16 = false;
     uint32_t r[NR], q[4];
     uint32_t scb, mnb; float d, dm;
     __device__ __forceinline__ void load(const uint8_t *row, int u, int g)
     {
         const uint8_t *blk = row + (uint32_t)(u >> 1) * 144u;
-        uint32_t a[4], b[4];
-        load_dwords<4>(blk, a);
+        uint32_t b[4];
+        r[4] = *reinterpret_cast<const uint32_t *>(blk + 4 * g);
         load_dwords<4>(blk + 16 + 64 * (u & 1) + 16 * g, b);
 #pragma unroll
-        for (int i = 0; i < 4; i++) { r[i] = b[i]; r[4 + i] = a[i]; }
+        for (int i = 0; i < 4; i++) r[i] = b[i];
     }
     // lane row (q1 q0) holds bytes 16 q0 .. of the unit's 64-element chunk q1; it keeps bytes 16 q0 + 8 q1 .. +8 of both
     __device__ __forceinline__ void open(int u, bool)
     {
+        uint32_t hd[4];
+        spread4u(r[4], hd);
 #pragma unroll
         for (int i = 0; i < 4; i++) q[i] = r[i];
         swap32(q[0], q[2]);
         swap32(q[1], q[3]);
         if ((u & 1) == 0) {
-            scb = r[5] & 0x3F3F3F3Fu;
-            mnb = r[6] & 0x3F3F3F3Fu;
+            scb = hd[1] & 0x3F3F3F3Fu;
+            mnb = hd[2] & 0x3F3F3F3Fu;
         } else {
-            scb = (r[7] & 0x0F0F0F0Fu) | ((r[5] >> 2) & 0x30303030u);
-            mnb = ((r[7] >> 4) & 0x0F0F0F0Fu) | ((r[6] >> 2) & 0x30303030u);
+            scb = (hd[3] & 0x0F0F0F0Fu) | ((hd[1] >> 2) & 0x30303030u);
+            mnb = ((hd[3] >> 4) & 0x0F0F0F0Fu) | ((hd[2] >> 2) & 0x30303030u);
         }
-        d = f16_bits_to_f32((uint16_t)r[4]);
-        dm = -f16_bits_to_f32((uint16_t)(r[4] >> 16));
+        d = f16_bits_to_f32((uint16_t)hd[0]);
+        dm = -f16_bits_to_f32((uint16_t)(hd[0] >> 16));
     }
     __device__ __forceinline__ v4u frag(int j) const
     {
@@ -330,52 +339,57 @@ template <> struct W<RFQ_Q6_K> {
 };
 
 template <> struct W<RFQ_GGUF_Q6_K> {
-    static constexpr int ORDER = HALVES_SWAPPED, PAIRS = P01, NR = 13;
+    static constexpr int ORDER = HALVES, PAIRS = P01, NR = 10;
     static constexpr bool MINS = false, SPLIT16 = true;
     uint32_t r[NR];
-    uint32_t a[2], b[2], c[2], s[2]; float d;
-    // Eight bytes at p, of which o (0 or 2) lie in the dword before: three aligned dwords, or two and the second again
-    static __device__ __forceinline__ void piece(const uint8_t *p, uint32_t o, uint32_t *out)
-    {
-        uint32_t v[2];
-        load_dwords<2>(p - o, v);
-        out[0] = v[0]; out[1] = v[1];
-        out[2] = *reinterpret_cast<const uint32_t *>(p - o + (o ? 8 : 4));
-    }
+    uint32_t q[4], c[2], s[2]; float d;
+    // Blocks start on multiples of 2 and every piece on a multiple of 4 from there: the aligned dwords around a piece, o (0
+    // or 2) bytes before it; the last is read only where it holds a byte of the piece.
     __device__ __forceinline__ void load(const uint8_t *row, int u, int g)
     {
         const uint8_t *blk = row + (uint32_t)(u >> 1) * 210u;
-        const int half = u & 1;
+        const int half = u & 1, gs = ((g & 1) << 1) | (g >> 1);
         const uint32_t o = (uint32_t)(reinterpret_cast<uintptr_t>(blk) & 3u);
-        piece(blk + 64 * half + 8 * g, o, r);
-        piece(blk + 64 * half + 32 + 8 * g, o, r + 3);
-        piece(blk + 128 + 32 * half + 8 * g, o, r + 6);
-        piece(blk + 192 + 8 * half, o, r + 9);
-        r[12] = *reinterpret_cast<const uint16_t *>(blk + 208) | (o << 16);
+        const uint8_t *a = blk - o;
+        uint32_t v[4], t[2];
+        load_dwords<4>(a + 64 * half + 16 * g, v);                // lower nibbles: 16 of the unit's 64 bytes
+        r[4] = *reinterpret_cast<const uint32_t *>(a + 64 * half + 16 * g + (o ? 16 : 12));
+        load_dwords<2>(a + 128 + 32 * half + 8 * gs, t);          // upper bit pairs: 8 of its 32 bytes
+        r[7] = *reinterpret_cast<const uint32_t *>(a + 128 + 32 * half + 8 * gs + (o ? 8 : 4));
+        // lanes 0 .. 2: the dwords of its eight scales, lane 3: d
+        r[8] = *reinterpret_cast<const uint32_t *>(a + (g == 3 ? 208 : 192 + 8 * half + (g == 2 && !o ? 4 : 4 * g)));
+        r[9] = o;
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] = v[i];
+        r[5] = t[0]; r[6] = t[1];
     }
-    // lane row (q1 q0) holds codes 8 q .. 8 q + 7 (of 32) of every group; after the exchange dword 0 holds four codes of
-    // the first 16, dword 1 of the second, both number 2 q0 + q1 of their four
+    // Lower nibbles: lane row (q1 q0) holds bytes 16 q0 .. of part q1 (groups with even / odd number); two exchanges give every
+    // lane row dword q of both halves of both parts.  Bit pairs: lane row (q1 q0) holds dwords 4 q0 + 2 q1, + 1 of eight; one
+    // exchange gives it dword q of both halves.
     __device__ __forceinline__ void open(int, bool)
     {
-        const uint32_t sel = 0x03020100u + __builtin_amdgcn_perm(0u, r[12] >> 16, 0u);
+        const uint32_t sel = 0x03020100u + __builtin_amdgcn_perm(0u, r[9], 0u);
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            a[i] = __builtin_amdgcn_perm(r[i + 1], r[i], sel);
-            b[i] = __builtin_amdgcn_perm(r[i + 4], r[i + 3], sel);
-            c[i] = __builtin_amdgcn_perm(r[i + 7], r[i + 6], sel);
-            s[i] = __builtin_amdgcn_perm(r[i + 10], r[i + 9], sel);
-        }
-        swap32(a[0], a[1]);
-        swap32(b[0], b[1]);
-        swap32(c[0], c[1]);
-        d = f16_bits_to_f32((uint16_t)r[12]);
+        for (int i = 0; i < 4; i++) q[i] = __builtin_amdgcn_perm(r[i + 1], r[i], sel);
+#pragma unroll
+        for (int i = 0; i < 2; i++) c[i] = __builtin_amdgcn_perm(r[i + 6], r[i + 5], sel);
+        swap32(q[0], q[2]);
+        swap32(q[1], q[3]);
+        swap16(q[0], q[1]);
+        swap16(q[2], q[3]);
+        swap16(c[0], c[1]);
+        uint32_t hd[4];
+        spread4u(r[8], hd);
+        s[0] = __builtin_amdgcn_perm(hd[1], hd[0], sel);
+        s[1] = __builtin_amdgcn_perm(hd[2], hd[1], sel);
+        d = f16_bits_to_f32((uint16_t)(hd[3] >> (8u * r[9])));
     }
     __device__ __forceinline__ v4u frag(int j) const
     {
         v4u o;
 #pragma unroll
         for (int e = 0; e < 2; e++) {
-            const uint32_t l = (((j & 1) ? b[e] : a[e]) >> (4 * (j >> 1))) & 0x0F0F0F0Fu;
+            const uint32_t l = (q[2 * (j & 1) + e] >> (4 * (j >> 1))) & 0x0F0F0F0Fu;
             const uint32_t t = (j < 2 ? c[e] << (4 - 2 * j) : c[e] >> (2 * j - 4)) & 0x30303030u;
             uint32_t p, r2;
             bytes2h(l | t, -32.f, p, r2);
@@ -502,7 +516,7 @@ template <int FMT> __device__ __forceinline__ W<FMT> placed(const W<FMT> &raw, i
 
 __device__ __forceinline__ int row_part(int order, int q)         // the number of the octet / quarter-half of lane row q
 {
-    return (order == OCTET_SWAPPED || order == HALVES_SWAPPED) ? ((q & 1) << 1) | (q >> 1) : q;
+    return order == OCTET_SWAPPED ? ((q & 1) << 1) | (q >> 1) : q;
 }
 
 template <int PAIRS> __device__ __forceinline__ constexpr int pair_of(int r, int h)  // element h of operand dword r
@@ -541,39 +555,43 @@ __device__ __forceinline__ void contract(const v4u &xa, const v4u &wf, v4f (&d)[
 constexpr int MAX_WAVES = 16;
 
 // ---- float32 x, m <= 8 -----------------------------------------------------------------------------------------------
-// blockDim = 64 * waves; blockIdx.y: the second of two matrices of the same shape that share x (w2, y2), when there are two.
+// blockDim = 64 * waves.  w2 != nullptr (TJ even): the odd row tiles come from w2, a second matrix of the same shape (gate and
+// up projections), and y[j] = swiglu(row j of w, row j of w2) as the reference defines it (kernels/swiglu.hip:40-62).  NORM:
+// x is RMSNorm(x) * norm_w (kernels/rms_norm.hip:40-84): x * norm_w is multiplied and the vector's factor
+// 1 / sqrt(mean(x^2) + eps) applied to its results.
 // LDS: per wavefront x_bytes for its unit of x as fp16 parts (plane hi, plane lo; vector; operand
 // order), later the wavefronts' results.
 // x goes global -> registers (sixteen lanes per vector, eight elements each: consecutive lanes on consecutive bytes) ->
 // two fp16 parts -> LDS -> operands: every element is converted once per workgroup and unit.
 constexpr int XROW = 256 + 16;                                    // bytes of a vector's 128 elements, bank-skewed
 template <int MV> constexpr int x_bytes() { return 2 * MV * XROW; }
-template <int TJ, int MV> constexpr int gemv_lds(int waves) { return waves * (x_bytes<MV>() > MV * 16 * TJ * 4 ? x_bytes<MV>() : MV * 16 * TJ * 4); }
+template <int TJ, int MV> constexpr int gemv_lds(int waves)
+{
+    // (the results are followed by the vectors' sums of squares)
+    return waves * (x_bytes<MV>() > MV * (16 * TJ + 1) * 4 ? x_bytes<MV>() : MV * (16 * TJ + 1) * 4);
+}
 
 // MV: 4 or 8 vectors, m <= MV.
-template <int FMT, int TJ, int MV, int D, int WAVES>
+template <int FMT, int TJ, int MV, int D, int WAVES, bool NORM>
 __global__ void __launch_bounds__(64 * WAVES)
 gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y, int m, int n, int k,
-                   const uint8_t *__restrict__ w2, float *__restrict__ y2)
+                   const uint8_t *__restrict__ w2, const float *__restrict__ norm_w, float eps)
 {
-    if (blockIdx.y != 0) {
-        w = w2;
-        y = y2;
-    }
     typedef W<FMT> WF;
     constexpr int P = MV / 4;                                     // octets of x per lane and unit
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
     const int groups = k >> 5, units = (groups + 3) >> 2;
-    const int n0 = blockIdx.x * (16 * TJ);
+    const bool glu = TJ >= 2 && w2 != nullptr;
+    const int n0 = blockIdx.x * (glu ? 8 * TJ : 16 * TJ);
     const size_t row_bytes = (size_t)(k / Fmt<FMT>::BE) * Fmt<FMT>::BB;
     const uint8_t *row[TJ];                                       // (weights: lane 4 * i + g fetches group g of row i)
     const int lg = lane & 3, from4 = 4 * (4 * i + q);
 #pragma unroll
     for (int t = 0; t < TJ; t++) {
-        const int r = n0 + 16 * t + (lane >> 2);
-        row[t] = w + (size_t)(r < n ? r : n - 1) * row_bytes;
+        const int r = n0 + 16 * (glu ? t >> 1 : t) + (lane >> 2);
+        row[t] = (glu && (t & 1) ? w2 : w) + (size_t)(r < n ? r : n - 1) * row_bytes;
     }
     // x: octet lane & 15 of the unit, vectors lane >> 4 and, with eight vectors, 4 + (lane >> 4)
     const float *xl[P];
@@ -596,7 +614,7 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
     const uint8_t *const xrd = area + (i & (MV - 1)) * XROW + q * 16;
 
     WF raw[D][TJ];
-    v4f xr[P][2];
+    v4f xr[P][2], nr[2];
     auto load_w = [&](WF (&dst)[TJ], int u) __attribute__((always_inline)) {
         const int uc = u < units ? u : units - 1;
         const int g = 4 * uc + lg < groups ? lg : groups - 1 - 4 * uc;  // (past the row's end: its last group, with scale 0)
@@ -611,7 +629,14 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
             xr[p][0] = *reinterpret_cast<const v4f *>(xl[p] + at);
             xr[p][1] = *reinterpret_cast<const v4f *>(xl[p] + at + 4);
         }
+        if constexpr (NORM) {
+            nr[0] = *reinterpret_cast<const v4f *>(norm_w + 8 * i + at);
+            nr[1] = *reinterpret_cast<const v4f *>(norm_w + 8 * i + at + 4);
+        }
     };
+    float ss[P];                                                  // NORM: this lane's part of its vectors' sums of squares
+#pragma unroll
+    for (int p = 0; p < P; p++) ss[p] = 0.0f;
     float s[P], lim[P];                                           // this lane's vectors: scale, and the largest |x| it can take
 #pragma unroll
     for (int p = 0; p < P; p++) { s[p] = 1.0f; lim[p] = 0.0f; }
@@ -641,6 +666,13 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                     if (Fmt<FMT>::BE < 128 && past) {
 #pragma unroll
                         for (int c = 0; c < 8; c++) e[p][c] = 0.0f;
+                    }
+                    if constexpr (NORM) {
+#pragma unroll
+                        for (int c = 0; c < 8; c++) {
+                            ss[p] = __builtin_fmaf(e[p][c], e[p][c], ss[p]);
+                            e[p][c] *= nr[c >> 2][c & 3];
+                        }
                     }
                     mx[p] = fmaxf(fmaxf(fmaxf(fabsf(e[p][0]), fabsf(e[p][1])), fmaxf(fabsf(e[p][2]), fabsf(e[p][3]))),
                                   fmaxf(fmaxf(fabsf(e[p][4]), fabsf(e[p][5])), fmaxf(fabsf(e[p][6]), fabsf(e[p][7]))));
@@ -759,13 +791,38 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
 #pragma unroll
             for (int t = 0; t < TJ; t++) red[(wave * MV + 4 * q + r) * (16 * TJ) + 16 * t + i] = acc[t][r] * inv[r];
     }
+    float *const squares = red + waves * MV * (16 * TJ);
+    if constexpr (NORM) {
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) ss[p] += __shfl_xor(ss[p], o);
+            if (i == 0) squares[wave * MV + 4 * p + q] = ss[p];
+        }
+    }
     __syncthreads();
-    for (int o = tid; o < MV * 16 * TJ; o += (int)blockDim.x) {
-        const int v = o / (16 * TJ), c = o % (16 * TJ);
-        if (v >= m || n0 + c >= n) continue;
+    auto total = [&](int v, int c) __attribute__((always_inline)) {
         float sum = 0.0f;
         for (int wv = 0; wv < waves; wv++) sum += red[(wv * MV + v) * (16 * TJ) + c];
-        y[(size_t)v * n + n0 + c] = sum;
+        return sum;
+    };
+    const int cols = glu ? 8 * TJ : 16 * TJ;
+    for (int o = tid; o < MV * cols; o += (int)blockDim.x) {
+        const int v = o / cols, c = o % cols;
+        if (v >= m || n0 + c >= n) continue;
+        float rinv = 1.0f;
+        if constexpr (NORM) {
+            float sq = 0.0f;
+            for (int wv = 0; wv < waves; wv++) sq += squares[wv * MV + v];
+            rinv = 1.0f / sqrtf(sq / (float)k + eps);
+        }
+        if (glu) {
+            const int at = 32 * (c >> 4) + (c & 15);
+            const float gate = total(v, at) * rinv, up = total(v, at + 16) * rinv;
+            y[(size_t)v * n + n0 + c] = gate * (up * (1.0f / (1.0f + expf(-up))));
+        } else {
+            y[(size_t)v * n + n0 + c] = total(v, c) * rinv;
+        }
     }
 }
 

@@ -113,3 +113,38 @@ def test_mx_exponents_beyond_the_clamp(fmt, oracle, cuda):
     got = ops.gemv(fmt, torch.from_numpy(w).to(cuda), torch.from_numpy(x).to(cuda), n, k)
     want = x.astype(np.float64) @ weights_of(oracle, fmt, w, n, k).T
     assert_close(got.cpu().numpy(), want, Q.NAMES[fmt], tol=TOL, plain_tol=2e-4)
+
+
+@pytest.mark.parametrize("fmt", BATCH_FORMATS)
+@pytest.mark.parametrize("m,n,k", [(2, 40, 256), (4, 1025, 768), (5, 16, 1280), (8, 5377, 1024)])
+def test_norm_taken_along(fmt, m, n, k, oracle, cuda):
+    import torch
+    from rocmforge_amd import ops
+    w = Q.make_weights(fmt, n, k, seed=fmt + m)
+    rng = np.random.default_rng(m * n)
+    x, nw = rng.standard_normal((m, k)).astype(np.float32) * 3, (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    got = ops.rms_norm_gemv(fmt, torch.from_numpy(w).to(cuda), torch.from_numpy(x).to(cuda), torch.from_numpy(nw).to(cuda), 1e-5, n, k)
+    x64 = x.astype(np.float64)
+    xn = x64 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + 1e-5) * nw
+    assert_close(got.cpu().numpy(), xn @ weights_of(oracle, fmt, w, n, k).T, f"{Q.NAMES[fmt]} {m}x{n}x{k}", tol=TOL, plain_tol=2e-4)
+
+
+@pytest.mark.parametrize("fmt", BATCH_FORMATS)
+@pytest.mark.parametrize("m,hidden,inter,norm", [(2, 256, 512, True), (3, 768, 1792, False), (5, 512, 6912, True), (8, 768, 2304, True)])
+def test_gate_and_up_in_one_launch(fmt, m, hidden, inter, norm, oracle, cuda):
+    import torch
+    from rocmforge_amd import ops
+    gate, up = Q.make_weights(fmt, inter, hidden, seed=fmt), Q.make_weights(fmt, inter, hidden, seed=fmt + 1)
+    down = Q.make_weights(Q.Q8_0, hidden, inter, seed=3)
+    rng = np.random.default_rng(m)
+    x, nw = rng.standard_normal((m, hidden)).astype(np.float32), (1 + 0.1 * rng.standard_normal(hidden)).astype(np.float32)
+    dev = [torch.from_numpy(t).to(cuda) for t in (gate, up, down, x, nw)]
+    got = ops.mlp_swiglu(fmt, dev[0], dev[1], Q.Q8_0, dev[2], dev[3], dev[4] if norm else None, 1e-5, hidden, inter)
+    xn = x.astype(np.float64)
+    if norm:
+        xn = xn / np.sqrt((xn * xn).mean(axis=1, keepdims=True) + 1e-5) * nw
+    g, u = (xn @ weights_of(oracle, fmt, t, inter, hidden).T for t in (gate, up))
+    h = g * (u / (1 + np.exp(-u)))
+    want = h @ weights_of(oracle, Q.Q8_0, down, hidden, inter).T
+    # (the product of two float32 sums, contracted once more: the errors of both add up)
+    assert_close(got.cpu().numpy(), want, f"{Q.NAMES[fmt]} {m}x{hidden}x{inter}", tol=3 * TOL, plain_tol=6e-4)
