@@ -17,7 +17,9 @@ from .quantize import BLOCK_BYTES, BLOCK_ELEMS
 
 
 def _stream() -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # torch.cuda.current_stream().cuda_stream without the Python object around the handle, which took a quarter of a small
+    # call's host time (2.7 us of 9.3; the handle alone 0.2).  The operators' tensors are on a device, so CUDA is initialised.
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def _ptr(t: torch.Tensor) -> C.c_void_p:
