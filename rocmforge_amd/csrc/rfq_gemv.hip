@@ -590,14 +590,12 @@ template <> struct Opened<RFQ_GGUF_Q6_K> {
 };
 template <> struct Unit<RFQ_GGUF_Q6_K> {
     static constexpr bool NEEDS_XSUM = true;
-    Window<8> wl, wh; uint16_t sc2, sc2b, d; int t;
+    Window<8> wl, wh; uint16_t sc2, d; int t;
     template <bool BYTES> __device__ __forceinline__ void load_as(const uint8_t *row, int u)
     {
         const uint8_t *blk = row + (size_t)(u >> 3) * 210;
         const int half = (u >> 2) & 1;
         t = u & 3;
-        // (the scales of quarter t | 2, which shares this unit's bytes: what the paired form multiplies as well)
-        sc2b = ld<uint16_t>(blk + 192 + 8 * half + 2 * (t | 2));
         if constexpr (BYTES) {
             wl.load_bytes<0>(blk + 64 * half + 32 * (t & 1));
             wh.load_bytes<0>(blk + 128 + 32 * half);
@@ -1404,11 +1402,57 @@ template <> struct IUnit<RFQ_GGUF_Q6_K> : Unit<RFQ_GGUF_Q6_K> {
     static __device__ __forceinline__ int pair_second(int p) { return pair_first(p) + 2; }
     static constexpr bool NIBBLE = false;
     static constexpr uint32_t TOPOFF = 0;
+    // The four lanes of a quad take the four pairs of one super-block (lane = 2 * half + t), and what a lane's windows lack
+    // another lane of the quad holds: the two lanes of a half share its 32 bytes of upper bits, 16 each; the ninth dword of the lower nibbles is the next lane's first (behind the last lane's
+    // begin the upper bits), the ninth of the upper bits the other half's first or the first of the scales, and the scales
+    // are fetched as one dword per lane.  Five loads instead of nine: the address unit, 33 clocks
+    // per load instruction and busy for two thirds of the time (the vector units for 41 %), was what bound this kernel.
+    uint32_t tw, t4;                                 // dword 4 * lane of the tail from byte 192 on, dword 16: o bytes earlier
+    __device__ __forceinline__ void load_pair(const uint8_t *row, int u)
+    {
+        const uint8_t *blk = row + (size_t)(u >> 3) * 210;
+        const int half = (u >> 2) & 1;
+        t = u & 3;
+        const uint32_t o = (uint32_t)(reinterpret_cast<uintptr_t>(blk) & 3u);
+        const uint8_t *a = blk - o;
+        wl.o = wh.o = o;
+        uint32_t v[8];
+        load_dwords_a4<8>(a + 64 * half + 32 * t, v);
+#pragma unroll
+        for (int i = 0; i < 8; i++) wl.d[i] = v[i];
+        uint32_t b[4];
+        load_dwords_a4<4>(a + 128 + 32 * half + 16 * t, b);
+#pragma unroll
+        for (int i = 0; i < 4; i++) wh.d[i] = b[i];
+        tw = *reinterpret_cast<const uint32_t *>(a + 192 + 4 * (2 * half + t));
+        t4 = *reinterpret_cast<const uint32_t *>(a + 208);       // (holds the block's last two bytes)
+    }
+    template <int CTRL> static __device__ __forceinline__ uint32_t quad(uint32_t v)
+    {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+    }
     __device__ __forceinline__ float idot_pair(const XPrep &xa, const XPrep &xb) const    // this unit (t < 2) and the one two on
     {
+        constexpr int NEXT = 0x39, L0 = 0x00, L2 = 0xAA, EVEN = 0xA0, ODD = 0xF5;    // quad_perm [1 2 3 0], [0 0 0 0], [2 2 2 2], [0 0 2 2], [1 1 3 3]
+        const int lane = threadIdx.x & 3;
+        const uint32_t next = quad<NEXT>(wl.d[0]), h0 = quad<L0>(wh.d[0]), h2 = quad<L2>(wh.d[0]);
+        const uint32_t ta = quad<EVEN>(tw), tb = quad<ODD>(tw), t0 = quad<L0>(tw), t2 = quad<L2>(tw);
+        Window<8> lower = wl, upper;
+        upper.o = wl.o;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            upper.d[i] = quad<EVEN>(wh.d[i]);
+            upper.d[4 + i] = quad<ODD>(wh.d[i]);
+        }
+        lower.d[8] = lane == 3 ? h0 : next;
+        upper.d[8] = lane < 2 ? h2 : t0;
+        const uint32_t sel = 0x03020100u + __builtin_amdgcn_perm(0u, wl.o + 2 * (uint32_t)t, 0u);
+        const uint16_t sc2 = (uint16_t)__builtin_amdgcn_perm(tb, ta, sel);
+        const uint16_t sc2b = (uint16_t)__builtin_amdgcn_perm(lane < 2 ? t2 : t4, tb, sel);
+        const uint16_t d = (uint16_t)(t4 >> (8u * wl.o));
         U8 ql, qh;
-        wl.piece<0>(ql.v);
-        wh.piece<0>(qh.v);
+        lower.piece<0>(ql.v);
+        upper.piece<0>(qh.v);
         const int shr = 2 * t;
         uint32_t alo[2] = {0, 0}, amid[2] = {0, 0}, blo[2] = {0, 0}, bmid[2] = {0, 0};
         int atop[2] = {0, 0}, btop[2] = {0, 0};
@@ -1729,9 +1773,9 @@ gemv_idot_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, flo
     int unit[UPL];
     if constexpr (IU::PAIR && UPL == 2) {
         // lane p owns the two units of pair p (the unit count of such a format is a multiple of eight: both live or
-        // both past the end)
+        // both past the end, four lanes of a quad alike: past the end they take the last super-block's four pairs)
         const bool in = 2 * tl < ku;
-        const int p = in ? tl : (ku >> 1) - 1;
+        const int p = in ? tl : (ku >> 1) - 4 + (tl & 3);
         live[0] = live[1] = in;
         unit[0] = IU::pair_first(p);
         unit[1] = IU::pair_second(p);
@@ -1774,7 +1818,8 @@ gemv_idot_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, flo
         if (r > row_last) r = row_last;
         const uint8_t *row = fused_row<FUSE>(w, f, r, rb);
         if constexpr (IU::PAIR && UPL == 2) {
-            buf[slot][0].load(row, unit[0]);          // one fetch serves both units of the pair
+            if constexpr (FMT == RFQ_GGUF_Q6_K) buf[slot][0].load_pair(row, unit[0]);
+            else buf[slot][0].load(row, unit[0]);     // one fetch serves both units of the pair
         } else {
 #pragma unroll
             for (int j = 0; j < UPL; j++) buf[slot][j].load(row, unit[j]);
