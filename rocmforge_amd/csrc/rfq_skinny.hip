@@ -92,26 +92,40 @@ int gemm_cfg(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, in
     return RFQ_OK;
 }
 
-// Rows of a slice: at most 16 * most, the slices as even as 16 rows allow.
+// 16-row operands per workgroup at most: six with one row tile (eight leave its registers one wavefront per SIMD: Q8_0
+// 4096 -> 1024, 100 rows, 28 us with eight, 160 rows 15 with twice five); eight with two (8192 rows of 4096, 100 rows: Q8_0
+// 28.8 us, 40 with two slices of four), but four for the scale-only 4-bit layouts, which would spill (Q4_0, 208 rows,
+// 1792 -> 5713: 79.7 us with eight, 45 with four).
+constexpr int most_tiles(int fmt, bool two) { return !two ? 6 : fmt == RFQ_Q4_0 || fmt == RFQ_GGUF_Q4_0 ? 4 : 8; }
+
+// The rows of a in slices of at most 16 * most_tiles, as even as 16 rows allow.  Where W gives fewer workgroups than the part
+// has CUs there are more slices, so that every CU gets one: a workgroup's time grows with its operands of 16 rows, and W that
+// small stays in the caches (4096 -> 1024, Q8_0: 48 rows 9.8 -> 6.2 us, 160 rows 15.2 -> 9.8; 1280 -> 1280 GGUF_Q4_K 100 rows
+// 8.9 -> 5.2).
 struct Slices { int count, tiles; };
-Slices slices_of(int m, int most)
+Slices slices_of(int fmt, int m, int n, bool two)
 {
-    const int tiles = (m + 15) / 16, count = (tiles + most - 1) / most;
-    return {count, (tiles + count - 1) / count};
+    const int tiles = (m + 15) / 16, most = most_tiles(fmt, two), groups = two ? (n + 31) / 32 : (n + 15) / 16;
+    int count = (tiles + most - 1) / most;
+    const int room = device_cu_count() / groups;
+    if (room > count) count = room < tiles ? room : tiles;
+    const int per = (tiles + count - 1) / count;
+    return {(tiles + per - 1) / per, per};
 }
-// Eight 16-row operands per workgroup; four where two row tiles of the scale-only 4-bit layouts would spill registers
-// (Q4_0, 208 rows, 1792 -> 5713: 79.7 us with eight, 30 with four; the other formats hold eight).
-constexpr int most_tiles(int fmt, bool two) { return two && (fmt == RFQ_Q4_0 || fmt == RFQ_GGUF_Q4_0) ? 4 : 8; }
+
 // Two row tiles per workgroup from about one workgroup per CU on: a workgroup reads all activations of its slice whether
 // it multiplies 16 rows of W or 32 (Q8_0, k = 4096, 48 rows: n = 8192 23.5 -> 18.7 us, n = 14336 43.2 -> 32.7; with fewer
 // workgroups than CUs one tile is ahead, n = 4096 11.4 against 13.7 us).
-bool two_tiles(int m, int n) { return (n + 15) / 16 * slices_of(m, 8).count > device_cu_count() + device_cu_count() / 8; }
+bool two_tiles(int fmt, int m, int n)
+{
+    return (n + 15) / 16 * slices_of(fmt, m, n, false).count > device_cu_count() + device_cu_count() / 8;
+}
 
 template <int FMT, int TJ, bool ARR>
 int gemm_mt(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int n, int k, hipStream_t s)
 {
     constexpr int MOST = most_tiles(FMT, TJ == 2);
-    const Slices sl = slices_of(m, MOST);
+    const Slices sl = slices_of(FMT, m, n, TJ == 2);
     const int rows = 16 * sl.tiles, slices = sl.count;
     // units of W in flight per wavefront: two, one where the registers of a unit leave no room for two
     constexpr int D = TJ * W<FMT>::NR > 9 ? 1 : 2;
@@ -121,10 +135,10 @@ int gemm_mt(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int
     case 3: return gemm_cfg<FMT, 3, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
     case 4: return gemm_cfg<FMT, 4, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
     default:
-        if constexpr (MOST == 8) {
+        if constexpr (MOST >= 6)
             if (sl.tiles <= 6) return gemm_cfg<FMT, 6, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
-            return gemm_cfg<FMT, 8, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
-        }
+        if constexpr (MOST >= 8)
+            if (sl.tiles <= 8) return gemm_cfg<FMT, 8, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
         return fail(RFQ_E_UNSUPPORTED, "rfq_gemm_f16: slices of %d rows", rows);
     }
 }
@@ -132,7 +146,7 @@ int gemm_mt(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int
 template <int FMT>
 int gemm_fmt(const uint8_t *w, const uint8_t *a, bool arranged, void *y, int f16_out, int m, int n, int k, hipStream_t s)
 {
-    if (two_tiles(m, n)) return arranged ? gemm_mt<FMT, 2, true>(w, a, y, f16_out, m, n, k, s) : gemm_mt<FMT, 2, false>(w, a, y, f16_out, m, n, k, s);
+    if (two_tiles(FMT, m, n)) return arranged ? gemm_mt<FMT, 2, true>(w, a, y, f16_out, m, n, k, s) : gemm_mt<FMT, 2, false>(w, a, y, f16_out, m, n, k, s);
     return arranged ? gemm_mt<FMT, 1, true>(w, a, y, f16_out, m, n, k, s) : gemm_mt<FMT, 1, false>(w, a, y, f16_out, m, n, k, s);
 }
 
@@ -187,8 +201,8 @@ int RFQ_SKINNY_CAT(launch_skinny_gemm_part, RFQ_SKINNY_PART)(int fmt, const uint
 bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts)
 {
     const double cus = device_cu_count(), ku = k / 1024.0;
-    const bool two = two_tiles(m, n);
-    const Slices sl = slices_of(m, most_tiles(fmt, two));
+    const bool two = two_tiles(fmt, m, n);
+    const Slices sl = slices_of(fmt, m, n, two);
     const int row_tiles = (n + 15) / 16 * sl.count;
     const double rounds = two ? 1.45 * (row_tiles / 2 > cus ? row_tiles / 2 / cus : 1.0) : 1.0;
     const double few = 3.0 + ku * rounds * (0.5 + 0.7 * (sl.tiles <= 4 ? sl.tiles : sl.tiles <= 6 ? 6 : 8));
