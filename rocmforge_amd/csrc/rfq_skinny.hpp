@@ -554,6 +554,15 @@ __device__ __forceinline__ void contract(const v4u &xa, const v4u &wf, v4f (&d)[
 
 constexpr int MAX_WAVES = 16;
 
+// Between a wavefront's writes to its own part of LDS and other lanes' reads of them (and before the part is written again):
+// the hardware completes a wavefront's LDS operations in order, this keeps the compiler from moving them across.  No instruction.
+__device__ __forceinline__ void wave_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---- float32 x, m <= 8 -----------------------------------------------------------------------------------------------
 // blockDim = 64 * waves.  w2 != nullptr (TJ even): the odd row tiles come from w2, a second matrix of the same shape (gate and
 // up projections), and y[j] = swiglu(row j of w, row j of w2) as the reference defines it (kernels/swiglu.hip:40-62).  NORM:
@@ -710,6 +719,7 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                         for (int t = 0; t < TJ; t++) acc[t][r] *= fr;
                     }
                 }
+                wave_order();                                     // (the unit before has been read)
 #pragma unroll
                 for (int p = 0; p < P; p++) {
                     uint32_t hi[4], lo[4];
@@ -737,7 +747,7 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                     cur[t] = placed<FMT>(raw[d][t], from4);
                     cur[t].open(u, Fmt<FMT>::BE < 128 && 4 * u + q >= groups);
                 }
-                // (a wavefront's LDS operations complete in order: no barrier between its writes and its reads)
+                wave_order();
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     const v4u hi = *reinterpret_cast<const v4u *>(xrd + j * 64);
@@ -954,7 +964,7 @@ gemm_skinny_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ a,
 #pragma unroll
                         for (int b = 0; b < MT; b++) xa[b] = ar[j % AD][b].ordered();
                     } else {
-                        // (a wavefront's LDS operations complete in order: no barrier around its own area)
+                        wave_order();                             // (the group before has been read)
 #pragma unroll
                         for (int b = 0; b < MT; b++) {
                             const v4u o = ar[j % AD][b].ordered();
@@ -965,6 +975,7 @@ gemm_skinny_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ a,
                                 *reinterpret_cast<v2u *>(area + b * ABLK + st1) = v2u{o[2], o[3]};
                             }
                         }
+                        wave_order();
 #pragma unroll
                         for (int b = 0; b < MT; b++) xa[b] = *reinterpret_cast<const v4u *>(area + b * ABLK + rd);
                     }
