@@ -52,13 +52,17 @@ int gemv_cfg(const SkinnyGemv &c, hipStream_t s)
 // Row tiles per workgroup: one up to 20 rows per CU, where a second tile would leave CUs without a workgroup, then two, four
 // from 52 on: every workgroup converts all of x (Q4_0, 8 vectors, k = 4096: n = 4096 8.8 / 10.7 / 14.5 us with 1 / 2 / 4,
 // n = 8192 12.7 / 11.5 / 14.9, n = 14336 23.4 / 18.8 / 18.4; MXFP4 n = 14336 22.8 / 22.1 / 18.8).  Two matrices take an even
-// number.
+// number.  Up to four vectors stay at two: converting half as much x matters less than a second workgroup per CU (14336 x 4096,
+// 4 vectors: MXFP4 18.4 / 17.2 us with 4 / 2, Q6_K 23.5 / 22.3, GGUF_Q4_K 16.5 / 15.9), but for pairs of MXFP matrices
+// (gate and up of 5120 -> 13824, 2 vectors, with the down projection: MXFP4 69.8 / 72.5).
 template <int FMT, int MV, bool NORM>
 int gemv_rows(const SkinnyGemv &c, hipStream_t s)
 {
+    constexpr bool MX = FMT == RFQ_MXFP4 || FMT == RFQ_MXFP6_E2M3;
     const int cus = device_cu_count();
     const long rows = c.w2 != nullptr ? 2L * c.n : c.n;
-    if (rows >= 52L * cus) return gemv_cfg<FMT, 4, MV, NORM>(c, s);
+    if constexpr (MV == 8 || MX)
+        if (rows >= 52L * cus && (MV == 8 || c.w2 != nullptr)) return gemv_cfg<FMT, 4, MV, NORM>(c, s);
     if (rows > 20L * cus || c.w2 != nullptr) return gemv_cfg<FMT, 2, MV, NORM>(c, s);
     return gemv_cfg<FMT, 1, MV, NORM>(c, s);
 }

@@ -15,8 +15,10 @@
 //     v_permlane16_swap until each holds its eight codes of every group.  Activations take the same way through LDS.
 //   * Mins (Q4_K): the sum of x over a group comes out of the same instruction with a weight operand of ones, already in
 //     the layout of the result: acc += min * sum(x).
-//   * float32 x is split into two fp16 parts hi + lo of 11 bits each under a power-of-two scale per wavefront and row that
-//     follows the largest |x| seen (slow path, rarely taken); both parts are multiplied, so 22 bits of x are kept.
+//   * float32 x is split into two fp16 parts of 11 bits each, hi and 2^11 times what hi leaves, under a power of two per vector
+//     and 128-element unit that takes the unit's largest |x| to 2^14 .. 2^15: 23 bits of every x down to 2^-28 of it.  The
+//     parts of eight vectors are the sixteen rows of one operand; a unit's sums are float32 and go, times the inverse power,
+//     into float64 accumulators, so that neither an outlier nor the length of a row costs a result its precision.
 //   * No split of k over workgroups: the wavefronts of a workgroup share 16 * TJ weight rows, take the 128-element units
 //     of k in turn and add their results through LDS: one launch, nothing to allocate.
 // Measured (cold weights, captured launches; the tiled kernel with its arrangement and its parts -> this one):
@@ -24,12 +26,15 @@
 //   9 x 1024 -> 1000       Q8_0 27.5 -> 3.1       GGUF_Q4_K 20.0 -> 3.2    GGUF_Q6_K 36.0 -> 4.3    Q4_K 16.1 -> 3.9
 //   48 x 4096 -> 14336     Q8_0 66.5 -> 32.7      GGUF_Q4_K 42.5 -> 23.3   GGUF_Q6_K 77.9 -> 42.0   Q4_K 40.6 -> 34.7
 // and decode batches (integer-dot batch kernel, or a launch per vector -> this one):
-//   8 x 4096 -> 4096       Q8_0 11.4 -> 9.7 us    GGUF_Q4_K 13.9 -> 8.7    Q6_K 33.4 -> 10.1        MXFP4 34.1 -> 9.4
-//   5 x 13824 -> 5120      Q8_0 62 -> 31          GGUF_Q4_K 60 -> 28       GGUF_Q6_K 90 -> 42       Q4_K 75 -> 33
-//   error against 64 bits (2-norm): 8e-8 .. 2e-7, the integer-dot kernel 3e-7 .. 1e-6
+//   8 x 4096 -> 4096       Q8_0 11.0 -> 8.7 us    GGUF_Q4_K 14.4 -> 8.4    Q6_K 34.1 -> 9.4         MXFP4 33.2 -> 8.7
+//   5 x 13824 -> 5120      Q8_0 61 -> 36          GGUF_Q4_K 61 -> 32       GGUF_Q6_K 90 -> 39       Q4_K 73 -> 34
+//   error against 64 bits (2-norm of the result), 512 x 13824, 5 vectors: Q6_K 1.07e-7 (float kernel) -> 8.1e-8, Q4_K 1.12e-7 ->
+//   7.4e-8, MXFP6 1.02e-7 -> 5.6e-8; (integer-dot kernel) GGUF_Q6_K 2.8e-7 -> 8.0e-8, 8 x 4096 -> 4096 Q8_0 2.7e-7 -> 7.7e-8
 // (10.5 us for 37 rows of GGUF_Q4_K is 0.9 TB/s of weights: what bounds it is the activations, 384 KB per workgroup
 // through LDS, and the instructions, about 60 per unit and 16-row operand.)
 #pragma once
+#include <type_traits>
+
 #include "rfq_common.hpp"
 
 namespace rfq {
@@ -524,14 +529,6 @@ template <int PAIRS> __device__ __forceinline__ constexpr int pair_of(int r, int
     return PAIRS == P04 ? r + 4 * h : PAIRS == P01 ? 2 * r + h : PAIRS == P02 ? (r >> 1) * 4 + (r & 1) + 2 * h : (r & 1) * 4 + (r >> 1) + 2 * h;
 }
 
-__device__ __forceinline__ uint32_t pack2h(float a, float b)
-{
-    const v2h h = {(_Float16)a, (_Float16)b};
-    uint32_t o;
-    __builtin_memcpy(&o, &h, 4);
-    return o;
-}
-
 template <bool SPLIT16>
 __device__ __forceinline__ void contract(const v4u &xa, const v4u &wf, v4f (&d)[2])
 {
@@ -573,11 +570,34 @@ __device__ __forceinline__ void wave_order()
 // x goes global -> registers (sixteen lanes per vector, eight elements each: consecutive lanes on consecutive bytes) ->
 // two fp16 parts -> LDS -> operands: every element is converted once per workgroup and unit.
 constexpr int XROW = 256 + 16;                                    // bytes of a vector's 128 elements, bank-skewed
-template <int MV> constexpr int x_bytes() { return 2 * MV * XROW; }
+// (the two parts of MV vectors as rows of the operand, and the vectors' inverse scales)
+template <int MV> constexpr int x_bytes() { return 2 * MV * XROW + MV * 4; }
 template <int TJ, int MV> constexpr int gemv_lds(int waves)
 {
     // (the results are followed by the vectors' sums of squares)
     return waves * (x_bytes<MV>() > MV * (16 * TJ + 1) * 4 ? x_bytes<MV>() : MV * (16 * TJ + 1) * 4);
+}
+
+// The largest magnitude (fmaxf of fabsf spends an instruction more per operand on signalling NaNs).
+__device__ __forceinline__ float max3_abs(float a, float b, float c)
+{
+    float o;
+    asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(o) : "v"(a), "v"(b), "v"(c));
+    return o;
+}
+
+// The largest of the sixteen lanes of a lane row, in all of them.
+__device__ __forceinline__ uint32_t max16(uint32_t v)
+{
+    auto step = [&](auto ctrl) {
+        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xF, 0xF, true);
+        v = v > o ? v : o;
+    };
+    step(std::integral_constant<int, 0xB1>{});                    // quad_perm [1 0 3 2]
+    step(std::integral_constant<int, 0x4E>{});                    // quad_perm [2 3 0 1]
+    step(std::integral_constant<int, 0x141>{});                   // row_half_mirror
+    step(std::integral_constant<int, 0x140>{});                   // row_mirror
+    return v;
 }
 
 // MV: 4 or 8 vectors, m <= MV.
@@ -588,6 +608,10 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
 {
     typedef W<FMT> WF;
     constexpr int P = MV / 4;                                     // octets of x per lane and unit
+    // With one row tile a unit's x is taken and its scale found (a chain of nine instructions) beside the sums of the unit
+    // before (GGUF_Q4_0 5 x 14336 -> 4096 22.2 -> 19.8 us); with more, the registers it needs would leave room for one
+    // workgroup per CU instead of two, or spill (GGUF_Q6_K 5 x 4096 -> 14336 28 -> 76 us).
+    constexpr bool AHEAD = TJ == 1;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
@@ -610,6 +634,7 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
         xl[p] = x + (size_t)(v < m ? v : m - 1) * k + 8 * i;
     }
     uint8_t *const area = lds + wave * x_bytes<MV>();
+    float *const area_inv = reinterpret_cast<float *>(area + 2 * MV * XROW);
     uint8_t *xw[P];
 #pragma unroll
     for (int p = 0; p < P; p++) {
@@ -620,7 +645,7 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
     // (halves: an octet is two operand halves, of the lane rows of parts 2 (o & 1) and 2 (o & 1) + 1)
     const int h0 = WF::ORDER > OCTET_SWAPPED ? row_part(WF::ORDER, 2 * (i & 1)) * 16 : 0;
     const int h1 = WF::ORDER > OCTET_SWAPPED ? row_part(WF::ORDER, 2 * (i & 1) + 1) * 16 : 0;
-    const uint8_t *const xrd = area + (i & (MV - 1)) * XROW + q * 16;
+    const uint8_t *const xrd = area + (i & (2 * MV - 1)) * XROW + q * 16;
 
     WF raw[D][TJ];
     v4f xr[P][2], nr[2];
@@ -646,90 +671,76 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
     float ss[P];                                                  // NORM: this lane's part of its vectors' sums of squares
 #pragma unroll
     for (int p = 0; p < P; p++) ss[p] = 0.0f;
-    float s[P], lim[P];                                           // this lane's vectors: scale, and the largest |x| it can take
+    // This lane's octets of unit u, and the power of two that takes the vector's largest |x| of the unit to 2^14 .. 2^15.
+    float e[P][8], s[P], inv_s[P];
+    auto take_x = [&](int u) __attribute__((always_inline)) {
+        const bool past = 128 * u + 8 * i >= k;
 #pragma unroll
-    for (int p = 0; p < P; p++) { s[p] = 1.0f; lim[p] = 0.0f; }
-    float acc[TJ][4];
+        for (int p = 0; p < P; p++) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) { e[p][c] = xr[p][0][c]; e[p][4 + c] = xr[p][1][c]; }
+            if (Fmt<FMT>::BE < 128 && past) {
+#pragma unroll
+                for (int c = 0; c < 8; c++) e[p][c] = 0.0f;
+            }
+            if constexpr (NORM) {
+                if (u < units) {
+#pragma unroll
+                    for (int c = 0; c < 8; c++) ss[p] = __builtin_fmaf(e[p][c], e[p][c], ss[p]);
+                }
+#pragma unroll
+                for (int c = 0; c < 8; c++) e[p][c] *= nr[c >> 2][c & 3];
+            }
+            const float mx = max3_abs(max3_abs(e[p][0], e[p][1], e[p][2]), max3_abs(e[p][3], e[p][4], e[p][5]), max3_abs(e[p][6], e[p][7], 0.0f));
+            const int ex = (int)(max16(__float_as_uint(mx)) >> 23);   // biased exponent
+            int se = 268 - ex;                                        // s = 2^(14 - (ex - 127))
+            se = se > 243 ? 243 : se;                                 // (2048 s stays finite)
+            s[p] = __uint_as_float((uint32_t)se << 23);
+            inv_s[p] = __uint_as_float((uint32_t)(254 - se) << 23);
+        }
+    };
+    double acc[TJ][4];
 #pragma unroll
     for (int t = 0; t < TJ; t++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) acc[t][r] = 0.0f;
+        for (int r = 0; r < 4; r++) acc[t][r] = 0.0;
     const v4u ones = {0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
 
     load_x(wave);
 #pragma unroll
     for (int d = 0; d < D; d++) load_w(raw[d], wave + d * waves);
+    if constexpr (AHEAD) {
+        take_x(wave);
+        load_x(wave + waves);
+    }
 
     for (int u0 = wave; u0 < units; u0 += D * waves) {
 #pragma unroll
         for (int d = 0; d < D; d++) {
             const int u = u0 + d * waves;
             if (u < units) {
-                float e[P][8], mx[P];
-                bool over = false;
-                const bool past = 128 * u + 8 * i >= k;
-#pragma unroll
-                for (int p = 0; p < P; p++) {
-#pragma unroll
-                    for (int c = 0; c < 4; c++) { e[p][c] = xr[p][0][c]; e[p][4 + c] = xr[p][1][c]; }
-                    if (Fmt<FMT>::BE < 128 && past) {
-#pragma unroll
-                        for (int c = 0; c < 8; c++) e[p][c] = 0.0f;
-                    }
-                    if constexpr (NORM) {
-#pragma unroll
-                        for (int c = 0; c < 8; c++) {
-                            ss[p] = __builtin_fmaf(e[p][c], e[p][c], ss[p]);
-                            e[p][c] *= nr[c >> 2][c & 3];
-                        }
-                    }
-                    mx[p] = fmaxf(fmaxf(fmaxf(fabsf(e[p][0]), fabsf(e[p][1])), fmaxf(fabsf(e[p][2]), fabsf(e[p][3]))),
-                                  fmaxf(fmaxf(fabsf(e[p][4]), fabsf(e[p][5])), fmaxf(fabsf(e[p][6]), fabsf(e[p][7]))));
-                    over |= mx[p] > lim[p];
-                }
-                load_x(u + waves);
-                if (__builtin_expect(__builtin_amdgcn_ballot_w64(over) != 0, 0)) {
-                    // |x| beyond what the scale takes: the vector's largest of this unit goes to 2^10 (up to 32 times as
-                    // much fits from then on), and what has been summed follows
-                    float f[P];
-#pragma unroll
-                    for (int p = 0; p < P; p++) {
-                        float t = mx[p];
-#pragma unroll
-                        for (int o = 1; o < 16; o <<= 1) t = fmaxf(t, __shfl_xor(t, o));
-                        f[p] = 1.0f;
-                        if (t > lim[p]) {
-                            const int ex = (int)(__float_as_uint(t) >> 23);  // biased exponent (255 for an infinity)
-                            int se = 264 - ex;                               // s = 2^(10 - (ex - 127))
-                            se = se > 252 ? 252 : se;
-                            const float s_new = __uint_as_float((uint32_t)se << 23);
-                            f[p] = s_new * (1.0f / s[p]);                    // (powers of two)
-                            s[p] = s_new;
-                            lim[p] = ex >= 249 ? 3.40282347e+38f : se == 252 ? __uint_as_float((uint32_t)17 << 23) : __uint_as_float((uint32_t)(ex + 5) << 23);
-                        }
-                    }
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {                            // (vector 4 q + r is row r of lanes, octet set q)
-                        float fr = __shfl(f[0], 16 * r);
-                        if constexpr (P == 2) {
-                            const float f1 = __shfl(f[1], 16 * r);
-                            fr = (q & 1) ? f1 : fr;
-                        }
-#pragma unroll
-                        for (int t = 0; t < TJ; t++) acc[t][r] *= fr;
-                    }
+                if constexpr (!AHEAD) {
+                    take_x(u);
+                    load_x(u + waves);
                 }
                 wave_order();                                     // (the unit before has been read)
+#pragma unroll
+                for (int p = 0; p < P; p++)
+                    if (i == 0) area_inv[4 * p + q] = inv_s[p];
 #pragma unroll
                 for (int p = 0; p < P; p++) {
                     uint32_t hi[4], lo[4];
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
-                        float a = e[p][pair_of<WF::PAIRS>(r, 0)] * s[p], b = e[p][pair_of<WF::PAIRS>(r, 1)] * s[p];
-                        asm("" : "+v"(a), "+v"(b));               // (one conversion of each product, not one per use)
-                        const v2h h = {(_Float16)a, (_Float16)b};
+                        // (x * s, x - hi / s and its multiple by 2048 s are exact: a part is rounded once, to fp16)
+                        const float a = e[p][pair_of<WF::PAIRS>(r, 0)], b = e[p][pair_of<WF::PAIRS>(r, 1)];
+                        v2h h = {(_Float16)__builtin_fmaf(a, s[p], 0.0f), (_Float16)__builtin_fmaf(b, s[p], 0.0f)};
                         __builtin_memcpy(&hi[r], &h, 4);
-                        lo[r] = pack2h(a - (float)h[0], b - (float)h[1]);
+                        asm("" : "+v"(hi[r]));                    // (one conversion of each product, not one per use)
+                        __builtin_memcpy(&h, &hi[r], 4);
+                        const float ra = __builtin_fmaf((float)h[0], -inv_s[p], a), rb = __builtin_fmaf((float)h[1], -inv_s[p], b);
+                        const v2h l = {(_Float16)__builtin_fmaf(ra, s[p] * 2048.0f, 0.0f), (_Float16)__builtin_fmaf(rb, s[p] * 2048.0f, 0.0f)};
+                        __builtin_memcpy(&lo[r], &l, 4);
                     }
                     if constexpr (WF::ORDER <= OCTET_SWAPPED) {
                         *reinterpret_cast<v4u *>(xw[p]) = v4u{hi[0], hi[1], hi[2], hi[3]};
@@ -748,59 +759,57 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                     cur[t].open(u, Fmt<FMT>::BE < 128 && 4 * u + q >= groups);
                 }
                 wave_order();
+                float sum[TJ][4];                                 // of this unit, in units of the vectors' inverse scales
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    const v4u hi = *reinterpret_cast<const v4u *>(xrd + j * 64);
-                    const v4u lo = *reinterpret_cast<const v4u *>(xrd + MV * XROW + j * 64);
+                    const v4u xa = *reinterpret_cast<const v4u *>(xrd + j * 64);
                     v4f xs[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-                    if constexpr (WF::MINS) {
-                        contract<false>(lo, ones, xs);
-                        contract<false>(hi, ones, xs);
-                    }
+                    if constexpr (WF::MINS) contract<false>(xa, ones, xs);
 #pragma unroll
                     for (int t = 0; t < TJ; t++) {
                         const v4u wf = cur[t].frag(j);
                         v4f p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-                        contract<WF::SPLIT16>(lo, wf, p);
-                        contract<WF::SPLIT16>(hi, wf, p);
+                        contract<WF::SPLIT16>(xa, wf, p);
                         const float s0 = cur[t].sc(j, 0);
 #pragma unroll
-                        for (int r = 0; r < 4; r++) acc[t][r] = __builtin_fmaf(s0, p[0][r], acc[t][r]);
+                        for (int r = 0; r < 4; r++) sum[t][r] = j == 0 ? s0 * p[0][r] : __builtin_fmaf(s0, p[0][r], sum[t][r]);
                         if constexpr (WF::SPLIT16) {
                             const float s1 = cur[t].sc(j, 1);
 #pragma unroll
-                            for (int r = 0; r < 4; r++) acc[t][r] = __builtin_fmaf(s1, p[1][r], acc[t][r]);
+                            for (int r = 0; r < 4; r++) sum[t][r] = __builtin_fmaf(s1, p[1][r], sum[t][r]);
                         }
                         if constexpr (WF::MINS) {
                             const float mn = cur[t].mn(j);
 #pragma unroll
-                            for (int r = 0; r < 4; r++) acc[t][r] = __builtin_fmaf(mn, xs[0][r], acc[t][r]);
+                            for (int r = 0; r < 4; r++) sum[t][r] = __builtin_fmaf(mn, xs[0][r], sum[t][r]);
                         }
                     }
+                }
+                const v4f inv = *reinterpret_cast<const v4f *>(area_inv + (4 * q & (MV - 1)));
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const double iv = (double)inv[r];
+#pragma unroll
+                    for (int t = 0; t < TJ; t++) acc[t][r] = __builtin_fma((double)sum[t][r], iv, acc[t][r]);
+                }
+                if constexpr (AHEAD) {
+                    take_x(u + waves);
+                    load_x(u + 2 * waves);
                 }
             }
             load_w(raw[d], u + D * waves);
         }
     }
-    // red[wave][vector][16 * TJ rows]; lane rows 0 .. P - 1 hold vectors 0 .. MV - 1
-    float inv[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        inv[r] = __shfl(s[0], 16 * r);
-        if constexpr (P == 2) {
-            const float s1 = __shfl(s[1], 16 * r);
-            inv[r] = (q & 1) ? s1 : inv[r];
-        }
-        inv[r] = 1.0f / inv[r];                                   // (a power of two)
-    }
+    // red[wave][vector][16 * TJ rows]; lane rows 0 .. P - 1 hold the hi parts of vectors 0 .. MV - 1, the next P the lo parts
     __syncthreads();
     float *const red = reinterpret_cast<float *>(lds);
-    if (q < P) {
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+    for (int r = 0; r < 4; r++)
 #pragma unroll
-            for (int t = 0; t < TJ; t++) red[(wave * MV + 4 * q + r) * (16 * TJ) + 16 * t + i] = acc[t][r] * inv[r];
-    }
+        for (int t = 0; t < TJ; t++) {
+            const double lo = __shfl_xor(acc[t][r], 16 * P);
+            if (q < P) red[(wave * MV + 4 * q + r) * (16 * TJ) + 16 * t + i] = (float)__builtin_fma(lo, 0x1p-11, acc[t][r]);
+        }
     float *const squares = red + waves * MV * (16 * TJ);
     if constexpr (NORM) {
 #pragma unroll
@@ -812,26 +821,27 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
     }
     __syncthreads();
     auto total = [&](int v, int c) __attribute__((always_inline)) {
-        float sum = 0.0f;
-        for (int wv = 0; wv < waves; wv++) sum += red[(wv * MV + v) * (16 * TJ) + c];
+        double sum = 0.0;
+        for (int wv = 0; wv < waves; wv++) sum += (double)red[(wv * MV + v) * (16 * TJ) + c];
         return sum;
     };
     const int cols = glu ? 8 * TJ : 16 * TJ;
     for (int o = tid; o < MV * cols; o += (int)blockDim.x) {
         const int v = o / cols, c = o % cols;
         if (v >= m || n0 + c >= n) continue;
-        float rinv = 1.0f;
-        if constexpr (NORM) {
-            float sq = 0.0f;
-            for (int wv = 0; wv < waves; wv++) sq += squares[wv * MV + v];
-            rinv = 1.0f / sqrtf(sq / (float)k + eps);
+        double rinv = 1.0;
+        if constexpr (NORM) {                                     // (one step of Newton's iteration: an error here is the whole vector's)
+            double sq = 0.0;
+            for (int wv = 0; wv < waves; wv++) sq += (double)squares[wv * MV + v];
+            const double mean = __builtin_fma(sq, 1.0 / (double)k, (double)eps), r0 = (double)(1.0f / sqrtf((float)mean));
+            rinv = r0 * __builtin_fma(-0.5 * mean, r0 * r0, 1.5);
         }
         if (glu) {
             const int at = 32 * (c >> 4) + (c & 15);
-            const float gate = total(v, at) * rinv, up = total(v, at + 16) * rinv;
+            const float gate = (float)(total(v, at) * rinv), up = (float)(total(v, at + 16) * rinv);
             y[(size_t)v * n + n0 + c] = gate * (up * (1.0f / (1.0f + expf(-up))));
         } else {
-            y[(size_t)v * n + n0 + c] = total(v, c) * rinv;
+            y[(size_t)v * n + n0 + c] = (float)(total(v, c) * rinv);
         }
     }
 }

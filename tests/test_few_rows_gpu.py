@@ -148,3 +148,42 @@ def test_gate_and_up_in_one_launch(fmt, m, hidden, inter, norm, oracle, cuda):
     want = h @ weights_of(oracle, Q.Q8_0, down, hidden, inter).T
     # (the product of two float32 sums, contracted once more: the errors of both add up)
     assert_close(got.cpu().numpy(), want, f"{Q.NAMES[fmt]} {m}x{hidden}x{inter}", tol=3 * TOL, plain_tol=6e-4)
+
+
+@pytest.mark.parametrize("fmt", BATCH_FORMATS)
+@pytest.mark.parametrize("m,n,k", [(4, 4000, 3072), (5, 96, 13824), (8, 256, 4096), (8, 96, 1024)])
+@pytest.mark.parametrize("outlier", [False, True])
+def test_decode_batches_keep_float32_precision(fmt, m, n, k, outlier, oracle, cuda):
+    """The 2-norm of the error: two fp16 parts keep 23 bits of x (errors of 2^-23 in a quarter of the values: 4e-8 rms), a
+    unit's sum of up to eight products rounds to 24 bits eight times (2.5e-8 rms each, partial sums growing like sqrt: 5e-8),
+    the matrix instruction as often again; together below 1e-7, and what a float32 kernel reaches is 1.1e-7 to 1.3e-7.  It
+    holds beside a value 2^14 times the others whose weights are zero, in the same unit and in those that follow."""
+    import torch
+    from rocmforge_amd import ops
+    w = Q.make_weights(fmt, n, k, seed=fmt + m).copy()
+    x = np.random.default_rng(m * n).standard_normal((m, k)).astype(np.float32)
+    if outlier:
+        w.reshape(n, -1)[:, : Q.BLOCK_BYTES[fmt]] = 0              # (a block of zero bytes decodes to zeros in every layout)
+        x[:, 5] = 2.0 ** 14
+    got = ops.gemv(fmt, torch.from_numpy(w).to(cuda), torch.from_numpy(x).to(cuda), n, k).cpu().numpy().astype(np.float64)
+    want = x.astype(np.float64) @ weights_of(oracle, fmt, w, n, k).T
+    error = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert np.linalg.norm(error) / np.sqrt(m) <= 1.3e-7, (Q.NAMES[fmt], error)
+
+
+@pytest.mark.parametrize("first", [120.5, 121.5, 122.5, 123.5, 126.5])
+def test_decode_batch_up_to_the_largest_value(first, oracle, cuda):
+    """The largest finite float after smaller ones of 2^first in the same wavefront's earlier unit (eight wavefronts take the
+    128-element units in turn)."""
+    import torch
+    from rocmforge_amd import ops
+    m, n, k = 5, 32, 2048
+    w = Q.make_weights(Q.Q4_0, n, k, seed=3).copy()
+    blocks = w.reshape(-1, 20)
+    blocks[:, :4] = np.frombuffer(np.float32(1e-4).tobytes(), np.uint8)
+    x = np.random.default_rng(1).standard_normal((m, k)).astype(np.float32)
+    x[:, 3] = 2.0 ** first
+    x[:, 1024 + 9] = np.finfo(np.float32).max
+    got = ops.gemv(Q.Q4_0, torch.from_numpy(w).to(cuda), torch.from_numpy(x).to(cuda), n, k).cpu().numpy()
+    want = x.astype(np.float64) @ weights_of(oracle, Q.Q4_0, w, n, k).T
+    assert np.all(np.abs(got - want) <= 1e-6 * np.abs(want) + 1e-7 * np.abs(want).max())
