@@ -612,6 +612,7 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
     // before (GGUF_Q4_0 5 x 14336 -> 4096 22.2 -> 19.8 us); with more, the registers it needs would leave room for one
     // workgroup per CU instead of two, or spill (GGUF_Q6_K 5 x 4096 -> 14336 28 -> 76 us).
     constexpr bool AHEAD = TJ == 1;
+    constexpr bool F32_SCALE = FMT == RFQ_Q4_0 || FMT == RFQ_Q8_0;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
@@ -671,8 +672,9 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
     float ss[P];                                                  // NORM: this lane's part of its vectors' sums of squares
 #pragma unroll
     for (int p = 0; p < P; p++) ss[p] = 0.0f;
-    // This lane's octets of unit u, and the power of two that takes the vector's largest |x| of the unit to 2^14 .. 2^15.
-    float e[P][8], s[P], inv_s[P];
+    // This lane's octets of unit u, and the biased exponent of the vector's largest |x| in the unit.
+    float e[P][8];
+    int ex[P];
     auto take_x = [&](int u) __attribute__((always_inline)) {
         const bool past = 128 * u + 8 * i >= k;
 #pragma unroll
@@ -692,11 +694,7 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                 for (int c = 0; c < 8; c++) e[p][c] *= nr[c >> 2][c & 3];
             }
             const float mx = max3_abs(max3_abs(e[p][0], e[p][1], e[p][2]), max3_abs(e[p][3], e[p][4], e[p][5]), max3_abs(e[p][6], e[p][7], 0.0f));
-            const int ex = (int)(max16(__float_as_uint(mx)) >> 23);   // biased exponent
-            int se = 268 - ex;                                        // s = 2^(14 - (ex - 127))
-            se = se > 243 ? 243 : se;                                 // (2048 s stays finite)
-            s[p] = __uint_as_float((uint32_t)se << 23);
-            inv_s[p] = __uint_as_float((uint32_t)(254 - se) << 23);
+            ex[p] = (int)(max16(__float_as_uint(mx)) >> 23);
         }
     };
     double acc[TJ][4];
@@ -723,10 +721,25 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                     take_x(u);
                     load_x(u + waves);
                 }
-                wave_order();                                     // (the unit before has been read)
+                int top = 14;                                     // the largest |x| goes to 2^top .. 2^(top + 1)
+                if constexpr (F32_SCALE) {
+                    // (a sum of 32 codes times 2^15 is below 2^28: a block scale from 2^100 on could take it past the largest
+                    // float where the result, with small x, is not.  With such a scale x loses bits below 2^-11 of the largest.)
+                    bool large = false;
 #pragma unroll
-                for (int p = 0; p < P; p++)
+                    for (int t = 0; t < TJ; t++) large |= fabsf(__uint_as_float(raw[d][t].r[0])) >= 0x1p100f;
+                    if (__builtin_amdgcn_ballot_w64(large) != 0) top = -14;
+                }
+                wave_order();                                     // (the unit before has been read)
+                float s[P], inv_s[P];
+#pragma unroll
+                for (int p = 0; p < P; p++) {
+                    int se = 254 + top - ex[p];                   // s = 2^(top - (ex - 127))
+                    se = se > 243 ? 243 : F32_SCALE && se < 1 ? 1 : se;   // (2048 s stays finite, s above zero)
+                    s[p] = __uint_as_float((uint32_t)se << 23);
+                    inv_s[p] = __uint_as_float((uint32_t)(254 - se) << 23);
                     if (i == 0) area_inv[4 * p + q] = inv_s[p];
+                }
 #pragma unroll
                 for (int p = 0; p < P; p++) {
                     uint32_t hi[4], lo[4];

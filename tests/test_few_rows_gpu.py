@@ -187,3 +187,28 @@ def test_decode_batch_up_to_the_largest_value(first, oracle, cuda):
     got = ops.gemv(Q.Q4_0, torch.from_numpy(w).to(cuda), torch.from_numpy(x).to(cuda), n, k).cpu().numpy()
     want = x.astype(np.float64) @ weights_of(oracle, Q.Q4_0, w, n, k).T
     assert np.all(np.abs(got - want) <= 1e-6 * np.abs(want) + 1e-7 * np.abs(want).max())
+
+
+@pytest.mark.parametrize("fmt", [Q.Q4_0, Q.Q8_0])
+@pytest.mark.parametrize("scale", [1e-37, 1e31, 1e33, 1e36])
+def test_decode_batch_with_scales_of_any_size(fmt, scale, oracle, cuda):
+    """The block scales of a 128-element unit near both ends of float32 against x that takes the results back to ordinary
+    sizes, beside ordinary units of the same row."""
+    import torch
+    from rocmforge_amd import ops
+    m, n, k = 6, 40, 1024
+    w = Q.make_weights(fmt, n, k, seed=8).copy()
+    blocks = w.reshape(n, k // 32, -1)
+    blocks[:, 4:8, :4] = np.frombuffer(np.float32(scale).tobytes(), np.uint8)
+    x = np.random.default_rng(2).standard_normal((m, k)).astype(np.float32)
+    x[:, 4 * 32 : 8 * 32] /= np.float32(scale)
+    got = ops.gemv(fmt, torch.from_numpy(w).to(cuda), torch.from_numpy(x).to(cuda), n, k).cpu().numpy()
+    want = x.astype(np.float64) @ weights_of(oracle, fmt, w, n, k).T
+    assert_close(got, want, f"{Q.NAMES[fmt]} scale {scale}", tol=TOL, plain_tol=2e-4)
+    x[2, 5 * 32 + 3] = 3e38                                        # (that vector's results lie beyond float32 or are large; the rest of its unit is lost beside it)
+    again = ops.gemv(fmt, torch.from_numpy(w).to(cuda), torch.from_numpy(x).to(cuda), n, k).cpu().numpy()
+    assert np.array_equal(np.delete(again, 2, 0), np.delete(got, 2, 0))
+    with np.errstate(over="ignore"):
+        large = (x[2].astype(np.float64) @ weights_of(oracle, fmt, w, n, k).T).astype(np.float32)
+    assert not np.isnan(again[2]).any() and np.array_equal(np.isinf(again[2]), np.isinf(large))
+    assert np.array_equal(np.sign(again[2][np.isinf(large)]), np.sign(large[np.isinf(large)]))
