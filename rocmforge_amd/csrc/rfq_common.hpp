@@ -124,10 +124,14 @@ struct SkinnyGemv {
     float eps;
     float *y;
     int m, n, k;
+    int keep_infinities;                                          // an infinity in x: see keeps_infinities; 0: its vector's results are NaN
 };
 int launch_skinny_gemv(int fmt, const SkinnyGemv &c, hipStream_t s);
 // Whether the above is the faster way for rows of x [m, k] and this matrix (m >= 2), alone and with what it takes along.
 bool few_rows_ahead(int fmt, int m, int n, int ku, bool batch_fits);
+// Whether a batch with an infinity in x gives infinities (NaN only against a zero weight) or NaN for all of the vector's
+// results, as the kernels do that take the format and shape in other batches.
+bool keeps_infinities(int fmt, int n, int ku, bool batch_fits);
 int launch_skinny_gemv_fused(int fmt, const uint8_t *d_w, const uint8_t *d_w2, const float *d_x, const float *d_norm_w, float eps, float *d_y,
                              int m, int n, int k, hipStream_t s);
 int launch_skinny_gemm(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, bool f16_out, int m, int n, int k,

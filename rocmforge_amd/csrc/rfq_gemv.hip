@@ -2359,6 +2359,20 @@ int run_generic(const uint8_t *w, const float *x, float *y, int n, int k, hipStr
     return RFQ_OK;
 }
 
+// Of the formats that have both kernels for single vectors (see run_rows): whether the float one takes this shape; true for
+// the format that has no other.
+bool float_rows(int fmt, int n, int ku)
+{
+    const int cus = device_cu_count();
+    if (fmt == RFQ_MXFP4) return !(ku > 256 || (ku <= 128 && (n <= cus * 16 || (n >= cus * 52 && n <= cus * 64))));
+    if (fmt == RFQ_Q6_K) return !((ku > 64 && ku <= 128 && n >= cus * 56 && n <= cus * 64) || ku > 256);
+    return fmt == RFQ_MXFP6_E2M3;
+}
+
+// Rows of at least eight million weights, and of this many units, go out as one launch per vector where no batch kernel takes
+// them (see run).
+bool launch_per_vector(int n, int ku) { return ku > 16 && ku <= 512 && (size_t)n * (size_t)ku >= ((size_t)1 << 18); }
+
 // m == 1, 16 < k / 32 <= 512: the kernels that keep x per lane.
 template <int FMT, bool FUSE>
 int run_rows(const uint8_t *w, const float *x, float *y, int n, int k, const GemvFuse &f, hipStream_t s)
@@ -2373,7 +2387,7 @@ int run_rows(const uint8_t *w, const float *x, float *y, int n, int k, const Gem
     // ahead (8192 x 8192 10.5 against 11.1 us, 32000 x 4096 16.8 against 18.8 us), and the fused forms keep it.
     if constexpr (FMT == RFQ_MXFP4) {
         const int cus = device_cu_count();
-        if (FUSE || !(ku > 256 || (ku <= 128 && (n <= cus * 16 || (n >= cus * 52 && n <= cus * 64))))) {
+        if (FUSE || float_rows(FMT, n, ku)) {
             if (ku <= 64) return run_idot<FMT, 1, 1, FUSE>(w, x, y, n, k, f, s, false);
             if (!FUSE && ku <= 128 && (n > cus * 16 || n <= cus * 8)) return run_idot<FMT, 1, 2, FUSE>(w, x, y, n, k, f, s, false);
             if (ku <= 128) return run_idot<FMT, 2, 1, FUSE>(w, x, y, n, k, f, s, false);
@@ -2383,7 +2397,7 @@ int run_rows(const uint8_t *w, const float *x, float *y, int n, int k, const Gem
     }
     if constexpr (FMT == RFQ_Q6_K) {
         const int cus = device_cu_count();
-        if (FUSE || !((ku > 64 && ku <= 128 && n >= cus * 56 && n <= cus * 64) || ku > 256)) {
+        if (FUSE || float_rows(FMT, n, ku)) {
             if (ku <= 64) return run_idot<FMT, 1, 1, FUSE>(w, x, y, n, k, f, s, false);
             if (!FUSE && ku <= 128 && (n > cus * 16 || n <= cus * 8)) return run_idot<FMT, 1, 2, FUSE>(w, x, y, n, k, f, s, false);
             if (ku <= 128) return run_idot<FMT, 2, 1, FUSE>(w, x, y, n, k, f, s, false);
@@ -2455,7 +2469,7 @@ int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStre
     const bool batch_fits = HasIdotBatch<FMT>::value && ku > 32 && ku <= 256;
     if (m > 1 && (reinterpret_cast<uintptr_t>(w) & 3u) == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && few_rows_ahead(FMT, m, n, ku, batch_fits)) {
         note_kernel("gemv_skinny_kernel<%s>", FMT, 0, 0, 0);
-        return launch_skinny_gemv(FMT, SkinnyGemv{w, nullptr, x, nullptr, 0.0f, y, m, n, k}, s);
+        return launch_skinny_gemv(FMT, SkinnyGemv{w, nullptr, x, nullptr, 0.0f, y, m, n, k, keeps_infinities(FMT, n, ku, batch_fits)}, s);
     }
     if (batch_fits && m > 1) {
         // the prepared vectors of a launch live in LDS (112 bytes per unit and vector): a batch that
@@ -2478,7 +2492,7 @@ int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStre
     // row): from eight million weights on, one decode launch per vector beats the one-row-per-wavefront kernel,
     // although it reads the weights m times (Q6_K, m = 8: 14336 x 4096 321 -> 91 us, 4096 x 4096 80 -> 37 us; at
     // 1024 x 2048 the single launch is the faster one, 11 against 22 us).
-    if (m > 1 && ku > 16 && ku <= 512 && (size_t)n * (size_t)k >= ((size_t)1 << 23)) {
+    if (m > 1 && launch_per_vector(n, ku)) {
         for (int v = 0; v < m; v++) {
             const int rc = run_rows<FMT, false>(w, x + (size_t)v * k, y + (size_t)v * n, n, k, GemvFuse{nullptr, nullptr, 0.0f, 0}, s);
             if (rc != RFQ_OK) return rc;
@@ -2607,6 +2621,14 @@ bool few_rows_ahead(int fmt, int m, int n, int ku, bool batch_fits)
     return n > cus * 16 || (n >= cus * 12 && ku <= 256);
 }
 
+// The integer-dot kernels turn a unit of x with an infinity into NaN.  The float kernels multiply it; the formats whose weights
+// are an offset from the code (all but the four here) then subtract infinities, which is NaN as well.
+bool keeps_infinities(int fmt, int n, int ku, bool batch_fits)
+{
+    if (fmt != RFQ_Q4_K && fmt != RFQ_Q6_K && fmt != RFQ_MXFP4 && fmt != RFQ_MXFP6_E2M3) return false;
+    return !batch_fits && (!launch_per_vector(n, ku) || float_rows(fmt, n, ku));
+}
+
 // The same for two to eight vectors through the few-row kernel: RFQ_E_UNSUPPORTED (without an error text) where the
 // separate steps are ahead.  Besides where the plain batch takes that kernel it is taken where the launches it saves (about
 // 3 us for the norm, 8 for norm, second projection and activation) are worth more than the difference: a norm up to 16
@@ -2626,7 +2648,7 @@ int launch_skinny_gemv_fused(int fmt, const uint8_t *d_w, const uint8_t *d_w2, c
     const bool taken = d_w2 != nullptr ? m >= 3 || n <= cus * 20 || few_rows_ahead(cf, m, n, ku, batch_fits)
                                        : n <= norm_rows || few_rows_ahead(cf, m, n, ku, batch_fits);
     if (!taken) return RFQ_E_UNSUPPORTED;
-    return launch_skinny_gemv(cf, SkinnyGemv{d_w, d_w2, d_x, d_norm_w, eps, d_y, m, n, k}, s);
+    return launch_skinny_gemv(cf, SkinnyGemv{d_w, d_w2, d_x, d_norm_w, eps, d_y, m, n, k, keeps_infinities(cf, n, ku, batch_fits)}, s);
 }
 
 // One launch for RMSNorm -> GEMV (norm_w != nullptr) and / or two GEMVs sharing

@@ -44,7 +44,7 @@ int gemv_cfg(const SkinnyGemv &c, hipStream_t s)
     const size_t lds = (size_t)gemv_lds<TJ, MV>(waves);
     const int rows = c.w2 != nullptr ? 8 * TJ : 16 * TJ;
     hipLaunchKernelGGL((gemv_skinny_kernel<FMT, TJ, MV, D, GEMV_WAVES, NORM>), dim3((c.n + rows - 1) / rows), dim3(64 * waves), lds, s, c.w, c.x,
-                       c.y, c.m, c.n, c.k, c.w2, c.norm_w, c.eps);
+                       c.y, c.m, c.n, c.k, c.w2, c.norm_w, c.eps, c.keep_infinities);
     RFQ_LAUNCH_CHECK("gemv_skinny_kernel");
     return RFQ_OK;
 }

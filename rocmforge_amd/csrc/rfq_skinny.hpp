@@ -602,9 +602,9 @@ __device__ __forceinline__ uint32_t max16(uint32_t v)
 
 // MV: 4 or 8 vectors, m <= MV.
 template <int FMT, int TJ, int MV, int D, int WAVES, bool NORM>
-__global__ void __launch_bounds__(64 * WAVES)
+__global__ void __launch_bounds__(64 * WAVES, (FMT == RFQ_MXFP4 && TJ == 2 && MV == 4 && !NORM ? 4 : 1))   // (128 registers, which it misses by two: two workgroups per CU)
 gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y, int m, int n, int k,
-                   const uint8_t *__restrict__ w2, const float *__restrict__ norm_w, float eps)
+                   const uint8_t *__restrict__ w2, const float *__restrict__ norm_w, float eps, int keep_infinities)
 {
     typedef W<FMT> WF;
     constexpr int P = MV / 4;                                     // octets of x per lane and unit
@@ -613,6 +613,7 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
     // workgroup per CU instead of two, or spill (GGUF_Q6_K 5 x 4096 -> 14336 28 -> 76 us).
     constexpr bool AHEAD = TJ == 1;
     constexpr bool F32_SCALE = FMT == RFQ_Q4_0 || FMT == RFQ_Q8_0;
+    constexpr bool INFINITIES = FMT == RFQ_Q4_K || FMT == RFQ_Q6_K || FMT == RFQ_MXFP4 || FMT == RFQ_MXFP6_E2M3;   // (see keeps_infinities)
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
@@ -732,8 +733,10 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                 }
                 wave_order();                                     // (the unit before has been read)
                 float s[P], inv_s[P];
+                unsigned long long infinite = 0;
 #pragma unroll
                 for (int p = 0; p < P; p++) {
+                    if (INFINITIES && keep_infinities) infinite |= __builtin_amdgcn_ballot_w64(ex[p] == 255);
                     int se = 254 + top - ex[p];                   // s = 2^(top - (ex - 127))
                     se = se > 243 ? 243 : F32_SCALE && se < 1 ? 1 : se;   // (2048 s stays finite, s above zero)
                     s[p] = __uint_as_float((uint32_t)se << 23);
@@ -763,6 +766,24 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                         *reinterpret_cast<v2u *>(xw[p] + h1) = v2u{hi[2], hi[3]};
                         *reinterpret_cast<v2u *>(xw[p] + MV * XROW + h0) = v2u{lo[0], lo[1]};
                         *reinterpret_cast<v2u *>(xw[p] + MV * XROW + h1) = v2u{lo[2], lo[3]};
+                    }
+                }
+                if constexpr (INFINITIES) {
+                    // (what an infinity leaves is a NaN: with it every result of the vector is NaN, without it the infinity's
+                    // product with a weight that is not zero stays one.  In LDS, where this costs the usual path no registers.)
+                    if (__builtin_expect(infinite != 0, 0)) {
+#pragma unroll
+                        for (int p = 0; p < P; p++)
+#pragma unroll
+                            for (int c = 0; c < 2; c++) {
+                                uint8_t *const at = xw[p] + (WF::ORDER <= OCTET_SWAPPED ? 8 * c : c ? h1 : h0);
+                                const v2u h = *reinterpret_cast<const v2u *>(at);
+                                v2u l = *reinterpret_cast<const v2u *>(at + MV * XROW);
+#pragma unroll
+                                for (int r = 0; r < 2; r++)
+                                    l[r] &= ((h[r] & 0x7FFFu) == 0x7C00u ? 0u : 0xFFFFu) | ((h[r] & 0x7FFF0000u) == 0x7C000000u ? 0u : 0xFFFF0000u);
+                                *reinterpret_cast<v2u *>(at + MV * XROW) = l;
+                            }
                     }
                 }
                 WF cur[TJ];

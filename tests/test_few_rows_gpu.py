@@ -66,7 +66,9 @@ def test_decode_batches(fmt, m, n, k, oracle, cuda):
 @pytest.mark.parametrize("fmt", [Q.Q4_0, Q.GGUF_Q4_K, Q.Q6_K, Q.MXFP4])
 def test_decode_batch_of_any_magnitude(fmt, oracle, cuda):
     """The fp16 parts of x follow its magnitude: vectors of very different size, sizes that grow and shrink by powers of
-    ten along k, zeros, subnormals; an infinity or a NaN turns its own vector's outputs into NaN and no other's."""
+    ten along k, zeros, subnormals; an infinity or a NaN changes its own vector's outputs and no other's: to NaN, or, for
+    the formats and shapes that other batches multiply in float32 (here Q6_K and MXFP4), an infinity to the infinity of its
+    product with the weight."""
     import torch
     from rocmforge_amd import ops
     m, n, k = 8, 48, 2048
@@ -93,7 +95,9 @@ def test_decode_batch_of_any_magnitude(fmt, oracle, cuda):
         y = x.copy()
         y[2, 700] = bad
         again = ops.gemv(fmt, dw, torch.from_numpy(y).to(cuda), n, k).cpu().numpy().astype(np.float64)
-        assert np.isnan(again[2]).all()
+        with np.errstate(invalid="ignore"):
+            product = w64[:, 700] * bad if fmt in (Q.Q6_K, Q.MXFP4) else np.full(n, np.nan)
+        assert np.array_equal(again[2], product, equal_nan=True)
         keep = [0, 1, 3, 4, 5, 6, 7]
         assert np.array_equal(again[keep], got[keep])
 
@@ -212,3 +216,33 @@ def test_decode_batch_with_scales_of_any_size(fmt, scale, oracle, cuda):
         large = (x[2].astype(np.float64) @ weights_of(oracle, fmt, w, n, k).T).astype(np.float32)
     assert not np.isnan(again[2]).any() and np.array_equal(np.isinf(again[2]), np.isinf(large))
     assert np.array_equal(np.sign(again[2][np.isinf(large)]), np.sign(large[np.isinf(large)]))
+
+
+@pytest.mark.parametrize("fmt,n,k,kept", [(Q.MXFP6_E2M3, 8400, 1024, True), (Q.MXFP6_E2M3, 40, 4096, True), (Q.Q6_K, 4096, 4096, True),
+                                          (Q.Q6_K, 64, 9216, True), (Q.Q6_K, 1024, 9216, False), (Q.MXFP4, 1024, 9216, False),
+                                          (Q.MXFP4, 64, 544, True), (Q.Q4_K, 256, 1024, True), (Q.Q4_K, 256, 1280, False), (Q.Q8_0, 256, 1024, False)])
+@pytest.mark.parametrize("m", [5, 8])
+def test_an_infinity_in_a_decode_batch(fmt, n, k, kept, m, oracle, cuda):
+    """kept: the product of an infinity and a weight that is not zero stays an infinity (one of zero is NaN; Q4_K multiplies
+    code and min apart, either of which may be zero, and adds the two); else all of that vector's results are NaN."""
+    import torch
+    from rocmforge_amd import ops
+    w = Q.make_weights(fmt, n, k, seed=4)
+    w64 = weights_of(oracle, fmt, w, n, k)
+    x = np.random.default_rng(5).standard_normal((m, k)).astype(np.float32)
+    dw = torch.from_numpy(w).to(cuda)
+    got = ops.gemv(fmt, dw, torch.from_numpy(x).to(cuda), n, k).cpu().numpy()
+    for at, bad in ((3, np.inf), (k - 1, -np.inf)):
+        y = x.copy()
+        y[m - 2, at] = bad
+        again = ops.gemv(fmt, dw, torch.from_numpy(y).to(cuda), n, k).cpu().numpy()
+        assert np.array_equal(np.delete(again, m - 2, 0), np.delete(got, m - 2, 0))
+        with np.errstate(invalid="ignore"):
+            product = w64[:, at] * bad
+        if not kept:
+            assert np.isnan(again[m - 2]).all()
+        elif fmt != Q.Q4_K:
+            assert np.array_equal(again[m - 2], product.astype(np.float32), equal_nan=True)
+        else:
+            inf = np.isinf(again[m - 2])
+            assert inf.any() and np.array_equal(again[m - 2][inf], product[inf].astype(np.float32)) and np.isnan(again[m - 2][~inf]).all()
