@@ -867,8 +867,14 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
         if constexpr (NORM) {                                     // (one step of Newton's iteration: an error here is the whole vector's)
             double sq = 0.0;
             for (int wv = 0; wv < waves; wv++) sq += (double)squares[wv * MV + v];
+            if (!(sq <= 3.40282347e+38)) {                        // (rarely: as the norm alone has it, x / infinity)
+                bool finite = sq == sq;
+                for (int j = 0; j < k && finite; j++) finite = fabsf(x[(size_t)v * k + j]) <= 3.40282347e+38f;
+                y[(size_t)v * n + n0 + c] = finite ? 0.0f : __uint_as_float(0x7FC00000u);
+                continue;
+            }
             const double mean = __builtin_fma(sq, 1.0 / (double)k, (double)eps), r0 = (double)(1.0f / sqrtf((float)mean));
-            rinv = r0 * __builtin_fma(-0.5 * mean, r0 * r0, 1.5);
+            rinv = r0 <= 3.40282347e+38 ? r0 * __builtin_fma(-0.5 * mean, r0 * r0, 1.5) : r0;
         }
         if (glu) {
             const int at = 32 * (c >> 4) + (c & 15);

@@ -246,3 +246,31 @@ def test_an_infinity_in_a_decode_batch(fmt, n, k, kept, m, oracle, cuda):
         else:
             inf = np.isinf(again[m - 2])
             assert inf.any() and np.array_equal(again[m - 2][inf], product[inf].astype(np.float32)) and np.isnan(again[m - 2][~inf]).all()
+
+
+@pytest.mark.parametrize("fmt", [Q.Q8_0, Q.Q4_K, Q.MXFP6_E2M3])
+@pytest.mark.parametrize("m", [3, 8])
+def test_norm_of_vectors_whose_squares_overflow(fmt, m, oracle, cuda):
+    """Finite x whose float32 sum of squares is infinite is zero after the norm (x / infinity), and so are its results, alone
+    and as gate and up projection; with an infinity or a NaN in x the vector's results are NaN; the others keep theirs."""
+    import torch
+    from rocmforge_amd import ops
+    n, k = 512, 1024
+    w, up = Q.make_weights(fmt, n, k, seed=1), Q.make_weights(fmt, n, k, seed=2)
+    down = Q.make_weights(Q.Q8_0, k, n, seed=3)
+    x = np.random.default_rng(3).standard_normal((m, k)).astype(np.float32)
+    dev = [torch.from_numpy(t).to(cuda) for t in (w, up, down, np.ones(k, np.float32))]
+
+    def both(x):
+        dx = torch.from_numpy(x).to(cuda)
+        return (ops.rms_norm_gemv(fmt, dev[0], dx, dev[3], 1e-5, n, k).cpu().numpy(),
+                ops.mlp_swiglu(fmt, dev[0], dev[1], Q.Q8_0, dev[2], dx, dev[3], 1e-5, k, n).cpu().numpy())
+    ordinary = both(x)
+    y = x.copy()
+    y[1] *= np.float32(3e37)
+    for got, before in zip(both(y), ordinary):
+        assert np.all(got[1] == 0) and np.array_equal(np.delete(got, 1, 0), np.delete(before, 1, 0))
+    for bad in (np.inf, -np.inf, np.nan):
+        y[1, 700] = bad
+        for got, before in zip(both(y), ordinary):
+            assert np.isnan(got[1]).all() and np.array_equal(np.delete(got, 1, 0), np.delete(before, 1, 0))
