@@ -937,7 +937,7 @@ gemm_skinny_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ a,
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
-    const int groups = k >> 5, units = (groups + 3) >> 2;
+    const int groups = k >> 5, units = groups >> 2;               // (whole units; what is left of a row comes after them)
     const int n0 = blockIdx.x * (16 * TJ);
     const size_t row_bytes = (size_t)(k / Fmt<FMT>::BE) * Fmt<FMT>::BB;
     const uint8_t *row[TJ];                                       // (weights: lane 4 * i + g fetches group g of row i)
@@ -970,8 +970,8 @@ gemm_skinny_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ a,
     WF raw[D][TJ];
     AF ar[AD][MT];
     auto load_w = [&](WF (&dst)[TJ], int u) __attribute__((always_inline)) {
-        const int uc = u < units ? u : units - 1;
-        const int g = 4 * uc + lg < groups ? lg : groups - 1 - 4 * uc;  // (past the row's end: its last group, as zeros)
+        const int uc = u < units ? u : units > 0 ? units - 1 : 0;
+        const int g = 4 * uc + lg < groups ? lg : groups - 1 - 4 * uc;  // (past the row's end: its last group)
 #pragma unroll
         for (int t = 0; t < TJ; t++) dst[t].load(row[t], uc, g);
     };
@@ -996,6 +996,55 @@ gemm_skinny_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ a,
 #pragma unroll
     for (int d = 0; d < D; d++) load_w(raw[d], wave + d * waves);
 
+    // one group's activations to operands
+    auto operands = [&](const AF (&src)[MT], v4u (&xa)[MT]) __attribute__((always_inline)) {
+        if constexpr (!AF::STAGED) {
+#pragma unroll
+            for (int b = 0; b < MT; b++) xa[b] = src[b].ordered();
+        } else {
+            wave_order();                                         // (the group before has been read)
+#pragma unroll
+            for (int b = 0; b < MT; b++) {
+                const v4u o = src[b].ordered();
+                if constexpr (AF::OCT) {
+                    *reinterpret_cast<v4u *>(area + b * ABLK + st0) = o;
+                } else {
+                    *reinterpret_cast<v2u *>(area + b * ABLK + st0) = v2u{o[0], o[1]};
+                    *reinterpret_cast<v2u *>(area + b * ABLK + st1) = v2u{o[2], o[3]};
+                }
+            }
+            wave_order();
+#pragma unroll
+            for (int b = 0; b < MT; b++) xa[b] = *reinterpret_cast<const v4u *>(area + b * ABLK + rd);
+        }
+    };
+    auto multiply = [&](const WF (&cur)[TJ], const v4u (&xa)[MT], int j) __attribute__((always_inline)) {
+        v4u wf[TJ];
+        float s0[TJ], s1[TJ], mn[TJ];
+#pragma unroll
+        for (int t = 0; t < TJ; t++) {
+            wf[t] = cur[t].frag(j);
+            s0[t] = cur[t].sc(j, 0);
+            s1[t] = WF::SPLIT16 ? cur[t].sc(j, 1) : 0.f;
+            mn[t] = WF::MINS ? cur[t].mn(j) : 0.f;
+        }
+#pragma unroll
+        for (int b = 0; b < MT; b++) {
+            v4f xs[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            if constexpr (WF::MINS) contract<false>(xa[b], ones, xs);
+#pragma unroll
+            for (int t = 0; t < TJ; t++) {
+                v4f p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                contract<WF::SPLIT16>(xa[b], wf[t], p);
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    acc[b][t][r] = __builtin_fmaf(s0[t], p[0][r], acc[b][t][r]);
+                    if constexpr (WF::SPLIT16) acc[b][t][r] = __builtin_fmaf(s1[t], p[1][r], acc[b][t][r]);
+                    if constexpr (WF::MINS) acc[b][t][r] = __builtin_fmaf(mn[t], xs[0][r], acc[b][t][r]);
+                }
+            }
+        }
+    };
     for (int u0 = wave; u0 < units; u0 += D * waves) {
 #pragma unroll
         for (int d = 0; d < D; d++) {
@@ -1005,65 +1054,43 @@ gemm_skinny_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ a,
 #pragma unroll
                 for (int t = 0; t < TJ; t++) {
                     cur[t] = placed<FMT>(raw[d][t], from4);
-                    cur[t].open(u, Fmt<FMT>::BE < 128 && 4 * u + q >= groups);
+                    cur[t].open(u, false);
                 }
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     v4u xa[MT];
-                    if constexpr (!AF::STAGED) {
-#pragma unroll
-                        for (int b = 0; b < MT; b++) xa[b] = ar[j % AD][b].ordered();
-                    } else {
-                        wave_order();                             // (the group before has been read)
-#pragma unroll
-                        for (int b = 0; b < MT; b++) {
-                            const v4u o = ar[j % AD][b].ordered();
-                            if constexpr (AF::OCT) {
-                                *reinterpret_cast<v4u *>(area + b * ABLK + st0) = o;
-                            } else {
-                                *reinterpret_cast<v2u *>(area + b * ABLK + st0) = v2u{o[0], o[1]};
-                                *reinterpret_cast<v2u *>(area + b * ABLK + st1) = v2u{o[2], o[3]};
-                            }
-                        }
-                        wave_order();
-#pragma unroll
-                        for (int b = 0; b < MT; b++) xa[b] = *reinterpret_cast<const v4u *>(area + b * ABLK + rd);
-                    }
+                    operands(ar[j % AD], xa);
                     load_a(ar[j % AD], j + AD < 4 ? u : u + waves, (j + AD) % 4);
-                    v4u wf[TJ];
-                    float s0[TJ], s1[TJ], mn[TJ];
-                    const bool dead = Fmt<FMT>::BE < 128 && 4 * u + j >= groups;
-#pragma unroll
-                    for (int t = 0; t < TJ; t++) {
-                        wf[t] = cur[t].frag(j);
-                        if (Fmt<FMT>::BE < 128) {
-#pragma unroll
-                            for (int r = 0; r < 4; r++) wf[t][r] = dead ? 0u : wf[t][r];
-                        }
-                        s0[t] = cur[t].sc(j, 0);
-                        s1[t] = WF::SPLIT16 ? cur[t].sc(j, 1) : 0.f;
-                        mn[t] = WF::MINS ? cur[t].mn(j) : 0.f;
-                    }
-#pragma unroll
-                    for (int b = 0; b < MT; b++) {
-                        v4f xs[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-                        if constexpr (WF::MINS) contract<false>(xa[b], ones, xs);
-#pragma unroll
-                        for (int t = 0; t < TJ; t++) {
-                            v4f p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-                            contract<WF::SPLIT16>(xa[b], wf[t], p);
-#pragma unroll
-                            for (int r = 0; r < 4; r++) {
-                                acc[b][t][r] = __builtin_fmaf(s0[t], p[0][r], acc[b][t][r]);
-                                if constexpr (WF::SPLIT16) acc[b][t][r] = __builtin_fmaf(s1[t], p[1][r], acc[b][t][r]);
-                                if constexpr (WF::MINS) acc[b][t][r] = __builtin_fmaf(mn[t], xs[0][r], acc[b][t][r]);
-                            }
-                        }
-                    }
+                    if constexpr (!AF::STAGED) __builtin_amdgcn_sched_barrier(0);   // (the loads go out before the group is multiplied)
+                    multiply(cur, xa, j);
                     if constexpr (MT >= 6) __builtin_amdgcn_sched_barrier(0);   // (the groups' operands side by side would not fit the registers)
                 }
             }
             load_w(raw[d], u + D * waves);
+        }
+    }
+    if constexpr (Fmt<FMT>::BE < 128) {
+        // The one to three groups behind the last whole unit, by the wavefront whose turn it is.  (As a unit filled up with
+        // zeros they would turn an infinity into NaN; a test before every group cost short rows 7 %.)
+        if ((groups & 3) != 0 && wave == units % waves) {
+            WF cur[TJ];
+#pragma unroll
+            for (int t = 0; t < TJ; t++) {
+                WF last;
+                last.load(row[t], units, 4 * units + lg < groups ? lg : 0);
+                cur[t] = placed<FMT>(last, from4);
+                cur[t].open(units, 4 * units + q >= groups);
+            }
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                if (4 * units + j < groups) {
+                    AF tail[MT];
+                    v4u xa[MT];
+                    load_a(tail, units, j);
+                    operands(tail, xa);
+                    multiply(cur, xa, j);
+                }
+            }
         }
     }
     // red[wave][row of a][16 * TJ rows of w]

@@ -274,3 +274,24 @@ def test_norm_of_vectors_whose_squares_overflow(fmt, m, oracle, cuda):
         y[1, 700] = bad
         for got, before in zip(both(y), ordinary):
             assert np.isnan(got[1]).all() and np.array_equal(np.delete(got, 1, 0), np.delete(before, 1, 0))
+
+
+@pytest.mark.parametrize("fmt", SHORT_BLOCKS)
+@pytest.mark.parametrize("k", [800, 832, 864, 896])
+@pytest.mark.parametrize("m,n", [(7, 72), (40, 9000)])
+def test_an_infinity_in_the_last_group_of_a_prompt_row(fmt, k, m, n, oracle, cuda):
+    """Rows that end inside a 128-element unit: what the kernel reads again to fill the unit is not multiplied, so that an
+    infinity among it does not become NaN: every output is the infinity's product with its weight."""
+    import torch
+    from rocmforge_amd import ops
+    w = Q.make_weights(fmt, n, k, seed=6)
+    a = np.random.default_rng(7).standard_normal((m, k)).astype(np.float16)
+    a[m // 2, k - 2] = -np.inf
+    dw, da = torch.from_numpy(w).to(cuda), torch.from_numpy(a).to(cuda)
+    with np.errstate(invalid="ignore"):
+        product = (weights_of(oracle, fmt, w, n, k)[:, k - 2] * -np.inf).astype(np.float32)
+    plain = ops.gemm_f16(fmt, dw, da, n, k, out_dtype=torch.float32).cpu().numpy()
+    arranged = ops.gemm_f16_arranged(fmt, dw, ops.ArrangedA(da), n, out_dtype=torch.float32).cpu().numpy()
+    for got in (plain, arranged):
+        assert np.array_equal(got[m // 2], product, equal_nan=True)
+        assert np.isfinite(np.delete(got, m // 2, 0)).all()
