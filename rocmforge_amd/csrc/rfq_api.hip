@@ -347,8 +347,12 @@ int rfq_rms_norm_gemv(int fmt, const void *d_w, size_t w_bytes, const float *d_x
     if (!d_scratch) return fail(RFQ_E_BADARG, "rfq_rms_norm_gemv: m=%d k=%d needs d_scratch (m * k floats)", m, k);
     if (k % 4 != 0 || !aligned16(d_x) || !aligned16(d_norm_weight) || !aligned16(d_scratch))
         return fail(RFQ_E_BADARG, "rfq_rms_norm_gemv: x, norm weight and scratch must be 16-byte aligned, k a multiple of 4");
-    rc = launch_skinny_gemv_fused(fmt, (const uint8_t *)d_w, nullptr, d_x, d_norm_weight, eps, d_y, m, n, k, s);
-    if (rc != RFQ_E_UNSUPPORTED) return rc;
+    // (a result written over x, or a norm in place: x is read before anything is written only by the separate steps)
+    const size_t x_bytes = (size_t)m * k * 4, y_bytes = (size_t)m * n * 4;
+    if (!overlap(d_y, y_bytes, d_x, x_bytes) && !overlap(d_y, y_bytes, d_norm_weight, (size_t)k * 4) && !overlap(d_scratch, x_bytes, d_x, x_bytes)) {
+        rc = launch_skinny_gemv_fused(fmt, (const uint8_t *)d_w, nullptr, d_x, d_norm_weight, eps, d_y, m, n, k, s);
+        if (rc != RFQ_E_UNSUPPORTED) return rc;
+    }
     rc = launch_rms_norm(RFQ_TABLE_F32, d_x, d_norm_weight, d_scratch, m, k, eps, s);
     if (rc != RFQ_OK) return rc;
     return launch_gemv(fmt, (const uint8_t *)d_w, d_scratch, d_y, m, n, k, s);

@@ -44,6 +44,11 @@ inline int fmt_block_elems(int fmt)
 // The loader's other K types (src/loader/dequant.rs:150-420): decoded by rfq_dequant*, on no matmul path.
 inline bool fmt_dequant_only(int fmt) { return fmt == RFQ_Q2_K || fmt == RFQ_Q3_K || fmt == RFQ_Q5_K; }
 // The matmul module's own decoders (src/kernels/matmul/quantized/): dequantisation and the two GEMV orientations.
+inline bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes)
+{
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return p < q + b_bytes && q < p + a_bytes;
+}
 inline bool fmt_mm_variant(int fmt) { return fmt == RFQ_MM_Q8_0 || fmt == RFQ_MM_Q4_K || fmt == RFQ_MM_Q6_K; }
 inline int fmt_block_bytes(int fmt)
 {

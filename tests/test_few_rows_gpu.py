@@ -295,3 +295,47 @@ def test_an_infinity_in_the_last_group_of_a_prompt_row(fmt, k, m, n, oracle, cud
     for got in (plain, arranged):
         assert np.array_equal(got[m // 2], product, equal_nan=True)
         assert np.isfinite(np.delete(got, m // 2, 0)).all()
+
+
+@pytest.mark.parametrize("m", [2, 5, 8])
+def test_norm_and_projection_over_their_own_input(m, cuda):
+    """rfq_rms_norm_gemv with the result written over x, and with x as its own scratch (then x holds the normalised rows):
+    the calls whose norm has to be a step of its own."""
+    import ctypes as C
+    import torch
+    from rocmforge_amd import _lib, ops
+    n = k = 1024
+    p = lambda t: C.c_void_p(t.data_ptr())
+    w = torch.from_numpy(Q.make_weights(Q.Q8_0, n, k, seed=1)).to(cuda)
+    gen = torch.Generator(device="cpu").manual_seed(2)
+    x, nw = torch.randn((m, k), generator=gen).to(cuda), torch.randn(k, generator=gen).to(cuda)
+    want = ops.rms_norm_gemv(Q.Q8_0, w, x, nw, 1e-5, n, k).cpu().numpy()
+    xn = ops.rms_norm(x, nw, 1e-5)
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for y, scratch in (("x", "own"), ("own", "x")):
+        into = x.clone()
+        own = torch.zeros((m, k), device=cuda)
+        _lib.check(_lib.lib().rfq_rms_norm_gemv(Q.Q8_0, p(w), w.numel(), p(into), p(nw), 1e-5, p(into if y == "x" else own), m, n, k,
+                                                p(into if scratch == "x" else own), stream))
+        assert_close((into if y == "x" else own).cpu().numpy(), want, f"result over {y}, scratch {scratch}", tol=TOL, plain_tol=2e-4)
+        if scratch == "x":
+            assert torch.equal(into, xn)
+
+
+@pytest.mark.parametrize("m,k,dtype", [(9, 1024, "f16"), (100, 1024, "f16"), (40, 2048, "f32")])
+def test_prompt_over_its_own_activations(m, k, dtype, cuda):
+    """The output in the activations' memory (n * size of an output = k * 2): read whole before it is written."""
+    import ctypes as C
+    import torch
+    from rocmforge_amd import _lib, ops
+    n = k if dtype == "f16" else k // 2
+    out_dtype = torch.float16 if dtype == "f16" else torch.float32
+    p = lambda t: C.c_void_p(t.data_ptr())
+    w = torch.from_numpy(Q.make_weights(Q.GGUF_Q4_K, n, k, seed=1)).to(cuda)
+    a = torch.randn((m, k), generator=torch.Generator(device="cpu").manual_seed(2)).to(cuda).half()
+    want = ops.gemm_f16(Q.GGUF_Q4_K, w, a, n, k, out_dtype=out_dtype).float().cpu().numpy()
+    into = a.clone()
+    _lib.check(_lib.lib().rfq_gemm_f16(Q.GGUF_Q4_K, p(w), w.numel(), p(into), p(into), _lib.F16 if dtype == "f16" else _lib.F32, m, n, k,
+                                       C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    got = into.view(out_dtype)[:, :n].float().cpu().numpy()
+    assert_close(got, want, f"{m}x{n}x{k} {dtype}", tol=2e-5 if dtype == "f32" else 2.0 ** -10, plain_tol=None)
