@@ -121,8 +121,8 @@ int launch_gemv_traced(int fmt, const uint8_t *d_w, const float *d_x, float *d_y
                        size_t capacity_waves, int *waves, hipStream_t s);
 // Few rows of activations on the matrix cores (rfq_skinny.hip, compiled in four parts): float32 x with m <= 8 (SkinnyGemv;
 // w2 != nullptr: y = swiglu over two matrices of one shape, norm_w != nullptr: x is RMSNorm(x) * norm_w), or float16 a (rows
-// or arranged).  The caller has checked formats, shapes and alignment (weights on multiples of 4, activations and the norm
-// weight of 16).
+// or arranged).  The caller has checked formats, shapes and alignment: few_rows_aligned for float32 x (and a norm weight on a
+// multiple of 16), weights on multiples of 4 and activations of 16 for float16.
 struct SkinnyGemv {
     const uint8_t *w, *w2;
     const float *x, *norm_w;
@@ -132,6 +132,7 @@ struct SkinnyGemv {
     int keep_infinities;                                          // an infinity in x: see keeps_infinities; 0: its vector's results are NaN
 };
 int launch_skinny_gemv(int fmt, const SkinnyGemv &c, hipStream_t s);
+bool few_rows_aligned(int fmt, const void *w, const void *w2, const void *x);
 // Whether the above is the faster way for rows of x [m, k] and this matrix (m >= 2), alone and with what it takes along.
 bool few_rows_ahead(int fmt, int m, int n, int ku, bool batch_fits);
 // Whether a batch with an infinity in x gives infinities (NaN only against a zero weight) or NaN for all of the vector's

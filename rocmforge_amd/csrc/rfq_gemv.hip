@@ -2467,7 +2467,7 @@ int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStre
     if (m == 1 && ku > 16 && ku <= 512)                        // (shorter rows leave most of a wavefront's lanes without a unit)
         return run_rows<FMT, false>(w, x, y, n, k, GemvFuse{nullptr, nullptr, 0.0f, 0}, s);
     const bool batch_fits = HasIdotBatch<FMT>::value && ku > 32 && ku <= 256;
-    if (m > 1 && (reinterpret_cast<uintptr_t>(w) & 3u) == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && few_rows_ahead(FMT, m, n, ku, batch_fits)) {
+    if (m > 1 && few_rows_aligned(FMT, w, nullptr, x) && few_rows_ahead(FMT, m, n, ku, batch_fits)) {
         note_kernel("gemv_skinny_kernel<%s>", FMT, 0, 0, 0);
         return launch_skinny_gemv(FMT, SkinnyGemv{w, nullptr, x, nullptr, 0.0f, y, m, n, k, keeps_infinities(FMT, n, ku, batch_fits)}, s);
     }
@@ -2594,6 +2594,15 @@ int launch_gemv(int fmt, const uint8_t *d_w, const float *d_x, float *d_y, int m
     }
 }
 
+// The few-row kernel loads x and the blocks that are whole dwords at any address (Q8_0 4096 x 4096 m = 8 with x off a 16-byte
+// boundary 8.1 us, 15.5 as two integer-dot launches); the other blocks come through aligned windows, which must not begin before the tensor.
+bool few_rows_aligned(int fmt, const void *w, const void *w2, const void *x)
+{
+    const bool windows = fmt == RFQ_GGUF_Q4_0 || fmt == RFQ_GGUF_Q8_0 || fmt == RFQ_GGUF_Q6_K || fmt == RFQ_MXFP4 || fmt == RFQ_MXFP6_E2M3;
+    if (windows && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(w2)) & 3u) != 0) return false;
+    return (reinterpret_cast<uintptr_t>(x) & 3u) == 0;
+}
+
 // Whether a batch goes through the matrix-core kernel for few rows (rfq_skinny.hip) instead of the integer-dot batch kernel
 // (batch_fits) or, where a format or row length has none, one decode launch per vector or the one-row-per-wavefront
 // kernel.  Its time hardly depends on m; measured on 512..14336 rows of 768..13824 for every format (us, there / here):
@@ -2638,9 +2647,7 @@ int launch_skinny_gemv_fused(int fmt, const uint8_t *d_w, const uint8_t *d_w2, c
 {
     const int cf = canonical_format(fmt), ku = k / 32, cus = device_cu_count();
     if (m < 2 || m > 8 || gemv_part_of(cf) < 0 || fmt_mm_variant(fmt)) return RFQ_E_UNSUPPORTED;
-    const uintptr_t ws = reinterpret_cast<uintptr_t>(d_w) | reinterpret_cast<uintptr_t>(d_w2);
-    const uintptr_t xs = reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_norm_w);
-    if ((ws & 3u) != 0 || (xs & 15u) != 0) return RFQ_E_UNSUPPORTED;
+    if (!few_rows_aligned(cf, d_w, d_w2, d_x) || (reinterpret_cast<uintptr_t>(d_norm_w) & 15u) != 0) return RFQ_E_UNSUPPORTED;
     const bool per_vector = cf == RFQ_Q6_K || cf == RFQ_MXFP4 || cf == RFQ_MXFP6_E2M3;
     const bool batch_fits = !per_vector && ku > 32 && ku <= 256;
     // (with two vectors the batch kernel of these two formats is further ahead: GGUF_Q6_K 2 x 3072 -> 4864 12.5 / 14.2 us)

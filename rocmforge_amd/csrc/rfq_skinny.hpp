@@ -44,6 +44,7 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v4f_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 
@@ -104,22 +105,23 @@ __device__ __forceinline__ void bytes2h(uint32_t d, float bias, uint32_t &p01, u
     p23 = add2h(__builtin_amdgcn_perm(0x64646464u, d, 0x04030402u), bias - 1024.0f);
 }
 
+// (any address: where a format's blocks are fetched through aligned windows the caller has rounded it down)
 template <int NW> __device__ __forceinline__ void load_dwords(const uint8_t *a, uint32_t (&d)[NW])
 {
-    typedef uint32_t v4a4 __attribute__((ext_vector_type(4), aligned(4)));
-    typedef uint32_t v2a4 __attribute__((ext_vector_type(2), aligned(4)));
+    typedef uint32_t v4a1 __attribute__((ext_vector_type(4), aligned(1)));
+    typedef uint32_t v2a1 __attribute__((ext_vector_type(2), aligned(1)));
     int i = 0;
 #pragma unroll
     for (; i + 4 <= NW; i += 4) {
-        const v4a4 v = *reinterpret_cast<const v4a4 *>(a + 4 * i);
+        const v4a1 v = *reinterpret_cast<const v4a1 *>(a + 4 * i);
         d[i] = v[0]; d[i + 1] = v[1]; d[i + 2] = v[2]; d[i + 3] = v[3];
     }
     if (i + 2 <= NW) {
-        const v2a4 v = *reinterpret_cast<const v2a4 *>(a + 4 * i);
+        const v2a1 v = *reinterpret_cast<const v2a1 *>(a + 4 * i);
         d[i] = v[0]; d[i + 1] = v[1];
         i += 2;
     }
-    if (i < NW) d[i] = *reinterpret_cast<const uint32_t *>(a + 4 * i);
+    if (i < NW) d[i] = ld<uint32_t>(a + 4 * i);
 }
 // Which eight elements of a group lane row q holds, and in which order its four operand dwords hold them.
 enum { OCTET, OCTET_SWAPPED, HALVES };                           // 8q..  |  8q'.. (q' = q with its bits swapped)  |  4q.. and 16+4q..
@@ -235,7 +237,7 @@ template <> struct W<RFQ_Q4_K> {                                 // 256-byte lay
         const uint8_t *blk = row + (uint32_t)(u >> 1) * 256u;
         const int h = u & 1;
         // (lanes 0, 1: two scales each; lanes 2, 3: the unit's four mins)
-        r[4] = *reinterpret_cast<const uint32_t *>(blk + (g < 2 ? 8 * h + 4 * g : 16 + 4 * h));
+        r[4] = ld<uint32_t>(blk + (g < 2 ? 8 * h + 4 * g : 16 + 4 * h));
         const U4 v = ld_once<U4>(blk + 32 + 28 * (4 * h + g));
 #pragma unroll
         for (int i = 0; i < 4; i++) r[i] = v.v[i];
@@ -261,7 +263,7 @@ template <> struct W<RFQ_GGUF_Q4_K> {
     {
         const uint8_t *blk = row + (uint32_t)(u >> 1) * 144u;
         uint32_t b[4];
-        r[4] = *reinterpret_cast<const uint32_t *>(blk + 4 * g);
+        r[4] = ld<uint32_t>(blk + 4 * g);
         load_dwords<4>(blk + 16 + 64 * (u & 1) + 16 * g, b);
 #pragma unroll
         for (int i = 0; i < 4; i++) r[i] = b[i];
@@ -305,7 +307,7 @@ template <> struct W<RFQ_Q6_K> {
     {
         const uint8_t *blk = row + (uint32_t)(u >> 1) * 256u;
         const int c = 4 * (u & 1) + g;
-        r[6] = *reinterpret_cast<const uint32_t *>(blk + 4 * c);
+        r[6] = ld<uint32_t>(blk + 4 * c);
         uint32_t v[6];
         load_dwords<6>(blk + 32 + 24 * c, v);
 #pragma unroll
@@ -662,8 +664,8 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
         const int at = 128 * uc + 8 * i < k ? 128 * uc : 128 * uc - 32 * (i >> 2);   // (past the end: the unit's first group)
 #pragma unroll
         for (int p = 0; p < P; p++) {
-            xr[p][0] = *reinterpret_cast<const v4f *>(xl[p] + at);
-            xr[p][1] = *reinterpret_cast<const v4f *>(xl[p] + at + 4);
+            xr[p][0] = *reinterpret_cast<const v4f_a4 *>(xl[p] + at);
+            xr[p][1] = *reinterpret_cast<const v4f_a4 *>(xl[p] + at + 4);
         }
         if constexpr (NORM) {
             nr[0] = *reinterpret_cast<const v4f *>(norm_w + 8 * i + at);

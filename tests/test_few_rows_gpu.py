@@ -339,3 +339,34 @@ def test_prompt_over_its_own_activations(m, k, dtype, cuda):
                                        C.c_void_p(torch.cuda.current_stream().cuda_stream)))
     got = into.view(out_dtype)[:, :n].float().cpu().numpy()
     assert_close(got, want, f"{m}x{n}x{k} {dtype}", tol=2e-5 if dtype == "f32" else 2.0 ** -10, plain_tol=None)
+
+
+@pytest.mark.parametrize("fmt", BATCH_FORMATS)
+@pytest.mark.parametrize("m,n,k", [(3, 3100, 3072), (6, 130, 1056), (8, 40, 13824)])
+def test_decode_batches_at_any_address(fmt, m, n, k, oracle, cuda):
+    """x on a 4-byte boundary and, where the blocks are whole dwords, weights at any byte: the same kernel and the same bits
+    as on a 16-byte boundary; elsewhere other kernels take the unaligned weights."""
+    import torch
+    from rocmforge_amd import _lib, ops
+    if fmt in FORMATS:
+        n, k = shape_of(fmt, n, k)
+    w = torch.from_numpy(Q.make_weights(fmt, n, k, seed=fmt)).to(cuda)
+    x = torch.randn((m, k), generator=torch.Generator(device="cpu").manual_seed(m)).to(cuda)
+    kernel = lambda: _lib.lib().rfq_bench_last_gemv_kernel().decode()
+    want = ops.gemv(fmt, w, x, n, k)
+    assert kernel().startswith("gemv_skinny_kernel")
+    space = torch.empty(m * k + 4, device=cuda)
+    for off in (1, 2, 3):
+        moved = space[off : off + m * k].view(m, k)
+        moved.copy_(x)
+        assert moved.data_ptr() % 16 == 4 * off
+        assert torch.equal(ops.gemv(fmt, w, moved, n, k), want) and kernel().startswith("gemv_skinny_kernel")
+    space = torch.empty(w.numel() + 4, dtype=torch.uint8, device=cuda)
+    windows = fmt in (Q.GGUF_Q4_0, Q.GGUF_Q8_0, Q.GGUF_Q6_K, Q.MXFP4, Q.MXFP6_E2M3)
+    for off in (2,) if windows else (1, 2, 3):
+        moved = space[off : off + w.numel()]
+        moved.copy_(w)
+        got = ops.gemv(fmt, moved, x, n, k)
+        assert kernel().startswith("gemv_skinny_kernel") != windows
+        assert_close(got.cpu().numpy(), want.cpu().numpy(), f"{Q.NAMES[fmt]} weights off by {off}", tol=TOL, plain_tol=2e-4)
+        assert windows or torch.equal(got, want)
