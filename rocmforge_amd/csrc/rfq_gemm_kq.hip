@@ -753,6 +753,7 @@ int launch_cfg(const uint8_t *w, const void *a, void *out, int m, int n, int k, 
     // four weight stages + the Q4_K min fragment (+ the integer-operand kernel's two header areas)
     constexpr int LDS = 4 * W_BYTES + BN * 48 + (FMT == KQ_GGUF_Q4_K_INT ? 2 * (2 * BN * 48 + 2 * BN * 4) : 0);
     static_assert(LDS <= 160 * 1024, "LDS budget");
+    constexpr int FORMAT = FMT == KQ_GGUF_Q4_K_INT ? (int)RFQ_GGUF_Q4_K : (int)FMT;
     // (both output types: a launch split along k writes f32 parts whatever the caller's type)
     static std::once_flag once;
     static hipError_t attr_err = hipSuccess;
@@ -769,6 +770,7 @@ int launch_cfg(const uint8_t *w, const void *a, void *out, int m, int n, int k, 
         // (the caller's buffer holds the arranged activations only: nowhere to put parts, no split along k)
         const v4u *at = reinterpret_cast<const v4u *>(arranged);
         const _Float16 *s2 = reinterpret_cast<const _Float16 *>(arranged + arranged_at_bytes(m, k));
+        note_kernel("gemm_kq_kernel<%s,%d,%d,arranged>", FORMAT, PLANES, 1, 0);
         hipLaunchKernelGGL((gemm_kq_kernel<FMT, OUT_F16, PLANES>), dim3(tiles), dim3(256), LDS, s, w, at, s2, out, m, n, k, 1);
         RFQ_LAUNCH_CHECK("gemm_kq_kernel");
         return RFQ_OK;
@@ -798,6 +800,7 @@ int launch_cfg(const uint8_t *w, const void *a, void *out, int m, int n, int k, 
     }
     v4u *at = reinterpret_cast<v4u *>(tmp);
     _Float16 *s2 = reinterpret_cast<_Float16 *>(tmp + at_bytes);
+    note_kernel("gemm_kq_kernel<%s,%d,%d>", FORMAT, PLANES, kparts, 0);
     hipLaunchKernelGGL((arrange_a_kernel<SUMS>), dim3((unsigned)(tiles32 * ((nst + 3) / 4))), dim3(256), 0, s,
                        reinterpret_cast<const _Float16 *>(a), at, s2, m, k, tiles32, nst);
     if (kparts > 1) {

@@ -58,7 +58,6 @@ namespace {
 
 // Which kernel the last GEMV launch of this thread took (name and template arguments), for the benchmark
 // driver's report: plain stores on the launch path, formatted only when asked for.
-inline void note_kernel(const char *name, int fmt, int a, int b, int c) { g_gemv_last_kernel = GemvLastKernel{name, fmt, a, b, c}; }
 
 // ---- wavefront reduction -----------------------------------------------------
 
@@ -2468,15 +2467,12 @@ int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStre
         return run_rows<FMT, false>(w, x, y, n, k, GemvFuse{nullptr, nullptr, 0.0f, 0}, s);
     const bool batch_fits = HasIdotBatch<FMT>::value && ku > 32 && ku <= 256;
     if (m > 1 && few_rows_aligned(FMT, w, nullptr, x) && few_rows_ahead(FMT, m, n, ku, batch_fits)) {
-        note_kernel("gemv_skinny_kernel<%s>", FMT, 0, 0, 0);
         return launch_skinny_gemv(FMT, SkinnyGemv{w, nullptr, x, nullptr, 0.0f, y, m, n, k, keeps_infinities(FMT, n, ku, batch_fits)}, s);
     }
     if (batch_fits && m > 1) {
-        // the prepared vectors of a launch live in LDS (112 bytes per unit and vector): a batch that
-        // does not fit goes out as launches of four or two vectors
-        const size_t lds_limit = 160 * 1024 - 4096;
-        int mb = m <= 2 ? 2 : 4;
-        while (mb > 2 && (size_t)mb * ku * 112 > lds_limit) mb /= 2;
+        // (four vectors at most: the prepared ones of a launch live in LDS, 112 bytes per unit and vector)
+        static_assert(4 * 256 * 112 <= 160 * 1024 - 4096, "the longest rows' prepared vectors fit");
+        const int mb = m <= 2 ? 2 : 4;
         for (int v0 = 0; v0 < m; v0 += mb) {
             const int mv = m - v0 < mb ? m - v0 : mb;
             const float *xv = x + (size_t)v0 * k;

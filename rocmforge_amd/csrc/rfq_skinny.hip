@@ -43,6 +43,7 @@ int gemv_cfg(const SkinnyGemv &c, hipStream_t s)
     static_assert(gemv_lds<TJ, MV>(GEMV_WAVES) <= 64 * 1024, "LDS a launch gets without asking");
     const size_t lds = (size_t)gemv_lds<TJ, MV>(waves);
     const int rows = c.w2 != nullptr ? 8 * TJ : 16 * TJ;
+    note_kernel(c.w2 != nullptr ? "gemv_skinny_kernel<%s,%d,%d,%d,pair>" : "gemv_skinny_kernel<%s,%d,%d,%d>", FMT, TJ, MV, NORM);
     hipLaunchKernelGGL((gemv_skinny_kernel<FMT, TJ, MV, D, GEMV_WAVES, NORM>), dim3((c.n + rows - 1) / rows), dim3(64 * waves), lds, s, c.w, c.x,
                        c.y, c.m, c.n, c.k, c.w2, c.norm_w, c.eps, c.keep_infinities);
     RFQ_LAUNCH_CHECK("gemv_skinny_kernel");
@@ -90,6 +91,7 @@ int gemm_cfg(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, in
         });
         if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(gemm_skinny_kernel)");
     }
+    note_kernel(ARR ? "gemm_skinny_kernel<%s,%d,%d,%d,arranged>" : "gemm_skinny_kernel<%s,%d,%d,%d>", FMT, MT, TJ, slices);
     hipLaunchKernelGGL((gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES>), dim3((n + 16 * TJ - 1) / (16 * TJ), slices), dim3(64 * waves), lds, s,
                        w, a, y, f16_out, m, n, k, rows);
     RFQ_LAUNCH_CHECK("gemm_skinny_kernel");

@@ -551,8 +551,6 @@ __device__ __forceinline__ void contract(const v4u &xa, const v4u &wf, v4f (&d)[
     }
 }
 
-constexpr int MAX_WAVES = 16;
-
 // Between a wavefront's writes to its own part of LDS and other lanes' reads of them (and before the part is written again):
 // the hardware completes a wavefront's LDS operations in order, this keeps the compiler from moving them across.  No instruction.
 __device__ __forceinline__ void wave_order()

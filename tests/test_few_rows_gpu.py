@@ -1,7 +1,6 @@
 """GPU: the matrix-core kernels for few rows of activations (short prompts through rfq_gemm_f16 and
-rfq_gemm_f16_arranged, decode batches of 2 to 8 through rfq_gemv) at the edges of their tiles: rows per operand (16), rows
-per slice (128), weight rows per workgroup (16 and 32), 128-element units of k and their remainders, more and fewer units
-than wavefronts; against the float64 contraction of the decoded weights."""
+rfq_gemm_f16_arranged, decode batches of 2 to 8 through rfq_gemv) at the edges of their tiles: rows per operand (16), weight
+rows per workgroup (16 and 32), 128-element units of k and their remainders, more and fewer units than wavefronts; against the float64 contraction of the decoded weights."""
 import numpy as np
 import pytest
 
@@ -134,7 +133,7 @@ def test_norm_taken_along(fmt, m, n, k, oracle, cuda):
 
 
 @pytest.mark.parametrize("fmt", BATCH_FORMATS)
-@pytest.mark.parametrize("m,hidden,inter,norm", [(2, 256, 512, True), (3, 768, 1792, False), (5, 512, 6912, True), (8, 768, 2304, True)])
+@pytest.mark.parametrize("m,hidden,inter,norm", [(2, 256, 512, True), (3, 768, 1792, False), (3, 256, 6912, True), (5, 512, 6912, True), (8, 768, 2304, True)])
 def test_gate_and_up_in_one_launch(fmt, m, hidden, inter, norm, oracle, cuda):
     import torch
     from rocmforge_amd import ops
@@ -370,3 +369,77 @@ def test_decode_batches_at_any_address(fmt, m, n, k, oracle, cuda):
         assert kernel().startswith("gemv_skinny_kernel") != windows
         assert_close(got.cpu().numpy(), want.cpu().numpy(), f"{Q.NAMES[fmt]} weights off by {off}", tol=TOL, plain_tol=2e-4)
         assert windows or torch.equal(got, want)
+
+
+def kernel_name():
+    from rocmforge_amd import _lib
+    return _lib.lib().rfq_bench_last_gemv_kernel().decode()
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_every_prompt_kernel(fmt, oracle, cuda):
+    """Every form of the fp16 kernel that the dispatch can pick (16-row operands, row tiles of W; rows or arranged), at
+    ragged sizes: that it is the one taken, its results, and that both orders of the activations give the same bits."""
+    import torch
+    from rocmforge_amd import ops
+    most = 4 if fmt in (Q.Q4_0, Q.GGUF_Q4_0) else 8
+    forms = [((1, 1), 13, 1003), ((2, 1), 24, 4001), ((3, 1), 37, 4090), ((4, 1), 61, 4001), ((6, 1), 90, 4090), ((6, 1), 75, 4001),
+             ((1, 2), 12, 9001), ((2, 2), 24, 9001), ((3, 2), 41, 8999), ((4, 2), 60, 9001), ((4, 2) if most == 4 else (6, 2), 105 if most == 4 else 90, 8200),
+             ((4, 2) if most == 4 else (8, 2), 121, 8200)]
+    k = 544 if fmt in SHORT_BLOCKS else 512
+    w = Q.make_weights(fmt, 9001, k, seed=fmt)
+    dw = torch.from_numpy(w).to(cuda)
+    w64 = weights_of(oracle, fmt, w, 9001, k)
+    for form, m, n in forms:
+        a = np.random.default_rng(m).standard_normal((m, k)).astype(np.float16)
+        da, part = torch.from_numpy(a).to(cuda), dw[: Q.packed_bytes(fmt, n * k)]
+        want = a.astype(np.float64) @ w64[:n].T
+        plain = ops.gemm_f16(fmt, part, da, n, k, out_dtype=torch.float32)
+        name = kernel_name()
+        assert name.startswith(f"gemm_skinny_kernel<{Q.NAMES[fmt]},{form[0]},{form[1]},") and "arranged" not in name, (name, form, m, n)
+        arranged = ops.gemm_f16_arranged(fmt, part, ops.ArrangedA(da), n, out_dtype=torch.float32)
+        assert kernel_name() == name[:-1] + ",arranged>"
+        assert torch.equal(plain, arranged)
+        assert_close(plain.cpu().numpy(), want, f"{Q.NAMES[fmt]} {m}x{n}x{k} {form}", tol=TOL, plain_tol=2e-4)
+
+
+@pytest.mark.parametrize("fmt", BATCH_FORMATS)
+@pytest.mark.parametrize("norm", [False, True])
+def test_every_decode_batch_kernel(fmt, norm, oracle, cuda):
+    """Every form of the float32 kernel (row tiles of W, vectors) alone and with the norm: that it is the one taken, and its
+    results."""
+    import torch
+    from rocmforge_amd import ops
+    k = 768
+    w = Q.make_weights(fmt, 13400, k, seed=fmt)
+    dw = torch.from_numpy(w).to(cuda)
+    w64 = weights_of(oracle, fmt, w, 13400, k)
+    nw = (1 + 0.1 * np.random.default_rng(1).standard_normal(k)).astype(np.float32)
+    for (tj, mv), m, n in [((1, 4), 4, 1101), ((2, 4), 3, 5401), ((2, 4), 4, 13399), ((1, 8), 5, 1101), ((2, 8), 8, 5401), ((4, 8), 7, 13399)]:
+        x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32) * 3
+        dx, part = torch.from_numpy(x).to(cuda), dw[: Q.packed_bytes(fmt, n * k)]
+        x64 = x.astype(np.float64)
+        if norm:
+            got = ops.rms_norm_gemv(fmt, part, dx, torch.from_numpy(nw).to(cuda), 1e-5, n, k)
+            x64 = x64 / np.sqrt((x64 * x64).mean(axis=1, keepdims=True) + 1e-5) * nw
+        else:
+            got = ops.gemv(fmt, part, dx, n, k)
+        label = "MXFP6" if fmt == Q.MXFP6_E2M3 else Q.NAMES[fmt]
+        assert kernel_name() == f"gemv_skinny_kernel<{label},{tj},{mv},{int(norm)}>"
+        assert_close(got.cpu().numpy(), x64 @ w64[:n].T, f"{Q.NAMES[fmt]} {m}x{n}x{k}", tol=TOL, plain_tol=2e-4)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(300, 96, 2048), (700, 200, 4096)])
+def test_arranged_prompts_of_many_rows(fmt, m, n, k, oracle, cuda):
+    """Arranged activations of 256 rows and more take the few-row kernel over narrow matrices (they cannot be split along k):
+    slices of 16 rows and of more."""
+    import torch
+    from rocmforge_amd import ops
+    w = Q.make_weights(fmt, n, k, seed=fmt)
+    a = np.random.default_rng(m).standard_normal((m, k)).astype(np.float16)
+    got = ops.gemm_f16_arranged(fmt, torch.from_numpy(w).to(cuda), ops.ArrangedA(torch.from_numpy(a).to(cuda)), n, out_dtype=torch.float32)
+    assert kernel_name().startswith("gemm_skinny_kernel") != (fmt == Q.Q4_K)       # (Q4_K: as plain ones, which are split)
+    # (Q4_K's tiled kernel multiplies q * scale rounded to fp16 once)
+    assert_close(got.cpu().numpy(), a.astype(np.float64) @ weights_of(oracle, fmt, w, n, k).T, f"{Q.NAMES[fmt]} {m}x{n}x{k}",
+                 tol=1e-3 if fmt == Q.Q4_K else TOL, plain_tol=None if fmt == Q.Q4_K else 2e-4)
