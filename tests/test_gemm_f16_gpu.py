@@ -79,12 +79,19 @@ def test_small_shapes_fp32_out(fmt, m, n, k, oracle, cuda):
                      plain_tol=2e-4)
 
 
+def kernel_name():
+    from rocmforge_amd import _lib
+    return _lib.lib().rfq_bench_last_gemv_kernel().decode()
+
+
 @pytest.mark.parametrize("fmt", [Q.Q4_0, Q.Q8_0, Q.GGUF_Q4_0, Q.GGUF_Q8_0])
-def test_k_not_a_multiple_of_the_stage(fmt, oracle, cuda):
+@pytest.mark.parametrize("m,kernel", [(40, "gemm_skinny_kernel"), (300, "gemm_kq_kernel")])
+def test_k_not_a_multiple_of_the_stage(fmt, m, kernel, oracle, cuda):
     import torch
-    m, n, k = 40, 96, 96 + 64 * 3                                        # k % 64 == 32
+    n, k = 96, 96 + 64 * 3                                               # k % 64 == 32
     w, a = weights(fmt, n, k, 7), acts(m, k, 8)
     out = run(fmt, w, a, n, k, cuda, torch.float32).cpu().numpy()
+    assert kernel_name().startswith(kernel)
     assert_close(out, oracle.qmatmul_nk(fmt, w, a.astype(np.float32), m, n, k), "k tail")
     assert_close(out, exact_weight_product(oracle, fmt, w, a, n, k), "k tail (float64 sums)", tol=2e-5, plain_tol=2e-4)
 
@@ -155,12 +162,13 @@ def test_one_plane_is_the_fp16_rounded_contraction(fmt, oracle, cuda):
     assert not np.array_equal(out, two)
 
 
-def test_gguf_q4_k_super_block_scales_of_any_size(oracle, cuda):
+@pytest.mark.parametrize("m,kernel", [(70, "gemm_skinny_kernel"), (300, "gemm_kq_kernel<GGUF_Q4_K,1,2>")])
+def test_gguf_q4_k_super_block_scales_of_any_size(m, kernel, oracle, cuda):
     """GGUF_Q4_K is contracted with integer operands and its accumulators run in units of the current super-block's d:
     super-blocks whose d is +0, -0, negative, or 2^+-8 times the neighbour's (also in a row's first and last block,
     and a whole row of zeros) must come out as the oracle's."""
     import torch
-    m, n, k = 70, 140, 2048                                               # 8 super-blocks per row
+    n, k = 140, 2048                                                      # 8 super-blocks per row
     w = weights(Q.GGUF_Q4_K, n, k, 51).copy()
     blocks = w.reshape(n, k // 256, 144)
     d = blocks[:, :, 0:2].copy().view("<f2")[..., 0]                      # [n, 8]
@@ -182,7 +190,7 @@ def test_gguf_q4_k_super_block_scales_of_any_size(oracle, cuda):
     blocks[:, :, 2:4] = dmin.astype("<f2")[..., None].view(np.uint8)
     a = acts(m, k, 53)
     out = run(Q.GGUF_Q4_K, w, a, n, k, cuda, torch.float32).cpu().numpy()
-    assert np.isfinite(out).all()
+    assert kernel_name().startswith(kernel) and np.isfinite(out).all()
     want = oracle.qmatmul_nk(Q.GGUF_Q4_K, w, a.astype(np.float32), m, n, k)
     exact = exact_weight_product(oracle, Q.GGUF_Q4_K, w, a, n, k)
     for col in range(n):                                                  # (each weight row against its own output size)
@@ -191,23 +199,32 @@ def test_gguf_q4_k_super_block_scales_of_any_size(oracle, cuda):
     A = torch.from_numpy(a).to(cuda)
     from rocmforge_amd import ops
     wd = torch.from_numpy(w).to(cuda)
-    # (this shape is split along k in two parts by rfq_gemm_f16; the arranged entry point takes it in one pass)
-    one_pass = ops.gemm_f16_arranged(Q.GGUF_Q4_K, wd, ops.ArrangedA(A), n, out_dtype=torch.float32).cpu().numpy()
+    # (300 rows are split along k in two parts by rfq_gemm_f16, and few rows taken as they are; one pass over k by the
+    # integer-operand kernel: arranged activations and a matrix wide enough for it, the same rows in front)
+    if m == 300:
+        wide = torch.from_numpy(weights(Q.GGUF_Q4_K, 14336, k, 54)).to(cuda)
+        wide[: wd.numel()] = wd
+        one_pass = ops.gemm_f16_arranged(Q.GGUF_Q4_K, wide, ops.ArrangedA(A), 14336, out_dtype=torch.float32)[:, :n].cpu().numpy()
+        assert kernel_name() == "gemm_kq_kernel<GGUF_Q4_K,1,1,arranged>"
+    else:
+        one_pass = ops.gemm_f16_arranged(Q.GGUF_Q4_K, wd, ops.ArrangedA(A), n, out_dtype=torch.float32).cpu().numpy()
     for col in range(n):
         assert_close(one_pass[:, col], want[:, col], f"one pass over k, weight row {col}")
         assert_close(one_pass[:, col], exact[:, col], f"one pass over k (float64 sums), weight row {col}", tol=2e-5, plain_tol=2e-4)
 
 
 @pytest.mark.parametrize("fmt", FORMATS)
-@pytest.mark.parametrize("m,n,k,parts", [(300, 200, 2048, 2), (64, 130, 4096, 4), (33, 70, 8192, 8)])
+@pytest.mark.parametrize("m,n,k,parts", [(300, 200, 2048, 2), (300, 130, 4096, 4), (257, 70, 8192, 8), (64, 130, 4096, 4), (33, 70, 8192, 8)])
 def test_split_along_k(fmt, m, n, k, parts, oracle, cuda):
     """Few output tiles and a long k: the launch is split along k into whole super-blocks, the parts' f32 tiles are
-    added in a fixed order: against the oracle, deterministic, and the fp16 output is the rounded fp32 output."""
+    added in a fixed order: against the oracle, deterministic, and the fp16 output is the rounded fp32 output.  (Fewer than
+    256 rows of such shapes go to the kernel for few rows, which does not split k, whatever rfq_gemm_f16_k_parts answers.)"""
     import torch
     from rocmforge_amd import _lib
     assert _lib.lib().rfq_gemm_f16_k_parts(m, n, k) == parts
     w, a = weights(fmt, n, k, 61 + fmt), acts(m, k, 62 + n)
     out = run(fmt, w, a, n, k, cuda, torch.float32)
+    assert kernel_name().startswith("gemm_kq_kernel") == (m >= 256) and (m < 256 or kernel_name().endswith(f",{parts}>"))
     again = run(fmt, w, a, n, k, cuda, torch.float32)
     assert torch.equal(out, again)
     assert torch.equal(run(fmt, w, a, n, k, cuda, torch.float16), out.to(torch.float16))
@@ -237,12 +254,12 @@ def test_k_parts_rule():
 
 def test_weights_at_a_4_byte_offset_and_kept_temporary(oracle, cuda):
     """The weight loads need 4-byte alignment only; the per-stream temporary is
-    reused by a smaller call after a larger one (and grown by a larger one)."""
+    reused by a smaller call after a larger one (and grown by a larger one).  256 rows and more: fewer take no temporary."""
     import torch
     from rocmforge_amd import ops
     fmt = Q.Q4_K
     outs = []
-    for m, n, k in [(64, 128, 512), (300, 256, 1024), (64, 128, 512)]:
+    for m, n, k in [(260, 128, 512), (400, 256, 1024), (260, 128, 512)]:
         w, a = weights(fmt, n, k, 6), acts(m, k, 7)
         buf = torch.zeros(w.size + 4, dtype=torch.uint8, device=cuda)
         buf[4:] = torch.from_numpy(w).to(cuda)
@@ -252,8 +269,15 @@ def test_weights_at_a_4_byte_offset_and_kept_temporary(oracle, cuda):
         outs.append(out.cpu().numpy())
     assert np.array_equal(outs[0], outs[2])
     from rocmforge_amd import _lib
+    assert kernel_name().startswith("gemm_kq_kernel")
+    # one pass of a large call: its kept buffer (48 MiB) shows in the device's free memory once it is released
+    big = torch.zeros((4096, 6144), dtype=torch.float16, device=cuda)
+    ops.gemm_f16(Q.Q8_0, torch.zeros(Q.packed_bytes(Q.Q8_0, 128 * 6144), dtype=torch.uint8, device=cuda), big, 128, 6144)
+    torch.cuda.synchronize()
+    held = torch.cuda.mem_get_info()[0]
     assert _lib.lib().rfq_release_temporaries() == _lib.OK               # the next call allocates again
-    w, a = weights(fmt, 128, 512, 6), acts(64, 512, 7)
+    assert torch.cuda.mem_get_info()[0] >= held + (40 << 20)
+    w, a = weights(fmt, 128, 512, 6), acts(260, 512, 7)
     again = ops.gemm_f16(fmt, torch.from_numpy(w).to(cuda), torch.from_numpy(a).to(cuda), 128, 512, out_dtype=torch.float32)
     torch.cuda.synchronize()
     assert np.array_equal(again.cpu().numpy(), outs[0])

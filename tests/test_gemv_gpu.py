@@ -67,9 +67,9 @@ def test_gemv_batches_as_decode_launches(fmt, n, k, m, oracle, cuda):
     assert_close(got, oracle.qmatmul_nk(fmt, w, x, m, n, k), f"{Q.NAMES[fmt]} {n}x{k} m={m}")
 
 
-# Q8_0 batches run on the matrix cores: 16 rows per workgroup, 16 wavefronts
-# that take every 16th unit, eight units at a time: odd unit counts, more than
-# one trip, fewer units than wavefronts, a ragged last row tile.
+# Q8_0 batches that run on the matrix cores: 16 rows per workgroup, eight wavefronts
+# that take the 128-element units of k in turn: odd unit counts, more than one trip,
+# fewer units than wavefronts, a ragged last row tile.
 @pytest.mark.parametrize("fmt", [Q.Q8_0, Q.GGUF_Q8_0])
 @pytest.mark.parametrize("m,n,k", [(2, 16, 96), (4, 50, 8224), (8, 33, 4096), (7, 1, 32)])
 def test_q8_0_batches_on_the_matrix_cores(fmt, m, n, k, oracle, cuda):
@@ -83,8 +83,9 @@ def test_q8_0_batches_on_the_matrix_cores(fmt, m, n, k, oracle, cuda):
 
 @pytest.mark.parametrize("fmt", [Q.Q4_0, Q.Q4_K])
 @pytest.mark.parametrize("m,k", [(8, 4096), (8, 8192), (5, 8192), (3, 8192)])
-def test_batches_whose_prepared_vectors_exceed_lds(fmt, m, k, oracle, cuda):
-    """Eight prepared vectors of k = 8192 need 229 KB of LDS: the batch goes out as launches of four."""
+def test_batches_of_the_longest_rows_with_a_batch_kernel(fmt, m, k, oracle, cuda):
+    """k = 8192: the prepared vectors of the integer-dot batch kernel take the most LDS (three run as four: 115 KB); from
+    five vectors on the batch goes to the few-row kernel."""
     n = 150
     w = Q.make_weights(fmt, n, k, seed=5200 + fmt)
     x = x_for(m, k, 6200 + m)

@@ -23,12 +23,12 @@ def test_gemv_sequence_replays(cuda):
     def step():
         for f, w, y in zip(fmts, ws, ys):
             ops.gemv(f, w, x, n, k, out=y)
-        ops.gemv(Q.Q8_0, ws[1], xb, n, k, out=yb)          # the batched matrix-core kernel (uses the kept temporary)
+        ops.gemv(Q.Q8_0, ws[1], xb, n, k, out=yb)          # a batch in one launch
 
     side = torch.cuda.Stream()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(side):
-        step()                                             # first use on this stream allocates the kept temporary
+        step()
         torch.cuda.synchronize()
         with torch.cuda.graph(graph, stream=side):
             step()
@@ -47,10 +47,11 @@ def test_gemv_sequence_replays(cuda):
             assert torch.equal(g, w_)
 
 
-def test_prefill_gemms_replay(cuda):
+@pytest.mark.parametrize("m,kernel", [(96, "gemm_skinny_kernel"), (300, "gemm_kq_kernel")])
+def test_prefill_gemms_replay(m, kernel, cuda):
     import torch
     from rocmforge_amd import _lib, ops
-    m, n, k = 96, 256, 512
+    n, k = 256, 512
     w = torch.from_numpy(Q.make_weights(Q.Q4_K, n, k, seed=3)).to(cuda)
     a = torch.zeros((m, k), dtype=torch.float16, device=cuda)
     out = torch.empty((m, n), dtype=torch.float16, device=cuda)
@@ -62,12 +63,13 @@ def test_prefill_gemms_replay(cuda):
 
     def step():
         ops.gemm_f16(Q.Q4_K, w, a, n, k, out_dtype=torch.float16, out=out)
+        assert _lib.lib().rfq_bench_last_gemv_kernel().decode().startswith(kernel)
         ops.gemm_mx(A, W, out_dtype=torch.bfloat16, out=out_mx)
 
     side = torch.cuda.Stream()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(side):
-        step()                                             # the temporary is kept per stream: warm this one too
+        step()                                             # the temporary (from 256 rows on) is kept per stream: warm this one too
         torch.cuda.synchronize()
         with torch.cuda.graph(graph, stream=side):
             step()
@@ -87,7 +89,7 @@ def test_capture_refuses_to_allocate_temporaries(cuda):
     RFQ_E_UNSUPPORTED instead of allocating (or growing, which would free memory an earlier graph holds)."""
     import torch
     from rocmforge_amd import _lib, ops
-    m, n, k = 64, 128, 512
+    m, n, k = 264, 128, 512                                # (fewer than 256 rows take no temporary)
     w = torch.from_numpy(Q.make_weights(Q.Q4_K, n, k, seed=8)).to(cuda)
     a = torch.zeros((m, k), dtype=torch.float16, device=cuda)
     a2 = torch.zeros((4 * m, k), dtype=torch.float16, device=cuda)
@@ -96,7 +98,15 @@ def test_capture_refuses_to_allocate_temporaries(cuda):
     side = torch.cuda.Stream()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(side):
-        ops.gemm_f16(Q.Q4_K, w, a, n, k, out=out)          # the stream now keeps a temporary for m = 64
+        refused = None
+        with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=side):
+            a.zero_()                                      # (a graph holds something)
+            try:
+                ops.gemm_f16(Q.Q4_K, w, a, n, k, out=out)  # nothing kept yet: would have to allocate
+            except _lib.RfqError as e:
+                refused = e
+        assert refused is not None and refused.status == _lib.E_UNSUPPORTED and "captur" in refused.message
+        ops.gemm_f16(Q.Q4_K, w, a, n, k, out=out)          # the stream now keeps a temporary for m = 264
         torch.cuda.synchronize()
         refused = None
         with torch.cuda.graph(graph, stream=side):
