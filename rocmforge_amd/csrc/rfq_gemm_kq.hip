@@ -1026,7 +1026,10 @@ int launch_gemm_f16(int fmt, const uint8_t *d_w, const void *d_a, void *d_out, i
     const int rival_parts = d_arranged != nullptr && fmt != RFQ_Q4_K ? 1 : k_parts_for(m, n, k);
     const bool known = fmt == RFQ_Q4_0 || fmt == RFQ_Q8_0 || fmt == RFQ_Q4_K || fmt == RFQ_Q6_K || fmt == RFQ_GGUF_Q4_0 ||
                        fmt == RFQ_GGUF_Q8_0 || fmt == RFQ_GGUF_Q4_K || fmt == RFQ_GGUF_Q6_K;
-    const bool static_fits = !use_static_scratch || arranged_at_bytes(m, k) + arranged_s2_bytes(m, k) <= RFQ_STATIC_SCRATCH_BYTES;
+    // (as launch_cfg sizes it: the group sums belong to two formats; what it refuses stays refused, what it takes gives the
+    // bits of the call without the static buffer)
+    const size_t sums = fmt == RFQ_Q4_K || fmt == RFQ_GGUF_Q4_K ? arranged_s2_bytes(m, k) : 0;
+    const bool static_fits = !use_static_scratch || arranged_at_bytes(m, k) + sums <= RFQ_STATIC_SCRATCH_BYTES;
     // (From 256 rows on, a whole tile, plain activations keep the tiled kernel and with it the rule that a stream under
     // capture must hold the call's temporary; arranged ones follow where both must give the same bits.)
     const bool rows_in_range = m < BM || (d_arranged != nullptr && fmt != RFQ_Q4_K && k_parts_for(m, n, k) > 1);

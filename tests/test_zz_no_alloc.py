@@ -26,6 +26,23 @@ def test_static_scratch_gemm_matches_the_allocating_entry_point(fmt, cuda):
             assert torch.equal(got, want), f"{Q.NAMES[fmt]} {m}x{n}x{k} {out_dtype}"
 
 
+def test_static_scratch_limit_counts_the_sums_of_their_formats_only(cuda):
+    """15.6 MiB of arranged activations fit the array, with the group sums of the Q4_K layouts they would not: Q8_0 has
+    none, so this call takes the kernel that rfq_gemm_f16 takes and gives its bits; GGUF_Q4_K is refused."""
+    import torch
+    from rocmforge_amd import _lib, ops
+    m, n, k = 230, 64, 32000
+    a = torch.from_numpy(np.random.default_rng(1).standard_normal((m, k)).astype(np.float16)).to(cuda)
+    w = torch.from_numpy(Q.make_weights(Q.Q8_0, n, k, seed=2)).to(cuda)
+    got = torch.full((m, n), float("nan"), device=cuda)
+    ops.gemm_f16_static(Q.Q8_0, w, a, n, k, out=got, out_dtype=torch.float32)
+    assert torch.equal(got, ops.gemm_f16(Q.Q8_0, w, a, n, k, out_dtype=torch.float32))
+    w = torch.from_numpy(Q.make_weights(Q.GGUF_Q4_K, n, k, seed=3)).to(cuda)
+    with pytest.raises(_lib.RfqError) as e:
+        ops.gemm_f16_static(Q.GGUF_Q4_K, w, a, n, k, out=got, out_dtype=torch.float32)
+    assert e.value.status == _lib.E_SIZE
+
+
 def test_static_scratch_limit_is_reported(cuda):
     import torch
     from rocmforge_amd import _lib
