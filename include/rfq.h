@@ -283,9 +283,12 @@ RFQ_API int rfq_dequant_rms_norm(int fmt, const void *d_packed, size_t packed_by
 /* d_y[m, n] = RMSNorm(d_x[m, k]; d_norm_weight, eps) . dequant(W)[n, k]^T: the
  * normalisation that precedes a projection in a decoder layer and the
  * projection (rfq_gemv) in one call.  For m = 1 and 512 < k <= 16384 it is one
- * launch and the normalised vector never exists in memory; other shapes run
- * rfq_rms_norm into d_scratch (m * k floats, 16-byte aligned; may be NULL when
- * the one-launch case applies) and then rfq_gemv.  The reference has the two
+ * launch and the normalised vector never exists in memory; other shapes need
+ * d_scratch (m * k floats, 16-byte aligned; may be NULL when that case
+ * applies): they run rfq_rms_norm into it and then rfq_gemv, or, for
+ * m = 2 .. 8 and by shape, one launch that leaves it as it is (its content
+ * afterwards is not part of the result).  With m = 2 .. 8 d_y may lie over
+ * d_x: such a call takes the two steps.  The reference has the two
  * steps only as separate f32 operations (kernels/rms_norm.hip, hipBLAS SGEMM:
  * src/ggml/hip_backend/op_dispatch.rs:1001-1014). */
 RFQ_API int rfq_rms_norm_gemv(int fmt, const void *d_w, size_t w_bytes, const float *d_x, const float *d_norm_weight,
@@ -315,7 +318,10 @@ RFQ_API int rfq_mlp_swiglu(int fmt_gate_up, const void *d_gate_w, const void *d_
 /* d_out[m, n] = d_a[m, k] (fp16) . dequant(W)[n, k]^T on the fp16 matrix
  * cores with fp32 accumulation; out_dtype is RFQ_F32 or RFQ_F16, optionally
  * or-ed with RFQ_GEMM_ONE_PLANE.  Formats: Q4_0, Q8_0, Q4_K, Q6_K and the four
- * GGUF file layouts.  Weights are decoded to f32 as the format defines and
+ * GGUF file layouts.  Fewer than 256 rows go, by shape, to a kernel for few rows
+ * that multiplies the integer codes and applies the scales in fp32 (no weight is
+ * rounded, in any format), in one launch and one pass over k, without temporary
+ * memory.  Otherwise weights are decoded to f32 as the format defines and
  * contracted as two fp16 operands, hi = fp16(v) and lo = fp16(v - hi) (v to
  * 2^-22: the result is that of an fp32 contraction, 5e-6 of rms(out) from the
  * reference's at 512 x 4096 x 14336); the 256-byte Q4_K layout, whose integer
@@ -330,7 +336,8 @@ RFQ_API int rfq_mlp_swiglu(int fmt_gate_up, const void *d_gate_w, const void *d_
  * allocates: run the call once on the stream before capturing it into a graph.)
  * A shape with few output tiles and a long k (an attention or down projection
  * of 512 tokens: 64 tiles of 256 x 128 for 256 CUs) is split along k into
- * rfq_gemm_f16_k_parts(m, n, k) parts of whole super-blocks, whose f32 tiles
+ * rfq_gemm_f16_k_parts(m, n, k) parts of whole super-blocks (unless the kernel
+ * for few rows takes it), whose f32 tiles
  * (parts * m * n * 4 more bytes of temporary) a second kernel adds in a fixed
  * order: the results are deterministic and differ from a single pass only in
  * the order of the fp32 sums.  The reference has no fused prefill GEMM (its matmul_q* hard-wire
@@ -368,13 +375,15 @@ RFQ_API int rfq_gemm_f16_static(int fmt, const void *d_w, size_t w_bytes, const 
  * rfq_gemm_f16_arranged multiplies any of the formats of rfq_gemm_f16 with it.
  * Results are bit-identical to rfq_gemm_f16 on the same A where that call takes
  * one pass over k (rfq_gemm_f16_k_parts(m, n, k) == 1; this entry point never
- * splits: it has no temporary for the parts).  Neither call
+ * splits: it has no temporary for the parts, and takes the kernel for few rows
+ * up to more rows instead).  Neither call
  * allocates or keeps anything, so both may be recorded under stream capture.
  * The reference has no fused prefill GEMM (see rfq_gemm_f16); its
  * counterpart is the shared input of the three SGEMMs of
  * HipBackend::mlp_swiglu (src/backend/hip_backend/backend.rs:1153-1278). */
 RFQ_API size_t rfq_gemm_f16_arranged_bytes(int m, int k);
-/* How many parts along k rfq_gemm_f16 takes for this shape (1 = a single pass). */
+/* How many parts along k rfq_gemm_f16's tiled kernel takes for this shape (1 = a single pass; the kernel for few rows,
+ * which may take fewer than 256 rows, never splits k). */
 RFQ_API int rfq_gemm_f16_k_parts(int m, int n, int k);
 RFQ_API int rfq_gemm_f16_arrange(const void *d_a_f16, int m, int k, void *d_arranged, size_t arranged_bytes,
                                  void *stream);

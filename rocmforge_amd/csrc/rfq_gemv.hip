@@ -1402,10 +1402,11 @@ template <> struct IUnit<RFQ_GGUF_Q6_K> : Unit<RFQ_GGUF_Q6_K> {
     static constexpr bool NIBBLE = false;
     static constexpr uint32_t TOPOFF = 0;
     // The four lanes of a quad take the four pairs of one super-block (lane = 2 * half + t), and what a lane's windows lack
-    // another lane of the quad holds: the two lanes of a half share its 32 bytes of upper bits, 16 each; the ninth dword of the lower nibbles is the next lane's first (behind the last lane's
-    // begin the upper bits), the ninth of the upper bits the other half's first or the first of the scales, and the scales
-    // are fetched as one dword per lane.  Five loads instead of nine: the address unit, 33 clocks
-    // per load instruction and busy for two thirds of the time (the vector units for 41 %), was what bound this kernel.
+    // another lane of the quad holds: the two lanes of a half share its 32 bytes of upper bits, 16 each; the ninth dword of
+    // the lower nibbles is the next lane's first (behind the last lane's begin the upper bits), the ninth of the upper bits
+    // the other half's first or the first of the scales, and the scales are fetched as one dword per lane.  Five loads instead
+    // of nine: the address unit, 34 clocks per load instruction and busy for 65 % of the time (the vector units for 40 %), was
+    // what bound this kernel (128256 x 4096 95.6 -> 86.6 us, the address unit now busy for 55 %).
     uint32_t tw, t4;                                 // dword 4 * lane of the tail from byte 192 on, dword 16: o bytes earlier
     __device__ __forceinline__ void load_pair(const uint8_t *row, int u)
     {
@@ -2602,8 +2603,8 @@ bool few_rows_aligned(int fmt, const void *w, const void *w2, const void *x)
 // Whether a batch goes through the matrix-core kernel for few rows (rfq_skinny.hip) instead of the integer-dot batch kernel
 // (batch_fits) or, where a format or row length has none, one decode launch per vector or the one-row-per-wavefront
 // kernel.  Its time hardly depends on m; measured on 512..14336 rows of 768..13824 for every format (us, there / here):
-//   m >= 5: always (Q8_0 4096 x 4096 m = 8 11.4 / 9.7, Q4_0 13.0 / 8.8, Q4_K 14336 x 4096 30.7 / 23.6, GGUF_Q6_K
-//     4096 x 13824 82 / 23, Q6_K 14336 x 4096 82 / 23, MXFP6 4096 x 4096 42.6 / 12.4);
+//   m >= 5: always (Q8_0 4096 x 4096 m = 8 11.0 / 8.7, Q4_0 13.0 / 8.5, Q4_K 14336 x 4096 30.7 / 23.1, GGUF_Q6_K
+//     4096 x 13824 82 / 24, Q6_K 14336 x 4096 82 / 25, MXFP6 4096 x 4096 42.6 / 11.9);
 //   m = 3, 4 against the batch kernel (which takes three as four): rows longer than 3000 with 12 or more of them per CU, up
 //     to 24 for the formats whose batch kernel streams well at many rows (4096 x 4096: Q8_0 9.5 / 8.3, GGUF_Q4_K 8.7 / 7.6;
 //     4096 x 8192 GGUF_Q6_K 12.9 / 14; 14336 x 4096: GGUF_Q4_0 18.4 / 15.7, but Q8_0 19.9 / 22.3, Q4_K 17.8 / 21.8);

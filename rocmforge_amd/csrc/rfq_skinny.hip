@@ -100,8 +100,8 @@ int gemm_cfg(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, in
 
 // 16-row operands per workgroup at most: six with one row tile (eight leave its registers one wavefront per SIMD: Q8_0
 // 4096 -> 1024, 100 rows, 28 us with eight, 160 rows 15 with twice five); eight with two (8192 rows of 4096, 100 rows: Q8_0
-// 28.8 us, 40 with two slices of four), but four for the scale-only 4-bit layouts, which would spill (Q4_0, 208 rows,
-// 1792 -> 5713: 79.7 us with eight, 45 with four).
+// 28.8 us, 40 with two slices of four), but four for the scale-only 4-bit layouts, whose forms of eight spilled (Q4_0, 208
+// rows, 1792 -> 5713: 79.7 us with eight, 45 with four).
 constexpr int most_tiles(int fmt, bool two) { return !two ? 6 : fmt == RFQ_Q4_0 || fmt == RFQ_GGUF_Q4_0 ? 4 : 8; }
 
 // The rows of a in slices of at most 16 * most_tiles, as even as 16 rows allow.  Where W gives fewer workgroups than the part
@@ -196,14 +196,15 @@ int RFQ_SKINNY_CAT(launch_skinny_gemm_part, RFQ_SKINNY_PART)(int fmt, const uint
 
 #if RFQ_SKINNY_PART == 0
 
-// Whether the few-row kernel is the faster one for a prompt, from estimates of both in microseconds fitted to 300 measured
-// shapes (Q4_K, Q8_0, GGUF_Q4_K, GGUF_Q6_K; n 768..14336, k 1024..14336, 16..256 rows).  The few-row kernel's time grows
-// with the 16-row operands a workgroup multiplies per 1024 k (all of them in every workgroup) and, beyond one workgroup
-// per CU, with the number of workgroups; the tiled kernel's is nearly flat up to 256 rows: a workgroup's own pass over k,
-// in `parts` parts, plus the f32 parts written and read again.  (tiled / few-row: Q8_0 16 x 4096 -> 4096 32.8 / 7.1 us,
-// 96 x 4096 -> 4096 35.9 / 20.6, 48 x 4096 -> 14336 66.5 / 32.7, 96 x 14336 -> 4096 65.8 / 63.1, 256 x 4096 -> 14336
-// 71.9 / 126.)  With parts == 1 the answer depends on the shape alone, so that arranged and plain activations take the
-// same kernel and give the same bits.
+// Whether the few-row kernel is the faster one for a prompt, from estimates of both in microseconds.  The few-row kernel's
+// time grows with the 16-row operands a workgroup multiplies per 1024 k (all of them in every workgroup) and, beyond one
+// workgroup per CU, with the number of workgroups; the tiled kernel's is nearly flat up to 256 rows: a workgroup's own pass
+// over k, in `parts` parts, plus the f32 parts written and read again.  (tiled / few-row: Q8_0 9 x 4096 -> 4096 33.3 / 6.6 us,
+// 112 x 4096 -> 4096 37.8 / 15.8, 56 x 4096 -> 14336 65.7 / 31.9, 80 x 14336 -> 4096 72.1 / 54.5, 255 x 4096 -> 14336
+// 72.9 / 99.9.)  The estimates lean to the tiled kernel: of 2640 shapes measured with both (the eight formats, n 768..14336, k
+// 1024..14336, 9..255 rows, plain and arranged) three that go to the few-row kernel are slower there by more than 4 % (7 % at
+// most), and some 250 that stay would gain more than 10 % by going.  With parts == 1 the answer depends on the shape alone, so
+// that arranged and plain activations take the same kernel and give the same bits.
 bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts)
 {
     const double cus = device_cu_count(), ku = k / 1024.0;

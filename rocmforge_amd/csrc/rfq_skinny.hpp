@@ -1,7 +1,7 @@
 // Matrix-core contraction for few rows of activations:  y[m, n] = x[m, k] . dequant(W)[n, k]^T, one launch, no temporary.
 //
 //   * float32 x, 2..8 rows  (decode batches, rfq_gemv)
-//   * float16 a, 9..160 rows (short prompts, rfq_gemm_f16 / rfq_gemm_f16_arranged)
+//   * float16 a, fewer than 256 rows, arranged ones also more (short prompts, rfq_gemm_f16 / rfq_gemm_f16_arranged)
 //
 // With so few rows every packed weight byte is wanted once and the matrix cores are nearly idle; what bounds the call is
 // the weight stream, the vector instructions that turn codes into operands, and the activations, which every workgroup
@@ -22,16 +22,17 @@
 //   * No split of k over workgroups: the wavefronts of a workgroup share 16 * TJ weight rows, take the 128-element units
 //     of k in turn and add their results through LDS: one launch, nothing to allocate.
 // Measured (cold weights, captured launches; the tiled kernel with its arrangement and its parts -> this one):
-//   37 x 4096 -> 4096      Q8_0 33.6 -> 10.7 us   GGUF_Q4_K 25.8 -> 10.5   GGUF_Q6_K 43.0 -> 12.3   Q4_K 22.2 -> 12.6
-//   9 x 1024 -> 1000       Q8_0 27.5 -> 3.1       GGUF_Q4_K 20.0 -> 3.2    GGUF_Q6_K 36.0 -> 4.3    Q4_K 16.1 -> 3.9
-//   48 x 4096 -> 14336     Q8_0 66.5 -> 32.7      GGUF_Q4_K 42.5 -> 23.3   GGUF_Q6_K 77.9 -> 42.0   Q4_K 40.6 -> 34.7
+//   37 x 4096 -> 4096      Q8_0 33.9 -> 10.8 us   GGUF_Q4_K 26.6 -> 10.4   GGUF_Q6_K 43.5 -> 11.3   Q4_K 22.5 -> 13.5
+//   9 x 1024 -> 768        Q8_0 27.9 -> 3.3       GGUF_Q4_K 20.2 -> 3.3    GGUF_Q6_K 36.5 -> 4.0    Q4_K 16.5 -> 4.0
+//   48 x 4096 -> 14336     Q8_0 63.8 -> 32.7      GGUF_Q4_K 44.7 -> 26.5   GGUF_Q6_K 82.1 -> 35.8   Q4_K 40.4 -> 33.7
 // and decode batches (integer-dot batch kernel, or a launch per vector -> this one):
 //   8 x 4096 -> 4096       Q8_0 11.0 -> 8.7 us    GGUF_Q4_K 14.4 -> 8.4    Q6_K 34.1 -> 9.4         MXFP4 33.2 -> 8.7
 //   5 x 13824 -> 5120      Q8_0 61 -> 36          GGUF_Q4_K 61 -> 32       GGUF_Q6_K 90 -> 39       Q4_K 73 -> 34
 //   error against 64 bits (2-norm of the result), 512 x 13824, 5 vectors: Q6_K 1.07e-7 (float kernel) -> 8.1e-8, Q4_K 1.12e-7 ->
 //   7.4e-8, MXFP6 1.02e-7 -> 5.6e-8; (integer-dot kernel) GGUF_Q6_K 2.8e-7 -> 8.0e-8, 8 x 4096 -> 4096 Q8_0 2.7e-7 -> 7.7e-8
-// (10.5 us for 37 rows of GGUF_Q4_K is 0.9 TB/s of weights: what bounds it is the activations, 384 KB per workgroup
-// through LDS, and the instructions, about 60 per unit and 16-row operand.)
+// (10.4 us for 37 rows of GGUF_Q4_K is 0.9 TB/s of weights: what bounds it is the activations, 384 KB per workgroup
+// through LDS, and the instructions, 12 vector instructions per matrix instruction; decode batches issue vector instructions
+// for 40 % of their time and wait for a third of their wavefronts' cycles.)
 #pragma once
 #include <type_traits>
 
