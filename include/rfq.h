@@ -110,7 +110,7 @@ typedef enum rfq_mx_kind { RFQ_MX_AUTO = 0, RFQ_MX_FP4 = 4, RFQ_MX_FP8 = 8, RFQ_
 RFQ_API int rfq_version(void);
 /* Thread-local description of the last failure on this thread ("" if none). */
 RFQ_API const char *rfq_last_error(void);
-/* rfq_gemm_f16 and rfq_gemv_kn keep up to 64 MiB of
+/* rfq_gemm_f16, rfq_gemv_kn and rfq_gemv (Q8_0 with m > 1 and d_y over d_x) keep up to 64 MiB of
  * temporary device memory per stream between calls (a stream's first call, or
  * a larger shape than before, allocates; a larger request replaces the
  * buffer).  Under stream capture such a call uses the buffer the stream

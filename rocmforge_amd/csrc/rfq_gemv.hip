@@ -2457,10 +2457,35 @@ int run_generic_m(const uint8_t *w, const float *x, float *y, int m, int n, int 
     }
 }
 
+// x as it was before the call, for a batch whose results are written over it.
+__global__ void __launch_bounds__(256)
+copy_x_kernel(const float *__restrict__ x, float *__restrict__ to, size_t count)
+{
+    const size_t at = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (at < count) to[at] = x[at];
+}
+
 template <int FMT>
 int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStream_t s)
 {
     const int ku = k / 32;
+    if constexpr (FMT == RFQ_Q8_0 || FMT == RFQ_GGUF_Q8_0) {
+        // (the kernels of these formats for batches read all of x in a step of its own once, and such calls worked)
+        const size_t count = (size_t)m * k;
+        if (m > 1 && overlap(x, count * 4, y, (size_t)m * n * 4)) {
+            uint8_t *tmp = nullptr;
+            bool transient = false;
+            if (int rc = workspace(s, count * 4, &tmp, &transient)) return rc;
+            hipLaunchKernelGGL(copy_x_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, x, reinterpret_cast<float *>(tmp), count);
+            int rc = hipGetLastError() == hipSuccess ? RFQ_OK : fail(RFQ_E_HIP, "copy_x_kernel");
+            if (rc == RFQ_OK) rc = run<FMT>(w, reinterpret_cast<const float *>(tmp), y, m, n, k, s);
+            if (transient) {
+                const hipError_t e = hipFreeAsync(tmp, s);
+                if (rc == RFQ_OK && e != hipSuccess) rc = hip_fail(e, "hipFreeAsync");
+            }
+            return rc;
+        }
+    }
     if constexpr (NeedsAlignedTensor<FMT>::value) {
         if (!tensor_aligned<FMT>(w, n, k)) return run_generic_m<FMT>(w, x, y, m, n, k, s);
     }

@@ -443,3 +443,16 @@ def test_arranged_prompts_of_many_rows(fmt, m, n, k, oracle, cuda):
     # (Q4_K's tiled kernel multiplies q * scale rounded to fp16 once)
     assert_close(got.cpu().numpy(), a.astype(np.float64) @ weights_of(oracle, fmt, w, n, k).T, f"{Q.NAMES[fmt]} {m}x{n}x{k}",
                  tol=1e-3 if fmt == Q.Q4_K else TOL, plain_tol=None if fmt == Q.Q4_K else 2e-4)
+
+
+@pytest.mark.parametrize("fmt", [Q.Q8_0, Q.GGUF_Q8_0])
+@pytest.mark.parametrize("m,k", [(2, 1024), (4, 1024), (5, 4096), (8, 4096)])
+def test_q8_0_batches_over_their_own_input(fmt, m, k, cuda):
+    import torch
+    from rocmforge_amd import ops
+    w = torch.from_numpy(Q.make_weights(fmt, k, k, seed=1)).to(cuda)
+    x = torch.randn((m, k), generator=torch.Generator(device="cpu").manual_seed(2)).to(cuda)
+    want = ops.gemv(fmt, w, x, k, k)
+    into = x.clone()
+    ops.gemv(fmt, w, into, k, k, out=into)
+    assert torch.equal(into, want)
