@@ -97,6 +97,22 @@ def test_k_not_a_multiple_of_the_stage(fmt, m, kernel, oracle, cuda):
 
 
 @pytest.mark.parametrize("fmt", FORMATS)
+def test_ragged_tiles_of_few_rows(fmt, oracle, cuda):
+    """Fewer than 256 rows over a matrix wide enough for the tiled kernel: one row tile, not full, and a ragged last column tile."""
+    import torch
+    m, n, k = 201, 14330, 2048
+    w, a = weights(fmt, n, k, 71), acts(m, k, 72)
+    out = run(fmt, w, a, n, k, cuda, torch.float32).cpu().numpy()
+    assert kernel_name().startswith("gemm_kq_kernel")
+    w64 = (gguf_q4_k_fused(w, n, k) if fmt == Q.GGUF_Q4_K else oracle.dequantize(fmt, w, n * k).reshape(n, k)).astype(np.float64)
+    # (the 256-byte Q4_K layout rounds q * scale to fp16: errors of at most 2^-11 of it, evenly spread between two of its
+    # codes' neighbours, 2^-11 / sqrt(12) = 1.4e-4 rms; the largest of three million normally distributed sums is 5.2 times that,
+    # 7.4e-4 of what q * scale contributes, which the opposite mins leave up to twice the output's size: 1.5e-3)
+    assert_close(out, a.astype(np.float64) @ w64.T, f"{Q.NAMES[fmt]} {m}x{n}x{k}", tol=1.5e-3 if fmt == Q.Q4_K else 2e-5,
+                 plain_tol=None if fmt == Q.Q4_K else 2e-4)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
 def test_fp16_output_is_the_rounded_fp32_output(fmt, cuda):
     import torch
     m, n, k = 130, 264, 512
