@@ -869,9 +869,14 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
             double sq = 0.0;
             for (int wv = 0; wv < waves; wv++) sq += (double)squares[wv * MV + v];
             if (!(sq <= 3.40282347e+38)) {                        // (rarely: as the norm alone has it, x / infinity)
-                bool finite = sq == sq;
-                for (int j = 0; j < k && finite; j++) finite = fabsf(x[(size_t)v * k + j]) <= 3.40282347e+38f;
-                y[(size_t)v * n + n0 + c] = finite ? 0.0f : __uint_as_float(0x7FC00000u);
+                float zero = 0.0f;                                // (NaN with an infinity or a NaN in x; no early end, so that loads run ahead)
+#pragma unroll 4
+                for (int j = 0; j < k; j += 4) {
+                    const v4f o = *reinterpret_cast<const v4f_a4 *>(x + (size_t)v * k + j);
+#pragma unroll
+                    for (int e4 = 0; e4 < 4; e4++) zero = __builtin_fmaf(o[e4], 0.0f, zero);
+                }
+                y[(size_t)v * n + n0 + c] = fabsf(zero);
                 continue;
             }
             const double mean = __builtin_fma(sq, 1.0 / (double)k, (double)eps), r0 = (double)(1.0f / sqrtf((float)mean));
