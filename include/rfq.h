@@ -321,7 +321,8 @@ RFQ_API int rfq_mlp_swiglu(int fmt_gate_up, const void *d_gate_w, const void *d_
  * GGUF file layouts.  Fewer than 256 rows go, by shape, to a kernel for few rows
  * that multiplies the integer codes and applies the scales in fp32 (no weight is
  * rounded, in any format), in one launch and one pass over k, without temporary
- * memory.  Otherwise weights are decoded to f32 as the format defines and
+ * memory.  Otherwise Q4_0, Q8_0 and their GGUF layouts are multiplied as integer codes too;
+ * the Q6_K layouts are decoded to f32 as the format defines and
  * contracted as two fp16 operands, hi = fp16(v) and lo = fp16(v - hi) (v to
  * 2^-22: the result is that of an fp32 contraction, 5e-6 of rms(out) from the
  * reference's at 512 x 4096 x 14336); the 256-byte Q4_K layout, whose integer

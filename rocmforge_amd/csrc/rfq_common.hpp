@@ -143,6 +143,11 @@ int launch_skinny_gemv_fused(int fmt, const uint8_t *d_w, const uint8_t *d_w2, c
                              int m, int n, int k, hipStream_t s);
 int launch_skinny_gemm(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, bool f16_out, int m, int n, int k,
                        hipStream_t s);
+// The tiled kernel on integer codes (rfq_gemm_codes.hip): arranged activations (s2: their group sums, GGUF_Q4_K); kparts > 1:
+// f32 parts [kparts][m][n] into out.  codes_rows: the rows of a workgroup's tile.
+constexpr bool codes_format(int fmt) { return fmt == RFQ_Q4_0 || fmt == RFQ_Q8_0 || fmt == RFQ_GGUF_Q4_0 || fmt == RFQ_GGUF_Q8_0 || fmt == RFQ_GGUF_Q4_K; }
+int codes_rows(int m, int n, int kparts);
+int launch_gemm_codes(int fmt, const uint8_t *w, const uint8_t *at, const uint8_t *s2, void *out, bool f16_out, int m, int n, int k, int kparts, hipStream_t s);
 bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts);
 #define RFQ_SKINNY_PART_DECL(N)                                                                                              \
     int launch_skinny_gemv_part##N(int fmt, const SkinnyGemv &c, hipStream_t s);                                             \

@@ -1,5 +1,6 @@
-// Prefill GEMM for the block formats with f16/f32 scales (Q4_0, Q8_0, Q4_K,
-// Q6_K): out[m, n] = A[m, k] (fp16) . dequant(W)[n, k]^T on the fp16 matrix
+// Prefill GEMM for the block formats with f16/f32 scales: Q4_K, Q6_K, GGUF_Q6_K, GGUF_Q4_K over whole tiles of 256 rows,
+// and every format as one rounded operand (RFQ_GEMM_ONE_PLANE); the others' codes go through rfq_gemm_codes.hip.
+// out[m, n] = A[m, k] (fp16) . dequant(W)[n, k]^T on the fp16 matrix
 // cores (v_mfma_f32_32x32x16_f16), fp32 accumulation.
 //
 // The weights are decoded with the reference's f32 arithmetic (the same
@@ -745,6 +746,22 @@ int k_parts_for(int m, int n, int k)
 size_t arranged_at_bytes(int m, int k) { return (size_t)((m + 31) / 32) * ((k + BK - 1) / BK) * 4096; }
 size_t arranged_s2_bytes(int m, int k) { return k % 256 == 0 ? (size_t)((m + 31) / 32) * (k / 256) * 1024 : 0; }
 
+// The parts of k of a call on plain activations: none where the static buffer has no room for them.
+int parts_in(const uint8_t *static_tmp, int m, int n, int k, bool sums)
+{
+    const int kparts = k_parts_for(m, n, k);
+    const size_t head = (arranged_at_bytes(m, k) + (sums ? arranged_s2_bytes(m, k) : 0) + 255) & ~(size_t)255;
+    return static_tmp != nullptr && kparts > 1 && head + (size_t)kparts * m * n * sizeof(float) > RFQ_STATIC_SCRATCH_BYTES ? 1 : kparts;
+}
+
+// The kernel on integer codes belongs to the same family: its rows per tile where the tiled kernel has its planes
+// (GGUF_Q4_K, whose operands are exact in one plane in both kernels, keeps that name).
+void note_codes(int fmt, int m, int n, int kparts, bool arranged)
+{
+    if (fmt == RFQ_GGUF_Q4_K) note_kernel(arranged ? "gemm_kq_kernel<%s,%d,%d,arranged>" : "gemm_kq_kernel<%s,%d,%d>", fmt, 1, kparts, 0);
+    else note_kernel(arranged ? "gemm_kq_kernel<%s,codes of %d,%d,arranged>" : "gemm_kq_kernel<%s,codes of %d,%d>", fmt, codes_rows(m, n, kparts), kparts, 0);
+}
+
 // `arranged` != nullptr: the caller's buffer from launch_arrange_a (activations and sums); a is not read.
 template <int FMT, bool OUT_F16, int PLANES>
 int launch_cfg(const uint8_t *w, const void *a, void *out, int m, int n, int k, uint8_t *static_tmp, const uint8_t *arranged,
@@ -755,61 +772,69 @@ int launch_cfg(const uint8_t *w, const void *a, void *out, int m, int n, int k, 
     static_assert(LDS <= 160 * 1024, "LDS budget");
     constexpr int FORMAT = FMT == KQ_GGUF_Q4_K_INT ? (int)RFQ_GGUF_Q4_K : (int)FMT;
     // (both output types: a launch split along k writes f32 parts whatever the caller's type)
-    static std::once_flag once;
-    static hipError_t attr_err = hipSuccess;
-    std::call_once(once, [] {
-        attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_kq_kernel<FMT, OUT_F16, PLANES>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-        if (attr_err == hipSuccess && OUT_F16)
-            attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_kq_kernel<FMT, false, PLANES>),
+    constexpr bool CODES = PLANES == 2 && codes_format(FMT);
+    if constexpr (!CODES) {
+        static std::once_flag once;
+        static hipError_t attr_err = hipSuccess;
+        std::call_once(once, [] {
+            attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_kq_kernel<FMT, OUT_F16, PLANES>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-    });
-    if (attr_err != hipSuccess) return hip_fail(attr_err, "hipFuncSetAttribute(gemm_kq_kernel)");
+            if (attr_err == hipSuccess && OUT_F16)
+                attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_kq_kernel<FMT, false, PLANES>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        });
+        if (attr_err != hipSuccess) return hip_fail(attr_err, "hipFuncSetAttribute(gemm_kq_kernel)");
+    }
     const int tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN);
     if (arranged != nullptr) {
         // (the caller's buffer holds the arranged activations only: nowhere to put parts, no split along k)
         const v4u *at = reinterpret_cast<const v4u *>(arranged);
         const _Float16 *s2 = reinterpret_cast<const _Float16 *>(arranged + arranged_at_bytes(m, k));
-        note_kernel("gemm_kq_kernel<%s,%d,%d,arranged>", FORMAT, PLANES, 1, 0);
-        hipLaunchKernelGGL((gemm_kq_kernel<FMT, OUT_F16, PLANES>), dim3(tiles), dim3(256), LDS, s, w, at, s2, out, m, n, k, 1);
-        RFQ_LAUNCH_CHECK("gemm_kq_kernel");
-        return RFQ_OK;
+        if constexpr (CODES) {
+            note_codes(FMT, m, n, 1, true);
+            return launch_gemm_codes(FMT, w, arranged, arranged + arranged_at_bytes(m, k), out, OUT_F16, m, n, k, 1, s);
+        } else {
+            note_kernel("gemm_kq_kernel<%s,%d,%d,arranged>", FORMAT, PLANES, 1, 0);
+            hipLaunchKernelGGL((gemm_kq_kernel<FMT, OUT_F16, PLANES>), dim3(tiles), dim3(256), LDS, s, w, at, s2, out, m, n, k, 1);
+            RFQ_LAUNCH_CHECK("gemm_kq_kernel");
+            return RFQ_OK;
+        }
     }
     // the temporary: the arranged activations, then the Q4_K group sums
     const int tiles32 = (m + 31) / 32, nst = (k + BK - 1) / BK;
     const size_t at_bytes = (size_t)tiles32 * nst * 4096;
-    constexpr bool SUMS = FMT == RFQ_Q4_K || FMT == KQ_GGUF_Q4_K_INT;
+    constexpr bool SUMS = FMT == RFQ_Q4_K || FMT == KQ_GGUF_Q4_K_INT || (CODES && FMT == RFQ_GGUF_Q4_K);
     const size_t s2_bytes = SUMS ? (size_t)tiles32 * (k / 256) * 1024 : 0;
     // Few output tiles and a long k (an attention or down projection of 512 tokens: 64 tiles for 256 CUs): the launch is
     // split along k, the parts' f32 tiles follow the arranged activations in the temporary, reduce_parts_kernel adds them.
-    int kparts = k_parts_for(m, n, k);
+    const int kparts = parts_in(static_tmp, m, n, k, SUMS);
     const size_t head_bytes = (at_bytes + s2_bytes + 255) & ~(size_t)255;
-    size_t parts_bytes = kparts > 1 ? (size_t)kparts * m * n * sizeof(float) : 0;
+    const size_t parts_bytes = kparts > 1 ? (size_t)kparts * m * n * sizeof(float) : 0;
     uint8_t *tmp = static_tmp;
     bool transient = false;
     if (static_tmp != nullptr) {
         if (at_bytes + s2_bytes > RFQ_STATIC_SCRATCH_BYTES)
             return fail(RFQ_E_SIZE, "rfq_gemm_f16_static: m=%d k=%d needs %zu bytes of temporary memory, the static buffer holds %zu",
                         m, k, at_bytes + s2_bytes, RFQ_STATIC_SCRATCH_BYTES);
-        if (head_bytes + parts_bytes > RFQ_STATIC_SCRATCH_BYTES) {                   // no room for parts: one pass over k
-            kparts = 1;
-            parts_bytes = 0;
-        }
     } else if (int rc = workspace(s, head_bytes + parts_bytes, &tmp, &transient)) {
         return rc;
     }
     v4u *at = reinterpret_cast<v4u *>(tmp);
     _Float16 *s2 = reinterpret_cast<_Float16 *>(tmp + at_bytes);
-    note_kernel("gemm_kq_kernel<%s,%d,%d>", FORMAT, PLANES, kparts, 0);
+    if constexpr (CODES) note_codes(FMT, m, n, kparts, false);
+    else note_kernel("gemm_kq_kernel<%s,%d,%d>", FORMAT, PLANES, kparts, 0);
     hipLaunchKernelGGL((arrange_a_kernel<SUMS>), dim3((unsigned)(tiles32 * ((nst + 3) / 4))), dim3(256), 0, s,
                        reinterpret_cast<const _Float16 *>(a), at, s2, m, k, tiles32, nst);
+    int code_rc = RFQ_OK;
     if (kparts > 1) {
         float *parts = reinterpret_cast<float *>(tmp + head_bytes);
         const size_t count = (size_t)m * n;
-        hipLaunchKernelGGL((gemm_kq_kernel<FMT, false, PLANES>), dim3(tiles * kparts), dim3(256), LDS, s, w, at, s2, parts, m, n, k, kparts);
+        if constexpr (CODES) code_rc = launch_gemm_codes(FMT, w, tmp, tmp + at_bytes, parts, false, m, n, k, kparts, s);
+        else hipLaunchKernelGGL((gemm_kq_kernel<FMT, false, PLANES>), dim3(tiles * kparts), dim3(256), LDS, s, w, at, s2, parts, m, n, k, kparts);
         hipLaunchKernelGGL((reduce_parts_kernel<OUT_F16>), dim3((unsigned)((count + 1023) / 1024)), dim3(256), 0, s, parts, out, count, kparts);
     } else {
-        hipLaunchKernelGGL((gemm_kq_kernel<FMT, OUT_F16, PLANES>), dim3(tiles), dim3(256), LDS, s, w, at, s2, out, m, n, k, 1);
+        if constexpr (CODES) code_rc = launch_gemm_codes(FMT, w, tmp, tmp + at_bytes, out, OUT_F16, m, n, k, 1, s);
+        else hipLaunchKernelGGL((gemm_kq_kernel<FMT, OUT_F16, PLANES>), dim3(tiles), dim3(256), LDS, s, w, at, s2, out, m, n, k, 1);
     }
     hipError_t launch_err = hipGetLastError();
     if (transient) {
@@ -817,7 +842,7 @@ int launch_cfg(const uint8_t *w, const void *a, void *out, int m, int n, int k, 
         if (launch_err == hipSuccess) launch_err = free_err;
     }
     if (launch_err != hipSuccess) return hip_fail(launch_err, "gemm_kq_kernel");
-    return RFQ_OK;
+    return code_rc;
 }
 
 #if RFQ_KQ_PART == 0
@@ -832,7 +857,12 @@ int launch_fmt(const uint8_t *w, const void *a, void *out, int out_dtype, int m,
         // exact in one pass: integer operands, d and dmin applied in f32
         if ((out_dtype & RFQ_GEMM_ONE_PLANE) == 0) {
             if (k % 256 != 0) return fail(RFQ_E_SIZE, "rfq_gemm_f16: k=%d is not whole Q4_K super-blocks", k);
-            return launch_gguf_q4_k_int(w, a, out, f16, m, n, k, static_tmp, arranged, s);
+            // (whole tiles of 256 rows: the kernel whose stages are laid out by hand is the faster one, 79 against 88 us for 512 x
+            // 4096 -> 14336; fewer rows per tile: 300 x 13824 -> 5120 91 -> 78 us, 64 x 14336 -> 4096 46 -> 28)
+            if (codes_rows(m, n, arranged != nullptr ? 1 : parts_in(static_tmp, m, n, k, true)) == 256)
+                return launch_gguf_q4_k_int(w, a, out, f16, m, n, k, static_tmp, arranged, s);
+            return f16 ? launch_cfg<FMT, true, 2>(w, a, out, m, n, k, static_tmp, arranged, s)
+                       : launch_cfg<FMT, false, 2>(w, a, out, m, n, k, static_tmp, arranged, s);
         }
     } else if constexpr (FMT != RFQ_Q4_K) {
         if ((out_dtype & RFQ_GEMM_ONE_PLANE) == 0)

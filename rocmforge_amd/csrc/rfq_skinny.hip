@@ -205,6 +205,9 @@ int RFQ_SKINNY_CAT(launch_skinny_gemm_part, RFQ_SKINNY_PART)(int fmt, const uint
 // 1024..14336, 9..255 rows, plain and arranged) three that go to the few-row kernel are slower there by more than 4 % (7 % at
 // most), and some 250 that stay would gain more than 10 % by going.  With parts == 1 the answer depends on the shape alone, so
 // that arranged and plain activations take the same kernel and give the same bits.
+// (The kernel on integer codes has since replaced the tiled one for five formats and is the faster one in part of what the
+// estimates leave here - Q8_0 64 x 14336 -> 4096 28 against 41 us - but adds longer runs of k in float32: its error against 64
+// bits is 1.2e-7 .. 1.5e-7 where this kernel's is 1.0e-7, GGUF_Q4_K 2.7e-7 .. 3.4e-7 against 1.3e-7.  The line stays.)
 bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts)
 {
     const double cus = device_cu_count(), ku = k / 1024.0;

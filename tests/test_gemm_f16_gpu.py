@@ -415,3 +415,40 @@ def test_arranged_activations_in_a_graph_and_bad_sizes(cuda):
                                    _lib.F16, m, n, k, None) == _lib.E_SIZE
     assert L.rfq_gemm_f16_arranged(fmt, C.c_void_p(w.data_ptr()), w.numel(), one, nbytes, C.c_void_p(out.data_ptr()),
                                    _lib.BF16, m, n, k, None) == _lib.E_BADARG
+
+
+# The kernel on integer codes, each of its row tiles at ragged sizes: one row, one column tile and more, k of one stage (128), of
+# whole stages, of a stage with one group and of one with three, in one part and in several.  Codes and activations are
+# exact, the sums float32: about sqrt(k) * 2^-24 of a typical output off.
+@pytest.mark.parametrize("fmt", [Q.Q4_0, Q.Q8_0, Q.GGUF_Q4_0, Q.GGUF_Q8_0, Q.GGUF_Q4_K])
+@pytest.mark.parametrize("m,n,k,rows,parts", [(257, 15, 32, 64, 1), (300, 1000, 160, 64, 1), (257, 129, 128, 64, 1), (300, 12000, 224, 192, 1), (512, 14340, 256, 256, 1),
+                                              (700, 3700, 384, 128, 1), (333, 4990, 3072, 192, 3), (511, 4000, 4096, 256, 4), (260, 40, 2048, 64, 2)])
+def test_integer_code_tiles(fmt, m, n, k, rows, parts, oracle, cuda):
+    import torch
+    from rocmforge_amd import _lib, ops
+    if fmt == Q.GGUF_Q4_K:
+        k = (k + 255) // 256 * 256
+    assert _lib.lib().rfq_gemm_f16_k_parts(m, n, k) == parts
+    w, a = weights(fmt, n, k, 7), acts(m, k, 8)
+    dw, da = torch.from_numpy(w).to(cuda), torch.from_numpy(a).to(cuda)
+    out = ops.gemm_f16(fmt, dw, da, n, k, out_dtype=torch.float32)
+    assert kernel_name() == (f"gemm_kq_kernel<GGUF_Q4_K,1,{parts}>" if fmt == Q.GGUF_Q4_K else f"gemm_kq_kernel<{Q.NAMES[fmt]},codes of {rows},{parts}>")
+    pick = np.unique(np.concatenate([np.arange(0, n, max(1, n // 97)), np.arange(max(0, n - 130), n)]))
+    want = a.astype(np.float64) @ (gguf_q4_k_fused(w, n, k) if fmt == Q.GGUF_Q4_K else oracle.dequantize(fmt, w, n * k).reshape(n, k))[pick].astype(np.float64).T
+    assert_close(out.cpu().numpy()[:, pick], want, f"{Q.NAMES[fmt]} {m}x{n}x{k}", tol=2e-5, plain_tol=2e-4)
+    assert torch.equal(ops.gemm_f16(fmt, dw, da, n, k), out.half())
+
+
+@pytest.mark.parametrize("fmt", [Q.Q4_0, Q.Q8_0])
+@pytest.mark.parametrize("scale", [1e-40, 1e30])
+def test_integer_codes_under_scales_of_any_size(fmt, scale, oracle, cuda):
+    """float32 block scales that fp16 operands could not carry."""
+    import torch
+    m, n, k = 260, 130, 256
+    w = weights(fmt, n, k, 3).reshape(-1, Q.BLOCK_BYTES[fmt]).copy()
+    w[:, :4] = (w[:, :4].copy().view("<f4") * np.float32(scale)).view(np.uint8)
+    a = acts(m, k, 4)
+    out = run(fmt, w.reshape(-1), a, n, k, cuda, torch.float32).cpu().numpy()
+    want = a.astype(np.float64) @ oracle.dequantize(fmt, w.reshape(-1), n * k).reshape(n, k).astype(np.float64).T
+    # (subnormal scales: a result is a sum of 8 products, each rounded to a multiple of 2^-149)
+    assert np.abs(out - want).max() <= 2e-5 * np.abs(want).max() + 16 * 2.0 ** -149
