@@ -1,0 +1,98 @@
+"""The operators' native call path: it gives what the Python text gives, leaves to that text every call with something unusual
+about it, and raises what the text raises."""
+import numpy as np
+import pytest
+import torch
+
+from rocmforge_amd import _lib, _native, ops, quantize as Q
+
+NAMES = ("gemv", "rms_norm_gemv", "mlp_swiglu", "gemm_f16", "arrange", "gemm_f16_arranged", "dequant")
+
+
+def test_unusual_arguments_are_left_to_the_python_text():
+    w, x = torch.zeros(20, dtype=torch.uint8), torch.zeros(32)
+    assert _native.gemv(Q.Q4_0, w, x, 1, 32, None) is None                 # host tensors
+    assert _native.gemv(Q.Q4_0, None, x, 1, 32, None) is None
+    assert _native.gemv(1.0, w, x, 1, 32, None) is None
+    assert _native.gemv(Q.Q4_0, w, x, 1 << 40, 32, None) is None
+    assert _native.gemv(Q.Q4_0, w, x, -1, 32, None) is None
+    assert _native.gemv(Q.Q4_0, torch.nn.Parameter(w, requires_grad=False), x, 1, 32, None) is None
+    assert _native.dequant(Q.Q4_0, w, 32, None) is None and _native.arrange(x) is None
+    with pytest.raises(TypeError):
+        _native.gemv(Q.Q4_0, w, x)
+
+
+@pytest.fixture
+def text_only(monkeypatch):
+    def switch():
+        for name in NAMES:
+            monkeypatch.setattr(_native, name, lambda *a: None)
+    return switch
+
+
+@pytest.mark.gpu
+def test_native_calls_equal_the_python_text(cuda, text_only):
+    n, k, fmt = 96, 256, Q.Q8_0
+    w = torch.from_numpy(Q.make_weights(fmt, n, k, seed=1)).to(cuda)
+    sq = torch.from_numpy(Q.make_weights(fmt, k, k, seed=2)).to(cuda)
+    rng = np.random.default_rng(3)
+    x = torch.from_numpy(rng.standard_normal((3, k)).astype(np.float32)).to(cuda)
+    nw = torch.ones(k, device=cuda) * 1.5
+    a = x.half()
+
+    def every():
+        out, f = torch.empty((3, n), device=cuda), torch.empty(n * k, device=cuda)
+        h = torch.empty((3, n), dtype=torch.float16, device=cuda)
+        A = ops.ArrangedA(a)
+        r = [ops.gemv(fmt, w, x, n, k), ops.gemv(fmt, w, x[0], n, k), ops.gemv(fmt, w, x, n, k, out=out), ops.rms_norm_gemv(fmt, w, x, nw, 1e-5, n, k),
+             ops.rms_norm_gemv(fmt, w, x[1], nw, 1e-5, n, k), ops.mlp_swiglu(fmt, sq, sq, fmt, sq, x, nw, 1e-5, k, k),
+             ops.mlp_swiglu(fmt, sq, sq, fmt, sq, x[2], None, 1e-5, k, k, scratch=torch.empty(16 * k, dtype=torch.uint8, device=cuda)),
+             ops.gemm_f16(fmt, w, a, n, k), ops.gemm_f16(fmt, w, a, n, k, out_dtype=torch.float32, one_plane=True), ops.gemm_f16(fmt, w, a, n, k, out=h),
+             ops.gemm_f16_arranged(fmt, w, A, n), ops.gemm_f16_arranged(fmt, w, A, n, out_dtype=torch.float32), ops.dequant(fmt, w, n * k), ops.dequant(fmt, w, n * k, out=f)]
+        assert r[2] is out and r[9] is h and r[13] is f and (A.m, A.k) == (3, k)
+        return r
+
+    got = every()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):                                           # the current stream is the one that is taken
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            captured = ops.gemv(fmt, w, x[0], n, k)
+        g.replay()
+        side.synchronize()
+    assert torch.equal(captured, got[1])
+    text_only()
+    for i, (p, q) in enumerate(zip(got, every())):
+        assert p.shape == q.shape and p.dtype == q.dtype and torch.equal(p, q), i
+
+
+@pytest.mark.gpu
+def test_native_errors_are_the_python_texts(cuda):
+    n, k = 8, 64
+    w = torch.from_numpy(Q.make_weights(Q.Q4_0, n, k, seed=1)).to(cuda)
+    x = torch.zeros((2, k), device=cuda)
+    with pytest.raises(_lib.RfqError):
+        ops.gemv(Q.Q4_0, w[:-20], x, n, k)                                   # bytes do not match the shape: the library refuses
+    with pytest.raises(_lib.RfqError):
+        ops.gemv(99, w, x, n, k)
+    with pytest.raises(ValueError):
+        ops.gemv(Q.Q4_0, w, x.t().contiguous().t(), n, k)                     # not contiguous
+    with pytest.raises(ValueError):
+        ops.gemm_f16(Q.Q4_0, w, x.half()[0], n, k)
+    with pytest.raises(ValueError):
+        ops.mlp_swiglu(Q.Q4_0, w, w[20:], Q.Q4_0, w, x, None, 1e-5, k, n)
+    with pytest.raises(KeyError):
+        ops.gemm_f16(Q.Q4_0, w, x.half(), n, k, out_dtype=torch.bfloat16)
+
+    class Listener(torch.overrides.TorchFunctionMode):
+        seen = 0
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            Listener.seen += 1
+            return func(*args, **(kwargs or {}))
+
+    with Listener():                                                        # whoever listens to torch functions hears the call
+        y = ops.gemv(Q.Q4_0, w, x, n, k)
+    assert Listener.seen > 0 and torch.equal(y, ops.gemv(Q.Q4_0, w, x, n, k))
+    assert not ops.gemv(Q.Q4_0, w, x.clone().requires_grad_(), n, k).requires_grad
