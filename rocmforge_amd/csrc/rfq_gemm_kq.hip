@@ -1065,7 +1065,9 @@ int launch_gemm_f16(int fmt, const uint8_t *d_w, const void *d_a, void *d_out, i
     const bool rows_in_range = m < BM || (d_arranged != nullptr && fmt != RFQ_Q4_K && k_parts_for(m, n, k) > 1);
     // (Activations that the output is written over are read whole before that by the arrangement only.)
     const bool apart = d_arranged != nullptr || !overlap(d_a, (size_t)m * k * 2, d_out, (size_t)m * n * ((out_dtype & ~RFQ_GEMM_ONE_PLANE) == RFQ_F16 ? 2 : 4));
-    if (known && (out_dtype & RFQ_GEMM_ONE_PLANE) == 0 && static_fits && rows_in_range && apart &&
+    // (the few-row kernel's offsets between plain rows are 32 bits wide)
+    const bool near = d_arranged != nullptr || k <= 1 << 24;
+    if (known && (out_dtype & RFQ_GEMM_ONE_PLANE) == 0 && static_fits && rows_in_range && apart && near &&
         prefer_skinny_gemm(fmt, m, n, k, rival_parts))
         return launch_skinny_gemm(fmt, d_w, static_cast<const uint8_t *>(d_arranged != nullptr ? d_arranged : d_a), d_arranged != nullptr,
                                   d_out, out_dtype == RFQ_F16, m, n, k, s);

@@ -74,28 +74,46 @@ template <int FMT> int gemv_fmt(const SkinnyGemv &c, hipStream_t s)
     return c.m <= 4 ? gemv_rows<FMT, 4, false>(c, s) : gemv_rows<FMT, 8, false>(c, s);
 }
 
-template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES>
-int gemm_cfg(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int n, int k, int rows, int slices, hipStream_t s)
+template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES, bool FULL, bool PAIR = in_pairs(FMT, MT, ARR, FULL)>
+int gemm_launch(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int n, int k, int rows, int slices, hipStream_t s)
 {
     constexpr bool STAGED = A16<W<FMT>::ORDER, W<FMT>::PAIRS, ARR>::STAGED;
-    constexpr int MOST_LDS = gemm_lds<MT, TJ, STAGED>(WAVES);
+    constexpr int MOST_LDS = gemm_lds<MT, TJ, STAGED, PAIR>(WAVES);
     static_assert(MOST_LDS <= 160 * 1024, "LDS");
     const int waves = waves_for(k, WAVES);
-    const size_t lds = (size_t)gemm_lds<MT, TJ, STAGED>(waves);
+    const size_t lds = (size_t)gemm_lds<MT, TJ, STAGED, PAIR>(waves);
     if constexpr (MOST_LDS > 64 * 1024) {
         static std::once_flag once;
         static hipError_t err = hipSuccess;
         std::call_once(once, [] {
-            err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES>),
+            err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES, FULL, PAIR>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, MOST_LDS);
         });
         if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(gemm_skinny_kernel)");
     }
     note_kernel(ARR ? "gemm_skinny_kernel<%s,%d,%d,%d,arranged>" : "gemm_skinny_kernel<%s,%d,%d,%d>", FMT, MT, TJ, slices);
-    hipLaunchKernelGGL((gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES>), dim3((n + 16 * TJ - 1) / (16 * TJ), slices), dim3(64 * waves), lds, s,
+    hipLaunchKernelGGL((gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES, FULL, PAIR>), dim3((n + 16 * TJ - 1) / (16 * TJ), slices), dim3(64 * waves), lds, s,
                        w, a, y, f16_out, m, n, k, rows);
     RFQ_LAUNCH_CHECK("gemm_skinny_kernel");
     return RFQ_OK;
+}
+
+// Two row tiles of W beside two to four operands of rows take 121 .. 172 registers, one workgroup per CU, and with a few spilled 128:
+// two per CU, which pays as soon as there are more workgroups than CUs (48 x 4096 -> 14336: GGUF_Q4_K 25.1 / 21.4 us, Q8_0 23.6 /
+// 22.3, GGUF_Q6_K 28.2 / 25.1; 282 workgroups, 37 x 2048 -> 9000: GGUF_Q4_K 14.4 / 12.0; with 160 workgroups, 64 x 1280 -> 5120: Q8_0 6.8 / 7.4, GGUF_Q4_0 6.7 / 8.0).
+template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES>
+int gemm_cfg(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int n, int k, int rows, int slices, hipStream_t s)
+{
+    const bool more = (long)((n + 16 * TJ - 1) / (16 * TJ)) * slices > device_cu_count();
+    if constexpr (TJ == 2 && MT >= 2 && MT <= 4 && !ARR)
+        if (more) return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, true>(w, a, y, f16_out, m, n, k, rows, slices, s);
+    // (single groups stay ahead in two places: long rows of the 4-bit GGUF layouts, 20 x 14336 -> 4096 GGUF_Q4_K 20.6 / 21.7 us, and six
+    // operands of the Q6_K layouts in several rounds, 160 x 3072 -> 6144 GGUF_Q6_K 33.0 / 34.3)
+    if constexpr (TJ == 1 && MT == 2 && !ARR && (FMT == RFQ_GGUF_Q4_0 || FMT == RFQ_GGUF_Q4_K))
+        if (k > 8192) return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, false, false>(w, a, y, f16_out, m, n, k, rows, slices, s);
+    if constexpr (TJ == 2 && MT == 6 && !ARR && (FMT == RFQ_Q6_K || FMT == RFQ_GGUF_Q6_K))
+        if (more) return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, false, false>(w, a, y, f16_out, m, n, k, rows, slices, s);
+    return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, false>(w, a, y, f16_out, m, n, k, rows, slices, s);
 }
 
 // 16-row operands per workgroup at most: six with one row tile (eight leave its registers one wavefront per SIMD: Q8_0

@@ -403,6 +403,27 @@ def test_every_prompt_kernel(fmt, oracle, cuda):
         assert_close(plain.cpu().numpy(), want, f"{Q.NAMES[fmt]} {m}x{n}x{k} {form}", tol=TOL, plain_tol=2e-4)
 
 
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(17, 40, 8224), (29, 3000, 8448), (20, 8193, 8192), (33, 8225, 416), (56, 8250, 352), (85, 8250, 192), (96, 16400, 256)])
+def test_rows_in_pairs_of_groups(fmt, m, n, k, oracle, cuda):
+    """Rows fetched as pairs of groups and as single ones, at the sizes where one takes over from the other (long rows; one workgroup
+    more than CUs at 32 rows of W each), last pairs of one group, and rows past the last that are not a multiple of eight."""
+    import torch
+    from rocmforge_amd import ops
+    n, k = shape_of(fmt, n, k)
+    w = Q.make_weights(fmt, n, k, seed=fmt)
+    a = np.random.default_rng(m).standard_normal((m, k)).astype(np.float16)
+    dw, da = torch.from_numpy(w).to(cuda), torch.from_numpy(a).to(cuda)
+    got = ops.gemm_f16(fmt, dw, da, n, k, out_dtype=torch.float32)
+    plain = kernel_name()
+    arranged = ops.gemm_f16_arranged(fmt, dw, ops.ArrangedA(da), n, out_dtype=torch.float32)
+    if plain.startswith("gemm_skinny_kernel"):
+        assert torch.equal(got, arranged)
+    pick = np.unique(np.concatenate([np.arange(0, n, max(1, n // 61)), np.arange(n - 20, n)]))
+    w64 = weights_of(oracle, fmt, w, n, k)[pick]
+    assert_close(got.cpu().numpy()[:, pick], a.astype(np.float64) @ w64.T, f"{Q.NAMES[fmt]} {m}x{n}x{k} {plain}", tol=TOL, plain_tol=2e-4)
+
+
 @pytest.mark.parametrize("fmt", BATCH_FORMATS)
 @pytest.mark.parametrize("norm", [False, True])
 def test_every_decode_batch_kernel(fmt, norm, oracle, cuda):
