@@ -111,7 +111,7 @@ int gemm_cfg(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, in
     // operands of the Q6_K layouts in several rounds, 160 x 3072 -> 6144 GGUF_Q6_K 33.0 / 34.3)
     if constexpr (TJ == 1 && MT == 2 && !ARR && (FMT == RFQ_GGUF_Q4_0 || FMT == RFQ_GGUF_Q4_K))
         if (k > 8192) return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, false, false>(w, a, y, f16_out, m, n, k, rows, slices, s);
-    if constexpr (TJ == 2 && MT == 6 && !ARR && (FMT == RFQ_Q6_K || FMT == RFQ_GGUF_Q6_K))
+    if constexpr (TJ == 2 && (MT == 5 || MT == 6) && !ARR && (FMT == RFQ_Q6_K || FMT == RFQ_GGUF_Q6_K))
         if (more) return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, false, false>(w, a, y, f16_out, m, n, k, rows, slices, s);
     return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, false>(w, a, y, f16_out, m, n, k, rows, slices, s);
 }
@@ -159,6 +159,12 @@ int gemm_mt(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int
     case 3: return gemm_cfg<FMT, 3, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
     case 4: return gemm_cfg<FMT, 4, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
     default:
+        // (five beside two row tiles: 160 x 4096 -> 4096 Q8_0 18.9 us as six, 17.7 as five, Q/K/V of 160 tokens GGUF_Q4_K 36.1 / 35.3; but
+        // GGUF_Q6_K in several rounds 17.9 / 18.6, 130 x 1280 -> 5120)
+        if constexpr (MOST >= 6 && TJ == 2) {
+            const bool rounds = (long)((n + 31) / 32) * slices > device_cu_count();
+            if (sl.tiles == 5 && !(FMT == RFQ_GGUF_Q6_K && rounds)) return gemm_cfg<FMT, 5, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
+        }
         if constexpr (MOST >= 6)
             if (sl.tiles <= 6) return gemm_cfg<FMT, 6, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
         if constexpr (MOST >= 8)

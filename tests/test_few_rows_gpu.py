@@ -404,10 +404,10 @@ def test_every_prompt_kernel(fmt, oracle, cuda):
 
 
 @pytest.mark.parametrize("fmt", FORMATS)
-@pytest.mark.parametrize("m,n,k", [(17, 40, 8224), (29, 3000, 8448), (20, 8193, 8192), (33, 8225, 416), (56, 8250, 352), (85, 8250, 192), (96, 16400, 256)])
+@pytest.mark.parametrize("m,n,k", [(17, 40, 8224), (29, 3000, 8448), (20, 8193, 8192), (33, 8225, 416), (56, 8250, 352), (85, 8250, 192), (96, 16400, 256), (75, 8000, 224), (80, 8300, 256), (150, 5001, 544)])
 def test_rows_in_pairs_of_groups(fmt, m, n, k, oracle, cuda):
     """Rows fetched as pairs of groups and as single ones, at the sizes where one takes over from the other (long rows; one workgroup
-    more than CUs at 32 rows of W each), last pairs of one group, and rows past the last that are not a multiple of eight."""
+    more than CUs at 32 rows of W each; five operands), last pairs of one group, and rows past the last that are not a multiple of eight."""
     import torch
     from rocmforge_amd import ops
     n, k = shape_of(fmt, n, k)
