@@ -350,7 +350,7 @@ int rfq_rms_norm_gemv(int fmt, const void *d_w, size_t w_bytes, const float *d_x
     // (a result written over x, or a norm in place: x is read before anything is written only by the separate steps)
     const size_t x_bytes = (size_t)m * k * 4, y_bytes = (size_t)m * n * 4;
     if (!overlap(d_y, y_bytes, d_x, x_bytes) && !overlap(d_y, y_bytes, d_norm_weight, (size_t)k * 4) && !overlap(d_scratch, x_bytes, d_x, x_bytes)) {
-        rc = launch_skinny_gemv_fused(fmt, (const uint8_t *)d_w, nullptr, d_x, d_norm_weight, eps, d_y, m, n, k, s);
+        rc = launch_skinny_gemv_fused(fmt, (const uint8_t *)d_w, nullptr, d_x, d_norm_weight, eps, d_y, m, n, k, s, nullptr);
         if (rc != RFQ_E_UNSUPPORTED) return rc;
     }
     rc = launch_rms_norm(RFQ_TABLE_F32, d_x, d_norm_weight, d_scratch, m, k, eps, s);
@@ -365,6 +365,19 @@ size_t rfq_mlp_scratch_bytes(int m, int hidden_size, int intermediate_size)
 {
     if (m <= 0 || hidden_size <= 0 || intermediate_size <= 0) return 0;
     return 3 * pad16((size_t)m * intermediate_size * 4) + pad16((size_t)m * hidden_size * 4);
+}
+
+// Whether x is prepared by a launch of its own (5 us, an eighth of them work) before a batch's projection, so that no workgroup
+// converts it: large matrices of the formats whose kernels are bound by vector instructions.  One step each, m = 6: GGUF_Q4_K gate
+// and up 5120 -> 13824 73.2 -> 65.2 us of the block, down 73.2 -> 66.6; MXFP4 79.3 -> 77.9 and -> 70.6; at 2560 -> 7168 (37 and 18
+// million weights) level or slower.  Up to four vectors only gate and up of the MXFP formats gain: 69.5 -> 62.2, 4 x 5120 -> 13824
+// MXFP4.  Q8_0, Q4_K and the Q6_K layouts were level or lost 1 to 5 % at any size.
+static bool prepare_pays(int fmt, int m, bool pair, size_t weights)
+{
+    const int cf = canonical_format(fmt);
+    const bool mx = cf == RFQ_MXFP4 || cf == RFQ_MXFP6_E2M3;
+    if (!prepared_format(cf) || m < 2 || (m < 5 && !(mx && pair))) return false;
+    return weights >= (pair ? (size_t)80000000 : (size_t)40000000);
 }
 
 int rfq_mlp_swiglu(int fmt_gate_up, const void *d_gate_w, const void *d_up_w, size_t gate_up_bytes, int fmt_down,
@@ -401,7 +414,9 @@ int rfq_mlp_swiglu(int fmt_gate_up, const void *d_gate_w, const void *d_up_w, si
         if (d_norm_weight && (hidden_size % 4 != 0 || !aligned16(d_x) || !aligned16(d_norm_weight)))
             return fail(RFQ_E_BADARG, "rfq_mlp_swiglu: x and norm weight must be 16-byte aligned, hidden_size a multiple of 4");
         rc = launch_skinny_gemv_fused(fmt_gate_up, (const uint8_t *)d_gate_w, (const uint8_t *)d_up_w, d_x, d_norm_weight, eps, h, m,
-                                      intermediate_size, hidden_size, s);
+                                      intermediate_size, hidden_size, s,
+                                      ready_bytes(m, hidden_size) <= need - mi && prepare_pays(fmt_gate_up, m, true, 2 * (size_t)intermediate_size * hidden_size)
+                                          ? base + mi : nullptr);
     }
     if (rc == RFQ_E_UNSUPPORTED) {
         const float *xin = d_x;
@@ -417,6 +432,10 @@ int rfq_mlp_swiglu(int fmt_gate_up, const void *d_gate_w, const void *d_up_w, si
         rc = launch_swiglu(gate, up, h, (size_t)m * intermediate_size, s);
     }
     if (rc != RFQ_OK) return rc;
+    if (ready_bytes(m, intermediate_size) <= need - mi && prepare_pays(fmt_down, m, false, (size_t)hidden_size * intermediate_size)) {
+        rc = launch_gemv_prepared(fmt_down, (const uint8_t *)d_down_w, h, d_out, m, hidden_size, intermediate_size, base + mi, s);
+        if (rc != RFQ_E_UNSUPPORTED) return rc;
+    }
     return launch_gemv(fmt_down, (const uint8_t *)d_down_w, h, d_out, m, hidden_size, intermediate_size, s);
 }
 

@@ -130,9 +130,17 @@ struct SkinnyGemv {
     float eps;
     float *y;
     int m, n, k;
+    const uint8_t *ready;                                         // x as launch_prepare_x wrote it (nullptr: every workgroup converts x)
     int keep_infinities;                                          // an infinity in x: see keeps_infinities; 0: its vector's results are NaN
 };
 int launch_skinny_gemv(int fmt, const SkinnyGemv &c, hipStream_t s);
+// x for SkinnyGemv::ready, ready_bytes(m, k) of it.
+constexpr size_t ready_bytes(int m, int k) { return (size_t)((k + 127) / 128) * (512 * m + 64); }
+constexpr bool prepared_format(int fmt)
+{
+    return fmt == RFQ_Q4_0 || fmt == RFQ_GGUF_Q4_0 || fmt == RFQ_GGUF_Q4_K || fmt == RFQ_MXFP4 || fmt == RFQ_MXFP6_E2M3;
+}
+int launch_prepare_x(int fmt, const SkinnyGemv &c, uint8_t *out, hipStream_t s);
 bool few_rows_aligned(int fmt, const void *w, const void *w2, const void *x);
 // Whether the above is the faster way for rows of x [m, k] and this matrix (m >= 2), alone and with what it takes along.
 bool few_rows_ahead(int fmt, int m, int n, int ku, bool batch_fits);
@@ -140,7 +148,8 @@ bool few_rows_ahead(int fmt, int m, int n, int ku, bool batch_fits);
 // results, as the kernels do that take the format and shape in other batches.
 bool keeps_infinities(int fmt, int n, int ku, bool batch_fits);
 int launch_skinny_gemv_fused(int fmt, const uint8_t *d_w, const uint8_t *d_w2, const float *d_x, const float *d_norm_w, float eps, float *d_y,
-                             int m, int n, int k, hipStream_t s);
+                             int m, int n, int k, hipStream_t s, uint8_t *ready);
+int launch_gemv_prepared(int fmt, const uint8_t *d_w, const float *d_x, float *d_y, int m, int n, int k, uint8_t *ready, hipStream_t s);
 int launch_skinny_gemm(int fmt, const uint8_t *w, const uint8_t *a, bool arranged, void *y, bool f16_out, int m, int n, int k,
                        hipStream_t s);
 // The tiled kernel on integer codes (rfq_gemm_codes.hip): arranged activations (s2: their group sums, GGUF_Q4_K); kparts > 1:

@@ -2493,7 +2493,7 @@ int run(const uint8_t *w, const float *x, float *y, int m, int n, int k, hipStre
         return run_rows<FMT, false>(w, x, y, n, k, GemvFuse{nullptr, nullptr, 0.0f, 0}, s);
     const bool batch_fits = HasIdotBatch<FMT>::value && ku > 32 && ku <= 256;
     if (m > 1 && few_rows_aligned(FMT, w, nullptr, x) && few_rows_ahead(FMT, m, n, ku, batch_fits)) {
-        return launch_skinny_gemv(FMT, SkinnyGemv{w, nullptr, x, nullptr, 0.0f, y, m, n, k, keeps_infinities(FMT, n, ku, batch_fits)}, s);
+        return launch_skinny_gemv(FMT, SkinnyGemv{w, nullptr, x, nullptr, 0.0f, y, m, n, k, nullptr, keeps_infinities(FMT, n, ku, batch_fits)}, s);
     }
     if (batch_fits && m > 1) {
         // (four vectors at most: the prepared ones of a launch live in LDS, 112 bytes per unit and vector)
@@ -2665,7 +2665,7 @@ bool keeps_infinities(int fmt, int n, int ku, bool batch_fits)
 // 3 us for the norm, 8 for norm, second projection and activation) are worth more than the difference: a norm up to 16
 // or 20 rows per CU, two matrices up to 40 (two vectors) or at any size (three and more).
 int launch_skinny_gemv_fused(int fmt, const uint8_t *d_w, const uint8_t *d_w2, const float *d_x, const float *d_norm_w, float eps, float *d_y,
-                             int m, int n, int k, hipStream_t s)
+                             int m, int n, int k, hipStream_t s, uint8_t *ready)
 {
     const int cf = canonical_format(fmt), ku = k / 32, cus = device_cu_count();
     if (m < 2 || m > 8 || gemv_part_of(cf) < 0 || fmt_mm_variant(fmt)) return RFQ_E_UNSUPPORTED;
@@ -2677,7 +2677,24 @@ int launch_skinny_gemv_fused(int fmt, const uint8_t *d_w, const uint8_t *d_w2, c
     const bool taken = d_w2 != nullptr ? m >= 3 || n <= cus * 20 || few_rows_ahead(cf, m, n, ku, batch_fits)
                                        : n <= norm_rows || few_rows_ahead(cf, m, n, ku, batch_fits);
     if (!taken) return RFQ_E_UNSUPPORTED;
-    return launch_skinny_gemv(cf, SkinnyGemv{d_w, d_w2, d_x, d_norm_w, eps, d_y, m, n, k, keeps_infinities(cf, n, ku, batch_fits)}, s);
+    const SkinnyGemv c{d_w, d_w2, d_x, d_norm_w, eps, d_y, m, n, k, ready, keeps_infinities(cf, n, ku, batch_fits)};
+    if (ready != nullptr)
+        if (int rc = launch_prepare_x(cf, c, ready, s)) return rc;
+    return launch_skinny_gemv(cf, c, s);
+}
+
+// y = x . W^T for a batch through x prepared in `ready` (ready_bytes): RFQ_E_UNSUPPORTED where a batch of this shape does not go
+// to the few-row kernel.
+int launch_gemv_prepared(int fmt, const uint8_t *d_w, const float *d_x, float *d_y, int m, int n, int k, uint8_t *ready, hipStream_t s)
+{
+    const int cf = canonical_format(fmt), ku = k / 32;
+    if (m < 2 || m > 8 || gemv_part_of(cf) < 0 || fmt_mm_variant(fmt) || !few_rows_aligned(cf, d_w, nullptr, d_x)) return RFQ_E_UNSUPPORTED;
+    const bool per_vector = cf == RFQ_Q6_K || cf == RFQ_MXFP4 || cf == RFQ_MXFP6_E2M3;
+    const bool batch_fits = !per_vector && ku > 32 && ku <= 256;
+    if (!few_rows_ahead(cf, m, n, ku, batch_fits)) return RFQ_E_UNSUPPORTED;
+    const SkinnyGemv c{d_w, nullptr, d_x, nullptr, 0.0f, d_y, m, n, k, ready, keeps_infinities(cf, n, ku, batch_fits)};
+    if (int rc = launch_prepare_x(cf, c, ready, s)) return rc;
+    return launch_skinny_gemv(cf, c, s);
 }
 
 // One launch for RMSNorm -> GEMV (norm_w != nullptr) and / or two GEMVs sharing

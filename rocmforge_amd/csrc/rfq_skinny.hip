@@ -35,7 +35,7 @@ int waves_for(int k, int most)
 
 constexpr int GEMV_WAVES = 8;
 
-template <int FMT, int TJ, int MV, bool NORM>
+template <int FMT, int TJ, int MV, bool NORM, bool READY>
 int gemv_cfg(const SkinnyGemv &c, hipStream_t s)
 {
     const int waves = waves_for(c.k, GEMV_WAVES);
@@ -43,9 +43,10 @@ int gemv_cfg(const SkinnyGemv &c, hipStream_t s)
     static_assert(gemv_lds<TJ, MV>(GEMV_WAVES) <= 64 * 1024, "LDS a launch gets without asking");
     const size_t lds = (size_t)gemv_lds<TJ, MV>(waves);
     const int rows = c.w2 != nullptr ? 8 * TJ : 16 * TJ;
-    note_kernel(c.w2 != nullptr ? "gemv_skinny_kernel<%s,%d,%d,%d,pair>" : "gemv_skinny_kernel<%s,%d,%d,%d>", FMT, TJ, MV, NORM);
-    hipLaunchKernelGGL((gemv_skinny_kernel<FMT, TJ, MV, D, GEMV_WAVES, NORM>), dim3((c.n + rows - 1) / rows), dim3(64 * waves), lds, s, c.w, c.x,
-                       c.y, c.m, c.n, c.k, c.w2, c.norm_w, c.eps, c.keep_infinities);
+    note_kernel(c.w2 != nullptr ? READY ? "gemv_skinny_kernel<%s,%d,%d,%d,pair,ready>" : "gemv_skinny_kernel<%s,%d,%d,%d,pair>"
+                                : READY ? "gemv_skinny_kernel<%s,%d,%d,%d,ready>" : "gemv_skinny_kernel<%s,%d,%d,%d>", FMT, TJ, MV, NORM);
+    hipLaunchKernelGGL((gemv_skinny_kernel<FMT, TJ, MV, D, GEMV_WAVES, NORM, READY>), dim3((c.n + rows - 1) / rows), dim3(64 * waves), lds, s, c.w, c.x,
+                       c.y, c.m, c.n, c.k, c.w2, c.norm_w, c.eps, c.keep_infinities, c.ready);
     RFQ_LAUNCH_CHECK("gemv_skinny_kernel");
     return RFQ_OK;
 }
@@ -59,13 +60,19 @@ int gemv_cfg(const SkinnyGemv &c, hipStream_t s)
 template <int FMT, int MV, bool NORM>
 int gemv_rows(const SkinnyGemv &c, hipStream_t s)
 {
+    // (prepared x: nothing to share between row tiles, so as many workgroups as the pair or the single matrix allows)
+    if constexpr (prepared_format(FMT)) {
+        if (c.ready != nullptr && c.w2 != nullptr) return gemv_cfg<FMT, 2, MV, NORM, true>(c, s);
+        if constexpr (!NORM)
+            if (c.ready != nullptr) return gemv_cfg<FMT, 1, MV, NORM, true>(c, s);
+    }
     constexpr bool MX = FMT == RFQ_MXFP4 || FMT == RFQ_MXFP6_E2M3;
     const int cus = device_cu_count();
     const long rows = c.w2 != nullptr ? 2L * c.n : c.n;
     if constexpr (MV == 8 || MX)
-        if (rows >= 52L * cus && (MV == 8 || c.w2 != nullptr)) return gemv_cfg<FMT, 4, MV, NORM>(c, s);
-    if (rows > 20L * cus || c.w2 != nullptr) return gemv_cfg<FMT, 2, MV, NORM>(c, s);
-    return gemv_cfg<FMT, 1, MV, NORM>(c, s);
+        if (rows >= 52L * cus && (MV == 8 || c.w2 != nullptr)) return gemv_cfg<FMT, 4, MV, NORM, false>(c, s);
+    if (rows > 20L * cus || c.w2 != nullptr) return gemv_cfg<FMT, 2, MV, NORM, false>(c, s);
+    return gemv_cfg<FMT, 1, MV, NORM, false>(c, s);
 }
 
 template <int FMT> int gemv_fmt(const SkinnyGemv &c, hipStream_t s)
@@ -245,6 +252,25 @@ bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts)
     double tiled = 8.0 + per_ku * ku / parts * (groups > cus ? groups / cus : 1.0);
     if (parts > 1) tiled += 4.0 + 8.0 * parts * m * (double)n / 5e6;
     return few < tiled;
+}
+
+int launch_prepare_x(int fmt, const SkinnyGemv &c, uint8_t *out, hipStream_t s)
+{
+    const dim3 grid((c.k + 127) / 128), block(c.m <= 4 ? 64 : 128);
+#define RFQ_PREPARE(F)                                                                                                                      \
+    hipLaunchKernelGGL((prepare_x_kernel<W<F>::ORDER, W<F>::PAIRS>), grid, block, 0, s, c.x, c.norm_w, c.m, c.k, out, c.keep_infinities); \
+    break
+    switch (fmt) {
+    case RFQ_Q4_0: RFQ_PREPARE(RFQ_Q4_0);
+    case RFQ_MXFP6_E2M3: RFQ_PREPARE(RFQ_MXFP6_E2M3);
+    case RFQ_GGUF_Q4_0: RFQ_PREPARE(RFQ_GGUF_Q4_0);
+    case RFQ_GGUF_Q4_K: RFQ_PREPARE(RFQ_GGUF_Q4_K);
+    case RFQ_MXFP4: RFQ_PREPARE(RFQ_MXFP4);
+    default: return fail(RFQ_E_UNSUPPORTED, "no few-row kernel on prepared x for format %d", fmt);
+    }
+#undef RFQ_PREPARE
+    RFQ_LAUNCH_CHECK("prepare_x_kernel");
+    return RFQ_OK;
 }
 
 int launch_skinny_gemv(int fmt, const SkinnyGemv &c, hipStream_t s)

@@ -641,7 +641,8 @@ constexpr int XROW = 256 + 16;                                    // bytes of a 
 template <int MV> constexpr int x_bytes() { return 2 * MV * XROW + MV * 4; }
 template <int TJ, int MV> constexpr int gemv_lds(int waves)
 {
-    // (the results are followed by the vectors' sums of squares)
+    // (the results are followed by the vectors' sums of squares, MV per wavefront, or of prepared x MV in double: x_bytes leaves room)
+    static_assert(x_bytes<MV>() >= MV * 16 * TJ * 4 + MV * 8, "room for the sums of squares");
     return waves * (x_bytes<MV>() > MV * (16 * TJ + 1) * 4 ? x_bytes<MV>() : MV * (16 * TJ + 1) * 4);
 }
 
@@ -667,18 +668,106 @@ __device__ __forceinline__ uint32_t max16(uint32_t v)
     return v;
 }
 
-// MV: 4 or 8 vectors, m <= MV.
-template <int FMT, int TJ, int MV, int D, int WAVES, bool NORM>
+// Octet e (8 consecutive elements of one vector; ex: the biased exponent of the vector's largest |x| in the unit) as the two
+// fp16 parts under a power of two that takes that largest to 2^top .. 2^(top + 1); inv: its inverse.
+template <int PAIRS, bool LOW>
+__device__ __forceinline__ void split_octet(const float (&e)[8], int ex, int top, uint32_t (&hi)[4], uint32_t (&lo)[4], float &inv)
+{
+    int se = 254 + top - ex;                                      // s = 2^(top - (ex - 127))
+    se = se > 243 ? 243 : LOW && se < 1 ? 1 : se;                 // (2048 s stays finite, s above zero)
+    const float s = __uint_as_float((uint32_t)se << 23);
+    inv = __uint_as_float((uint32_t)(254 - se) << 23);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        // (x * s, x - hi / s and its multiple by 2048 s are exact: a part is rounded once, to fp16)
+        const float a = e[pair_of<PAIRS>(r, 0)], b = e[pair_of<PAIRS>(r, 1)];
+        v2h h = {(_Float16)__builtin_fmaf(a, s, 0.0f), (_Float16)__builtin_fmaf(b, s, 0.0f)};
+        __builtin_memcpy(&hi[r], &h, 4);
+        asm("" : "+v"(hi[r]));                                    // (one conversion of each product, not one per use)
+        __builtin_memcpy(&h, &hi[r], 4);
+        const float ra = __builtin_fmaf((float)h[0], -inv, a), rb = __builtin_fmaf((float)h[1], -inv, b);
+        const v2h l = {(_Float16)__builtin_fmaf(ra, s * 2048.0f, 0.0f), (_Float16)__builtin_fmaf(rb, s * 2048.0f, 0.0f)};
+        __builtin_memcpy(&lo[r], &l, 4);
+    }
+}
+// What an infinity leaves as its lower part is a NaN, and with it every result of the vector; without it the infinity's product
+// with a weight that is not zero stays one.
+__device__ __forceinline__ uint32_t without_infinities(uint32_t hi, uint32_t lo)
+{
+    return lo & (((hi & 0x7FFFu) == 0x7C00u ? 0u : 0xFFFFu) | ((hi & 0x7FFF0000u) == 0x7C000000u ? 0u : 0xFFFF0000u));
+}
+
+// x prepared for several workgroups (SkinnyGemv::ready), in the caller's scratch memory: per unit, group and lane row the operands
+// of the m vectors' upper parts and then of their lower parts, 16 bytes each; behind all units, eight floats per unit
+// each, the vectors' inverse scales and (norm) their sums of squares.
+__host__ __device__ constexpr size_t ready_squares(int m, int units) { return (size_t)units * (512 * m + 32); }
+
+template <int ORDER, int PAIRS>
+__global__ void __launch_bounds__(128)
+prepare_x_kernel(const float *__restrict__ x, const float *__restrict__ norm_w, int m, int k, uint8_t *__restrict__ out, int keep_infinities)
+{
+    const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4, u = blockIdx.x, units = gridDim.x;
+    const int v = 4 * (int)(threadIdx.x >> 6) + q, at = 128 * u + 8 * i;
+    float e[8], ss = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 8; c++) e[c] = 0.0f;
+    if (at < k) {
+        const float *p = x + (size_t)(v < m ? v : m - 1) * k + at;
+        const v4f a = *reinterpret_cast<const v4f_a4 *>(p), b = *reinterpret_cast<const v4f_a4 *>(p + 4);
+#pragma unroll
+        for (int c = 0; c < 4; c++) { e[c] = a[c]; e[4 + c] = b[c]; }
+        if (norm_w != nullptr) {
+            const v4f na = *reinterpret_cast<const v4f *>(norm_w + at), nb = *reinterpret_cast<const v4f *>(norm_w + at + 4);
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                ss = __builtin_fmaf(e[c], e[c], ss);
+                e[c] *= c < 4 ? na[c & 3] : nb[c & 3];
+            }
+        }
+    }
+    const float mx = max3_abs(max3_abs(e[0], e[1], e[2]), max3_abs(e[3], e[4], e[5]), max3_abs(e[6], e[7], 0.0f));
+    const int ex = (int)(max16(__float_as_uint(mx)) >> 23);
+    uint32_t hi[4], lo[4];
+    float inv;
+    split_octet<PAIRS, false>(e, ex, 14, hi, lo, inv);
+    if (keep_infinities && ex == 255) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) lo[r] = without_infinities(hi[r], lo[r]);
+    }
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) ss += __shfl_xor(ss, o);
+    if (v >= m) return;
+    uint8_t *const unit = out + (size_t)u * (512 * m);
+    const int o = i & 3, j4 = (i >> 2) * 4;                       // octet o of group i >> 2
+    if constexpr (ORDER <= OCTET_SWAPPED) {
+        uint8_t *const to = unit + ((j4 + row_part(ORDER, o)) * (2 * m) + v) * 16;
+        *reinterpret_cast<v4u *>(to) = v4u{hi[0], hi[1], hi[2], hi[3]};
+        *reinterpret_cast<v4u *>(to + m * 16) = v4u{lo[0], lo[1], lo[2], lo[3]};
+    } else {
+        uint8_t *const t0 = unit + ((j4 + 2 * (o & 1)) * (2 * m) + v) * 16 + (o >> 1) * 8, *const t1 = t0 + 2 * m * 16;
+        *reinterpret_cast<v2u *>(t0) = v2u{hi[0], hi[1]};
+        *reinterpret_cast<v2u *>(t0 + m * 16) = v2u{lo[0], lo[1]};
+        *reinterpret_cast<v2u *>(t1) = v2u{hi[2], hi[3]};
+        *reinterpret_cast<v2u *>(t1 + m * 16) = v2u{lo[2], lo[3]};
+    }
+    if (i == 0) {
+        reinterpret_cast<float *>(out + (size_t)units * (512 * m))[u * 8 + v] = inv;
+        reinterpret_cast<float *>(out + ready_squares(m, units))[u * 8 + v] = ss;
+    }
+}
+
+// MV: 4 or 8 vectors, m <= MV.  READY: x comes prepared (prepare_x_kernel) and no workgroup converts it.
+template <int FMT, int TJ, int MV, int D, int WAVES, bool NORM, bool READY>
 __global__ void __launch_bounds__(64 * WAVES, (FMT == RFQ_MXFP4 && TJ == 2 && MV == 4 && !NORM ? 4 : 1))   // (128 registers, which it misses by two: two workgroups per CU)
 gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y, int m, int n, int k,
-                   const uint8_t *__restrict__ w2, const float *__restrict__ norm_w, float eps, int keep_infinities)
+                   const uint8_t *__restrict__ w2, const float *__restrict__ norm_w, float eps, int keep_infinities, const uint8_t *__restrict__ ready)
 {
     typedef W<FMT> WF;
     constexpr int P = MV / 4;                                     // octets of x per lane and unit
     // With one row tile a unit's x is taken and its scale found (a chain of nine instructions) beside the sums of the unit
     // before (GGUF_Q4_0 5 x 14336 -> 4096 22.2 -> 19.8 us); with more, the registers it needs would leave room for one
     // workgroup per CU instead of two, or spill (GGUF_Q6_K 5 x 4096 -> 14336 28 -> 76 us).
-    constexpr bool AHEAD = TJ == 1;
+    constexpr bool AHEAD = TJ == 1 && !READY;
     constexpr bool F32_SCALE = FMT == RFQ_Q4_0 || FMT == RFQ_Q8_0;
     constexpr bool INFINITIES = FMT == RFQ_Q4_K || FMT == RFQ_Q6_K || FMT == RFQ_MXFP4 || FMT == RFQ_MXFP6_E2M3;   // (see keeps_infinities)
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -772,9 +861,24 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
         for (int r = 0; r < 4; r++) acc[t][r] = 0.0;
     const v4u ones = {0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
 
-    load_x(wave);
+    // READY: a unit's operands and inverse scales, fetched with its weights
+    v4u xq[D][4];
+    v4f iq[D];
+    const int xi = i & (2 * MV - 1), xv = xi & (MV - 1);
+    const float *const iq_lane = READY ? reinterpret_cast<const float *>(ready + (size_t)units * (512 * m)) + (4 * q & (MV - 1)) : nullptr;
+    const uint8_t *const xq_lane = READY ? ready + (q * (2 * m) + (xv < m ? xv : m - 1) + (xi < MV ? 0 : m)) * 16 : nullptr;
+    auto load_ready = [&](int d, int u) __attribute__((always_inline)) {
+        const int uc = u < units ? u : units - 1;
 #pragma unroll
-    for (int d = 0; d < D; d++) load_w(raw[d], wave + d * waves);
+        for (int j = 0; j < 4; j++) xq[d][j] = *reinterpret_cast<const v4u *>(xq_lane + (size_t)uc * (512 * m) + j * (128 * m));
+        iq[d] = *reinterpret_cast<const v4f *>(iq_lane + (size_t)uc * 8);
+    };
+    if constexpr (!READY) load_x(wave);
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+        load_w(raw[d], wave + d * waves);
+        if constexpr (READY) load_ready(d, wave + d * waves);
+    }
     if constexpr (AHEAD) {
         take_x(wave);
         load_x(wave + waves);
@@ -785,72 +889,55 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
         for (int d = 0; d < D; d++) {
             const int u = u0 + d * waves;
             if (u < units) {
-                if constexpr (!AHEAD) {
+                if constexpr (!AHEAD && !READY) {
                     take_x(u);
                     load_x(u + waves);
                 }
-                int top = 14;                                     // the largest |x| goes to 2^top .. 2^(top + 1)
+                // (a sum of 32 codes times 2^15 is below 2^28: a block scale from 2^100 on could take it past the largest
+                // float where the result, with small x, is not)
+                bool large = false;
                 if constexpr (F32_SCALE) {
-                    // (a sum of 32 codes times 2^15 is below 2^28: a block scale from 2^100 on could take it past the largest
-                    // float where the result, with small x, is not.  With such a scale x loses bits below 2^-11 of the largest.)
-                    bool large = false;
 #pragma unroll
                     for (int t = 0; t < TJ; t++) large |= fabsf(__uint_as_float(raw[d][t].r[0])) >= 0x1p100f;
-                    if (__builtin_amdgcn_ballot_w64(large) != 0) top = -14;
+                    large = __builtin_amdgcn_ballot_w64(large) != 0;
                 }
-                wave_order();                                     // (the unit before has been read)
-                float s[P], inv_s[P];
-                unsigned long long infinite = 0;
+                if constexpr (!READY) {
+                    // (with such a scale x loses bits below 2^-11 of the largest)
+                    const int top = large ? -14 : 14;
+                    wave_order();                                 // (the unit before has been read)
+                    unsigned long long infinite = 0;
 #pragma unroll
-                for (int p = 0; p < P; p++) {
-                    if (INFINITIES && keep_infinities) infinite |= __builtin_amdgcn_ballot_w64(ex[p] == 255);
-                    int se = 254 + top - ex[p];                   // s = 2^(top - (ex - 127))
-                    se = se > 243 ? 243 : F32_SCALE && se < 1 ? 1 : se;   // (2048 s stays finite, s above zero)
-                    s[p] = __uint_as_float((uint32_t)se << 23);
-                    inv_s[p] = __uint_as_float((uint32_t)(254 - se) << 23);
-                    if (i == 0) area_inv[4 * p + q] = inv_s[p];
-                }
-#pragma unroll
-                for (int p = 0; p < P; p++) {
-                    uint32_t hi[4], lo[4];
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        // (x * s, x - hi / s and its multiple by 2048 s are exact: a part is rounded once, to fp16)
-                        const float a = e[p][pair_of<WF::PAIRS>(r, 0)], b = e[p][pair_of<WF::PAIRS>(r, 1)];
-                        v2h h = {(_Float16)__builtin_fmaf(a, s[p], 0.0f), (_Float16)__builtin_fmaf(b, s[p], 0.0f)};
-                        __builtin_memcpy(&hi[r], &h, 4);
-                        asm("" : "+v"(hi[r]));                    // (one conversion of each product, not one per use)
-                        __builtin_memcpy(&h, &hi[r], 4);
-                        const float ra = __builtin_fmaf((float)h[0], -inv_s[p], a), rb = __builtin_fmaf((float)h[1], -inv_s[p], b);
-                        const v2h l = {(_Float16)__builtin_fmaf(ra, s[p] * 2048.0f, 0.0f), (_Float16)__builtin_fmaf(rb, s[p] * 2048.0f, 0.0f)};
-                        __builtin_memcpy(&lo[r], &l, 4);
+                    for (int p = 0; p < P; p++) {
+                        if (INFINITIES && keep_infinities) infinite |= __builtin_amdgcn_ballot_w64(ex[p] == 255);
+                        uint32_t hi[4], lo[4];
+                        float inv_s;
+                        split_octet<WF::PAIRS, F32_SCALE>(e[p], ex[p], top, hi, lo, inv_s);
+                        if (i == 0) area_inv[4 * p + q] = inv_s;
+                        if constexpr (WF::ORDER <= OCTET_SWAPPED) {
+                            *reinterpret_cast<v4u *>(xw[p]) = v4u{hi[0], hi[1], hi[2], hi[3]};
+                            *reinterpret_cast<v4u *>(xw[p] + MV * XROW) = v4u{lo[0], lo[1], lo[2], lo[3]};
+                        } else {
+                            *reinterpret_cast<v2u *>(xw[p] + h0) = v2u{hi[0], hi[1]};
+                            *reinterpret_cast<v2u *>(xw[p] + h1) = v2u{hi[2], hi[3]};
+                            *reinterpret_cast<v2u *>(xw[p] + MV * XROW + h0) = v2u{lo[0], lo[1]};
+                            *reinterpret_cast<v2u *>(xw[p] + MV * XROW + h1) = v2u{lo[2], lo[3]};
+                        }
                     }
-                    if constexpr (WF::ORDER <= OCTET_SWAPPED) {
-                        *reinterpret_cast<v4u *>(xw[p]) = v4u{hi[0], hi[1], hi[2], hi[3]};
-                        *reinterpret_cast<v4u *>(xw[p] + MV * XROW) = v4u{lo[0], lo[1], lo[2], lo[3]};
-                    } else {
-                        *reinterpret_cast<v2u *>(xw[p] + h0) = v2u{hi[0], hi[1]};
-                        *reinterpret_cast<v2u *>(xw[p] + h1) = v2u{hi[2], hi[3]};
-                        *reinterpret_cast<v2u *>(xw[p] + MV * XROW + h0) = v2u{lo[0], lo[1]};
-                        *reinterpret_cast<v2u *>(xw[p] + MV * XROW + h1) = v2u{lo[2], lo[3]};
-                    }
-                }
-                if constexpr (INFINITIES) {
-                    // (what an infinity leaves is a NaN: with it every result of the vector is NaN, without it the infinity's
-                    // product with a weight that is not zero stays one.  In LDS, where this costs the usual path no registers.)
-                    if (__builtin_expect(infinite != 0, 0)) {
+                    if constexpr (INFINITIES) {
+                        // (in LDS, where this costs the usual path no registers)
+                        if (__builtin_expect(infinite != 0, 0)) {
 #pragma unroll
-                        for (int p = 0; p < P; p++)
+                            for (int p = 0; p < P; p++)
 #pragma unroll
-                            for (int c = 0; c < 2; c++) {
-                                uint8_t *const at = xw[p] + (WF::ORDER <= OCTET_SWAPPED ? 8 * c : c ? h1 : h0);
-                                const v2u h = *reinterpret_cast<const v2u *>(at);
-                                v2u l = *reinterpret_cast<const v2u *>(at + MV * XROW);
+                                for (int c = 0; c < 2; c++) {
+                                    uint8_t *const at = xw[p] + (WF::ORDER <= OCTET_SWAPPED ? 8 * c : c ? h1 : h0);
+                                    const v2u h = *reinterpret_cast<const v2u *>(at);
+                                    v2u l = *reinterpret_cast<const v2u *>(at + MV * XROW);
 #pragma unroll
-                                for (int r = 0; r < 2; r++)
-                                    l[r] &= ((h[r] & 0x7FFFu) == 0x7C00u ? 0u : 0xFFFFu) | ((h[r] & 0x7FFF0000u) == 0x7C000000u ? 0u : 0xFFFF0000u);
-                                *reinterpret_cast<v2u *>(at + MV * XROW) = l;
-                            }
+                                    for (int r = 0; r < 2; r++) l[r] = without_infinities(h[r], l[r]);
+                                    *reinterpret_cast<v2u *>(at + MV * XROW) = l;
+                                }
+                        }
                     }
                 }
                 WF cur[TJ];
@@ -859,11 +946,21 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                     cur[t] = placed<FMT>(raw[d][t], from4);
                     cur[t].open(u, Fmt<FMT>::BE < 128 && 4 * u + q >= groups);
                 }
-                wave_order();
+                if constexpr (READY && F32_SCALE) {
+                    if (__builtin_expect(large, 0)) {
+#pragma unroll
+                        for (int t = 0; t < TJ; t++)
+#pragma unroll
+                            for (int j = 0; j < 4; j++) cur[t].sc4[j] *= 0x1p-28f;
+                    }
+                }
+                if constexpr (!READY) wave_order();
                 float sum[TJ][4];                                 // of this unit, in units of the vectors' inverse scales
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    const v4u xa = *reinterpret_cast<const v4u *>(xrd + j * 64);
+                    v4u xa;
+                    if constexpr (READY) xa = xq[d][j];
+                    else xa = *reinterpret_cast<const v4u *>(xrd + j * 64);
                     v4f xs[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
                     if constexpr (WF::MINS) contract<false>(xa, ones, xs);
 #pragma unroll
@@ -886,10 +983,14 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                         }
                     }
                 }
-                const v4f inv = *reinterpret_cast<const v4f *>(area_inv + (4 * q & (MV - 1)));
+                v4f inv;
+                if constexpr (READY) inv = iq[d];
+                else inv = *reinterpret_cast<const v4f *>(area_inv + (4 * q & (MV - 1)));
+                const double back = READY && F32_SCALE && large ? 0x1p28 : 1.0;
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const double iv = (double)inv[r];
+                    double iv = (double)inv[r];
+                    if constexpr (READY && F32_SCALE) iv *= back;
 #pragma unroll
                     for (int t = 0; t < TJ; t++) acc[t][r] = __builtin_fma((double)sum[t][r], iv, acc[t][r]);
                 }
@@ -899,6 +1000,7 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                 }
             }
             load_w(raw[d], u + D * waves);
+            if constexpr (READY) load_ready(d, u + D * waves);
         }
     }
     // red[wave][vector][16 * TJ rows]; lane rows 0 .. P - 1 hold the hi parts of vectors 0 .. MV - 1, the next P the lo parts
@@ -912,7 +1014,17 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
             if (q < P) red[(wave * MV + 4 * q + r) * (16 * TJ) + 16 * t + i] = (float)__builtin_fma(lo, 0x1p-11, acc[t][r]);
         }
     float *const squares = red + waves * MV * (16 * TJ);
-    if constexpr (NORM) {
+    if constexpr (NORM && READY) {
+        // (a vector's units over the lanes of a wavefront)
+        for (int v = wave; v < m; v += waves) {
+            const float *const sq = reinterpret_cast<const float *>(ready + ready_squares(m, units));
+            double sum = 0.0;
+            for (int u = lane; u < units; u += 64) sum += (double)sq[u * 8 + v];
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o);
+            if (lane == 0) reinterpret_cast<double *>(squares)[v] = sum;
+        }
+    } else if constexpr (NORM) {
 #pragma unroll
         for (int p = 0; p < P; p++) {
 #pragma unroll
@@ -933,7 +1045,8 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
         double rinv = 1.0;
         if constexpr (NORM) {                                     // (one step of Newton's iteration: an error here is the whole vector's)
             double sq = 0.0;
-            for (int wv = 0; wv < waves; wv++) sq += (double)squares[wv * MV + v];
+            if constexpr (READY) sq = reinterpret_cast<const double *>(squares)[v];
+            else for (int wv = 0; wv < waves; wv++) sq += (double)squares[wv * MV + v];
             if (!(sq <= 3.40282347e+38)) {                        // (rarely: as the norm alone has it, x / infinity)
                 float zero = 0.0f;                                // (NaN with an infinity or a NaN in x; no early end, so that loads run ahead)
 #pragma unroll 4

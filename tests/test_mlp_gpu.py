@@ -203,3 +203,35 @@ def test_mlp_rejects_bad_arguments(cuda):
     with pytest.raises(_lib.RfqError) as e:   # more rows than the decode kernels take
         ops.mlp_swiglu(Q.Q4_0, wg, wg, Q.Q4_0, wd, dev(gauss((9, hidden), 4), cuda), None, 1e-5, hidden, inter)
     assert e.value.status == _lib.E_UNSUPPORTED
+
+
+@pytest.mark.parametrize("fmt", [Q.Q4_0, Q.GGUF_Q4_0, Q.GGUF_Q4_K, Q.MXFP4, Q.MXFP6_E2M3])
+@pytest.mark.parametrize("m,hidden,inter,norm", [(2, 4128, 9792, True), (5, 4096, 9984, True), (7, 3424, 11712, False), (8, 4128, 9792, True)])
+def test_batches_over_large_matrices_on_prepared_x(fmt, m, hidden, inter, norm, cuda):
+    """x (and h) prepared by a launch of its own: rows of whole units and rows that end inside one, four and eight vectors, with and
+    without the norm; an outlier, and a vector of zeros.  Against the float64 block over the decoded weights."""
+    import torch
+    from rocmforge_amd import _lib, ops
+    if fmt == Q.GGUF_Q4_K:
+        hidden, inter = (hidden + 255) // 256 * 256, (inter + 255) // 256 * 256
+    rows = 997                                                            # made once and repeated: rows are independent
+    make = lambda n, k, seed: torch.from_numpy(Q.make_weights(fmt, rows, k, seed=seed)).to(cuda).view(rows, -1).repeat(n // rows + 1, 1)[:n].reshape(-1)
+    gate, up, down = make(inter, hidden, 1), make(inter, hidden, 2), make(hidden, inter, 3)
+    g = torch.Generator(device="cpu").manual_seed(m)
+    x, nw = torch.randn((m, hidden), generator=g), 1 + 0.1 * torch.randn(hidden, generator=g)
+    x[0, 7] = 3000.0
+    x[1] = 0.0
+    x, nw = x.to(cuda), nw.to(cuda)
+    got = ops.mlp_swiglu(fmt, gate, up, fmt, down, x, nw if norm else None, 1e-5, hidden, inter)
+    name = _lib.lib().rfq_bench_last_gemv_kernel().decode()
+    assert name.endswith(",ready>") == (m >= 5), name                      # (the down projection's)
+    dec = lambda w, n, k: ops.dequant(fmt, w, n * k).view(n, k).double()
+    xd = x.double()
+    if norm:
+        xd = xd / (xd.pow(2).mean(1, keepdim=True) + 1e-5).sqrt() * nw.double()
+    u = xd @ dec(up, inter, hidden).t().contiguous()
+    h = (xd @ dec(gate, inter, hidden).t().contiguous()) * (u * torch.sigmoid(u))
+    want = h @ dec(down, hidden, inter).t().contiguous()
+    # (float32 results of gate and up through the activation, then a float32 sum: 1e-6 of a vector's typical output or less)
+    err = (got.double() - want).norm(dim=1) / want.norm(dim=1).clamp_min(1e-30)
+    assert torch.isfinite(got).all() and float(err[torch.arange(m, device=cuda) != 1].max()) < 1e-5 and float(got[1].abs().max()) == 0.0, err
