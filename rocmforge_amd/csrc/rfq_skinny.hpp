@@ -668,15 +668,18 @@ __device__ __forceinline__ uint32_t max16(uint32_t v)
     return v;
 }
 
-// Octet e (8 consecutive elements of one vector; ex: the biased exponent of the vector's largest |x| in the unit) as the two
-// fp16 parts under a power of two that takes that largest to 2^top .. 2^(top + 1); inv: its inverse.
-template <int PAIRS, bool LOW>
-__device__ __forceinline__ void split_octet(const float (&e)[8], int ex, int top, uint32_t (&hi)[4], uint32_t (&lo)[4], float &inv)
+// The power of two that takes a vector's largest |x| in a unit (ex: its biased exponent) to 2^top .. 2^(top + 1), and its inverse.
+template <bool LOW> __device__ __forceinline__ void octet_scale(int ex, int top, float &s, float &inv)
 {
     int se = 254 + top - ex;                                      // s = 2^(top - (ex - 127))
     se = se > 243 ? 243 : LOW && se < 1 ? 1 : se;                 // (2048 s stays finite, s above zero)
-    const float s = __uint_as_float((uint32_t)se << 23);
+    s = __uint_as_float((uint32_t)se << 23);
     inv = __uint_as_float((uint32_t)(254 - se) << 23);
+}
+// Octet e (8 consecutive elements of one vector) under that power of two as the two fp16 parts.
+template <int PAIRS>
+__device__ __forceinline__ void split_octet(const float (&e)[8], float s, float inv, uint32_t (&hi)[4], uint32_t (&lo)[4])
+{
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         // (x * s, x - hi / s and its multiple by 2048 s are exact: a part is rounded once, to fp16)
@@ -728,8 +731,9 @@ prepare_x_kernel(const float *__restrict__ x, const float *__restrict__ norm_w, 
     const float mx = max3_abs(max3_abs(e[0], e[1], e[2]), max3_abs(e[3], e[4], e[5]), max3_abs(e[6], e[7], 0.0f));
     const int ex = (int)(max16(__float_as_uint(mx)) >> 23);
     uint32_t hi[4], lo[4];
-    float inv;
-    split_octet<PAIRS, false>(e, ex, 14, hi, lo, inv);
+    float s, inv;
+    octet_scale<false>(ex, 14, s, inv);
+    split_octet<PAIRS>(e, s, inv, hi, lo);
     if (keep_infinities && ex == 255) {
 #pragma unroll
         for (int r = 0; r < 4; r++) lo[r] = without_infinities(hi[r], lo[r]);
@@ -905,14 +909,18 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                     // (with such a scale x loses bits below 2^-11 of the largest)
                     const int top = large ? -14 : 14;
                     wave_order();                                 // (the unit before has been read)
+                    float s[P], inv_s[P];
                     unsigned long long infinite = 0;
 #pragma unroll
                     for (int p = 0; p < P; p++) {
                         if (INFINITIES && keep_infinities) infinite |= __builtin_amdgcn_ballot_w64(ex[p] == 255);
+                        octet_scale<F32_SCALE>(ex[p], top, s[p], inv_s[p]);
+                        if (i == 0) area_inv[4 * p + q] = inv_s[p];
+                    }
+#pragma unroll
+                    for (int p = 0; p < P; p++) {
                         uint32_t hi[4], lo[4];
-                        float inv_s;
-                        split_octet<WF::PAIRS, F32_SCALE>(e[p], ex[p], top, hi, lo, inv_s);
-                        if (i == 0) area_inv[4 * p + q] = inv_s;
+                        split_octet<WF::PAIRS>(e[p], s[p], inv_s[p], hi, lo);
                         if constexpr (WF::ORDER <= OCTET_SWAPPED) {
                             *reinterpret_cast<v4u *>(xw[p]) = v4u{hi[0], hi[1], hi[2], hi[3]};
                             *reinterpret_cast<v4u *>(xw[p] + MV * XROW) = v4u{lo[0], lo[1], lo[2], lo[3]};
