@@ -754,12 +754,10 @@ int parts_in(const uint8_t *static_tmp, int m, int n, int k, bool sums)
     return static_tmp != nullptr && kparts > 1 && head + (size_t)kparts * m * n * sizeof(float) > RFQ_STATIC_SCRATCH_BYTES ? 1 : kparts;
 }
 
-// The kernel on integer codes belongs to the same family: its rows per tile where the tiled kernel has its planes
-// (GGUF_Q4_K, whose operands are exact in one plane in both kernels, keeps that name).
+// The kernel on integer codes belongs to the same family: its rows per tile where the tiled kernel has its planes.
 void note_codes(int fmt, int m, int n, int kparts, bool arranged)
 {
-    if (fmt == RFQ_GGUF_Q4_K) note_kernel(arranged ? "gemm_kq_kernel<%s,%d,%d,arranged>" : "gemm_kq_kernel<%s,%d,%d>", fmt, 1, kparts, 0);
-    else note_kernel(arranged ? "gemm_kq_kernel<%s,codes of %d,%d,arranged>" : "gemm_kq_kernel<%s,codes of %d,%d>", fmt, codes_rows(m, n, kparts), kparts, 0);
+    note_kernel(arranged ? "gemm_kq_kernel<%s,codes of %d,%d,arranged>" : "gemm_kq_kernel<%s,codes of %d,%d>", fmt, codes_rows(m, n, kparts), kparts, 0);
 }
 
 // `arranged` != nullptr: the caller's buffer from launch_arrange_a (activations and sums); a is not read.

@@ -178,55 +178,60 @@ def test_one_plane_is_the_fp16_rounded_contraction(fmt, oracle, cuda):
     assert not np.array_equal(out, two)
 
 
-@pytest.mark.parametrize("m,kernel", [(70, "gemm_skinny_kernel"), (300, "gemm_kq_kernel<GGUF_Q4_K,1,2>")])
-def test_gguf_q4_k_super_block_scales_of_any_size(m, kernel, oracle, cuda):
-    """GGUF_Q4_K is contracted with integer operands and its accumulators run in units of the current super-block's d:
-    super-blocks whose d is +0, -0, negative, or 2^+-8 times the neighbour's (also in a row's first and last block,
-    and a whole row of zeros) must come out as the oracle's."""
+@pytest.mark.parametrize("m,n,k,arranged,kernel", [(70, 140, 2048, False, "gemm_skinny_kernel<GGUF_Q4_K,"), (70, 140, 2048, True, "gemm_skinny_kernel<GGUF_Q4_K,"),
+                                                   (300, 140, 2048, False, "gemm_kq_kernel<GGUF_Q4_K,codes of 64,2>"),
+                                                   (700, 3700, 2048, True, "gemm_kq_kernel<GGUF_Q4_K,codes of 128,1,arranged>"),
+                                                   (300, 14336, 2048, True, "gemm_kq_kernel<GGUF_Q4_K,codes of 192,1,arranged>"),
+                                                   (512, 14336, 2048, False, "gemm_kq_kernel<GGUF_Q4_K,1,1>"),
+                                                   (512, 14336, 2048, True, "gemm_kq_kernel<GGUF_Q4_K,1,1,arranged>"),
+                                                   (511, 4000, 4096, False, "gemm_kq_kernel<GGUF_Q4_K,1,4>")])
+def test_gguf_q4_k_super_block_scales_of_any_size(m, n, k, arranged, kernel, oracle, cuda):
+    """GGUF_Q4_K is contracted with integer operands and the tiled kernels' accumulators run in units of the current super-block's
+    d: super-blocks whose d is +0, -0, negative, or 2^+-8 times the neighbour's (also in a row's first and last block,
+    and a whole row of zeros) must come out as the oracle's.  Each of the kernels, the special rows in front of a matrix wide
+    enough for it: few rows, codes over row tiles that fit, whole tiles of 256 rows in one pass over k and in parts."""
     import torch
-    n, k = 140, 2048                                                      # 8 super-blocks per row
-    w = weights(Q.GGUF_Q4_K, n, k, 51).copy()
-    blocks = w.reshape(n, k // 256, 144)
-    d = blocks[:, :, 0:2].copy().view("<f2")[..., 0]                      # [n, 8]
+    from rocmforge_amd import ops
+    special, nb = 140, k // 256
+    w = weights(Q.GGUF_Q4_K, special, k, 51).copy()
+    blocks = w.reshape(special, nb, 144)
+    d = blocks[:, :, 0:2].copy().view("<f2")[..., 0]                      # [special, nb]
     rng = np.random.Generator(np.random.PCG64(52))
     d[0, :] = 0.0                                                         # a row without any scale (its mins remain)
     d[1, 0] = 0.0                                                         # zero first, later not
-    d[2, 7] = 0.0
+    d[2, nb - 1] = 0.0
     d[3, 3] = -0.0
     d[4, :] = -d[4, :]
     d[5, 1::2] *= np.float16(256.0)
     d[6, 1::2] /= np.float16(256.0)
-    pick = rng.integers(0, 8, size=n)
-    for r in range(7, n, 3): d[r, pick[r]] = 0.0
-    for r in range(8, n, 5): d[r, pick[r]] *= np.float16(-64.0)
+    pick = rng.integers(0, nb, size=special)
+    for r in range(7, special, 3): d[r, pick[r]] = 0.0
+    for r in range(8, special, 5): d[r, pick[r]] *= np.float16(-64.0)
     blocks[:, :, 0:2] = d.astype("<f2")[..., None].view(np.uint8)
     dmin = blocks[:, :, 2:4].copy().view("<f2")[..., 0]
     dmin[9::4, 2] = 0.0
     dmin[10::7, :] = -dmin[10::7, :]
     blocks[:, :, 2:4] = dmin.astype("<f2")[..., None].view(np.uint8)
     a = acts(m, k, 53)
-    out = run(Q.GGUF_Q4_K, w, a, n, k, cuda, torch.float32).cpu().numpy()
-    assert kernel_name().startswith(kernel) and np.isfinite(out).all()
-    want = oracle.qmatmul_nk(Q.GGUF_Q4_K, w, a.astype(np.float32), m, n, k)
-    exact = exact_weight_product(oracle, Q.GGUF_Q4_K, w, a, n, k)
-    for col in range(n):                                                  # (each weight row against its own output size)
+    wd = torch.from_numpy(w).to(cuda)
+    if n > special:
+        wide = torch.from_numpy(weights(Q.GGUF_Q4_K, n, k, 54)).to(cuda)
+        wide[: wd.numel()] = wd
+        wd = wide
+    da = torch.from_numpy(a).to(cuda)
+    if arranged:
+        out = ops.gemm_f16_arranged(Q.GGUF_Q4_K, wd, ops.ArrangedA(da), n, out_dtype=torch.float32)
+    else:
+        out = ops.gemm_f16(Q.GGUF_Q4_K, wd, da, n, k, out_dtype=torch.float32)
+    name = kernel_name()
+    assert name == kernel or (kernel.endswith(",") and name.startswith(kernel)), name
+    assert torch.isfinite(out).all()
+    out = out[:, :special].cpu().numpy()
+    want = oracle.qmatmul_nk(Q.GGUF_Q4_K, w, a.astype(np.float32), m, special, k)
+    exact = exact_weight_product(oracle, Q.GGUF_Q4_K, w, a, special, k)
+    for col in range(special):                                            # (each weight row against its own output size)
         assert_close(out[:, col], want[:, col], f"GGUF_Q4_K special super-block scales, weight row {col}")
         assert_close(out[:, col], exact[:, col], f"same (float64 sums), weight row {col}", tol=2e-5, plain_tol=2e-4)
-    A = torch.from_numpy(a).to(cuda)
-    from rocmforge_amd import ops
-    wd = torch.from_numpy(w).to(cuda)
-    # (300 rows are split along k in two parts by rfq_gemm_f16, and few rows taken as they are; one pass over k by the
-    # integer-operand kernel: arranged activations and a matrix wide enough for it, the same rows in front)
-    if m == 300:
-        wide = torch.from_numpy(weights(Q.GGUF_Q4_K, 14336, k, 54)).to(cuda)
-        wide[: wd.numel()] = wd
-        one_pass = ops.gemm_f16_arranged(Q.GGUF_Q4_K, wide, ops.ArrangedA(A), 14336, out_dtype=torch.float32)[:, :n].cpu().numpy()
-        assert kernel_name() == "gemm_kq_kernel<GGUF_Q4_K,1,1,arranged>"
-    else:
-        one_pass = ops.gemm_f16_arranged(Q.GGUF_Q4_K, wd, ops.ArrangedA(A), n, out_dtype=torch.float32).cpu().numpy()
-    for col in range(n):
-        assert_close(one_pass[:, col], want[:, col], f"one pass over k, weight row {col}")
-        assert_close(one_pass[:, col], exact[:, col], f"one pass over k (float64 sums), weight row {col}", tol=2e-5, plain_tol=2e-4)
 
 
 @pytest.mark.parametrize("fmt", FORMATS)
@@ -432,7 +437,9 @@ def test_integer_code_tiles(fmt, m, n, k, rows, parts, oracle, cuda):
     w, a = weights(fmt, n, k, 7), acts(m, k, 8)
     dw, da = torch.from_numpy(w).to(cuda), torch.from_numpy(a).to(cuda)
     out = ops.gemm_f16(fmt, dw, da, n, k, out_dtype=torch.float32)
-    assert kernel_name() == (f"gemm_kq_kernel<GGUF_Q4_K,1,{parts}>" if fmt == Q.GGUF_Q4_K else f"gemm_kq_kernel<{Q.NAMES[fmt]},codes of {rows},{parts}>")
+    # (GGUF_Q4_K over whole tiles of 256 rows keeps the kernel laid out by hand)
+    form = "1" if fmt == Q.GGUF_Q4_K and rows == 256 else f"codes of {rows}"
+    assert kernel_name() == f"gemm_kq_kernel<{Q.NAMES[fmt]},{form},{parts}>"
     pick = np.unique(np.concatenate([np.arange(0, n, max(1, n // 97)), np.arange(max(0, n - 130), n)]))
     want = a.astype(np.float64) @ (gguf_q4_k_fused(w, n, k) if fmt == Q.GGUF_Q4_K else oracle.dequantize(fmt, w, n * k).reshape(n, k))[pick].astype(np.float64).T
     assert_close(out.cpu().numpy()[:, pick], want, f"{Q.NAMES[fmt]} {m}x{n}x{k}", tol=2e-5, plain_tol=2e-4)
