@@ -772,6 +772,9 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
     // before (GGUF_Q4_0 5 x 14336 -> 4096 22.2 -> 19.8 us); with more, the registers it needs would leave room for one
     // workgroup per CU instead of two, or spill (GGUF_Q6_K 5 x 4096 -> 14336 28 -> 76 us).
     constexpr bool AHEAD = TJ == 1 && !READY;
+    // (e and xr then both go round the loop.  Left free, the compiler gives these forms' e the registers of xr, fetches into others and
+    // waits at once to move them: GGUF_Q4_0 4 x 4096 -> 4096 and MXFP4 lost 3 to 5 %)
+    constexpr bool MOVED = AHEAD && !NORM && MV == 4 && (FMT == RFQ_Q4_0 || FMT == RFQ_GGUF_Q4_0 || FMT == RFQ_MXFP4 || FMT == RFQ_MXFP6_E2M3);
     constexpr bool F32_SCALE = FMT == RFQ_Q4_0 || FMT == RFQ_Q8_0;
     constexpr bool INFINITIES = FMT == RFQ_Q4_K || FMT == RFQ_Q6_K || FMT == RFQ_MXFP4 || FMT == RFQ_MXFP6_E2M3;   // (see keeps_infinities)
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -841,7 +844,10 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
 #pragma unroll
         for (int p = 0; p < P; p++) {
 #pragma unroll
-            for (int c = 0; c < 4; c++) { e[p][c] = xr[p][0][c]; e[p][4 + c] = xr[p][1][c]; }
+            for (int c = 0; c < 8; c++) {
+                if constexpr (MOVED) asm("v_mov_b32 %0, %1" : "=&v"(e[p][c]) : "v"(xr[p][c >> 2][c & 3]));
+                else e[p][c] = xr[p][c >> 2][c & 3];
+            }
             if (Fmt<FMT>::BE < 128 && past) {
 #pragma unroll
                 for (int c = 0; c < 8; c++) e[p][c] = 0.0f;
@@ -907,7 +913,9 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
                 }
                 if constexpr (!READY) {
                     // (with such a scale x loses bits below 2^-11 of the largest)
-                    const int top = large ? -14 : 14;
+                    int top = 14;
+                    if constexpr (F32_SCALE)
+                        if (large) top = -14;
                     wave_order();                                 // (the unit before has been read)
                     float s[P], inv_s[P];
                     unsigned long long infinite = 0;
