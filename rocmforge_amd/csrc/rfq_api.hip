@@ -367,17 +367,29 @@ size_t rfq_mlp_scratch_bytes(int m, int hidden_size, int intermediate_size)
     return 3 * pad16((size_t)m * intermediate_size * 4) + pad16((size_t)m * hidden_size * 4);
 }
 
-// Whether x is prepared by a launch of its own (5 us, an eighth of them work) before a batch's projection, so that no workgroup
-// converts it: large matrices of the formats whose kernels are bound by vector instructions.  One step each, m = 6: GGUF_Q4_K gate
-// and up 5120 -> 13824 73.2 -> 65.2 us of the block, down 73.2 -> 66.6; MXFP4 79.3 -> 77.9 and -> 70.6; at 2560 -> 7168 (37 and 18
-// million weights) level or slower.  Up to four vectors only gate and up of the MXFP formats gain: 69.5 -> 62.2, 4 x 5120 -> 13824
-// MXFP4.  Q8_0, Q4_K and the Q6_K layouts were level or lost 1 to 5 % at any size.
-static bool prepare_pays(int fmt, int m, bool pair, size_t weights)
+// Whether x [m, k] is prepared by a launch of its own (5 us, an eighth of them work) before a batch's projection of n rows (`pair`:
+// gate and up, n each), so that no workgroup converts it.  Formats whose kernels are bound by vector instructions; Q8_0, Q4_K and the
+// Q6_K layouts were level or lost 1 to 5 % at any size.  Times of the block with one step prepared over none:
+//   * Gate and up: a workgroup that converts x takes 32 rows of each, one on prepared x takes 16.  What decides is whether the former
+//     leave CUs idle in their last round.  More than one per CU (n > 32 per CU; hidden 1536..5120 x 8448..12288, 5 and 8 vectors): Q4_0
+//     0.78..0.89, GGUF_Q4_0 0.79..0.87, GGUF_Q4_K 0.76..0.88, MXFP4 0.83..0.96, MXFP6 0.81..0.93; with hidden 1024 up to 1.03.
+//     Two whole rounds: MXFP formats of 5 and more vectors 1.01..1.04 at 2560 x 16384 (84 million weights), 0.96..0.99 at 6144 x 16384.
+//     One round (5120 x 7936, 6144 x 8192, 8192 x 8192): GGUF_Q4_K 0.95..0.98, MXFP6 0.95..1.006, Q4_0 0.98..1.02, GGUF_Q4_0
+//     0.99..1.013, MXFP4 0.98..1.03; up to four vectors MXFP4 0.93..0.98, MXFP6 0.92..0.96 (two vectors level), and 1.0 at 50 million weights.
+//   * Down: on prepared x one row tile to a workgroup.  As many without (n <= 20 per CU): 4096 x 9984, 5120 x 13824 0.96..0.99 with 5
+//     vectors, 0.97..1.013 with 8 (MXFP formats 0.92..0.97); below 40 million weights 0.95..1.02.  Two row tiles without: Q4_0 and
+//     GGUF_Q4_0 1.03..1.10, GGUF_Q4_K 1.0..1.045, MXFP4 0.985..1.03, MXFP6 0.93..0.97.
+//   * Up to four vectors nothing else gains: Q4_0 and the GGUF layouts 0.99..1.11.
+static bool prepare_pays(int fmt, int m, bool pair, int n, int k)
 {
-    const int cf = canonical_format(fmt);
+    const int cf = canonical_format(fmt), cus = device_cu_count();
     const bool mx = cf == RFQ_MXFP4 || cf == RFQ_MXFP6_E2M3;
     if (!prepared_format(cf) || m < 2 || (m < 5 && !(mx && pair))) return false;
-    return weights >= (pair ? (size_t)80000000 : (size_t)40000000);
+    const size_t weights = (pair ? 2 : 1) * (size_t)n * k;
+    if (!pair) return weights >= 40000000 && (n <= 20 * cus || cf == RFQ_MXFP6_E2M3);
+    const int round = 32 * cus, last = n % round;                 // rows of a round of workgroups, and of the last one (0: whole)
+    if (n > round) return k >= 1536 && !(mx && m >= 5 && (last == 0 || 10 * last > 9 * round) && weights < 160000000);
+    return weights >= 80000000 && (cf == RFQ_GGUF_Q4_K || cf == RFQ_MXFP6_E2M3 || (cf == RFQ_MXFP4 && m < 5));
 }
 
 int rfq_mlp_swiglu(int fmt_gate_up, const void *d_gate_w, const void *d_up_w, size_t gate_up_bytes, int fmt_down,
@@ -415,7 +427,7 @@ int rfq_mlp_swiglu(int fmt_gate_up, const void *d_gate_w, const void *d_up_w, si
             return fail(RFQ_E_BADARG, "rfq_mlp_swiglu: x and norm weight must be 16-byte aligned, hidden_size a multiple of 4");
         rc = launch_skinny_gemv_fused(fmt_gate_up, (const uint8_t *)d_gate_w, (const uint8_t *)d_up_w, d_x, d_norm_weight, eps, h, m,
                                       intermediate_size, hidden_size, s,
-                                      ready_bytes(m, hidden_size) <= need - mi && prepare_pays(fmt_gate_up, m, true, 2 * (size_t)intermediate_size * hidden_size)
+                                      ready_bytes(m, hidden_size) <= need - mi && prepare_pays(fmt_gate_up, m, true, intermediate_size, hidden_size)
                                           ? base + mi : nullptr);
     }
     if (rc == RFQ_E_UNSUPPORTED) {
@@ -432,7 +444,7 @@ int rfq_mlp_swiglu(int fmt_gate_up, const void *d_gate_w, const void *d_up_w, si
         rc = launch_swiglu(gate, up, h, (size_t)m * intermediate_size, s);
     }
     if (rc != RFQ_OK) return rc;
-    if (ready_bytes(m, intermediate_size) <= need - mi && prepare_pays(fmt_down, m, false, (size_t)hidden_size * intermediate_size)) {
+    if (ready_bytes(m, intermediate_size) <= need - mi && prepare_pays(fmt_down, m, false, hidden_size, intermediate_size)) {
         rc = launch_gemv_prepared(fmt_down, (const uint8_t *)d_down_w, h, d_out, m, hidden_size, intermediate_size, base + mi, s);
         if (rc != RFQ_E_UNSUPPORTED) return rc;
     }

@@ -206,7 +206,7 @@ def test_mlp_rejects_bad_arguments(cuda):
 
 
 @pytest.mark.parametrize("fmt", [Q.Q4_0, Q.GGUF_Q4_0, Q.GGUF_Q4_K, Q.MXFP4, Q.MXFP6_E2M3])
-@pytest.mark.parametrize("m,hidden,inter,norm", [(2, 4128, 9792, True), (5, 4096, 9984, True), (7, 3424, 11712, False), (8, 4128, 9792, True)])
+@pytest.mark.parametrize("m,hidden,inter,norm", [(2, 4128, 9792, True), (5, 4096, 9984, True), (7, 3424, 11712, False), (8, 4128, 9792, True), (8, 6144, 8192, True)])
 def test_batches_over_large_matrices_on_prepared_x(fmt, m, hidden, inter, norm, cuda):
     """x (and h) prepared by a launch of its own: rows of whole units and rows that end inside one, four and eight vectors, with and
     without the norm; an outlier, and a vector of zeros.  Against the float64 block over the decoded weights."""
@@ -224,7 +224,8 @@ def test_batches_over_large_matrices_on_prepared_x(fmt, m, hidden, inter, norm, 
     x, nw = x.to(cuda), nw.to(cuda)
     got = ops.mlp_swiglu(fmt, gate, up, fmt, down, x, nw if norm else None, 1e-5, hidden, inter)
     name = _lib.lib().rfq_bench_last_gemv_kernel().decode()
-    assert name.endswith(",ready>") == (m >= 5), name                      # (the down projection's)
+    # (the down projection's; where two row tiles go to a workgroup that converts x, only MXFP6 is ahead on prepared x)
+    assert name.endswith(",ready>") == (m >= 5 and (hidden <= 5120 or fmt == Q.MXFP6_E2M3)), name
     dec = lambda w, n, k: ops.dequant(fmt, w, n * k).view(n, k).double()
     xd = x.double()
     if norm:
