@@ -81,7 +81,21 @@ template <int FMT> int gemv_fmt(const SkinnyGemv &c, hipStream_t s)
     return c.m <= 4 ? gemv_rows<FMT, 4, false>(c, s) : gemv_rows<FMT, 8, false>(c, s);
 }
 
-template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES, bool FULL, bool PAIR = in_pairs(FMT, MT, ARR, FULL)>
+// How a workgroup fetches and orders its activations (see gemm_skinny_kernel).
+struct Form { bool full, pair, deep, turn; };
+// Pairs of groups, two ahead where one row tile leaves registers for it.
+[[maybe_unused]] constexpr Form usual(int fmt, int mt, int tj, bool arr) { return {false, in_pairs(fmt, mt, arr, false), mt <= 2 && tj == 1, false}; }
+[[maybe_unused]] constexpr Form deep(Form f) { f.deep = true; return f; }
+[[maybe_unused]] constexpr Form single(Form f) { f.pair = f.deep = false; return f; }
+[[maybe_unused]] constexpr Form turned(Form f) { f.turn = true; return f; }
+// (one form took 152 registers instead of 118 with the codes turned: GGUF_Q4_0 200 x 1280 -> 5120 15.4 -> 17.5 us)
+[[maybe_unused]] constexpr Form full(int fmt, int mt, bool arr)
+{
+    const bool pair = in_pairs(fmt, mt, arr, true);
+    return {true, pair, false, !arr && !pair && fmt == RFQ_GGUF_Q4_0};
+}
+
+template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES, bool FULL, bool PAIR, bool DEEP, bool TURN>
 int gemm_launch(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int n, int k, int rows, int slices, hipStream_t s)
 {
     constexpr bool STAGED = A16<W<FMT>::ORDER, W<FMT>::PAIRS, ARR>::STAGED;
@@ -93,14 +107,14 @@ int gemm_launch(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m,
         static std::once_flag once;
         static hipError_t err = hipSuccess;
         std::call_once(once, [] {
-            err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES, FULL, PAIR>),
+            err = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES, FULL, PAIR, DEEP, TURN>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, MOST_LDS);
         });
         if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(gemm_skinny_kernel)");
     }
     note_kernel(ARR ? "gemm_skinny_kernel<%s,%d,%d,%d,arranged>" : "gemm_skinny_kernel<%s,%d,%d,%d>", FMT, MT, TJ, slices);
-    hipLaunchKernelGGL((gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES, FULL, PAIR>), dim3((n + 16 * TJ - 1) / (16 * TJ), slices), dim3(64 * waves), lds, s,
-                       w, a, y, f16_out, m, n, k, rows);
+    hipLaunchKernelGGL((gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES, FULL, PAIR, DEEP, TURN>), dim3((n + 16 * TJ - 1) / (16 * TJ), slices),
+                       dim3(64 * waves), lds, s, w, a, y, f16_out, m, n, k, rows);
     RFQ_LAUNCH_CHECK("gemm_skinny_kernel");
     return RFQ_OK;
 }
@@ -108,19 +122,55 @@ int gemm_launch(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m,
 // Two row tiles of W beside two to four operands of rows take 121 .. 172 registers, one workgroup per CU, and with a few spilled 128:
 // two per CU, which pays as soon as there are more workgroups than CUs (48 x 4096 -> 14336: GGUF_Q4_K 25.1 / 21.4 us, Q8_0 23.6 /
 // 22.3, GGUF_Q6_K 28.2 / 25.1; 282 workgroups, 37 x 2048 -> 9000: GGUF_Q4_K 14.4 / 12.0; with 160 workgroups, 64 x 1280 -> 5120: Q8_0 6.8 / 7.4, GGUF_Q4_0 6.7 / 8.0).
+// Not GGUF_Q8_0 with four operands, which spills most (60 x 1024 -> 14336 16.0 against 13.9 without, 60 x 4096 -> 8320 34.6 / 30.8).
 template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES>
 int gemm_cfg(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int n, int k, int rows, int slices, hipStream_t s)
 {
+    constexpr Form USUAL = usual(FMT, MT, TJ, ARR);
+#define RFQ_GEMM_FORM(F)                                                                                     \
+    do {                                                                                                     \
+        constexpr Form form = F;                                                                             \
+        return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, form.full, form.pair, form.deep, form.turn>(w, a, y, f16_out, m, n, k, rows, slices, s); \
+    } while (0)
     const bool more = (long)((n + 16 * TJ - 1) / (16 * TJ)) * slices > device_cu_count();
-    if constexpr (TJ == 2 && MT >= 2 && MT <= 4 && !ARR)
-        if (more) return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, true>(w, a, y, f16_out, m, n, k, rows, slices, s);
-    // (single groups stay ahead in two places: long rows of the 4-bit GGUF layouts, 20 x 14336 -> 4096 GGUF_Q4_K 20.6 / 21.7 us, and six
-    // operands of the Q6_K layouts in several rounds, 160 x 3072 -> 6144 GGUF_Q6_K 33.0 / 34.3)
-    if constexpr (TJ == 1 && MT == 2 && !ARR && (FMT == RFQ_GGUF_Q4_0 || FMT == RFQ_GGUF_Q4_K))
-        if (k > 8192) return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, false, false>(w, a, y, f16_out, m, n, k, rows, slices, s);
-    if constexpr (TJ == 2 && (MT == 5 || MT == 6) && !ARR && (FMT == RFQ_Q6_K || FMT == RFQ_GGUF_Q6_K))
-        if (more) return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, false, false>(w, a, y, f16_out, m, n, k, rows, slices, s);
-    return gemm_launch<FMT, MT, TJ, ARR, D, WAVES, false>(w, a, y, f16_out, m, n, k, rows, slices, s);
+    if constexpr (ARR) {
+        // Arranged: codes turned once for all operands, but activations where that cost registers or came too late behind the load of W
+        // (17 x 1024 -> 14336 Q8_0 11.6 -> 10.5 us; 17 x 11264 -> 1536 15.7 -> 14.4; with short rows the codes, 9 x 1024 -> 768 3.58 / 3.42).
+        if constexpr (FMT == RFQ_Q8_0 && TJ == 2 && MT == 2) RFQ_GEMM_FORM(turned(USUAL));
+        if constexpr ((FMT == RFQ_Q8_0 || FMT == RFQ_GGUF_Q8_0) && TJ == 1 && MT == 1)
+            if (k > 2048) RFQ_GEMM_FORM(turned(USUAL));
+        if constexpr (FMT == RFQ_Q8_0 && TJ == 1 && MT == 2)
+            if (k > 4096) RFQ_GEMM_FORM(turned(USUAL));
+        // (two registers over the 128 for two workgroups per CU: 17 x 1024 -> 14336 8.7 -> 7.2 us; with 192 workgroups 7.35 / 7.7)
+        if constexpr (FMT == RFQ_GGUF_Q4_K && TJ == 2 && MT == 2)
+            if (more) RFQ_GEMM_FORM(full(FMT, MT, ARR));
+        RFQ_GEMM_FORM(USUAL);
+    } else {
+        // (one unit of k to a wavefront: single groups, whose second fetch does not wait for a whole pair; 60 x 1024 -> 14336 Q8_0 13.6 /
+        // 12.8 us, 90 rows GGUF_Q8_0 17.9 / 17.2, 33 x 1024 -> 4096 4.8 / 4.6, 75 x 2048 -> 1792 6.45 / 6.1, 75 x 3072 -> 1536 7.9 / 7.45)
+        if constexpr (TJ == 2 && ((FMT == RFQ_Q8_0 && MT == 4) || (FMT == RFQ_GGUF_Q8_0 && MT == 6)))
+            if (more && k <= 1024) RFQ_GEMM_FORM(single(USUAL));
+        if constexpr (FMT == RFQ_GGUF_Q8_0 && TJ == 1 && MT == 3) {
+            if (k < 4096) RFQ_GEMM_FORM(single(USUAL));
+            // (its ten registers a unit leave one unit of W in flight: activations further ahead, 33 x 4096 -> 4096 11.9 -> 10.6 us)
+            RFQ_GEMM_FORM(deep(USUAL));
+        }
+        if constexpr (TJ == 2 && MT >= 2 && MT <= 4 && !(FMT == RFQ_GGUF_Q8_0 && MT == 4))
+            if (more) RFQ_GEMM_FORM(full(FMT, MT, ARR));
+        // One workgroup per CU has registers for two pairs ahead: long rows of the 4- and 6-bit layouts with nothing else to wait behind
+        // (9 x 8192 -> 5120 Q4_K 20.5 -> 18.4 us, Q6_K 20.2 -> 18.9, GGUF_Q4_K 15.7 -> 14.4, Q4_0 16.5 -> 15.6; Q4_K short ones too, 6.8 -> 6.2
+        // with k = 1280, where Q4_0 and GGUF_Q4_K lose 2 %; the 8-bit layouts lose 1 to 7 %).
+        if constexpr (TJ == 2 && MT <= 2 && (FMT == RFQ_Q4_K || FMT == RFQ_Q6_K || FMT == RFQ_Q4_0 || FMT == RFQ_GGUF_Q4_K))
+            if (!more && (FMT == RFQ_Q4_K || k >= 4096)) RFQ_GEMM_FORM(deep(USUAL));
+        // (single groups stay ahead in two places: long rows of the 4-bit GGUF layouts, 20 x 14336 -> 4096 GGUF_Q4_K 20.6 / 21.7 us, and six
+        // operands of the Q6_K layouts in several rounds, 160 x 3072 -> 6144 GGUF_Q6_K 33.0 / 34.3)
+        if constexpr (TJ == 1 && MT == 2 && (FMT == RFQ_GGUF_Q4_0 || FMT == RFQ_GGUF_Q4_K))
+            if (k > 8192) RFQ_GEMM_FORM(single(USUAL));
+        if constexpr (TJ == 2 && (MT == 5 || MT == 6) && (FMT == RFQ_Q6_K || FMT == RFQ_GGUF_Q6_K))
+            if (more) RFQ_GEMM_FORM(single(USUAL));
+        RFQ_GEMM_FORM(USUAL);
+    }
+#undef RFQ_GEMM_FORM
 }
 
 // 16-row operands per workgroup at most: six with one row tile (eight leave its registers one wavefront per SIMD: Q8_0
@@ -167,10 +217,10 @@ int gemm_mt(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m, int
     case 4: return gemm_cfg<FMT, 4, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
     default:
         // (five beside two row tiles: 160 x 4096 -> 4096 Q8_0 18.9 us as six, 17.7 as five, Q/K/V of 160 tokens GGUF_Q4_K 36.1 / 35.3; but
-        // GGUF_Q6_K in several rounds 17.9 / 18.6, 130 x 1280 -> 5120)
+        // GGUF_Q6_K in several rounds 17.9 / 18.6, 130 x 1280 -> 5120, and arranged 10.7 / 11.05, 75 x 1280 -> 5120, 41.0 / 42.0 with k = 8192)
         if constexpr (MOST >= 6 && TJ == 2) {
             const bool rounds = (long)((n + 31) / 32) * slices > device_cu_count();
-            if (sl.tiles == 5 && !(FMT == RFQ_GGUF_Q6_K && rounds)) return gemm_cfg<FMT, 5, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
+            if (sl.tiles == 5 && !(FMT == RFQ_GGUF_Q6_K && (ARR || rounds))) return gemm_cfg<FMT, 5, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);
         }
         if constexpr (MOST >= 6)
             if (sl.tiles <= 6) return gemm_cfg<FMT, 6, TJ, ARR, D, 8>(w, a, y, f16_out, m, n, k, rows, slices, s);

@@ -1092,19 +1092,19 @@ gemv_skinny_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, f
 // operands.  Arranged activations (ARR, the order arrange_a_kernel writes: unit (32 rows, 64 k) of 4 KiB, octet c of half h
 // of row fr at ((c * 64) + 32 h + fr) * 16 bytes, its dwords the element pairs (0,4)(1,5)(2,6)(3,7)) are loaded as operands
 // where a lane takes whole octets, through LDS where it takes halves of two.
-// TURN: rows are brought into the order of the codes (P02) after all.
+// TURN: activations are brought into the order of the codes after all.
 template <int ORDER, int PAIRS, bool ARR, bool TURN = false> struct A16 {
-    static_assert(!TURN || (!ARR && PAIRS == P02), "rows to P02");
     static constexpr bool OCT = ORDER <= OCTET_SWAPPED;
     static constexpr bool STAGED = !ARR || !OCT;
+    static_assert(!TURN || (ARR ? OCT && PAIRS == P01 : PAIRS == P02), "orders that a turn is written for");
     v4u v;
     __device__ __forceinline__ void load(const uint8_t *p, uint32_t at) { v = *reinterpret_cast<const v4u *>(p + at); }
     // the order in which the operand holds an octet: as it comes, but in order where halves of it go to different lanes
-    static constexpr int AS = TURN ? (int)P02 : ARR && OCT ? (int)P04 : (int)P01;
+    static constexpr int AS = TURN ? PAIRS : ARR && OCT ? (int)P04 : (int)P01;
     __device__ __forceinline__ v4u ordered() const
     {
         constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;
-        if constexpr (ARR && !OCT)
+        if constexpr (ARR && (TURN || !OCT))
             return v4u{__builtin_amdgcn_perm(v[1], v[0], LO), __builtin_amdgcn_perm(v[3], v[2], LO),
                        __builtin_amdgcn_perm(v[1], v[0], HI), __builtin_amdgcn_perm(v[3], v[2], HI)};
         else if constexpr (TURN)
@@ -1138,16 +1138,16 @@ template <int MT, int TJ, bool STAGED, bool PAIR> constexpr int gemm_lds(int wav
 
 // blockDim = 64 * waves; LDS: gemm_lds.  a: rows [m, k] or the arranged buffer; blockIdx.y: slices of rows_per_slice (a
 // multiple of 16, at most 16 * MT) rows each.
-// FULL: for more workgroups than CUs, two of them to a CU (128 registers).  PAIR: rows are fetched as pairs of groups.
-template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES, bool FULL, bool PAIR>
-__global__ void __launch_bounds__(64 * WAVES, FULL && PAIR ? 4 : 1)
+// FULL: for more workgroups than CUs, two of them to a CU (128 registers).  PAIR: rows are fetched as pairs of groups; DEEP: two
+// pairs ahead.  TURN: see A16.
+template <int FMT, int MT, int TJ, bool ARR, int D, int WAVES, bool FULL, bool PAIR, bool DEEP, bool TURN>
+__global__ void __launch_bounds__(64 * WAVES, FULL && (PAIR || ARR) ? 4 : 1)
 gemm_skinny_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ a, void *__restrict__ y, int f16_out, int m, int n, int k,
                    int rows_per_slice)
 {
     typedef W<FMT> WF;
-    // (one form took 152 registers instead of 118 with the codes turned: GGUF_Q4_0 200 x 1280 -> 5120 15.4 -> 17.5 us)
-    typedef A16<WF::ORDER, WF::PAIRS, ARR, FULL && !PAIR && FMT == RFQ_GGUF_Q4_0> AF;
-    constexpr int PAIRS_AHEAD = MT <= 2 && TJ == 1 ? 2 : 1;
+    typedef A16<WF::ORDER, WF::PAIRS, ARR, TURN> AF;
+    constexpr int PAIRS_AHEAD = DEEP ? 2 : 1;
     constexpr int AD = PAIR ? 2 * PAIRS_AHEAD : MT <= 2 ? 4 : MT * TJ < 12 ? 2 : 1;  // groups of activations in flight (registers)
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, q = lane >> 4;
