@@ -55,7 +55,8 @@ RFQ_API int rfq_bench_get_rows(int fmt, const void *d_table, size_t table_bytes,
  * rfq_mlp_swiglu (its down projection) / rfq_gemm_f16* launch took ("" before the first), e.g.
  * "gemv_idot_kernel<Q4_K,1,2,7>": lets the driver name the kernel it timed, and a test the one it checks, from the
  * dispatch actually taken instead of a constant.  gemv_skinny_kernel: row tiles of W, vectors, norm; gemm_skinny_kernel:
- * 16-row operands of A, row tiles of W, slices of A; gemm_kq_kernel: operands per weight
+ * 16-row operands of A, row tiles of W, slices of A, and how A is fetched ("arranged", in "pairs" of groups, two of them
+ * ahead: "deep", two workgroups to a CU: "full", put in the order of the codes: "turned"); gemm_kq_kernel: operands per weight
  * or, on integer codes, "codes of" the rows of a tile, then the parts along k. */
 RFQ_API const char *rfq_bench_last_gemv_kernel(void);
 

@@ -112,7 +112,10 @@ int gemm_launch(const uint8_t *w, const uint8_t *a, void *y, int f16_out, int m,
         });
         if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(gemm_skinny_kernel)");
     }
-    note_kernel(ARR ? "gemm_skinny_kernel<%s,%d,%d,%d,arranged>" : "gemm_skinny_kernel<%s,%d,%d,%d>", FMT, MT, TJ, slices);
+    constexpr const char *name = ARR ? FULL ? "gemm_skinny_kernel<%s,%d,%d,%d,arranged,full>" : TURN ? "gemm_skinny_kernel<%s,%d,%d,%d,arranged,turned>" : "gemm_skinny_kernel<%s,%d,%d,%d,arranged>"
+        : FULL ? PAIR ? "gemm_skinny_kernel<%s,%d,%d,%d,pairs,full>" : TURN ? "gemm_skinny_kernel<%s,%d,%d,%d,full,turned>" : "gemm_skinny_kernel<%s,%d,%d,%d,full>"
+        : PAIR ? DEEP ? "gemm_skinny_kernel<%s,%d,%d,%d,pairs,deep>" : "gemm_skinny_kernel<%s,%d,%d,%d,pairs>" : "gemm_skinny_kernel<%s,%d,%d,%d>";
+    note_kernel(name, FMT, MT, TJ, slices);
     hipLaunchKernelGGL((gemm_skinny_kernel<FMT, MT, TJ, ARR, D, WAVES, FULL, PAIR, DEEP, TURN>), dim3((n + 16 * TJ - 1) / (16 * TJ), slices),
                        dim3(64 * waves), lds, s, w, a, y, f16_out, m, n, k, rows);
     RFQ_LAUNCH_CHECK("gemm_skinny_kernel");

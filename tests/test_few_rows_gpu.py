@@ -398,30 +398,61 @@ def test_every_prompt_kernel(fmt, oracle, cuda):
         name = kernel_name()
         assert name.startswith(f"gemm_skinny_kernel<{Q.NAMES[fmt]},{form[0]},{form[1]},") and "arranged" not in name, (name, form, m, n)
         arranged = ops.gemm_f16_arranged(fmt, part, ops.ArrangedA(da), n, out_dtype=torch.float32)
-        assert kernel_name() == name[:-1] + ",arranged>"
+        base = ",".join(name[:-1].split(",")[:4]) + ",arranged"
+        assert kernel_name() in [base + how for how in (">", ",turned>", ",full>")]
         assert torch.equal(plain, arranged)
         assert_close(plain.cpu().numpy(), want, f"{Q.NAMES[fmt]} {m}x{n}x{k} {form}", tol=TOL, plain_tol=2e-4)
 
 
+# m, n, k; the forms that rows of these sizes take on a part of 256 CUs (16-row operands, row tiles of W, slices, then how they are
+# fetched) with their formats, "" all others; arranged activations where not the same tiles, "arranged".
+FETCHES = [
+    (17, 40, 8224, {"1,1,2,pairs,deep": ""}, {"1,1,2,arranged,turned": "Q8_0 GGUF_Q8_0"}),
+    (9, 300, 2048, {"1,1,1,pairs,deep": ""}, {}),
+    (29, 3000, 8448, {"2,1,1": "GGUF_Q4_0 GGUF_Q4_K", "2,1,1,pairs,deep": ""}, {"2,1,1,arranged,turned": "Q8_0"}),
+    (17, 3000, 4096, {"2,1,1,pairs,deep": ""}, {}),
+    (33, 4090, 1056, {"3,1,1": "GGUF_Q8_0", "3,1,1,pairs": ""}, {}),
+    (33, 4090, 4096, {"3,1,1,pairs,deep": "GGUF_Q8_0", "3,1,1,pairs": ""}, {}),
+    (9, 5000, 256, {"1,2,1,pairs,deep": "Q4_K", "1,2,1,pairs": ""}, {}),
+    (9, 5000, 4096, {"1,2,1,pairs,deep": "Q4_0 Q4_K Q6_K GGUF_Q4_K", "1,2,1,pairs": ""}, {}),
+    (17, 5000, 4128, {"2,2,1,pairs,deep": "Q4_0 Q4_K Q6_K GGUF_Q4_K", "2,2,1,pairs": ""}, {"2,2,1,arranged,turned": "Q8_0"}),
+    (20, 8193, 8192, {"2,2,1,pairs,full": ""}, {"2,2,1,arranged,turned": "Q8_0", "2,2,1,arranged,full": "GGUF_Q4_K"}),
+    (33, 8225, 416, {"3,2,1,full": "Q4_K", "3,2,1,pairs,full": ""}, {}),
+    (56, 8250, 352, {"4,2,1,full": "Q4_0 Q6_K", "4,2,1,full,turned": "GGUF_Q4_0", "4,2,1": "Q8_0", "4,2,1,pairs": "GGUF_Q8_0", "4,2,1,pairs,full": ""}, {}),
+    (60, 8208, 1280, {"4,2,1,full": "Q4_0 Q6_K", "4,2,1,full,turned": "GGUF_Q4_0", "4,2,1,pairs": "GGUF_Q8_0", "4,2,1,pairs,full": ""}, {}),
+    (75, 8000, 224, {"3,2,2,pairs,full": "Q4_0 GGUF_Q4_0", "5,2,1,pairs": ""}, {"6,2,1,arranged": "GGUF_Q6_K"}),
+    (80, 8300, 256, {"3,2,2,pairs,full": "Q4_0 GGUF_Q4_0", "5,2,1": "Q6_K", "6,2,1": "GGUF_Q6_K", "5,2,1,pairs": ""}, {}),
+    (85, 8250, 192, {"3,2,2,pairs,full": "Q4_0 GGUF_Q4_0", "6,2,1": "Q6_K GGUF_Q6_K GGUF_Q8_0", "6,2,1,pairs": ""}, {}),
+    (90, 8208, 1280, {"3,2,2,pairs,full": "Q4_0 GGUF_Q4_0", "6,2,1": "Q6_K GGUF_Q6_K", "6,2,1,pairs": ""}, {}),
+    (96, 16400, 256, {"3,2,2,pairs,full": "Q4_0 GGUF_Q4_0", "6,2,1": "Q6_K GGUF_Q6_K GGUF_Q8_0", "6,2,1,pairs": ""}, {}),
+    (150, 5001, 544, {"4,2,3,full": "Q4_0", "4,2,3,full,turned": "GGUF_Q4_0", "5,2,2": "Q6_K", "6,2,2": "GGUF_Q6_K", "5,2,2,pairs": ""}, {}),
+]
+
+
 @pytest.mark.parametrize("fmt", FORMATS)
-@pytest.mark.parametrize("m,n,k", [(17, 40, 8224), (29, 3000, 8448), (20, 8193, 8192), (33, 8225, 416), (56, 8250, 352), (85, 8250, 192), (96, 16400, 256), (75, 8000, 224), (80, 8300, 256), (150, 5001, 544)])
-def test_rows_in_pairs_of_groups(fmt, m, n, k, oracle, cuda):
-    """Rows fetched as pairs of groups and as single ones, at the sizes where one takes over from the other (long rows; one workgroup
-    more than CUs at 32 rows of W each; five operands), last pairs of one group, and rows past the last that are not a multiple of eight."""
+@pytest.mark.parametrize("m,n,k,rows,others", FETCHES, ids=lambda v: str(v) if isinstance(v, int) else "")
+def test_rows_in_pairs_of_groups(m, n, k, rows, others, fmt, oracle, cuda):
+    """Rows fetched as pairs of groups and as single ones, one and two pairs ahead, with registers for one and two workgroups per CU;
+    arranged activations with either operand turned, at the sizes where one form takes over from the other; last pairs of one group, and rows
+    past the last that are not a multiple of eight: that it is the form taken, its results, and that both orders of the activations give
+    the same bits."""
     import torch
     from rocmforge_amd import ops
     n, k = shape_of(fmt, n, k)
     w = Q.make_weights(fmt, n, k, seed=fmt)
     a = np.random.default_rng(m).standard_normal((m, k)).astype(np.float16)
     dw, da = torch.from_numpy(w).to(cuda), torch.from_numpy(a).to(cuda)
+    label = Q.NAMES[fmt]
+    form = next(f for f, formats in rows.items() if formats == "" or label in formats.split())
     got = ops.gemm_f16(fmt, dw, da, n, k, out_dtype=torch.float32)
-    plain = kernel_name()
+    assert kernel_name() == f"gemm_skinny_kernel<{label},{form}>"
     arranged = ops.gemm_f16_arranged(fmt, dw, ops.ArrangedA(da), n, out_dtype=torch.float32)
-    if plain.startswith("gemm_skinny_kernel"):
-        assert torch.equal(got, arranged)
+    other = next((f for f, formats in others.items() if label in formats.split()), ",".join(form.split(",")[:3]) + ",arranged")
+    assert kernel_name() == f"gemm_skinny_kernel<{label},{other}>"
+    assert torch.equal(got, arranged)
     pick = np.unique(np.concatenate([np.arange(0, n, max(1, n // 61)), np.arange(n - 20, n)]))
     w64 = weights_of(oracle, fmt, w, n, k)[pick]
-    assert_close(got.cpu().numpy()[:, pick], a.astype(np.float64) @ w64.T, f"{Q.NAMES[fmt]} {m}x{n}x{k} {plain}", tol=TOL, plain_tol=2e-4)
+    assert_close(got.cpu().numpy()[:, pick], a.astype(np.float64) @ w64.T, f"{label} {m}x{n}x{k} {form}", tol=TOL, plain_tol=2e-4)
 
 
 @pytest.mark.parametrize("fmt", BATCH_FORMATS)
