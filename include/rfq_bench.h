@@ -59,6 +59,8 @@ RFQ_API int rfq_bench_get_rows(int fmt, const void *d_table, size_t table_bytes,
  * ahead: "deep", two workgroups to a CU: "full", put in the order of the codes: "turned"); gemm_kq_kernel: operands per weight
  * or, on integer codes, "codes of" the rows of a tile, then the parts along k. */
 RFQ_API const char *rfq_bench_last_gemv_kernel(void);
+/* The launch before that one (rfq_mlp_swiglu: gate and up). */
+RFQ_API const char *rfq_bench_gemv_kernel_before(void);
 
 /* The floor of a one-launch step that has to fetch `bytes` from HBM: a kernel that only reads copy i % copies
  * (16-byte loads, consecutive lanes on consecutive addresses, `depth` = 4, 8 or 16 loads of a thread in flight at

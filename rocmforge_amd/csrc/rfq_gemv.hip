@@ -50,7 +50,7 @@ constexpr int gemv_part_of(int canonical)
 }
 
 #if RFQ_GEMV_PART == 0
-thread_local GemvLastKernel g_gemv_last_kernel = {"", 0, 0, 0, 0};
+thread_local GemvLastKernel g_gemv_last_kernel = {"", 0, 0, 0, 0}, g_gemv_kernel_before = {"", 0, 0, 0, 0};
 thread_local GemvTraceRequest g_gemv_trace_request = {nullptr, 0, 0};
 #endif
 
@@ -2744,10 +2744,8 @@ int launch_gemv_traced(int fmt, const uint8_t *d_w, const float *d_x, float *d_y
 } // namespace rfq
 
 #if RFQ_GEMV_PART == 0
-extern "C" RFQ_API const char *rfq_bench_last_gemv_kernel(void)
+static const char *kernel_text(const rfq::GemvLastKernel &k, char (&text)[128])
 {
-    static thread_local char text[128];
-    const rfq::GemvLastKernel &k = rfq::g_gemv_last_kernel;
     const char *f = "?";
     switch (k.fmt) {
     case RFQ_Q4_0: f = "Q4_0"; break;
@@ -2767,5 +2765,15 @@ extern "C" RFQ_API const char *rfq_bench_last_gemv_kernel(void)
     }
     snprintf(text, sizeof text, k.name, f, k.a, k.b, k.c);
     return text;
+}
+extern "C" RFQ_API const char *rfq_bench_last_gemv_kernel(void)
+{
+    static thread_local char text[128];
+    return kernel_text(rfq::g_gemv_last_kernel, text);
+}
+extern "C" RFQ_API const char *rfq_bench_gemv_kernel_before(void)
+{
+    static thread_local char text[128];
+    return kernel_text(rfq::g_gemv_kernel_before, text);
 }
 #endif // part 0

@@ -223,9 +223,13 @@ def test_batches_over_large_matrices_on_prepared_x(fmt, m, hidden, inter, norm, 
     x[1] = 0.0
     x, nw = x.to(cuda), nw.to(cuda)
     got = ops.mlp_swiglu(fmt, gate, up, fmt, down, x, nw if norm else None, 1e-5, hidden, inter)
-    name = _lib.lib().rfq_bench_last_gemv_kernel().decode()
+    L, mx = _lib.lib(), fmt in (Q.MXFP4, Q.MXFP6_E2M3)
+    name, first = L.rfq_bench_last_gemv_kernel().decode(), L.rfq_bench_gemv_kernel_before().decode()
     # (the down projection's; where two row tiles go to a workgroup that converts x, only MXFP6 is ahead on prepared x)
     assert name.endswith(",ready>") == (m >= 5 and (hidden <= 5120 or fmt == Q.MXFP6_E2M3)), name
+    # (gate and up: more than one round of 32 rows per CU, or one round and the formats that are ahead there; two vectors of MXFP6 take
+    # other kernels over so many rows)
+    assert first.endswith(",pair,ready>") == ((m >= 5 or mx and (m > 2 or fmt == Q.MXFP4)) and (inter > 8192 or fmt in (Q.GGUF_Q4_K, Q.MXFP6_E2M3))), first
     dec = lambda w, n, k: ops.dequant(fmt, w, n * k).view(n, k).double()
     xd = x.double()
     if norm:
@@ -236,3 +240,85 @@ def test_batches_over_large_matrices_on_prepared_x(fmt, m, hidden, inter, norm, 
     # (float32 results of gate and up through the activation, then a float32 sum: 1e-6 of a vector's typical output or less)
     err = (got.double() - want).norm(dim=1) / want.norm(dim=1).clamp_min(1e-30)
     assert torch.isfinite(got).all() and float(err[torch.arange(m, device=cuda) != 1].max()) < 1e-5 and float(got[1].abs().max()) == 0.0, err
+
+
+@pytest.mark.parametrize("fmt", [Q.Q4_0, Q.GGUF_Q4_0, Q.GGUF_Q4_K, Q.MXFP4, Q.MXFP6_E2M3])
+@pytest.mark.parametrize("m", [3, 5, 8])
+def test_prepared_x_at_its_limits(fmt, m, cuda):
+    """Infinities, NaN, squares that overflow, tiny and huge x through prepared x: gate and up against the same rows in a block small
+    enough to convert x in every workgroup, down against rfq_gemv on the same h; the other vectors keep their bits."""
+    import torch
+    from rocmforge_amd import _lib, ops
+    hidden, inter, few, rows = 4864, 8448, 512, 997
+    make = lambda n, k, seed: torch.from_numpy(Q.make_weights(fmt, rows, k, seed=seed)).to(cuda).view(rows, -1).repeat(n // rows + 1, 1)[:n].reshape(-1)
+    gate, up, down = make(inter, hidden, 1), make(inter, hidden, 2), make(hidden, inter, 3)
+    small, small_down = Q.packed_bytes(fmt, few * hidden), make(hidden, few, 4)
+    L, mx = _lib.lib(), fmt in (Q.MXFP4, Q.MXFP6_E2M3)
+    g = torch.Generator(device="cpu").manual_seed(m)
+    x0, nw = torch.randn((m, hidden), generator=g), (1 + 0.1 * torch.randn(hidden, generator=g)).to(cuda)
+
+    def block(x, norm):
+        """h (what the call leaves at the start of its scratch memory) and the output, of the block and of its first rows."""
+        scratch = torch.empty(L.rfq_mlp_scratch_bytes(m, hidden, inter), dtype=torch.uint8, device=cuda)
+        h = lambda i: scratch[: m * i * 4].clone().view(torch.float32).view(m, i)
+        out = ops.mlp_swiglu(fmt, gate, up, fmt, down, x, norm, 1e-5, hidden, inter, scratch=scratch)
+        assert L.rfq_bench_gemv_kernel_before().decode().endswith(",pair,ready>") == (m >= 5 or mx)
+        assert L.rfq_bench_last_gemv_kernel().decode().endswith(",ready>") == (m >= 5)
+        all_h = h(inter)
+        ops.mlp_swiglu(fmt, gate[:small], up[:small], fmt, small_down, x, norm, 1e-5, hidden, few, scratch=scratch)
+        assert "ready" not in L.rfq_bench_gemv_kernel_before().decode()
+        return all_h, h(few), out
+
+    def same(got, want, what):
+        """NaN and infinities in the same places, the rest to the float32 sums' rounding of a vector's typical value."""
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf()), what
+        assert torch.equal(got[got.isinf()], want[want.isinf()]), what
+        a, b = got.double().nan_to_num(0, 0, 0), want.double().nan_to_num(0, 0, 0)
+        assert bool(((a - b).abs().amax(1) <= 1e-6 * b.abs().amax(1) + 2.0 ** -140).all()), what
+
+    for norm in (None, nw):
+        ordinary = block(x0.to(cuda), norm)
+        for what, change in (("none", lambda v: None), ("inf", lambda v: v.__setitem__(700, float("inf"))), ("-inf at the end", lambda v: v.__setitem__(hidden - 1, -float("inf"))),
+                             ("nan", lambda v: v.__setitem__(701, float("nan"))), ("squares overflow", lambda v: v.mul_(3e37)), ("tiny", lambda v: v.mul_(1e-38)),
+                             ("subnormal", lambda v: v.mul_(1e-42)), ("outlier", lambda v: v.__setitem__(5, 1e15)), ("zero", lambda v: v.zero_())):
+            x = x0.clone()
+            change(x[1])
+            what = f"{Q.NAMES[fmt]} {m} vectors, norm {norm is not None}, {what}"
+            h, h_few, out = block(x.to(cuda), norm)
+            same(h[:, :few], h_few, "gate and up, " + what)
+            same(out, ops.gemv(fmt, down, h, hidden, inter), "down, " + what)
+            for got, before in zip((h, out), (ordinary[0], ordinary[2])):
+                keep = [v for v in range(m) if v != 1]
+                assert torch.equal(got[keep], before[keep]), what
+            if norm is not None and "squares overflow" in what:
+                assert not h[1].any() and not out[1].any()
+
+
+@pytest.mark.parametrize("scale", [2.0 ** 99, 2.0 ** 110, -(2.0 ** 120)])
+def test_block_scales_beyond_2_100_on_prepared_x(scale, cuda):
+    """Q4_0 blocks whose scale times a sum of scaled x would pass the largest float32 beside small x (gate and up) and small h (down)."""
+    import torch
+    from rocmforge_amd import _lib, ops
+    m, hidden, inter, rows, fmt = 5, 4864, 8448, 997, Q.Q4_0
+    make = lambda n, k, seed: torch.from_numpy(Q.make_weights(fmt, rows, k, seed=seed)).to(cuda).view(rows, -1).repeat(n // rows + 1, 1)[:n].contiguous()
+    gate, up, down = make(inter, hidden, 1), make(inter, hidden, 2), make(hidden, inter, 3)
+
+    def scale_by(w, rows, blocks, by):                                        # float32 scales at the start of 20-byte blocks
+        v = w.view(w.shape[0], -1, 20)
+        s = v[rows, blocks, :4].contiguous().view(torch.float32) * by
+        v[rows, blocks, :4] = s.view(torch.uint8)
+    every = slice(None)
+    x = torch.randn((m, hidden), generator=torch.Generator(device="cpu").manual_seed(7)).to(cuda)
+    for w in (gate, up): scale_by(w, every, slice(4, 8), scale)
+    x[:, 128:256] /= scale
+    scale_by(gate, slice(256, 384), every, 1 / scale)                           # h of one 128-element unit of the down projection is small
+    scale_by(down, every, slice(8, 12), scale)
+    out = ops.mlp_swiglu(fmt, gate.view(-1), up.view(-1), fmt, down.view(-1), x, None, 1e-5, hidden, inter)
+    L = _lib.lib()
+    assert L.rfq_bench_gemv_kernel_before().decode().endswith(",pair,ready>") and L.rfq_bench_last_gemv_kernel().decode().endswith(",ready>")
+    dec = lambda w, n, k: ops.dequant(fmt, w.reshape(-1), n * k).view(n, k).double()
+    u = x.double() @ dec(up, inter, hidden).t().contiguous()
+    h = (x.double() @ dec(gate, inter, hidden).t().contiguous()) * (u * torch.sigmoid(u))
+    want = h @ dec(down, hidden, inter).t().contiguous()
+    # (float32 results of gate and up through the activation, then a float32 sum: 1e-6 of a vector's typical output or less)
+    assert torch.isfinite(out).all() and float(((out.double() - want).norm(dim=1) / want.norm(dim=1)).max()) < 1e-5
