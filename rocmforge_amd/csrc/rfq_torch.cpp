@@ -262,4 +262,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nu
 
 } // namespace
 
-PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&module); }
+// (the version whose C++ interface this was compiled over: nothing promises that another one's is the same)
+PyMODINIT_FUNC PyInit__native()
+{
+    PyObject *m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", RFQ_TORCH_VERSION) < 0) Py_CLEAR(m);
+    return m;
+}

@@ -8,21 +8,39 @@ and the dequant launches (src/kernels/quant/q4_0.rs:107-153).
 from __future__ import annotations
 
 import ctypes as C
+import os
 
 import torch
 
 from . import _lib
 from ._lib import check, lib
-try:
-    # The calls that need nothing said about them, natively (csrc/rfq_torch.cpp): None for all others, which the text below
-    # checks, answers or refuses.  4864 x 896 Q4_0, one vector: 6.7 -> 4.3 us of host time.
-    from . import _native
-except ImportError as e:
-    raise ImportError("rocmforge_amd/_native.so is missing or does not load: build it with `make -C rocmforge_amd/csrc` "
-                      "(or __graft_entry__.build())") from e
 from .quantize import BLOCK_BYTES, BLOCK_ELEMS
 
-_native.set_check(check)
+
+class _TextAlone:
+    """Where _native.so is not built (the library alone, no torch headers): every call goes through the text below."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _native_calls():
+    # The calls that need nothing said about them, natively (csrc/rfq_torch.cpp): None for all others, which the text below
+    # checks, answers or refuses.  4864 x 896 Q4_0, one vector: 6.7 -> 4.3 us of host time.
+    if not os.path.exists(os.path.join(os.path.dirname(os.path.abspath(__file__)), "_native.so")):
+        return _TextAlone()
+    again = "build it again with `make -C rocmforge_amd/csrc` (or __graft_entry__.build())"
+    try:
+        from . import _native as calls
+    except ImportError as e:
+        raise ImportError(f"rocmforge_amd/_native.so does not load: {again}") from e
+    if calls.torch_version != torch.__version__:
+        raise ImportError(f"rocmforge_amd/_native.so was built for torch {calls.torch_version}, this is {torch.__version__}: {again}")
+    calls.set_check(check)
+    return calls
+
+
+_native = _native_calls()
 
 
 def _stream() -> C.c_void_p:

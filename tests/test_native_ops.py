@@ -1,11 +1,16 @@
 """The operators' native call path: it gives what the Python text gives, leaves to that text every call with something unusual
 about it, and raises what the text raises."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
 
 from rocmforge_amd import _lib, _native, ops, quantize as Q
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 NAMES = ("gemv", "rms_norm_gemv", "mlp_swiglu", "gemm_f16", "arrange", "gemm_f16_arranged", "dequant")
 
 
@@ -22,11 +27,45 @@ def test_unusual_arguments_are_left_to_the_python_text():
         _native.gemv(Q.Q4_0, w, x)
 
 
+def python(code, *argv, **env):
+    return subprocess.run([sys.executable, "-c", code, *argv], cwd=ROOT, env={**os.environ, **env}, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=110)
+
+
+def test_the_library_is_built_without_torch():
+    """C++ and Rust programs need librfq.so alone: its targets ask for neither Python nor torch, and the default target does not fail
+    where they are not there."""
+    for args in (["lib"], ["all", "PYTHON=false"], ["PYTHON=/no/such/python"]):
+        p = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "rocmforge_amd", "csrc"), *args], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        assert p.returncode == 0 and "-shared" in p.stdout and "rfq_api.hip" in p.stdout and "rfq_torch.cpp" not in p.stdout, (args, p.stdout[-2000:])
+    p = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "rocmforge_amd", "csrc")], stdout=subprocess.PIPE, text=True)
+    assert p.returncode == 0 and "rfq_torch.cpp" in p.stdout
+
+
+def test_another_torch_than_the_one_built_for_is_refused():
+    p = python("import torch; torch.__version__ = '0.0.0'; import rocmforge_amd.ops")
+    assert p.returncode != 0 and f"was built for torch {torch.__version__}" in p.stdout and "0.0.0" in p.stdout
+
+
+def test_operators_without_their_native_calls(tmp_path):
+    """The library alone beside the package: the operators import, and every call goes through the text."""
+    here = os.path.join(ROOT, "rocmforge_amd")
+    package = tmp_path / "rocmforge_amd"
+    package.mkdir()
+    for name in os.listdir(here):
+        if name.endswith(".py") or name == "librfq.so":
+            (package / name).symlink_to(os.path.join(here, name))
+    p = python("import sys; sys.path.insert(0, sys.argv[1])\n"
+               "import torch; from rocmforge_amd import ops, _lib; assert _lib.lib().rfq_version() > 0 and ops.__file__.startswith(sys.argv[1])\n"
+               "try: ops.gemv(2, torch.zeros(20, dtype=torch.uint8), torch.zeros(32), 1, 32)\n"
+               "except ValueError as e: print('text:', e)\n", str(tmp_path))
+    assert p.returncode == 0 and "text: packed weights must be" in p.stdout, p.stdout
+
+
 @pytest.fixture
 def text_only(monkeypatch):
     def switch():
         for name in NAMES:
-            monkeypatch.setattr(_native, name, lambda *a: None)
+            monkeypatch.setattr(ops._native, name, lambda *a: None)
     return switch
 
 
