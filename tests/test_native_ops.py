@@ -61,6 +61,14 @@ def test_operators_without_their_native_calls(tmp_path):
     assert p.returncode == 0 and "text: packed weights must be" in p.stdout, p.stdout
 
 
+def test_one_library_in_the_process(tmp_path):
+    """The library beside the package, once, whatever other librfq.so the loader would find first (a C++ program's installation)."""
+    subprocess.run(["gcc", "-shared", "-fPIC", "-x", "c", os.devnull, "-o", str(tmp_path / "librfq.so")], check=True)
+    p = python("import rocmforge_amd.ops as o; o.lib()\n"
+               "print(sorted({l.split()[-1] for l in open('/proc/self/maps') if 'librfq' in l}))", LD_LIBRARY_PATH=str(tmp_path) + ":" + os.environ.get("LD_LIBRARY_PATH", ""))
+    assert p.returncode == 0 and str([os.path.join(os.path.realpath(ROOT), "rocmforge_amd", "librfq.so")]) in p.stdout, p.stdout
+
+
 @pytest.fixture
 def text_only(monkeypatch):
     def switch():
