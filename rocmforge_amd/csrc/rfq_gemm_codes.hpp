@@ -29,46 +29,16 @@
 #include <type_traits>
 #include <utility>
 
-#include "rfq_common.hpp"
+#include "rfq_code_operands.hpp"
 
 namespace rfq {
 namespace codes {
 
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 typedef uint32_t v4u_a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int N> struct IC { static constexpr int value = N; };
 // f(IC<0>{}) ... f(IC<N - 1>{}): a loop that is unrolled whatever its size
 template <typename F, int... X> __device__ __forceinline__ void each(F &&f, std::integer_sequence<int, X...>) { (f(IC<X>{}), ...); }
 template <int N, typename F> __device__ __forceinline__ void each(F &&f) { each(f, std::make_integer_sequence<int, N>{}); }
-
-__device__ __forceinline__ uint32_t add2h(uint32_t bits, float bias)
-{
-    v2h h;
-    __builtin_memcpy(&h, &bits, 4);
-    h = h + v2h{(_Float16)bias, (_Float16)bias};
-    uint32_t o;
-    __builtin_memcpy(&o, &h, 4);
-    return o;
-}
-// nibbles at bits SHIFT and SHIFT + 16 as an fp16 pair of nibble + bias (0x6400 | c reads 1024 + c)
-template <int SHIFT> __device__ __forceinline__ uint32_t nib2h(uint32_t d, float bias)
-{
-    uint32_t mask = 0x000F000Fu, magic = 0x64006400u;
-    asm("" : "+s"(mask));
-    asm("" : "+v"(magic));
-    return add2h(((d >> SHIFT) & mask) | magic, bias - 1024.0f);
-}
-// bytes (0, 1) and (2, 3) of a dword as fp16 pairs of byte + bias
-__device__ __forceinline__ void bytes2h(uint32_t d, float bias, uint32_t &p01, uint32_t &p23)
-{
-    p01 = add2h(__builtin_amdgcn_perm(0x64646464u, d, 0x04010400u), bias - 1024.0f);
-    p23 = add2h(__builtin_amdgcn_perm(0x64646464u, d, 0x04030402u), bias - 1024.0f);
-}
 
 // Group<FMT>: the bytes of one 32-element group of a weight row.  octet<o>(): elements 8 o .. 8 o + 7 as fp16 codes in the
 // order of arranged activations, (0,4)(1,5)(2,6)(3,7).

@@ -849,7 +849,7 @@ int launch_fmt(const uint8_t *w, const void *a, void *out, int out_dtype, int m,
                const uint8_t *arranged, hipStream_t s)
 {
     // The 256-byte Q4_K layout is contracted in one plane (its large part, the integer mins, is exact and q * scale is
-    // small beside it); every other format in two unless the caller asks for one.
+    // small beside it); the Q6_K layouts in two and the others as integer codes (launch_cfg), unless the caller asks for one.
     const bool f16 = (out_dtype & ~RFQ_GEMM_ONE_PLANE) == RFQ_F16;
     if constexpr (FMT == RFQ_GGUF_Q4_K) {
         // exact in one pass: integer operands, d and dmin applied in f32

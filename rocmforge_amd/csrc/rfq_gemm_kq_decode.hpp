@@ -61,6 +61,18 @@ template <bool BOTH> __device__ __forceinline__ void fp16_parts(float v, _Float1
     if constexpr (BOTH) fp16_pair(v, hi, lo);
     else hi = (_Float16)v;
 }
+// step T (see below) of a format that decodes element by element: elements 3 (T % 3) .. of chunk T / 3
+template <bool BOTH, class R> __device__ __forceinline__ void step_values(const R &raw, int T, v8h (&h)[4], v8h (&l)[4])
+{
+    const int c = T / 3, e0 = 3 * (T % 3), e1 = e0 + 3 < 8 ? e0 + 3 : 8;
+#pragma unroll
+    for (int e = e0; e < e1; e++) {
+        _Float16 hi, lo = (_Float16)0.0f;
+        fp16_parts<BOTH>(raw.value(8 * c + e), hi, lo);
+        h[c][chunk_pos(e)] = hi;
+        if constexpr (BOTH) l[c][chunk_pos(e)] = lo;
+    }
+}
 
 // Every format decodes a 32-element group in 12 steps (chunk c = T/3 of 8
 // elements, three steps each) so that the work can be spread evenly between
@@ -89,14 +101,8 @@ template <> struct Raw32<RFQ_Q4_0> {
     }
     template <bool BOTH> __device__ __forceinline__ void step(int T, v8h (&h)[4], v8h (&l)[4], v2h (&)[4]) const
     {
-        const int c = T / 3, e0 = 3 * (T % 3), e1 = e0 + 3 < 8 ? e0 + 3 : 8;
-#pragma unroll
-        for (int e = e0; e < e1; e++) {
-            _Float16 hi, lo = (_Float16)0.0f;
-            fp16_parts<BOTH>(value(8 * c + e), hi, lo);
-            h[c][chunk_pos(e)] = hi;
-            if constexpr (BOTH) l[c][chunk_pos(e)] = lo;
-        }
+        static_assert(!BOTH, "two operands: the codes themselves are one (rfq_gemm_codes.hpp)");
+        step_values<BOTH>(*this, T, h, l);
     }
 };
 
@@ -128,14 +134,8 @@ template <> struct Raw32<RFQ_Q8_0> {
     }
     template <bool BOTH> __device__ __forceinline__ void step(int T, v8h (&h)[4], v8h (&l)[4], v2h (&)[4]) const
     {
-        const int c = T / 3, e0 = 3 * (T % 3), e1 = e0 + 3 < 8 ? e0 + 3 : 8;
-#pragma unroll
-        for (int e = e0; e < e1; e++) {
-            _Float16 hi, lo = (_Float16)0.0f;
-            fp16_parts<BOTH>(value(8 * c + e), hi, lo);
-            h[c][chunk_pos(e)] = hi;
-            if constexpr (BOTH) l[c][chunk_pos(e)] = lo;
-        }
+        static_assert(!BOTH, "two operands: the codes themselves are one (rfq_gemm_codes.hpp)");
+        step_values<BOTH>(*this, T, h, l);
     }
 };
 
@@ -219,17 +219,7 @@ template <> struct Raw32<RFQ_Q6_K> {
         uint64_t two = (uint64_t)d[1 + w] | ((uint64_t)d[1 + (w < 5 ? w + 1 : w)] << 32);
         return (float)sbfe6((uint32_t)(two >> o), 0) * scale;
     }
-    template <bool BOTH> __device__ __forceinline__ void step(int T, v8h (&h)[4], v8h (&l)[4], v2h (&)[4]) const
-    {
-        const int c = T / 3, e0 = 3 * (T % 3), e1 = e0 + 3 < 8 ? e0 + 3 : 8;
-#pragma unroll
-        for (int e = e0; e < e1; e++) {
-            _Float16 hi, lo = (_Float16)0.0f;
-            fp16_parts<BOTH>(value(8 * c + e), hi, lo);
-            h[c][chunk_pos(e)] = hi;
-            if constexpr (BOTH) l[c][chunk_pos(e)] = lo;
-        }
-    }
+    template <bool BOTH> __device__ __forceinline__ void step(int T, v8h (&h)[4], v8h (&l)[4], v2h (&)[4]) const { step_values<BOTH>(*this, T, h, l); }
 };
 
 // ---- the block layouts of GGUF model files (ggml-common.h, ggml-quants.c) --------
@@ -259,14 +249,8 @@ template <> struct Raw32<RFQ_GGUF_Q4_0> {
     }
     template <bool BOTH> __device__ __forceinline__ void step(int T, v8h (&h)[4], v8h (&l)[4], v2h (&)[4]) const
     {
-        const int c = T / 3, e0 = 3 * (T % 3), e1 = e0 + 3 < 8 ? e0 + 3 : 8;
-#pragma unroll
-        for (int e = e0; e < e1; e++) {
-            _Float16 hi, lo = (_Float16)0.0f;
-            fp16_parts<BOTH>(value(8 * c + e), hi, lo);
-            h[c][chunk_pos(e)] = hi;
-            if constexpr (BOTH) l[c][chunk_pos(e)] = lo;
-        }
+        static_assert(!BOTH, "two operands: the codes themselves are one (rfq_gemm_codes.hpp)");
+        step_values<BOTH>(*this, T, h, l);
     }
 };
 
@@ -296,14 +280,8 @@ template <> struct Raw32<RFQ_GGUF_Q8_0> {
     }
     template <bool BOTH> __device__ __forceinline__ void step(int T, v8h (&h)[4], v8h (&l)[4], v2h (&)[4]) const
     {
-        const int c = T / 3, e0 = 3 * (T % 3), e1 = e0 + 3 < 8 ? e0 + 3 : 8;
-#pragma unroll
-        for (int e = e0; e < e1; e++) {
-            _Float16 hi, lo = (_Float16)0.0f;
-            fp16_parts<BOTH>(value(8 * c + e), hi, lo);
-            h[c][chunk_pos(e)] = hi;
-            if constexpr (BOTH) l[c][chunk_pos(e)] = lo;
-        }
+        static_assert(!BOTH, "two operands: the codes themselves are one (rfq_gemm_codes.hpp)");
+        step_values<BOTH>(*this, T, h, l);
     }
 };
 
@@ -357,14 +335,8 @@ template <> struct Raw32<RFQ_GGUF_Q4_K> {
     }
     template <bool BOTH> __device__ __forceinline__ void step(int T, v8h (&h)[4], v8h (&l)[4], v2h (&)[4]) const
     {
-        const int c = T / 3, e0 = 3 * (T % 3), e1 = e0 + 3 < 8 ? e0 + 3 : 8;
-#pragma unroll
-        for (int e = e0; e < e1; e++) {
-            _Float16 hi, lo = (_Float16)0.0f;
-            fp16_parts<BOTH>(value(8 * c + e), hi, lo);
-            h[c][chunk_pos(e)] = hi;
-            if constexpr (BOTH) l[c][chunk_pos(e)] = lo;
-        }
+        static_assert(!BOTH, "two operands: the codes themselves are one (rfq_gemm_codes.hpp)");
+        step_values<BOTH>(*this, T, h, l);
     }
 };
 
@@ -556,17 +528,7 @@ template <> struct Raw32<RFQ_GGUF_Q6_K> {
         const uint32_t q = (d[e >> 2] >> (8 * (e & 3))) & 255u;
         return __builtin_fmaf(__uint_as_float(d[8 + (e >> 4)]), (float)q, __uint_as_float(d[10 + (e >> 4)]));
     }
-    template <bool BOTH> __device__ __forceinline__ void step(int T, v8h (&h)[4], v8h (&l)[4], v2h (&)[4]) const
-    {
-        const int c = T / 3, e0 = 3 * (T % 3), e1 = e0 + 3 < 8 ? e0 + 3 : 8;
-#pragma unroll
-        for (int e = e0; e < e1; e++) {
-            _Float16 hi, lo = (_Float16)0.0f;
-            fp16_parts<BOTH>(value(8 * c + e), hi, lo);
-            h[c][chunk_pos(e)] = hi;
-            if constexpr (BOTH) l[c][chunk_pos(e)] = lo;
-        }
-    }
+    template <bool BOTH> __device__ __forceinline__ void step(int T, v8h (&h)[4], v8h (&l)[4], v2h (&)[4]) const { step_values<BOTH>(*this, T, h, l); }
 };
 
 } // namespace kq

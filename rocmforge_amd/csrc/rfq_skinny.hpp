@@ -36,18 +36,12 @@
 #pragma once
 #include <type_traits>
 
-#include "rfq_common.hpp"
+#include "rfq_code_operands.hpp"
 
 namespace rfq {
 namespace skinny {
 
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v4f_a4 __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 
 // out[j] in lane (q, i) = in[q] of lane (j, i): a 4 x 4 transposition over the four 16-lane rows.
 __device__ __forceinline__ void swap32(uint32_t &a, uint32_t &b)
@@ -79,31 +73,6 @@ __device__ __forceinline__ void spread4u(uint32_t v, uint32_t (&out)[4])
 {
     out[0] = out[1] = out[2] = out[3] = v;
     transpose4(out[0], out[1], out[2], out[3]);
-}
-
-__device__ __forceinline__ uint32_t add2h(uint32_t bits, float bias)
-{
-    v2h h;
-    __builtin_memcpy(&h, &bits, 4);
-    h = h + v2h{(_Float16)bias, (_Float16)bias};
-    uint32_t o;
-    __builtin_memcpy(&o, &h, 4);
-    return o;
-}
-// nibbles (n, n + 4) of a dword, n = shift / 4, as an fp16 pair of code + bias (0x6400 | c reads 1024 + c).  One and-or
-// after the shift: the instruction takes no literal here, so the mask is kept in a scalar and the magic in a vector register.
-template <int SHIFT> __device__ __forceinline__ uint32_t nib2h(uint32_t d, float bias)
-{
-    uint32_t mask = 0x000F000Fu, magic = 0x64006400u;
-    asm("" : "+s"(mask));
-    asm("" : "+v"(magic));
-    return add2h(((d >> SHIFT) & mask) | magic, bias - 1024.0f);
-}
-// bytes (0, 1) and (2, 3) of a dword as fp16 pairs of byte + bias
-__device__ __forceinline__ void bytes2h(uint32_t d, float bias, uint32_t &p01, uint32_t &p23)
-{
-    p01 = add2h(__builtin_amdgcn_perm(0x64646464u, d, 0x04010400u), bias - 1024.0f);
-    p23 = add2h(__builtin_amdgcn_perm(0x64646464u, d, 0x04030402u), bias - 1024.0f);
 }
 
 // the eight nibbles of a dword in their order, as fp16 pairs of nibble + bias
