@@ -459,3 +459,32 @@ def test_integer_codes_under_scales_of_any_size(fmt, scale, oracle, cuda):
     want = a.astype(np.float64) @ oracle.dequantize(fmt, w.reshape(-1), n * k).reshape(n, k).astype(np.float64).T
     # (subnormal scales: a result is a sum of 8 products, each rounded to a multiple of 2^-149)
     assert np.abs(out - want).max() <= 2e-5 * np.abs(want).max() + 16 * 2.0 ** -149
+
+
+@pytest.mark.parametrize("fmt", [Q.Q4_0, Q.Q8_0, Q.GGUF_Q4_0, Q.GGUF_Q8_0, Q.GGUF_Q4_K])
+@pytest.mark.parametrize("m,n,k,rows,parts", [(257, 129, 32, 64, 1), (300, 1000, 160, 64, 1), (300, 12000, 224, 192, 1), (512, 14340, 352, 256, 1), (700, 3700, 96, 128, 1),
+                                              (333, 4990, 3072, 192, 3)])
+def test_infinities_and_nan_under_integer_codes(fmt, m, n, k, rows, parts, oracle, cuda):
+    """An infinity or a NaN in a row of the activations, in its first group, between and in the last, which may end inside a stage of 128
+    (there the padding's products must add nothing): the outputs of that row are the infinity's products with its weights (one of
+    zero is NaN) or NaN, every other row keeps its bits.  GGUF_Q4_K multiplies the mins with sums of the activations, whose two
+    fp16 parts an infinity leaves as infinity and NaN: NaN."""
+    import torch
+    from rocmforge_amd import ops
+    if fmt == Q.GGUF_Q4_K:
+        k = (k + 255) // 256 * 256
+    w, a = weights(fmt, n, k, 9), acts(m, k, 10)
+    dw = torch.from_numpy(w).to(cuda)
+    clean = ops.gemm_f16(fmt, dw, torch.from_numpy(a).to(cuda), n, k, out_dtype=torch.float32).cpu().numpy()
+    bad = {0: (0, np.inf), 17: (k // 2, -np.inf), 64: (k - 1, np.nan), m - 2: (max(0, k - 33), np.inf), m - 1: (k - 1, -np.inf)}
+    for row, (at, value) in bad.items(): a[row, at] = value
+    got = ops.gemm_f16(fmt, dw, torch.from_numpy(a).to(cuda), n, k, out_dtype=torch.float32).cpu().numpy()
+    form = "1" if fmt == Q.GGUF_Q4_K and rows == 256 else f"codes of {rows}"
+    assert kernel_name() == f"gemm_kq_kernel<{Q.NAMES[fmt]},{form},{parts}>"
+    w32 = oracle.dequantize(fmt, w, n * k).reshape(n, k)
+    for row, (at, value) in bad.items():
+        with np.errstate(invalid="ignore"):
+            want = np.full(n, np.nan, np.float32) if fmt == Q.GGUF_Q4_K else w32[:, at] * np.float32(value)
+        assert np.array_equal(got[row], want, equal_nan=True), (row, at, value)
+    others = np.setdiff1d(np.arange(m), list(bad))
+    assert np.array_equal(got[others], clean[others])
