@@ -27,6 +27,16 @@ def test_unusual_arguments_are_left_to_the_python_text():
         _native.gemv(Q.Q4_0, w, x)
 
 
+def test_fake_tensors_are_left_to_the_python_text():
+    """Device tensors by every property, but without memory: in their mode, and after it."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        w, x = torch.empty(20, dtype=torch.uint8, device="cuda"), torch.empty(32, device="cuda")
+        assert w.is_cuda and _native.gemv(Q.Q4_0, w, x, 1, 32, None) is None
+    assert _native.gemv(Q.Q4_0, w, x, 1, 32, None) is None
+    assert _native.dequant(Q.Q4_0, w, 32, None) is None
+
+
 def python(code, *argv, **env):
     return subprocess.run([sys.executable, "-c", code, *argv], cwd=ROOT, env={**os.environ, **env}, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=110)
 
@@ -143,3 +153,60 @@ def test_native_errors_are_the_python_texts(cuda):
         y = ops.gemv(Q.Q4_0, w, x, n, k)
     assert Listener.seen > 0 and torch.equal(y, ops.gemv(Q.Q4_0, w, x, n, k))
     assert not ops.gemv(Q.Q4_0, w, x.clone().requires_grad_(), n, k).requires_grad
+
+
+@pytest.mark.gpu
+def test_calls_under_transforms_and_modes_end_as_the_python_texts(cuda, text_only):
+    """Tensors without storage of their own (vmap, functional transforms), tangents and dispatch modes: the same result, or the same
+    error, with the native calls as without them, and a mode hears as much."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+    n, k, fmt = 8, 64, Q.Q4_0
+    w = torch.from_numpy(Q.make_weights(fmt, n, k, seed=1)).to(cuda)
+    wide = torch.from_numpy(Q.make_weights(fmt, k, k, seed=2)).to(cuda)
+    x = torch.randn((3, k), device=cuda)
+    calls = {"gemv": lambda v: ops.gemv(fmt, w, v, n, k), "norm": lambda v: ops.rms_norm_gemv(fmt, w, v, torch.ones(k, device=cuda), 1e-5, n, k),
+             "mlp": lambda v: ops.mlp_swiglu(fmt, wide, wide, fmt, wide, v, None, 1e-5, k, k), "gemm": lambda v: ops.gemm_f16(fmt, w, v.half(), n, k),
+             "arrange": lambda v: ops.ArrangedA(v.half()).buf, "dequant": lambda v: ops.dequant(fmt, w, n * k, out=v.new_empty(n * k))}
+
+    class Heard(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    def dispatch(f):
+        with Heard() as mode:
+            y = f(x)
+        assert mode.names
+        return y, tuple(mode.names)
+
+    def dual(f):
+        with forward_ad.dual_level():
+            y = forward_ad.unpack_dual(f(forward_ad.make_dual(x, torch.ones_like(x))))
+            return y.primal, y.tangent is None
+
+    contexts = {"vmap": lambda f: torch.func.vmap(f)(x.reshape(3, 1, k)), "grad": lambda f: torch.func.grad(lambda v: f(v).float().sum())(x),
+                "jvp": lambda f: torch.func.jvp(f, (x,), (torch.ones_like(x),)), "dispatch": dispatch, "dual": dual,
+                "inference": torch.inference_mode()(lambda f: f(x)), "grad mode": lambda f: f(x.clone().requires_grad_()).requires_grad}
+
+    def outcome(context, f):
+        try:
+            return context(f)
+        except Exception as e:                                              # (whatever torch says there)
+            return type(e), str(e).splitlines()[0]
+
+    def same(a, b):
+        if isinstance(a, torch.Tensor): return isinstance(b, torch.Tensor) and a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
+        if isinstance(a, tuple): return isinstance(b, tuple) and len(a) == len(b) and all(same(p, q) for p, q in zip(a, b))
+        return a == b
+
+    got = {(c, f): outcome(contexts[c], calls[f]) for c in contexts for f in calls}
+    text_only()
+    for (c, f), r in got.items():
+        want = outcome(contexts[c], calls[f])
+        assert same(r, want), (c, f, r, want)
+    assert isinstance(got["dispatch", "gemv"][0], torch.Tensor) and isinstance(got["inference", "mlp"], torch.Tensor)
