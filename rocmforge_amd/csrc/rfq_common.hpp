@@ -159,7 +159,7 @@ int launch_skinny_gemm(int fmt, const uint8_t *w, const uint8_t *a, bool arrange
 // The tiled kernel on integer codes (rfq_gemm_codes.hip): arranged activations (s2: their group sums, GGUF_Q4_K); kparts > 1:
 // f32 parts [kparts][m][n] into out.  codes_rows: the rows of a workgroup's tile.
 constexpr bool codes_format(int fmt) { return fmt == RFQ_Q4_0 || fmt == RFQ_Q8_0 || fmt == RFQ_GGUF_Q4_0 || fmt == RFQ_GGUF_Q8_0 || fmt == RFQ_GGUF_Q4_K; }
-int codes_rows(int m, int n, int kparts);
+int codes_rows(int fmt, int m, int n, int kparts);
 int launch_gemm_codes(int fmt, const uint8_t *w, const uint8_t *at, const uint8_t *s2, void *out, bool f16_out, int m, int n, int k, int kparts, hipStream_t s);
 bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts);
 #define RFQ_SKINNY_PART_DECL(N)                                                                                              \

@@ -757,7 +757,7 @@ int parts_in(const uint8_t *static_tmp, int m, int n, int k, bool sums)
 // The kernel on integer codes belongs to the same family: its rows per tile where the tiled kernel has its planes.
 void note_codes(int fmt, int m, int n, int kparts, bool arranged)
 {
-    note_kernel(arranged ? "gemm_kq_kernel<%s,codes of %d,%d,arranged>" : "gemm_kq_kernel<%s,codes of %d,%d>", fmt, codes_rows(m, n, kparts), kparts, 0);
+    note_kernel(arranged ? "gemm_kq_kernel<%s,codes of %d,%d,arranged>" : "gemm_kq_kernel<%s,codes of %d,%d>", fmt, codes_rows(fmt, m, n, kparts), kparts, 0);
 }
 
 // `arranged` != nullptr: the caller's buffer from launch_arrange_a (activations and sums); a is not read.
@@ -855,9 +855,10 @@ int launch_fmt(const uint8_t *w, const void *a, void *out, int out_dtype, int m,
         // exact in one pass: integer operands, d and dmin applied in f32
         if ((out_dtype & RFQ_GEMM_ONE_PLANE) == 0) {
             if (k % 256 != 0) return fail(RFQ_E_SIZE, "rfq_gemm_f16: k=%d is not whole Q4_K super-blocks", k);
-            // (whole tiles of 256 rows: the kernel whose stages are laid out by hand is the faster one, 79 against 88 us for 512 x
-            // 4096 -> 14336; fewer rows per tile: 300 x 13824 -> 5120 91 -> 78 us, 64 x 14336 -> 4096 46 -> 28)
-            if (codes_rows(m, n, arranged != nullptr ? 1 : parts_in(static_tmp, m, n, k, true)) == 256)
+            // (tiles of 256 rows: the kernel whose stages are laid out by hand is the faster one, 79 against 88 us for 512 x 4096 ->
+            // 14336, and so it is where fewer rows per tile only spread the same work over more rounds, 800 x 1024 -> 13824 47.9 / 54.4;
+            // else fewer rows per tile: 300 x 13824 -> 5120 91 -> 78 us, 64 x 14336 -> 4096 46 -> 28)
+            if (codes_rows(FMT, m, n, arranged != nullptr ? 1 : parts_in(static_tmp, m, n, k, true)) == 256)
                 return launch_gguf_q4_k_int(w, a, out, f16, m, n, k, static_tmp, arranged, s);
             return f16 ? launch_cfg<FMT, true, 2>(w, a, out, m, n, k, static_tmp, arranged, s)
                        : launch_cfg<FMT, false, 2>(w, a, out, m, n, k, static_tmp, arranged, s);
