@@ -104,11 +104,15 @@ int launch_gemv(int fmt, const uint8_t *d_w, const float *d_x, float *d_y, int m
 // rfq_gemv.hip is compiled in four parts (the kernels of some formats each; part 0 also holds launch_gemv and
 // launch_gemv_fused, which hand a call to its format's part).  `fuse` points at the part-internal GemvFuse.
 struct GemvLastKernel { const char *name; int fmt, a, b, c; };
-extern thread_local GemvLastKernel g_gemv_last_kernel, g_gemv_kernel_before;   // which kernels this thread's last two GEMV or fp16 GEMM launches took
+// Which kernels this thread's last two GEMV or fp16 GEMM launches took, `at[last]` the later.  (__thread: no call of an initialiser on
+// the way to it; a small decode call is bound by the host.)
+struct GemvLastKernels { GemvLastKernel at[2]; int last; };
+extern __thread GemvLastKernels g_gemv_last_kernels;
 inline void note_kernel(const char *name, int fmt, int a, int b, int c)
 {
-    g_gemv_kernel_before = g_gemv_last_kernel;
-    g_gemv_last_kernel = GemvLastKernel{name, fmt, a, b, c};
+    GemvLastKernels &k = g_gemv_last_kernels;
+    k.last ^= 1;
+    k.at[k.last] = GemvLastKernel{name, fmt, a, b, c};
 }
 struct GemvTraceRequest { unsigned long long *d_buf; size_t capacity_waves; int waves_written; };
 extern thread_local GemvTraceRequest g_gemv_trace_request;   // set around a launch that is to stamp its timeline

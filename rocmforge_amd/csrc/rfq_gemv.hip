@@ -50,7 +50,7 @@ constexpr int gemv_part_of(int canonical)
 }
 
 #if RFQ_GEMV_PART == 0
-thread_local GemvLastKernel g_gemv_last_kernel = {"", 0, 0, 0, 0}, g_gemv_kernel_before = {"", 0, 0, 0, 0};
+__thread GemvLastKernels g_gemv_last_kernels = {{{"", 0, 0, 0, 0}, {"", 0, 0, 0, 0}}, 0};
 thread_local GemvTraceRequest g_gemv_trace_request = {nullptr, 0, 0};
 #endif
 
@@ -2769,11 +2769,11 @@ static const char *kernel_text(const rfq::GemvLastKernel &k, char (&text)[128])
 extern "C" RFQ_API const char *rfq_bench_last_gemv_kernel(void)
 {
     static thread_local char text[128];
-    return kernel_text(rfq::g_gemv_last_kernel, text);
+    return kernel_text(rfq::g_gemv_last_kernels.at[rfq::g_gemv_last_kernels.last], text);
 }
 extern "C" RFQ_API const char *rfq_bench_gemv_kernel_before(void)
 {
     static thread_local char text[128];
-    return kernel_text(rfq::g_gemv_kernel_before, text);
+    return kernel_text(rfq::g_gemv_last_kernels.at[rfq::g_gemv_last_kernels.last ^ 1], text);
 }
 #endif // part 0
