@@ -283,15 +283,17 @@ int RFQ_SKINNY_CAT(launch_skinny_gemm_part, RFQ_SKINNY_PART)(int fmt, const uint
 // Whether the few-row kernel is the faster one for a prompt, from estimates of both in microseconds.  The few-row kernel's
 // time grows with the 16-row operands a workgroup multiplies per 1024 k (all of them in every workgroup) and, beyond one
 // workgroup per CU, with the number of workgroups; the tiled kernel's is nearly flat up to 256 rows: a workgroup's own pass
-// over k, in `parts` parts, plus the f32 parts written and read again.  (tiled / few-row: Q8_0 9 x 4096 -> 4096 33.3 / 6.6 us,
-// 112 x 4096 -> 4096 37.8 / 15.8, 56 x 4096 -> 14336 65.7 / 31.9, 80 x 14336 -> 4096 72.1 / 54.5, 255 x 4096 -> 14336
-// 72.9 / 99.9.)  The estimates lean to the tiled kernel: of 2640 shapes measured with both (the eight formats, n 768..14336, k
-// 1024..14336, 9..255 rows, plain and arranged) three that go to the few-row kernel are slower there by more than 4 % (7 % at
-// most), and some 250 that stay would gain more than 10 % by going.  With parts == 1 the answer depends on the shape alone, so
+// over k, in `parts` parts, plus the f32 parts written and read again.  With parts == 1 the answer depends on the shape alone, so
 // that arranged and plain activations take the same kernel and give the same bits.
-// (The kernel on integer codes has since replaced the tiled one for five formats and is the faster one in part of what the
-// estimates leave here - Q8_0 64 x 14336 -> 4096 28 against 41 us - but adds longer runs of k in float32: its error against 64
-// bits is 1.2e-7 .. 1.5e-7 where this kernel's is 1.0e-7, GGUF_Q4_K 2.7e-7 .. 3.4e-7 against 1.3e-7.  The line stays.)
+// Q4_K and the Q6_K layouts: the estimates lean to the tiled kernel; of the shapes measured with both (n 768..14336, k
+// 1024..14336, 9..255 rows, plain and arranged) three that go to the few-row kernel are slower there by more than 4 % (7 % at most).
+// Q4_0, Q8_0, their GGUF layouts and GGUF_Q4_K: the other kernel is the one on integer codes, and the line is drawn by precision.  That
+// kernel adds a row in float32 in longer runs: error against 64 bits up to 4.1e-7, 1.5 times the few-row kernel's (0.93..2.9, at
+// most 1.6e-7 there), GGUF_Q4_K up to 8.4e-7, 2.7 times (1.4..4.3, at most 2.1e-7).  So a call of few rows goes to it only where it is
+// far ahead.  (codes / few-row: Q8_0 9 x 4096 -> 4096 18.7 / 8.0 us, 112 x 4096 -> 4096 23.2 / 16.7, 56 x 4096 -> 14336 29.8 / 33.5, 80 x
+// 14336 -> 4096 37.2 / 48.3, 64 x 14336 -> 4096 30.4 / 38.3, 255 x 4096 -> 14336 57.8 / 102.7.  Of 5250 calls measured with both, 4646 go to
+// the few-row kernel, 209 of them more than 10 % slower than the other would be, at most 1.67 times; 604 stay, and 40 of those would
+// gain more than 10 % by going.)
 bool prefer_skinny_gemm(int fmt, int m, int n, int k, int parts)
 {
     const double cus = device_cu_count(), ku = k / 1024.0;

@@ -30,9 +30,9 @@
 //   5 x 13824 -> 5120      Q8_0 61 -> 36          GGUF_Q4_K 61 -> 32       GGUF_Q6_K 90 -> 39       Q4_K 73 -> 34
 //   error against 64 bits (2-norm of the result), 512 x 13824, 5 vectors: Q6_K 1.07e-7 (float kernel) -> 8.1e-8, Q4_K 1.12e-7 ->
 //   7.4e-8, MXFP6 1.02e-7 -> 5.6e-8; (integer-dot kernel) GGUF_Q6_K 2.8e-7 -> 8.0e-8, 8 x 4096 -> 4096 Q8_0 2.7e-7 -> 7.7e-8
-// (9.2 us for 37 rows of GGUF_Q4_K is 1 TB/s of weights: what bounds it is the activations, 384 KB per workgroup
-// through L2 and LDS, and the instructions, 12 vector instructions per matrix instruction; decode batches issue vector instructions
-// for 40 % of their time and wait for a third of their wavefronts' cycles.)
+// (9.2 us for 37 rows of GGUF_Q4_K is 1 TB/s of weights: what bounds it is vector instructions, 11 per matrix instruction, eight of
+// them for scale and min, issued for 59 % of the cycles, and behind them the activations, 384 KB per workgroup through L2 and LDS;
+// decode batches issue vector instructions for 40 % of their time and wait for a third of their wavefronts' cycles.)
 #pragma once
 #include <type_traits>
 
