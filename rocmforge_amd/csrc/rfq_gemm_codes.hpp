@@ -1,5 +1,5 @@
 // Prefill GEMM on integer codes:  out[m, n] = A[m, k] (fp16, arranged) . dequant(W)[n, k]^T  for the formats whose scale
-// belongs to 32 elements (Q4_0, Q8_0, GGUF_Q4_0, GGUF_Q8_0), and for GGUF_Q4_K where rows do not fill tiles of 256.
+// belongs to 32 elements (Q4_0, Q8_0, GGUF_Q4_0, GGUF_Q8_0), and for GGUF_Q4_K where tiles of fewer than 256 rows save time (codes_rows).
 //
 // What bounds these calls is the matrix pipe and, behind it, the vector instructions: they do not run beside each other
 // freely (a v_mfma_f32_16x16x32_f16 followed by no / one / two / three / four v_fma_f32 takes 9.0 / 9.3 / 10.2 / 11.4 / 13.1

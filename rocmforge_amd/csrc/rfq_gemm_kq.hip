@@ -1,4 +1,4 @@
-// Prefill GEMM for the block formats with f16/f32 scales: Q4_K, Q6_K, GGUF_Q6_K, GGUF_Q4_K over whole tiles of 256 rows,
+// Prefill GEMM for the block formats with f16/f32 scales: Q4_K, Q6_K, GGUF_Q6_K, GGUF_Q4_K over tiles of 256 rows,
 // and every format as one rounded operand (RFQ_GEMM_ONE_PLANE); the others' codes go through rfq_gemm_codes.hip.
 // out[m, n] = A[m, k] (fp16) . dequant(W)[n, k]^T on the fp16 matrix
 // cores (v_mfma_f32_32x32x16_f16), fp32 accumulation.
